@@ -10,11 +10,19 @@
 //   forward output   Y = H W^T + b                          (FP32)
 //   backward         dZ_below = (dZ W) * GELU'(Z_below)     (FP32 + BF16)
 //   weight gradient  dW = dZ^T H                            (FP32)
-// Operands are addressed by (row stride, column stride), so transposes are
-// free; a 256-thread workgroup computes a 64 x 64 tile as four waves of
-// 2 x 2 MFMA blocks, staging 64 x 32 slices of A and B^T in LDS.
 // Master weights, gradients and Adam moments are FP32; the BF16 weight
-// copy the GEMMs read is refreshed by the optimizer step.
+// copies the GEMMs read are refreshed by the optimizer step.
+//
+// Networks whose widths fit in LDS (mlp_fits_rows) run two kernels per
+// training step: k_mlp_rows takes 16 batch rows per workgroup through every
+// layer forward and back, k_mlp_weights forms every weight gradient and
+// applies Adam to it where it stands.  Wider networks, and fg_bf16_gemm,
+// run k_gemm_bf16 layer by layer: operands addressed by (row stride, column
+// stride), a 256-thread workgroup per 64 x 64 tile as four waves of 2 x 2
+// MFMA blocks, 64 x 32 slices of A and B^T staged in LDS.  Both accumulate
+// every output over k in the same 32-wide MFMA steps, so they give the same
+// bits.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -42,6 +50,13 @@ __device__ __forceinline__ float bf2f(bf16_t h) { return __uint_as_float((unsign
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
 __device__ __forceinline__ float gelu_d(float x) {
   return 0.5f * (1.0f + erff(x * 0.70710678118654752f)) + x * 0.39894228040143268f * expf(-0.5f * x * x);
+}
+
+// both at once, each from the same operations
+__device__ __forceinline__ float gelu_both(float x, float &d) {
+  const float e = 1.0f + erff(x * 0.70710678118654752f);
+  d = 0.5f * e + x * 0.39894228040143268f * expf(-0.5f * x * x);
+  return 0.5f * x * e;
 }
 
 enum { EPI_STORE = 0, EPI_GELU = 1, EPI_GELU_BACK = 2 };
@@ -173,6 +188,447 @@ __global__ void k_adam(float *w, const float *gr, float *m, float *v, bf16_t *wb
   wb[l] = f2bf(x);
 }
 
+// ------------------------------------------------- networks in LDS -----
+// (pointers to global memory: as generic ones, loaded from memory, every access
+// would be a flat instruction)
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(1))) float mlp_f;
+typedef __attribute__((address_space(1))) bf16_t mlp_b;
+typedef __attribute__((address_space(1))) bf16x8 mlp_b8;
+typedef __attribute__((address_space(1))) u32x2 mlp_u2;
+
+// Matrices that the MFMAs read as operands are stored tile by tile in the
+// operand's own order: a tile is 16 columns x 32 of the contracted index k,
+// lane (c % 16) + 16 (k % 32 / 8) holding eight consecutive k of column c, so
+// that a wave's operand is one contiguous kilobyte.  (Row by row, a lane's 16
+// bytes lie a row apart from its neighbour's and each takes a cache access of
+// its own: 5.1 us a layer in k_mlp_rows.)  Tiles of a column block follow
+// each other in k, ksteps of them; whatever no weight or value fills is zero.
+#define MLP_TILE 512
+__device__ __forceinline__ long mlp_tile(int c, int k, int ksteps) {
+  return ((long)(c >> 4) * ksteps + (k >> 5)) * MLP_TILE + ((c & 15) + 16 * ((k & 31) >> 3)) * 8 + (k & 7);
+}
+
+// One dense layer as the two kernels below see it, in device memory (uniform
+// loads, two cache lines a layer).  kp and np are K and N rounded up to 128
+// (whole groups of four steps); the batch is padded to ldb, a multiple of 32.
+struct mlp_layer {
+  int K, N, kp, np;
+  mlp_f *bias;     // in the flat parameters
+  mlp_b *Wb, *Wt;  // tiles of W: columns n over k, and columns k over n
+  mlp_f *Z;        // batch x N: GELU' of the pre-activations; the last layer's output
+  mlp_f *dZ;       // batch x N: their gradients
+  mlp_b *Ht;       // tiles of the layer's input: columns k over the batch
+  mlp_b *dZt;      // tiles of the gradients: columns n over the batch
+};
+
+// One wave's work in k_mlp_weights
+enum { JOB_LOSS = 0, JOB_BIAS = 1, JOB_WEIGHT = 2 };
+struct mlp_job {
+  int kind, n0, k0, K, N, kp, np, unused;
+  long at;  // the bias or weight matrix in the flat parameters
+  mlp_b *Wb, *Wt, *Ht, *dZt;
+  mlp_f *dZ;
+};
+
+#define MLP_ROWS_TPB 1024  // 16 waves, one 16-column block of the layer each
+#define MLP_PAD 8          // LDS row padding (16 bytes)
+
+// the squared error's partial sums (k_mlp_weights) to one number, in the
+// order of k_mse's tree; one workgroup of MLP_ROWS_TPB threads
+__device__ __forceinline__ void mlp_loss_tree(const float *lossp, long n, float *red, float *loss) {
+  red[threadIdx.x] = lossp[threadIdx.x];
+  __syncthreads();
+  for (int w = MLP_ROWS_TPB / 2; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *loss = red[0] / (float)n;
+}
+
+// One wave's weights for the first 8 steps (256 of k) of a 16-column block,
+// and its column's bias: loaded a layer ahead, so that their latency passes
+// behind the layer before and its barrier.
+struct mlp_ahead {
+  bf16x8 b[8];
+  float bias;
+  // tile: the block's first tile
+  __device__ __forceinline__ void load(const mlp_b *tile, int kp) {
+    const mlp_b *q = tile + (threadIdx.x & 63) * 8;
+#pragma unroll
+    for (int u = 0; u < 4; u++) b[u] = *(const mlp_b8 *)(q + MLP_TILE * u);
+    if (kp > 128) {
+#pragma unroll
+      for (int u = 4; u < 8; u++) b[u] = *(const mlp_b8 *)(q + MLP_TILE * u);
+    }
+  }
+};
+
+// A 16 x 16 block of act (this lane's row in LDS) times a weight copy's
+// column block, k < kp, the first 256 of k loaded ahead: one accumulator,
+// 32-wide steps in increasing k
+__device__ __forceinline__ f32x4 mlp_block(const bf16_t *act, const mlp_ahead &w, const mlp_b *tile, int kp) {
+  const int lane = threadIdx.x & 63;
+  const bf16_t *a = act + (lane >> 4) * 8;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < 4; u++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8 *)(a + 32 * u), w.b[u], acc, 0, 0, 0);
+  if (kp > 128) {
+#pragma unroll
+    for (int u = 4; u < 8; u++)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8 *)(a + 32 * u), w.b[u], acc, 0, 0, 0);
+  }
+  const mlp_b *b = tile + lane * 8;
+#pragma unroll 2
+  for (int k = 256; k < kp; k += 128) {
+    bf16x8 bv[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) bv[u] = *(const mlp_b8 *)(b + (long)k * (MLP_TILE / 32) + MLP_TILE * u);
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8 *)(a + k + 32 * u), bv[u], acc, 0, 0, 0);
+  }
+  return acc;
+}
+
+// V consecutive k of one column of a tile
+template <int V>
+__device__ __forceinline__ void mlp_store_rows(mlp_b *t, const bf16_t (&h)[V]) {
+  if constexpr (V == 4)
+    *(mlp_u2 *)t = u32x2{h[0] | (unsigned)h[1] << 16, h[2] | (unsigned)h[3] << 16};
+  else if constexpr (V == 2)
+    *(__attribute__((address_space(1))) unsigned *)t = h[0] | (unsigned)h[1] << 16;
+  else
+    *t = h[0];
+}
+
+// Forward pass of 4 V rows through every layer and, when TRAIN, the MSE
+// gradient back through every layer.  Rows are independent of each other,
+// so one workgroup carries its rows through the whole network: the
+// activations stay in LDS (BF16), the weights stream from L2 straight into
+// MFMA operands, and a layer costs one
+// barrier instead of a launch.
+// The MFMA block has 16 rows; row r of it holds the workgroup's row
+// (r / 4) V + min(r % 4, V - 1), so that with few rows every lane still has
+// V results: GELU (erff, ~100 instructions) on them and the weights'
+// passage through the CU's L1 (1.3 MB both ways for the emulator network)
+// are what bounds the kernel, the products are not.  GELU' is formed on the
+// way up, where erff is at hand, and kept for the way back.
+// 512 rows of 5-256-256-256-256-512: 28.6 us; with k_mlp_weights 41 us a
+// training step, where fourteen k_gemm_bf16, five k_colsum (114 us each), k_mse
+// and k_adam took 1160 us.  Forward alone, 128 rows: 13 us, was 5 x 24 us.
+// Workgroups are dispatched round-robin over the 8 XCDs; each XCD takes a
+// contiguous run of rows, so that the tiles they fill together are written
+// through one L2 (with neighbouring rows on different XCDs, k_mlp_weights
+// read the partly written lines 55 us slower).
+// The last workgroup of a launch with loss != NULL reduces the previous
+// step's loss partials instead.
+template <int V, bool TRAIN>
+__global__ __launch_bounds__(MLP_ROWS_TPB) void k_mlp_rows(const mlp_layer *__restrict__ net, int L,
+                                                           const float *__restrict__ X, const float *__restrict__ T,
+                                                           int batch, int ldb, int ld, const float *lossp,
+                                                           float *loss) {
+  extern __shared__ __attribute__((aligned(16))) bf16_t lds_mlp[];
+  if (TRAIN && loss && blockIdx.x == gridDim.x - 1) {
+    mlp_loss_tree(lossp, (long)batch * net[L - 1].N, (float *)lds_mlp, loss);
+    return;
+  }
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int lr = lane & 15, rq = V * (lane >> 4);  // this lane's column and first row of a block
+  const int per = (int)gridDim.x / 8;  // (the grid is 8 per, plus the one above)
+  const int i0 = ((int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8)) * 4 * V;
+  const int bsteps = ldb / 32;
+  if (i0 >= (TRAIN ? (batch + 31) / 32 * 32 : batch)) return;
+  const int jw = wave * 16 + lr;  // its column in the wave's first block
+  bf16_t *cur = lds_mlp, *nxt = lds_mlp + 4 * V * ld;
+  const int arow = ((lr >> 2) * V + min(lr & 3, V - 1)) * ld;  // its MFMA row in LDS
+  mlp_ahead ah;
+  // what the wave's first block of pass q reads: q < L forward layer q, then
+  // back through layers L - 1 .. 1
+  auto ahead = [&](int q) {
+    if (q < L) {
+      const mlp_layer &n = net[q];
+      if (wave * 16 < n.np) ah.load(n.Wb + (long)wave * (n.kp / 32) * MLP_TILE, n.kp);
+      ah.bias = n.bias[min(jw, n.N - 1)];
+    } else if (TRAIN && q < 2 * L - 1) {
+      const mlp_layer &n = net[2 * L - 1 - q];
+      if (wave * 16 < n.kp) ah.load(n.Wt + (long)wave * (n.np / 32) * MLP_TILE, n.np);
+    }
+  };
+  ahead(0);
+  {
+    const int K = net[0].K, kp = net[0].kp;
+    for (int e = tid; e < 4 * V * kp; e += MLP_ROWS_TPB) {
+      const int r = e / kp, k = e - r * kp;
+      const bool in = i0 + r < batch && k < K;
+      const bf16_t h = in ? f2bf(X[(long)(i0 + r) * K + k]) : (bf16_t)0;
+      cur[r * ld + k] = h;
+      if (TRAIN && k < K) net[0].Ht[mlp_tile(k, i0 + r, bsteps)] = h;
+    }
+  }
+  __syncthreads();
+  for (int l = 0; l < L; l++) {
+    const mlp_layer n = net[l];
+    const bool last = l == L - 1;
+    const float scale = 2.0f / (float)((long)batch * n.N);
+    mlp_b *tr = TRAIN ? (last ? n.dZt : net[l + 1].Ht) : nullptr;
+    if (wave * 16 >= n.np) ahead(l + 1);  // (a wave without a block here)
+    for (int j0 = wave * 16; j0 < n.np; j0 += MLP_ROWS_TPB / 4) {
+      const int j = j0 + lr, jc = min(j, n.N - 1);
+      const mlp_b *tile = n.Wb + (long)(j0 / 16) * (n.kp / 32) * MLP_TILE;
+      if (j0 != wave * 16) {  // (a wave's first block was loaded ahead)
+        ah.load(tile, n.kp);
+        ah.bias = n.bias[jc];
+      }
+      float t[V];
+      if (TRAIN && last) {
+#pragma unroll
+        for (int v = 0; v < V; v++) t[v] = T[(long)min(i0 + rq + v, batch - 1) * n.N + jc];
+      }
+      const f32x4 acc = mlp_block(cur + arow, ah, tile, n.kp);
+      const float bj = ah.bias;
+      if (j0 + MLP_ROWS_TPB / 4 >= n.np) ahead(l + 1);
+      bf16_t h[V];
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        const int i = i0 + rq + v;
+        const bool in = i < batch && j < n.N;
+        const float x = acc[v] + bj;
+        const long o = (long)i * n.N + j;
+        h[v] = 0;
+        if (!last) {
+          float d;
+          const float y = gelu_both(x, d);
+          if (in) {
+            h[v] = f2bf(y);
+            if (TRAIN) n.Z[o] = d;
+          }
+        } else if (in) {
+          n.Z[o] = x;
+          if (TRAIN) {  // dY = 2 (Y - T) / n
+            const float d = x - t[v];
+            const float gd = scale * d;
+            n.dZ[o] = gd;
+            h[v] = f2bf(gd);
+          }
+        }
+        if (TRAIN || !last) nxt[(rq + v) * ld + j] = h[v];
+      }
+      if (TRAIN && j < n.N) mlp_store_rows<V>(tr + mlp_tile(j, i0 + rq, bsteps), h);
+    }
+    __syncthreads();
+    bf16_t *s = cur;
+    cur = nxt;
+    nxt = s;
+  }
+  if constexpr (TRAIN) {
+    for (int l = L - 1; l >= 1; l--) {  // dZ below = (dZ W) * GELU'(Z below)
+      const mlp_layer n = net[l], below = net[l - 1];
+      if (wave * 16 >= n.kp) ahead(2 * L - l);
+      for (int j0 = wave * 16; j0 < n.kp; j0 += MLP_ROWS_TPB / 4) {
+        const int j = j0 + lr, jc = min(j, n.K - 1);
+        const mlp_b *tile = n.Wt + (long)(j0 / 16) * (n.np / 32) * MLP_TILE;
+        if (j0 != wave * 16) ah.load(tile, n.np);
+        float d[V];  // (this lane stored them on the way up)
+#pragma unroll
+        for (int v = 0; v < V; v++) d[v] = below.Z[(long)min(i0 + rq + v, batch - 1) * n.K + jc];
+        const f32x4 acc = mlp_block(cur + arow, ah, tile, n.np);
+        if (j0 + MLP_ROWS_TPB / 4 >= n.kp) ahead(2 * L - l);
+        bf16_t h[V];
+#pragma unroll
+        for (int v = 0; v < V; v++) {
+          const int i = i0 + rq + v;
+          h[v] = 0;
+          if (i < batch && j < n.K) {
+            const float x = acc[v] * d[v];
+            below.dZ[(long)i * n.K + j] = x;
+            h[v] = f2bf(x);
+          }
+          nxt[(rq + v) * ld + j] = h[v];
+        }
+        if (j < n.K) mlp_store_rows<V>(below.dZt + mlp_tile(j, i0 + rq, bsteps), h);
+      }
+      __syncthreads();
+      bf16_t *s = cur;
+      cur = nxt;
+      nxt = s;
+    }
+  }
+}
+
+struct adam_args {
+  float lr, b1, b2, eps, c1, c2;
+};
+
+// one parameter's Adam step (bias-corrected): its moments updated, its new
+// value returned
+__device__ __forceinline__ float adam_step(float p, float &m, float &v, float g, const adam_args &a) {
+  m = a.b1 * m + (1.f - a.b1) * g;
+  v = a.b2 * v + (1.f - a.b2) * g * g;
+  return p - a.lr * (m / a.c1) / (sqrtf(v / a.c2) + a.eps);
+}
+
+#define MLP_CS_U 128  // rows a lane has in flight in a column sum
+#define MLP_LS_U 64   // values of each array in the squared error's sums
+
+// Everything of a training step after k_mlp_rows, one wave per job, the
+// long sequential ones first:
+//   - 16 waves: the squared error's 1024 partial sums (k_mse's order);
+//   - 64 columns per wave: the bias gradient (rows in order) and its step;
+//   - 32 x 32 weights per wave: dW = dZ^T H over the batch as 2 x 2 MFMA
+//     blocks, 32 rows per step, then Adam on the accumulators and both BF16
+//     copies of the new weights.
+// ADAM false stores the gradient instead (fg_mlp_gradient).  Every operand
+// is stored in tiles over the batch, so the fragments load straight from
+// memory, and a job's new weights fill whole tiles of both copies; 32 x 32
+// weights a job give the 330k-weight network 330 waves, where the 64 x 64 workgroups of
+// k_gemm_bf16 gave 4 to 32 a layer.  Bound: the latency of reading what
+// other XCDs have just written, a few round trips deep, so every job has as
+// much in flight as its registers hold.
+// 512 rows of that network: 13 us (20 us with half as many loads in flight).
+template <bool ADAM>
+__global__ __launch_bounds__(64) void k_mlp_weights(const mlp_job *__restrict__ jobs, const float *__restrict__ Y,
+                                                    const float *__restrict__ T, int nout, int batch, int ldb,
+                                                    mlp_f *p, mlp_f *g, mlp_f *m, mlp_f *v, mlp_f *lossp,
+                                                    adam_args ad) {
+  const int lane = threadIdx.x;
+  const mlp_job job = jobs[blockIdx.x];
+  if (job.kind == JOB_LOSS) {
+    const long n = (long)batch * nout;
+    const int t = job.n0 + lane;
+    float s = 0.f;
+    // whole chunks without a condition on the sums: loads that only a
+    // condition needs sink into it, one latency each
+    long l0 = t;
+    for (; l0 - t + (long)MLP_ROWS_TPB * MLP_LS_U <= n; l0 += (long)MLP_ROWS_TPB * MLP_LS_U) {
+      float y[MLP_LS_U], z[MLP_LS_U];
+#pragma unroll
+      for (int u = 0; u < MLP_LS_U; u++) {
+        y[u] = Y[l0 + (long)MLP_ROWS_TPB * u];
+        z[u] = T[l0 + (long)MLP_ROWS_TPB * u];
+      }
+#pragma unroll
+      for (int u = 0; u < MLP_LS_U; u++) {
+        const float d = y[u] - z[u];
+        s += d * d;
+      }
+    }
+    for (; l0 < n; l0 += MLP_ROWS_TPB) {
+      const float d = Y[l0] - T[l0];
+      s += d * d;
+    }
+    lossp[t] = s;
+    return;
+  }
+  if (job.kind == JOB_BIAS) {
+    const int j = job.n0 + lane, jc = min(j, job.N - 1);
+    const mlp_f *dZ = job.dZ + jc;
+    const long q = job.at + jc;
+    float pv = 0.f, mv = 0.f, vv = 0.f;
+    if (ADAM) {
+      pv = p[q];
+      mv = m[q];
+      vv = v[q];
+    }
+    float s = 0.f;
+    int i0 = 0;
+    for (; i0 + MLP_CS_U <= batch; i0 += MLP_CS_U) {
+      float x[MLP_CS_U];
+#pragma unroll
+      for (int u = 0; u < MLP_CS_U; u++) x[u] = dZ[(long)(i0 + u) * job.N];
+#pragma unroll
+      for (int u = 0; u < MLP_CS_U; u++) s += x[u];
+    }
+#pragma unroll 16
+    for (; i0 < batch; i0++) s += dZ[(long)i0 * job.N];
+    if (j < job.N) {
+      if constexpr (ADAM) {
+        p[q] = adam_step(pv, mv, vv, s, ad);
+        m[q] = mv;
+        v[q] = vv;
+      } else {
+        g[q] = s;
+      }
+    }
+    return;
+  }
+  const int n0 = job.n0, k0 = job.k0, N = job.N, K = job.K;
+  const int lr = lane & 15, kq = (lane >> 4) * 8, rq = 4 * (lane >> 4);
+  // a lane holds rows n0 + 16 x + rq .. + 3 of column k0 + 16 y + lr of each
+  // block; the parameters and moments of all of them load together, first
+  float pv[2][2][4], mv[2][2][4], vv[2][2][4];
+  if constexpr (ADAM) {
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+      for (int y = 0; y < 2; y++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const int n = min(n0 + 16 * x + rq + u, N - 1), k = min(k0 + 16 * y + lr, K - 1);
+          const long q = job.at + (long)n * K + k;
+          pv[x][y][u] = p[q];
+          mv[x][y][u] = m[q];
+          vv[x][y][u] = v[q];
+        }
+  }
+  const long bs = (long)(ldb / 32) * MLP_TILE;  // a column block of the batch's tiles
+  const mlp_b *a0 = job.dZt + n0 / 16 * bs + lane * 8, *a1 = a0 + bs;
+  const mlp_b *b0 = job.Ht + k0 / 16 * bs + lane * 8, *b1 = b0 + bs;
+  f32x4 acc[2][2] = {};
+#pragma unroll 8
+  for (long b = 0; b < (long)(batch + 31) / 32 * MLP_TILE; b += MLP_TILE) {
+    const bf16x8 av[2] = {*(const mlp_b8 *)(a0 + b), *(const mlp_b8 *)(a1 + b)};
+    const bf16x8 bv[2] = {*(const mlp_b8 *)(b0 + b), *(const mlp_b8 *)(b1 + b)};
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+      for (int y = 0; y < 2; y++) acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[x], bv[y], acc[x][y], 0, 0, 0);
+  }
+#pragma unroll
+  for (int x = 0; x < 2; x++)
+#pragma unroll
+    for (int y = 0; y < 2; y++) {
+      const int k = k0 + 16 * y + lr, nq = n0 + 16 * x + rq;
+      if (k >= K) continue;
+      bf16_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int n = nq + u;
+        if (n >= N) continue;
+        const long q = job.at + (long)n * K + k;
+        if constexpr (ADAM) {
+          const float pn = adam_step(pv[x][y][u], mv[x][y][u], vv[x][y][u], acc[x][y][u], ad);
+          p[q] = pn;
+          m[q] = mv[x][y][u];
+          v[q] = vv[x][y][u];
+          w[u] = f2bf(pn);
+          job.Wb[mlp_tile(n, k, job.kp / 32)] = w[u];
+        } else {
+          g[q] = acc[x][y][u];
+        }
+      }
+      if (ADAM && nq < N) mlp_store_rows<4>(job.Wt + mlp_tile(k, nq, job.np / 32), w);
+    }
+}
+
+// the last step's loss partials (grid of one workgroup)
+__global__ __launch_bounds__(MLP_ROWS_TPB) void k_mlp_loss(const float *lossp, long n, float *loss) {
+  __shared__ float red[MLP_ROWS_TPB];
+  mlp_loss_tree(lossp, n, red, loss);
+}
+
+// both BF16 copies of the weights (layer blockIdx.y; p: its FP32 weights
+// precede its bias)
+__global__ void k_mlp_copies(const mlp_layer *__restrict__ net) {
+  const mlp_layer n = net[blockIdx.y];
+  const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= (long)n.N * n.K) return;
+  const int i = (int)(q / n.K), k = (int)(q - (long)i * n.K);
+  const bf16_t w = f2bf(n.bias[q - (long)n.N * n.K]);
+  n.Wb[mlp_tile(i, k, n.kp / 32)] = w;
+  n.Wt[mlp_tile(k, i, n.np / 32)] = w;
+}
+
 // ------------------------------------------------------------ host ----
 struct fg_mlp {
   int L;                        // dense layers
@@ -191,7 +647,37 @@ struct fg_mlp {
   float *loss;                   // per-step losses of the last fg_mlp_train call
   int loss_cap;
   long step;                     // Adam steps taken
+  // networks in LDS (mlp_fits_rows): the kernels' view of the arrays, the
+  // padded arrays it points to in one allocation, and fg_mlp_train's
+  // samples (kept for the next call, grown when a larger set comes)
+  mlp_layer *net;                // device copy; NULL: layer by layer
+  mlp_job *jobs;                 // k_mlp_weights's work list, njobs entries
+  int njobs;
+  char *padded;
+  float *lossp;                  // MLP_ROWS_TPB partial sums of the squared error
+  int ld, ldb;                   // LDS row length of k_mlp_rows, row length of the transposes
+  float *Xall, *Tall;
+  size_t all_cap;                // samples they hold
 };
+
+// Rows per workgroup of k_mlp_rows, 4 V: few, so that the chip's CUs share
+// the GELUs, until every CU has a workgroup; then more rows for each passage
+// of the weights.  Microseconds per training step with 4, 8, 16 rows:
+// batch 512 40.6, 42.2, 53.5; 1024 53.1, 53.9, 64.8; 2048 95.7, 76.2, 86.0;
+// 4096 176, 135, 122.
+static int mlp_rows_v(int batch) { return batch <= 4 * 256 ? 1 : batch <= 8 * 256 ? 2 : 4; }
+
+// k_mlp_rows keeps two sets of up to 16 activation rows in LDS: networks up
+// to 896 wide fit 64 KB.  Wider ones run layer by layer (k_gemm_bf16).
+static int mlp_rows_ld(const fg_mlp *m) {
+  int kp = 0;
+  for (int l = 0; l <= m->L; l++) kp = std::max(kp, (m->width[l] + 127) / 128 * 128);
+  return kp + MLP_PAD;
+}
+static bool mlp_fits_rows(int ld) { return (size_t)2 * 16 * ld * sizeof(bf16_t) <= 65536; }
+static size_t mlp_rows_lds(int ld, int v) {  // (the loss tree of the last workgroup reuses it)
+  return std::max((size_t)2 * 4 * v * ld * sizeof(bf16_t), (size_t)MLP_ROWS_TPB * sizeof(float));
+}
 
 static fg_status mlp_gemm(fg_mlp *m, const gemm_args &g) {
   dim3 grid((g.N + GT - 1) / GT, (g.M + GT - 1) / GT);
@@ -212,7 +698,7 @@ extern "C" fg_status fg_mlp_set_params(fg_mlp *m, const float *params);
 extern "C" fg_status fg_mlp_destroy(fg_mlp *m) {
   if (!m) return FG_OK;
   (void)hipStreamSynchronize(m->stream);
-  void *ptrs[] = {m->p, m->g, m->m, m->v, m->pb, m->X, m->T, m->loss};
+  void *ptrs[] = {m->p, m->g, m->m, m->v, m->pb, m->X, m->T, m->loss, m->net, m->jobs, m->padded, m->lossp, m->Xall, m->Tall};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   for (int l = 0; l < MLP_MAX_LAYERS; l++) {
@@ -267,16 +753,75 @@ extern "C" fg_status fg_mlp_create(const int *widths, int nlayers, int max_batch
   MLP_TRY(hipMalloc((void **)&m->g, P * 4));
   MLP_TRY(hipMalloc((void **)&m->m, P * 4));
   MLP_TRY(hipMalloc((void **)&m->v, P * 4));
-  MLP_TRY(hipMalloc((void **)&m->pb, P * 2));
   MLP_TRY(hipMemset(m->m, 0, P * 4));
   MLP_TRY(hipMemset(m->v, 0, P * 4));
   MLP_TRY(hipMemset(m->g, 0, P * 4));
+  m->ld = mlp_rows_ld(m);
+  const bool rows = mlp_fits_rows(m->ld);
+  if (!rows) MLP_TRY(hipMalloc((void **)&m->pb, P * 2));
   for (int l = 0; l < nlayers; l++) {
     const size_t in = (size_t)max_batch * widths[l], outn = (size_t)max_batch * widths[l + 1];
-    MLP_TRY(hipMalloc((void **)&m->H[l], in * 2));
     MLP_TRY(hipMalloc((void **)&m->Z[l], outn * 4));
     MLP_TRY(hipMalloc((void **)&m->dZ[l], outn * 4));
+    if (rows) continue;
+    MLP_TRY(hipMalloc((void **)&m->H[l], in * 2));
     MLP_TRY(hipMalloc((void **)&m->dZb[l], outn * 2));
+  }
+  if (rows) {
+    m->ldb = (max_batch + 31) / 32 * 32;
+    mlp_layer net[MLP_MAX_LAYERS] = {};
+    size_t at[MLP_MAX_LAYERS][4], end = 0;
+    auto take = [&](size_t count) {  // (256-byte aligned pieces)
+      const size_t o = end;
+      end += (count * sizeof(bf16_t) + 255) / 256 * 256;
+      return o;
+    };
+    for (int l = 0; l < nlayers; l++) {
+      mlp_layer &n = net[l];
+      n.K = widths[l];
+      n.N = widths[l + 1];
+      n.kp = (n.K + 127) / 128 * 128;
+      n.np = (n.N + 127) / 128 * 128;
+      at[l][0] = take((size_t)n.np * n.kp);
+      at[l][1] = take((size_t)n.kp * n.np);
+      at[l][2] = take((size_t)n.kp * m->ldb);
+      at[l][3] = take((size_t)n.np * m->ldb);
+    }
+    MLP_TRY(hipMalloc((void **)&m->padded, end));
+    MLP_TRY(hipMemset(m->padded, 0, end));  // the padding stays zero
+    MLP_TRY(hipMalloc((void **)&m->lossp, MLP_ROWS_TPB * sizeof(float)));
+    std::vector<mlp_job> jobs;
+    for (int t = 0; t < MLP_ROWS_TPB; t += 64) {
+      mlp_job j{};
+      j.kind = JOB_LOSS;
+      j.n0 = t;
+      jobs.push_back(j);
+    }
+    for (int l = 0; l < nlayers; l++) {
+      mlp_layer &n = net[l];
+      n.Wb = (mlp_b *)(m->padded + at[l][0]);
+      n.Wt = (mlp_b *)(m->padded + at[l][1]);
+      n.Ht = (mlp_b *)(m->padded + at[l][2]);
+      n.dZt = (mlp_b *)(m->padded + at[l][3]);
+      n.bias = (mlp_f *)(m->p + m->offb[l]);
+      n.Z = (mlp_f *)m->Z[l];
+      n.dZ = (mlp_f *)m->dZ[l];
+    }
+    auto push = [&](int kind, int l, int n0, int k0) {
+      const mlp_layer &n = net[l];
+      jobs.push_back({kind, n0, k0, n.K, n.N, n.kp, n.np, 0, kind == JOB_BIAS ? m->offb[l] : m->offW[l], n.Wb, n.Wt, n.Ht,
+                      n.dZt, n.dZ});
+    };
+    for (int l = 0; l < nlayers; l++)
+      for (int n0 = 0; n0 < widths[l + 1]; n0 += 64) push(JOB_BIAS, l, n0, 0);
+    for (int l = 0; l < nlayers; l++)
+      for (int n0 = 0; n0 < widths[l + 1]; n0 += 32)
+        for (int k0 = 0; k0 < widths[l]; k0 += 32) push(JOB_WEIGHT, l, n0, k0);
+    m->njobs = (int)jobs.size();
+    MLP_TRY(hipMalloc((void **)&m->net, sizeof net));
+    MLP_TRY(hipMemcpy(m->net, net, sizeof net, hipMemcpyHostToDevice));
+    MLP_TRY(hipMalloc((void **)&m->jobs, jobs.size() * sizeof(mlp_job)));
+    MLP_TRY(hipMemcpy(m->jobs, jobs.data(), jobs.size() * sizeof(mlp_job), hipMemcpyHostToDevice));
   }
   MLP_TRY(hipMalloc((void **)&m->X, (size_t)max_batch * widths[0] * 4));
   MLP_TRY(hipMalloc((void **)&m->T, (size_t)max_batch * widths[nlayers] * 4));
@@ -302,8 +847,14 @@ extern "C" fg_status fg_mlp_create(const int *widths, int nlayers, int max_batch
 extern "C" fg_status fg_mlp_set_params(fg_mlp *m, const float *params) {
   if (!m || !params) return FG_E_INVALID;
   FG_HIP(hipMemcpyAsync(m->p, params, m->nparam * 4, hipMemcpyHostToDevice, m->stream));
-  hipLaunchKernelGGL(k_f32_to_bf16, dim3(fg_blocks(m->nparam, 256)), dim3(256), 0, m->stream, m->p, m->pb,
-                     m->nparam);
+  if (m->net) {
+    long most = 0;
+    for (int l = 0; l < m->L; l++) most = std::max(most, (long)m->width[l] * m->width[l + 1]);
+    hipLaunchKernelGGL(k_mlp_copies, dim3(fg_blocks(most, 256), m->L), dim3(256), 0, m->stream, m->net);
+  } else {
+    hipLaunchKernelGGL(k_f32_to_bf16, dim3(fg_blocks(m->nparam, 256)), dim3(256), 0, m->stream, m->p, m->pb,
+                       m->nparam);
+  }
   FG_LAUNCH_CHECK();
   FG_HIP(hipStreamSynchronize(m->stream));
   return FG_OK;
@@ -318,9 +869,56 @@ extern "C" fg_status fg_mlp_get_params(fg_mlp *m, float *params) {
   return FG_OK;
 }
 
+// networks in LDS: forward pass of `batch` rows of x (device); output in
+// Z[L-1].  With t (device targets) also the gradients of the
+// pre-activations; *prev_loss, when not NULL, takes the loss of the step
+// before this one.
+template <int V>
+static fg_status mlp_rows_launch(fg_mlp *m, const float *x, const float *t, int batch, float *prev_loss) {
+  const size_t lds = mlp_rows_lds(m->ld, V);
+  if (t) {
+    // rows up to the next multiple of 32 are written (as zeros), which the
+    // weight gradients' last step over the batch reads
+    const int blocks = fg_blocks((batch + 31) / 32 * (32 / (4 * V)), 8) * 8 + (prev_loss ? 1 : 0);
+    hipLaunchKernelGGL((k_mlp_rows<V, true>), dim3(blocks), dim3(MLP_ROWS_TPB), lds, m->stream, m->net, m->L, x, t,
+                       batch, m->ldb, m->ld, m->lossp, prev_loss);
+  } else {
+    hipLaunchKernelGGL((k_mlp_rows<V, false>), dim3(fg_blocks(fg_blocks(batch, 4 * V), 8) * 8), dim3(MLP_ROWS_TPB), lds,
+                       m->stream, m->net, m->L, x, nullptr, batch, m->ldb, m->ld, nullptr, nullptr);
+  }
+  FG_LAUNCH_CHECK();
+  return FG_OK;
+}
+static fg_status mlp_rows(fg_mlp *m, const float *x, const float *t, int batch, float *prev_loss) {
+  switch (mlp_rows_v(batch)) {
+    case 1: return mlp_rows_launch<1>(m, x, t, batch, prev_loss);
+    case 2: return mlp_rows_launch<2>(m, x, t, batch, prev_loss);
+    default: return mlp_rows_launch<4>(m, x, t, batch, prev_loss);
+  }
+}
+
+// the weight gradients of mlp_rows(x, t): stored (adam NULL), or applied
+static fg_status mlp_weights(fg_mlp *m, const float *t, int batch, const adam_args *adam) {
+  auto kernel = adam ? k_mlp_weights<true> : k_mlp_weights<false>;
+  hipLaunchKernelGGL(kernel, dim3(m->njobs), dim3(64), 0, m->stream, m->jobs, m->Z[m->L - 1], t, m->width[m->L],
+                     batch, m->ldb, (mlp_f *)m->p, (mlp_f *)m->g, (mlp_f *)m->m, (mlp_f *)m->v, (mlp_f *)m->lossp,
+                     adam ? *adam : adam_args{});
+  FG_LAUNCH_CHECK();
+  return FG_OK;
+}
+
+// the loss of the last mlp_weights
+static fg_status mlp_loss(fg_mlp *m, int batch, float *loss) {
+  hipLaunchKernelGGL(k_mlp_loss, dim3(1), dim3(MLP_ROWS_TPB), 0, m->stream, m->lossp, (long)batch * m->width[m->L],
+                     loss);
+  FG_LAUNCH_CHECK();
+  return FG_OK;
+}
+
 // forward pass of the batch in m->X (rows = batch); output in Z[L-1]
 static fg_status mlp_forward(fg_mlp *m, int batch) {
   const int L = m->L;
+  if (m->net) return mlp_rows(m, m->X, nullptr, batch, nullptr);
   hipLaunchKernelGGL(k_f32_to_bf16, dim3(fg_blocks((long)batch * m->width[0], 256)), dim3(256), 0, m->stream, m->X,
                      m->H[0], (long)batch * m->width[0]);
   FG_LAUNCH_CHECK();
@@ -429,8 +1027,14 @@ extern "C" fg_status fg_mlp_gradient(fg_mlp *m, const float *x, const float *t, 
     FG_HIP(hipMalloc((void **)&m->loss, 4));
     m->loss_cap = 1;
   }
-  if (fg_status s = mlp_forward(m, batch)) return s;
-  if (fg_status s = mlp_backward(m, batch, m->loss)) return s;
+  if (m->net) {
+    if (fg_status s = mlp_rows(m, m->X, m->T, batch, nullptr)) return s;
+    if (fg_status s = mlp_weights(m, m->T, batch, nullptr)) return s;
+    if (fg_status s = mlp_loss(m, batch, m->loss)) return s;
+  } else {
+    if (fg_status s = mlp_forward(m, batch)) return s;
+    if (fg_status s = mlp_backward(m, batch, m->loss)) return s;
+  }
   if (grad) FG_HIP(hipMemcpyAsync(grad, m->g, m->nparam * 4, hipMemcpyDeviceToHost, m->stream));
   if (loss) FG_HIP(hipMemcpyAsync(loss, m->loss, 4, hipMemcpyDeviceToHost, m->stream));
   FG_HIP(hipStreamSynchronize(m->stream));
@@ -448,44 +1052,57 @@ extern "C" fg_status fg_mlp_train(fg_mlp *m, const float *x, const float *t, int
     return FG_E_INVALID;
   }
   const int din = m->width[0], dout = m->width[m->L];
-  float *Xall = nullptr, *Tall = nullptr;
-  FG_HIP(hipMalloc((void **)&Xall, (size_t)n * din * 4));
-  FG_HIP(hipMalloc((void **)&Tall, (size_t)n * dout * 4));
   fg_status st = FG_OK;
+  if (m->all_cap < (size_t)n) {
+    if (m->Xall) (void)hipFree(m->Xall);
+    if (m->Tall) (void)hipFree(m->Tall);
+    m->Xall = m->Tall = nullptr;
+    m->all_cap = 0;
+    FG_HIP(hipMalloc((void **)&m->Xall, (size_t)n * din * 4));
+    FG_HIP(hipMalloc((void **)&m->Tall, (size_t)n * dout * 4));
+    m->all_cap = (size_t)n;
+  }
   if (m->loss_cap < steps) {
     if (m->loss) (void)hipFree(m->loss);
     m->loss = nullptr;
-    if (hipMalloc((void **)&m->loss, (size_t)steps * 4) != hipSuccess) st = FG_E_NOMEM;
-    m->loss_cap = steps;
+    m->loss_cap = 0;
+    if (hipMalloc((void **)&m->loss, (size_t)steps * 4) != hipSuccess)
+      st = FG_E_NOMEM;
+    else
+      m->loss_cap = steps;
   }
-  if (!st && (hipMemcpyAsync(Xall, x, (size_t)n * din * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
-              hipMemcpyAsync(Tall, t, (size_t)n * dout * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess))
+  if (!st && (hipMemcpyAsync(m->Xall, x, (size_t)n * din * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
+              hipMemcpyAsync(m->Tall, t, (size_t)n * dout * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess))
     st = FG_E_HIP;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const int nb = n / batch;
   for (int s = 0; s < steps && !st; s++) {
     const int q = s % nb;
-    if (hipMemcpyAsync(m->X, Xall + (size_t)q * batch * din, (size_t)batch * din * 4, hipMemcpyDeviceToDevice,
-                       m->stream) != hipSuccess ||
-        hipMemcpyAsync(m->T, Tall + (size_t)q * batch * dout, (size_t)batch * dout * 4, hipMemcpyDeviceToDevice,
-                       m->stream) != hipSuccess) {
+    const float *xs = m->Xall + (size_t)q * batch * din, *ts = m->Tall + (size_t)q * batch * dout;
+    m->step++;
+    const float c1 = 1.0f - powf(b1, (float)m->step), c2 = 1.0f - powf(b2, (float)m->step);
+    if (m->net) {
+      const adam_args adam = {lr, b1, b2, eps, c1, c2};
+      if ((st = mlp_rows(m, xs, ts, batch, s > 0 ? m->loss + s - 1 : nullptr))) break;
+      st = mlp_weights(m, ts, batch, &adam);
+      continue;
+    }
+    if (hipMemcpyAsync(m->X, xs, (size_t)batch * din * 4, hipMemcpyDeviceToDevice, m->stream) != hipSuccess ||
+        hipMemcpyAsync(m->T, ts, (size_t)batch * dout * 4, hipMemcpyDeviceToDevice, m->stream) != hipSuccess) {
       st = FG_E_HIP;
       break;
     }
     if ((st = mlp_forward(m, batch))) break;
     if ((st = mlp_backward(m, batch, m->loss + s))) break;
-    m->step++;
-    const float c1 = 1.0f - powf(b1, (float)m->step), c2 = 1.0f - powf(b2, (float)m->step);
     hipLaunchKernelGGL(k_adam, dim3(fg_blocks(m->nparam, 256)), dim3(256), 0, m->stream, m->p, m->g, m->m, m->v,
                        m->pb, m->nparam, lr, b1, b2, eps, c1, c2);
     if (hipGetLastError() != hipSuccess) st = FG_E_HIP;
   }
+  if (!st && m->net) st = mlp_loss(m, batch, m->loss + steps - 1);
   if (!st && losses &&
       hipMemcpyAsync(losses, m->loss, (size_t)steps * 4, hipMemcpyDeviceToHost, m->stream) != hipSuccess)
     st = FG_E_HIP;
   (void)hipStreamSynchronize(m->stream);
-  (void)hipFree(Xall);
-  (void)hipFree(Tall);
   if (st && st != FG_E_NOMEM) fg_set_error("fg_mlp_train: HIP error");
   return st;
 }
