@@ -122,6 +122,23 @@ extern "C" fg_status fg_create(const fg_params *p, const fg_tables *t, int devic
   TRY(dev_upload(&d.visc_pow15, t->visc_pow15, R));
   TRY(dev_upload(&d.visc_cav_on, t->visc_cav_on, R));
   TRY(dev_upload(&d.visc_cav, t->visc_cav, R));
+  {
+    std::vector<double> rings(R * RG_NU, 0.0);
+    for (size_t i = 0; i < R; i++) {
+      double *r = &rings[i * RG_NU];
+      r[RG_MED] = t->Rmed[i];
+      r[RG_IMED] = t->invRmed[i];
+      r[RG_IDMED] = t->invdiffRmed[i];
+      r[RG_INF] = t->Rinf[i];
+      r[RG_IINF] = t->invRinf[i];
+      r[RG_IDXT] = t->invdxtheta[i];
+      r[RG_SUPP] = t->supp_torque[i];
+      r[RG_IDSUP] = t->invdiffRsup[i];
+      r[RG_SUP] = t->Rsup[i];
+      r[RG_CS] = t->cs_iso[i];
+    }
+    TRY(dev_upload(&d.rings, rings.data(), rings.size()));
+  }
   TRY(dev_upload(&d.cos_cell, t->cos_cell, NS));
   TRY(dev_upload(&d.sin_cell, t->sin_cell, NS));
   TRY(dev_upload(&d.cos_pot, t->cos_pot, NS));
@@ -236,7 +253,7 @@ extern "C" fg_status fg_destroy(fg_ctx *c) {
                   c->t.ev_zone,    c->t.ev_coef,    c->t.ev_period,   c->t.ev_vtheta_arg, c->t.visc_const,
                   c->t.visc_pow15, c->t.visc_cav,   c->t.visc_cav_on, c->t.cos_cell,     c->t.sin_cell,
                   c->t.cos_pot,    c->t.sin_pot,    c->t.sg_Kr,       c->t.sg_Kt,        c->t.sg_norm_r,
-                  c->t.sg_norm_t,  c->t.sg_sqrt_ratio, c->t.sg_ratio, c->DRR,            c->DPP,
+                  c->t.sg_norm_t,  c->t.sg_sqrt_ratio, c->t.sg_ratio, c->t.rings,       c->DRR,            c->DPP,
                   c->DRP,          c->Work,         c->QRStar,        c->DensStar,       c->dq,
                   c->TempShift,    c->Vradial,      c->Vazimutal,     c->Vmoy,           c->newDT,
                   c->DT1D,         c->VMed,         c->nu,            c->cs_mean,        c->sgacc_mean,

@@ -2,10 +2,11 @@
 // fg_steps.hip (same expressions, same rounding), regrouped so that one
 // substep makes five passes over HBM instead of ~100:
 //
-//   k_src   2D tile (TH x TW cells + halo) staged in LDS:
-//           CorrectVtheta, evanescent damping, pressure, potential,
-//           Substep1, viscous stress, viscous update, artificial
-//           viscosity, velocity update, second damping pass
+//   k_src   a wave per column strip and ring band, marching over the rings
+//           with its windows in registers: CorrectVtheta, evanescent
+//           damping, pressure, potential, Substep1, viscous stress, viscous
+//           update, artificial viscosity, velocity update, second damping
+//           pass
 //           state A -> state B
 //   k_trad  column-marching radial van Leer sweep of the five transported
 //           quantities (each slope and flux evaluated once), plus one wave
@@ -39,22 +40,6 @@
 #include "fg_cell.h"
 #include "fg_internal.h"
 #include "fg_reduce.h"
-
-#define TH 16
-#define TW 64
-#define HALO_R 4  // rows above the tile (i - 4 .. )
-#define HALO_B 2  // rows below the tile ( .. i + TH + 1)
-#define HALO_C 4  // columns on each side
-#define HC (TW + 2 * HALO_C)
-// sector of a staged column j0 - HALO_C + c (j0 = the tile's first column):
-// at most one ring length outside [0, ns) once ns reaches the staged width,
-// so a compare and an add or subtract replace the two runtime modulos
-__device__ __forceinline__ int wrap_col(int x, int ns) {
-  if (x < 0) x += ns;
-  while (x >= ns) x -= ns;
-  return x;
-}
-#define SRC64_TPB 512  // k_src: two 80 KB workgroups per CU, four waves per SIMD
 
 fg_status fg_disk_force_async(fg_ctx *c, const double *dens, double x, double y, double rs, double *out_dev);
 
@@ -98,30 +83,49 @@ struct src_args {
   fg_dev_tables t;
   fg_planets_arg P;
   double dt, omega_frame, domega;
-  int nr, ns, indirect, evanescent, corotating;
+  int nr, ns, indirect, evanescent;
+  int plain;  // planet_potential_plain applies
+  int nstrips, width, band;  // strips of `width` columns, bands of `band` rings
 };
 
-// potential at one cell (FillForcesArraysKernel, Kernels.cu:1234-1252)
-// InvDistance = 1.0 / Rm is passed in: the ring table holds the same
-// correctly rounded quotient
-__device__ __forceinline__ double cell_potential(const fg_planets_arg &P, double Rm, double InvDistance, double cosp,
-                                                 double sinp, int indirect) {
-  const double x = Rm * cosp, y = Rm * sinp;
-  double acc = 0.0;
-  for (int k = 0; k < P.nb; k++) {
-    double xp = P.x[k], yp = P.y[k], m = P.m[k];
-    double distance = (x - xp) * (x - xp) + (y - yp) * (y - yp);
-    double distancesmooth = sqrt(distance + P.smooth[k]);
-    double pv = -1.0 * m / distancesmooth;
-    if (indirect) pv += 1.0 * m * P.invd3[k] * (x * xp + y * yp);
-    acc += pv;
-    if (k == 0) {
-      pv = -1.0 * 1.0 * InvDistance;
-      pv -= P.ix * x + P.iy * y;
-      acc += pv;
-    }
-  }
-  return acc;
+// a planet's contribution to the potential at (x, y), and then, behind the
+// first planet's, the star's (FillForcesArraysKernel, Kernels.cu:1234-1252)
+__device__ __forceinline__ double planet_potential(double x, double y, double xp, double yp, double m, double smooth,
+                                                   double invd3, int indirect) {
+  const double distance = (x - xp) * (x - xp) + (y - yp) * (y - yp);
+  const double distancesmooth = sqrt(distance + smooth);
+  double pv = -1.0 * m / distancesmooth;
+  if (indirect) pv += 1.0 * m * invd3 * (x * xp + y * yp);
+  return pv;
+}
+// The same where the host found every operand far from the ends of the
+// exponent range (plain_potential): neither the square root nor the quotient
+// needs its operands scaled, and the root's own iteration (Goldschmidt's, with
+// Markstein's corrections) leaves half the reciprocal that the quotient takes,
+// after one Newton step.  Both results are the correctly rounded ones: 16
+// instructions instead of 29.
+__device__ __forceinline__ double planet_potential_plain(double x, double y, double xp, double yp, double m,
+                                                         double smooth, double invd3, int indirect) {
+  const double d = (x - xp) * (x - xp) + (y - yp) * (y - yp) + smooth;
+  const double y0 = __builtin_amdgcn_rsq(d);
+  double r = d * y0, h = 0.5 * y0;  // towards sqrt(d) and 1 / (2 sqrt(d))
+  const double t = fma(-h, r, 0.5);
+  r = fma(r, t, r);
+  h = fma(h, t, h);
+  r = fma(fma(-r, r, d), h, r);
+  r = fma(fma(-r, r, d), h, r);
+  double i = h + h;
+  i = fma(i, fma(-r, i, 1.0), i);
+  double pv = recip64(r, i).div(-1.0 * m);
+  if (indirect) pv += 1.0 * m * invd3 * (x * xp + y * yp);
+  return pv;
+}
+// InvDistance = 1.0 / Rm (the ring table holds the same correctly rounded
+// quotient), (ix, iy) the indirect term of the star
+__device__ __forceinline__ double star_potential(double x, double y, double InvDistance, double ix, double iy) {
+  double pv = -1.0 * 1.0 * InvDistance;
+  pv -= ix * x + iy * y;
+  return pv;
 }
 
 // evanescent damping constants of ring i for a step (Kernels.cu:978-1004);
@@ -137,319 +141,349 @@ __device__ __forceinline__ void ev_consts(const fg_dev_tables &t, const double *
   vrad0 = -3.0 * nu[i] / Rm * t.vrad0_slope;
 }
 
-// per-ring tables the source stages read, staged per tile row in LDS
-enum { RT_MED, RT_IMED, RT_IDMED, RT_INF, RT_IINF, RT_IDXT, RT_SUPP, RT_IDSUP, RT_SUP, RT_NU, RT_CS, RT_SMED, RT_EVZ, RT_EMED, RT_N };
-__device__ __forceinline__ const double *ring_table(const fg_dev_tables &t, const double *nu, int x) {
-  switch (x) {
-    case RT_MED: return t.Rmed;
-    case RT_IMED: return t.invRmed;
-    case RT_IDMED: return t.invdiffRmed;
-    case RT_INF: return t.Rinf;
-    case RT_IINF: return t.invRinf;
-    case RT_IDXT: return t.invdxtheta;
-    case RT_SUPP: return t.supp_torque;
-    case RT_IDSUP: return t.invdiffRsup;
-    case RT_SUP: return t.Rsup;
-    case RT_NU: return nu;
-    case RT_CS: return t.cs_iso;
-    default: return t.SigmaMed;
-  }
+// x of lane l-1 (lane 0 reads 0): DPP wave_shr:1 on each dword
+__device__ __forceinline__ double lane_prev(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x138, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x138, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
+
+// x of lane l+1 (lane 63 reads 0): DPP wave_shl:1 on each dword
+__device__ __forceinline__ double lane_next(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x130, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x130, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// Workgroups are dispatched round-robin over the 8 XCDs.  The block of a list
+// of n that this workgroup of a grid of 8 ceil(n / 8) takes, each XCD a
+// contiguous run, so that neighbouring blocks, which read each other's halos,
+// share an L2; -1: none.
+#define FG_NXCD 8
+__device__ __forceinline__ int xcd_block(int n) {
+  const int b = (int)(blockIdx.x % FG_NXCD) * ((int)gridDim.x / FG_NXCD) + (int)(blockIdx.x / FG_NXCD);
+  return b < n ? b : -1;
+}
+static inline int xcd_grid(int n) { return (n + FG_NXCD - 1) / FG_NXCD * FG_NXCD; }
+
+// k_src's strips: one wave marches over the rings of a band, a lane per
+// column.  SRC_HL / SRC_HR columns at the ends of the wave are halo (a
+// result depends on the inputs up to three columns to the left and two to
+// the right), and so are the SRC_HT rings above and SRC_HB below the band.
+#define SRC_HL 3
+#define SRC_HR 2
+#define SRC_HT 3
+#define SRC_HB 2
+#define SRC_W (64 - SRC_HL - SRC_HR)  // most columns a strip outputs
+#define SRC_ROWS 32
+#define SRC_MAX_BAND (SRC_ROWS - SRC_HT - SRC_HB)
+// damping constants of a ring: 1 + lambda and its reciprocal refinement,
+// lambda times what Sigma, the energy, vrad and vtheta relax to (the last
+// two in the first pass, then in the second)
+enum { EV_D, EV_R, EV_S, EV_E, EV_VR1, EV_VT1, EV_VR2, EV_VT2, EV_N };
+
+// (q + lambda q0) / (1 + lambda), Kernels.cu:1006-1012
+__device__ __forceinline__ double ev_damp(double q, const double *ev, int which) {
+  return recip64(ev[EV_D], ev[EV_R]).div(q + ev[which]);
+}
+
+// element at byte offset `off` of a row: the scalar row address plus a 32-bit
+// lane offset is the memory instructions' own form, no vector arithmetic
+__device__ __forceinline__ double &at(double *row, unsigned off) { return *(double *)((char *)row + off); }
+__device__ __forceinline__ double at(const double *row, unsigned off) { return *(const double *)((const char *)row + off); }
 
 // MODE bit 1: adiabatic (energy damped, P = (gamma - 1) e, EnergyInt out);
 // bit 2: self-gravity kick after Substep1
-template <int KTH, int KTW, int KTPB, int MODE>
-__global__ __launch_bounds__(KTPB) void k_src(src_args a) {
+//
+// One step of the march takes in ring m and completes ring m - 2; what the
+// stages need of earlier rings stays in registers (slot ring mod 3, so a
+// step is instantiated per m mod 3 and nothing is shifted), the neighbours
+// in azimuth come from the neighbouring lanes by DPP.  So there is no LDS
+// tile, no barrier, no index
+// arithmetic per cell, and a band of H rings by 59 columns evaluates
+// (H + 5) / H x 64 / 59 cells per cell, where the 16 x 64 LDS tile with its
+// halo of four evaluated 1.55.
+// Bound: HBM on large grids (2048 x 4096: 442 MB by the counters, of which
+// 403 are the fields read and written once, in 104 us, was 238 us; 1024 x 3072:
+// 47 us, was 89), the waves' own issue on small ones (a dependent FP64
+// operation every nine cycles; 128 x 384: 9 us, was 13).  Three waves per SIMD
+// (168 VGPRs) and two rings in flight without energy and self-gravity; with
+// them two waves and one ring (177 to 191 VGPRs), since the third wave would
+// spill (512 x 1536 with both 29 us, was 34; 37 with three).
+template <int MODE>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE ? 2 : 3))) void k_src(src_args a) {
+  constexpr int AHEAD = MODE ? 1 : 2;  // rings whose loads are in flight
   constexpr bool ADI = MODE & 1, SGK = MODE & 2;
-  constexpr int KHR = KTH + HALO_R + HALO_B, KHC = KTW + 2 * HALO_C;
-  constexpr int KPT = (KHR * KHC + KTPB - 1) / KTPB;
-  __shared__ double sS[KHR][KHC];   // Sigma after the first damping
-  __shared__ double sA[KHR][KHC];   // pressure, then VradInt
-  __shared__ double sB[KHR][KHC];   // potential, then VthetaInt
-  __shared__ double sC[KHR][KHC];   // vtheta, then TAURR, then Qr
-  __shared__ double sD[KHR][KHC];   // vrad, then TAUPP, then Qtheta
-  __shared__ double sE[KHR][KHC];   // TAURP
-  const int nr = a.nr, ns = a.ns;
-  const int i0 = blockIdx.y * KTH, j0 = blockIdx.x * KTW;
-  const int tid = threadIdx.x;
+  __shared__ double tab[SRC_ROWS][RG_N], evc[SRC_ROWS][EV_N];
+  const int nr = a.nr, ns = a.ns, lane = threadIdx.x;
+  const int block = xcd_block(a.nstrips * ((nr + a.band) / a.band));
+  if (block < 0) return;
+  const int strip = block % a.nstrips, i0 = block / a.nstrips * a.band;
+  const int i1 = min(i0 + a.band, nr + 1);  // rings i0 .. i1 - 1 (the ghost ring with the last band)
   const fg_dev_tables &t = a.t;
-  const double dt = a.dt;
-#define GI(r) (i0 - HALO_R + (r))
-#define GJ(c) wrap_col(j0 - HALO_C + (c), ns)
-
-  // ---- S0: load, CorrectVtheta, damping #1, pressure, potential ----
-  // all of a thread's loads are issued before any of them is used
-  double ls[KPT], lvr[KPT], lvt[KPT], le[ADI ? KPT : 1], lkr[SGK ? KPT : 1], lkt[SGK ? KPT : 1];
+  const double dt = a.dt, OF = a.omega_frame;
+  const int g = strip * a.width - SRC_HL + lane;  // this lane's column, unwrapped
+  const int j = (g % ns + ns) % ns;
+  unsigned jb = 8u * j;  // in bytes
+  const bool mine = lane >= SRC_HL && lane < SRC_HL + a.width && g < ns;
+  const double cosp = t.cos_pot[j], sinp = t.sin_pot[j];
+  // ring m's inputs are loaded AHEAD steps ahead (rings clamped into the
+  // grid), slot ring mod 3 as below
+  double n_s[3], n_vr[3], n_vt[3], n_e[3], n_kr[3], n_kt[3];
+  auto fetch = [&](int m, auto phase) __attribute__((always_inline)) {
+    constexpr int X = decltype(phase)::value % 3;
+    const long l = (long)min(max(m, 0), nr) * ns;
+    n_s[X] = at(a.dens + l, jb);
+    n_vr[X] = at(a.vr + l, jb);
+    n_vt[X] = at(a.vt + l, jb);
+    if constexpr (ADI) n_e[X] = at(a.energy + l, jb);
+    if constexpr (SGK) {
+      n_kr[X] = at(a.kick_r + l, jb);
+      n_kt[X] = at(a.kick_t + l, jb);
+    }
+  };
+#define LVL(n) std::integral_constant<int, n>()
+  fetch(i0 - SRC_HT, LVL(0));
+  if (AHEAD > 1) fetch(i0 - SRC_HT + 1, LVL(1));
+  // the tables of the rings the band reads and their damping constants
+  // (Kernels.cu:978-1004), a ring per lane, into LDS, from where each step
+  // takes them with a uniform address: held in scalar registers they would
+  // need three times as many as there are, read through the scalar cache
+  // every use is a round trip (1.26 us a step for a lone wave)
+  bool damped = false;
+  if (lane < i1 - i0 + SRC_HT + SRC_HB) {
+    const int i = i0 - SRC_HT + lane, ic = min(max(i, 0), nr - 1);
+    double r[RG_NU];
 #pragma unroll
-  for (int k = 0; k < KPT; k++) {
-    const int q = tid + k * KTPB;
-    ls[k] = lvr[k] = lvt[k] = 0.0;
-    if constexpr (ADI) le[k] = 0.0;
-    if constexpr (SGK) lkr[k] = lkt[k] = 0.0;
-    if (q < KHR * KHC) {
-      const int r = q / KHC, cc = q - r * KHC, i = GI(r);
-      if (i >= 0 && i <= nr) {
-        const int j = GJ(cc);
-        const long l = (long)i * ns + j;
-        ls[k] = a.dens[l];
-        lvr[k] = a.vr[l];
-        lvt[k] = a.vt[l];
-        if constexpr (ADI) le[k] = a.energy[l];
-        if constexpr (SGK)
-          if (i < nr) {
-            lkr[k] = a.kick_r[l];
-            lkt[k] = a.kick_t[l];
-          }
-      }
+    for (int x = 0; x < RG_NU; x++) r[x] = t.rings[(long)ic * RG_NU + x];
+    const double v = a.nu[ic];
+    damped = a.evanescent && i == ic && t.ev_zone[ic];
+#pragma unroll
+    for (int x = 0; x < RG_NU; x++) tab[lane][x] = r[x];
+    tab[lane][RG_NU] = v;
+    if (damped) {
+      double lambda, vr0, vt0, *ev = evc[lane];
+      ev_consts(t, a.nu1, i, dt, OF, lambda, vr0, vt0, a.sg1);
+      const recip64 d(1.0 + lambda);
+      ev[EV_D] = d.d;
+      ev[EV_R] = d.r;
+      ev[EV_S] = lambda * t.SigmaMed[i];
+      ev[EV_E] = ADI ? lambda * t.EnergyMed[i] : 0.0;
+      ev[EV_VR1] = lambda * vr0;
+      ev[EV_VT1] = lambda * vt0;
+      ev_consts(t, a.nu, i, dt, OF, lambda, vr0, vt0, a.sg2);
+      ev[EV_VR2] = lambda * vr0;
+      ev[EV_VT2] = lambda * vt0;
     }
   }
-  // The per-ring tables of the tile's rows (rings clamped into the table;
-  // rows outside the disk are never read) and the potential's cos/sin of
-  // its columns, staged in LDS while the loads above are in flight: every
-  // stage below reads them from there.  Read from memory inside a stage,
-  // each would be a dependent round trip.  Each wave loads every fourth
-  // table, lane r row r.
-  __shared__ double rt[RT_N][KHR];
-  __shared__ double ct[2][KHC];
-  {
-    const int w = tid >> 6, ln = tid & 63;
-    if (w < 4 && ln < KHR) {
-      const int i = min(max(GI(ln), 0), nr - 1);
-      // wave w: tables w, w + 4, w + 8 and (wave 0) the ev_zone flags;
-      // all loads issued before the first LDS write
-      const double v0 = ring_table(t, a.nu, w)[i], v1 = ring_table(t, a.nu, w + 4)[i];
-      const double v2 = ring_table(t, a.nu, w + 8)[i];
-      const int ez = t.ev_zone[i];
-      rt[w][ln] = v0;
-      rt[w + 4][ln] = v1;
-      rt[w + 8][ln] = v2;
-      if (w == 0) rt[RT_EVZ][ln] = (double)ez;
-      if (ADI && w == 1) rt[RT_EMED][ln] = t.EnergyMed[i];
-    }
-    for (int c = tid; c < KHC; c += KTPB) {
-      const int j = GJ(c);
-      ct[0][c] = t.cos_pot[j];
-      ct[1][c] = t.sin_pot[j];
-    }
-  }
-  // damping constants of the tile's rings, once per ring (Kernels.cu:978-1004):
-  // lambda, then vrad0 and vtheta0 of the first pass, then of the second
-  __shared__ double evc[KHR][5];
-  if (a.evanescent) {
-    for (int r = tid; r < KHR; r += KTPB) {
-      const int i = GI(r);
-      if (i >= 0 && i < nr && t.ev_zone[i]) {
-        ev_consts(t, a.nu1, i, dt, a.omega_frame, evc[r][0], evc[r][1], evc[r][2], a.sg1);
-        ev_consts(t, a.nu, i, dt, a.omega_frame, evc[r][0], evc[r][3], evc[r][4], a.sg2);
-      }
-    }
-  }
+  const unsigned zones = (unsigned)__ballot(damped);  // bit r: ring i0 - SRC_HT + r is damped
   __syncthreads();
-#pragma unroll
-  for (int k = 0; k < KPT; k++) {
-    const int q = tid + k * KTPB;
-    if (q >= KHR * KHC) break;
-    int r = q / KHC, cc = q - r * KHC;
-    int i = GI(r);
-    double s = 0.0, vr = 0.0, vt = 0.0, p = 0.0, phi = 0.0;
-    if (i >= 0 && i <= nr) {
-      s = ls[k];
-      vr = lvr[k];
-      vt = lvt[k];
-      if (i < nr) {
-        if (a.corotating) vt = vt - a.domega * rt[RT_MED][r];
-        double e = ADI ? le[k] : 0.0;
-        if (a.evanescent && rt[RT_EVZ][r] != 0.0) {
-          vr = damp_toward(vr, evc[r][0], evc[r][1]);
-          vt = damp_toward(vt, evc[r][0], evc[r][2]);
-          s = damp_toward(s, evc[r][0], rt[RT_SMED][r]);
-          if (ADI) e = damp_toward(e, evc[r][0], rt[RT_EMED][r]);
-        }
-        if (ADI) {
-          p = (a.gamma - 1.0) * e;  // Kernels.cu:196
-        } else {
-          const double cs = rt[RT_CS][r];
-          p = s * cs * cs;
-        }
-        phi = cell_potential(a.P, rt[RT_MED][r], rt[RT_IMED][r], ct[0][cc], ct[1][cc], a.indirect);
+  // the first planet and the indirect term in registers, further planets where
+  // the launch put them (indexed by a loop, a by-value copy would live in
+  // scratch)
+  const auto &more = ((__attribute__((address_space(4))) const src_args *)__builtin_amdgcn_kernarg_segment_ptr())->P;
+  double px = a.P.x[0], py = a.P.y[0], pm = a.P.m[0], ps = a.P.smooth[0], pi3 = a.P.invd3[0], ix = a.P.ix, iy = a.P.iy;
+  asm volatile("" : "+s"(px), "+s"(py), "+s"(pm), "+s"(ps), "+s"(pi3), "+s"(ix), "+s"(iy));
+  const double invdphi = t.invdphi, onethird = 1.0 / 3.0;
+  // windows, ring x in slot x mod 3: Sigma, its left neighbour, pressure,
+  // potential, vtheta and its right neighbour; VradInt / VthetaInt after
+  // Substep1 and VradInt after the viscous update; stresses; radial
+  // artificial pressure; the halved sums Sigma_i + Sigma_i-1 and
+  // Sigma_j + Sigma_j-1 with their reciprocal refinements, which divide in
+  // S1, S3 and S5 (x * 2 / d is x / (d / 2), both scalings exact)
+  double S[3] = {}, Sl[3] = {}, P[3] = {}, F[3] = {}, T[3] = {}, Tn[3] = {}, EN[3] = {};
+  double A1[3] = {}, B1[3] = {}, A3[3] = {}, RR[3] = {}, PP[3] = {}, RP[3] = {}, QR[3] = {};
+  double hr[3] = {}, hrr[3] = {}, ha[3] = {}, har[3] = {};
+  // LEVEL: how many of the stages ring m's step evaluates (the first steps
+  // of a band only fill the windows); IN: rings m - 3 .. m + 1 lie strictly
+  // inside the disk, which drops the edge cases
+  auto step = [&](int m, auto level, auto phase, auto inner) __attribute__((always_inline)) {
+    constexpr int LV = decltype(level)::value, C = decltype(phase)::value, M1 = (C + 2) % 3, M2 = (C + 1) % 3;
+    constexpr bool IN = decltype(inner)::value;
+    double s = n_s[C], vr = n_vr[C], vt = n_vt[C], e = ADI ? n_e[C] : 0.0;
+    const double kr = SGK ? n_kr[C] : 0.0, kt = SGK ? n_kt[C] : 0.0;
+    fetch(m + AHEAD, LVL(C + AHEAD));
+    // (keeps the lane offset apart from the row address: added up before the
+    // loop they would be a vector pointer per field)
+    asm volatile("" : "+v"(jb));
+    const int row = m - i0 + SRC_HT;  // rings m, k, o in the tables
+    const double *Rm = tab[row], *Rk = tab[max(row - 1, 0)], *Ro = tab[max(row - 2, 0)];
+    const int k = m - 1, o = m - 2;
+    // ---- S0: CorrectVtheta, damping #1, pressure, potential of ring m ----
+    double p = 0.0, phi = 0.0;
+    if (IN || (m >= 0 && m < nr)) {
+      vt = vt - a.domega * Rm[RG_MED];
+      if (zones >> row & 1) {
+        const double *ev = evc[row];
+        vr = ev_damp(vr, ev, EV_VR1);
+        vt = ev_damp(vt, ev, EV_VT1);
+        s = ev_damp(s, ev, EV_S);
+        if (ADI) e = ev_damp(e, ev, EV_E);
       }
+      if (ADI) {
+        p = (a.gamma - 1.0) * e;  // Kernels.cu:196
+      } else {
+        const double cs = Rm[RG_CS];
+        p = s * cs * cs;
+      }
+      const double x = Rm[RG_MED] * cosp, y = Rm[RG_MED] * sinp;
+      if (a.P.nb > 0) {
+        phi = 0.0 + (a.plain ? planet_potential_plain(x, y, px, py, pm, ps, pi3, a.indirect)
+                             : planet_potential(x, y, px, py, pm, ps, pi3, a.indirect));
+        phi += star_potential(x, y, Rm[RG_IMED], ix, iy);
+      }
+      for (int q = 1; q < a.P.nb; q++)
+        phi += planet_potential(x, y, more.x[q], more.y[q], more.m[q], more.smooth[q], more.invd3[q], a.indirect);
+      if (a.opress && mine && m >= i0 && m < i1) at(a.opress + (long)m * ns, jb) = p;  // for the temperature output
+    } else if (m != nr) {
+      s = vr = vt = 0.0;
     }
-    sS[r][cc] = s;
-    sA[r][cc] = p;
-    sB[r][cc] = phi;
-    sC[r][cc] = vt;
-    sD[r][cc] = vr;
-  }
-  __syncthreads();
-
-  // ---- S1: Substep1 (Kernels.cu:13-53) on rows [1, KHR), cols [1, KHC-1) ----
-  // The divisors of S1's pressure gradients, Sigma_i + Sigma_i-1 (radial)
-  // and Sigma_j + Sigma_j-1 (azimuthal), reappear halved in S3; x * 2 / d is
-  // x / (d / 2) (both scalings exact), so S1 divides by the halved sums and
-  // keeps their reciprocal refinements (recip64) for S3 in the same thread.
-  double regA[KPT], regB[KPT], hrad[KPT], hazi[KPT];
-  {
-#pragma unroll
-    for (int k = 0; k < KPT; k++) {
-      const int q = tid + k * KTPB;
-      if (q >= KHR * KHC) break;
-      int r = q / KHC, cc = q - r * KHC;
-      int i = GI(r);
+    S[C] = s;
+    P[C] = p;
+    F[C] = phi;
+    T[C] = vt;
+    Tn[C] = lane_next(vt);
+    Sl[C] = lane_prev(s);
+    if (ADI) EN[C] = e;
+    // ---- S1: Substep1 (Kernels.cu:13-53) of ring m ----
+    if constexpr (LV >= 1) {
       double vri = 0.0, vti = 0.0;
-      hrad[k] = hazi[k] = 0.0;
-      if (r >= 1 && cc >= 1 && cc < KHC - 1 && i >= 0 && i < nr) {
-        if (i > 0) {
-          const recip64 hd(0.5 * (sS[r][cc] + sS[r - 1][cc]));
-          hrad[k] = hd.r;
-          double gradp = hd.div(sA[r][cc] - sA[r - 1][cc]) * rt[RT_IDMED][r];
-          double gradphi = (sB[r][cc] - sB[r - 1][cc]) * rt[RT_IDMED][r];
-          double vt2 = sC[r][cc] + sC[r][cc + 1] + sC[r - 1][cc] + sC[r - 1][cc + 1];
-          vt2 = vt2 / 4.0 + a.omega_frame * rt[RT_INF][r];
+      hr[C] = hrr[C] = ha[C] = har[C] = 0.0;
+      if (IN || (m >= 0 && m < nr)) {
+        if (IN || m > 0) {
+          const recip64 hd(0.5 * (s + S[M1]));
+          hr[C] = hd.d;
+          hrr[C] = hd.r;
+          const double idm = Rm[RG_IDMED];
+          const double gradp = hd.div(p - P[M1]) * idm;
+          const double gradphi = (phi - F[M1]) * idm;
+          double vt2 = T[C] + Tn[C] + T[M1] + Tn[M1];
+          vt2 = vt2 / 4.0 + OF * Rm[RG_INF];
           vt2 = vt2 * vt2;
-          double vr_src = -gradp - gradphi;
-          double vradint2 = vr_src + vt2 * rt[RT_IINF][r];
-          vri = sD[r][cc] + dt * vradint2;
+          const double vr_src = -gradp - gradphi;
+          const double vradint2 = vr_src + vt2 * Rm[RG_IINF];
+          vri = vr + dt * vradint2;
         }
-        const double invdxtheta = rt[RT_IDXT][r];
-        const recip64 hd(0.5 * (sS[r][cc] + sS[r][cc - 1]));
-        hazi[k] = hd.r;
-        double gradp = hd.div(sA[r][cc] - sA[r][cc - 1]) * invdxtheta;
-        double gradphi = (sB[r][cc] - sB[r][cc - 1]) * invdxtheta;
-        double v = sC[r][cc] - dt * (gradp + gradphi);
-        v += dt * rt[RT_SUPP][r];
+        const double invdxtheta = Rm[RG_IDXT];
+        const recip64 hd(0.5 * (s + Sl[C]));
+        ha[C] = hd.d;
+        har[C] = hd.r;
+        const double gradp = hd.div(p - lane_prev(p)) * invdxtheta;
+        const double gradphi = (phi - lane_prev(phi)) * invdxtheta;
+        double v = vt - dt * (gradp + gradphi);
+        v += dt * Rm[RG_SUPP];
         vti = v;
+        if constexpr (SGK) {  // self-gravity kick (0 on ring 0 of VradInt)
+          vri = vri + kr;
+          vti = vti + kt;
+        }
       }
-      // self-gravity kick on VradInt / VthetaInt (0 on ring 0 and outside)
-      regA[k] = SGK ? vri + lkr[k] : vri;
-      regB[k] = SGK ? vti + lkt[k] : vti;
+      A1[C] = vri;  // VradInt (0 on rings 0 and NRAD, as never written)
+      B1[C] = vti;  // VthetaInt
     }
-    if (a.opress) {  // pressure for the temperature output, own cells only
-      for (int q = tid; q < KTH * KTW; q += KTPB) {
-        int r = q / KTW + HALO_R, cc = q % KTW + HALO_C;
-        int i = GI(r), j = j0 + cc - HALO_C;
-        if (i < nr && j < ns) a.opress[(long)i * ns + j] = sA[r][cc];
+    // ---- S2: viscous stress (Kernels.cu:733-771) of ring k ----
+    if constexpr (LV >= 2) {
+      if (IN || (k >= 0 && k < nr)) {
+        const double invRm = Rk[RG_IMED], idsup = Rk[RG_IDSUP], Rinf = Rk[RG_INF], v = Rk[RG_NU];
+        const double bn = lane_next(B1[M1]), b = B1[M1], vrl = A1[M1], vrn = A1[C];
+        const double drr = (vrn - vrl) * idsup;
+        const double dpp = (bn - b) * invdphi * invRm + 0.5 * (vrn + vrl) * invRm;
+        double dv = (vrn * Rk[RG_SUP] - vrl * Rinf) * idsup * invRm;
+        dv += (bn - b) * invdphi * invRm;
+        RR[M1] = 2.0 * S[M1] * v * (drr - onethird * dv);
+        PP[M1] = 2.0 * S[M1] * v * (dpp - onethird * dv);
+        if (LV >= 3 && (IN || k > 0)) {
+          const double drp = 0.5 * (Rinf * (b * invRm - B1[M2] * Ro[RG_IMED]) * Rk[RG_IDMED] +
+                                    (vrl - lane_prev(vrl)) * invdphi * Rk[RG_IINF]);
+          RP[M1] = 2.0 * 0.25 * (S[M1] + S[M2] + Sl[M1] + Sl[M2]) * v * drp;
+        }
       }
     }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < KPT; k++) {
-      const int q = tid + k * KTPB;
-      if (q >= KHR * KHC) break;
-      int r = q / KHC, cc = q - r * KHC;
-      sA[r][cc] = regA[k];  // VradInt (0 on rows 0 and NRAD, as never written)
-      sB[r][cc] = regB[k];  // VthetaInt
+    // ---- S3: viscous velocity update (Kernels.cu:118-150): VradInt of ring k ----
+    if constexpr (LV >= 3) {
+      A3[M1] = A1[M1];
+      if (IN || (k >= 1 && k < nr))
+        A3[M1] += recip64(hr[M1], hrr[M1])
+                      .div(dt * Rk[RG_IINF] *
+                           ((Rk[RG_MED] * RR[M1] - Ro[RG_MED] * RR[M2]) * Rk[RG_IDMED] +
+                            (lane_next(RP[M1]) - RP[M1]) * invdphi - 0.5 * (PP[M1] + PP[M2])));
     }
-  }
-  __syncthreads();
-
-  // ---- S2: viscous stress (Kernels.cu:733-771) on rows [1, KHR-1), cols [2, KHC-2) ----
-  const double invdphi = t.invdphi;
-  const double onethird = 1.0 / 3.0;
-#pragma unroll
-  for (int kq = 0; kq < KPT; kq++) {
-    const int q = tid + kq * KTPB;
-    if (q >= KHR * KHC) break;
-    int r = q / KHC, cc = q - r * KHC;
-    int i = GI(r);
-    if (r < 1 || r >= KHR - 1 || cc < 2 || cc >= KHC - 2 || i < 0 || i >= nr) continue;
-    const double *VrR = &sA[r][0];
-    const double invRm = rt[RT_IMED][r], idsup = rt[RT_IDSUP][r];
-    double drr = (sA[r + 1][cc] - VrR[cc]) * idsup;
-    double dpp = (sB[r][cc + 1] - sB[r][cc]) * invdphi * invRm + 0.5 * (sA[r + 1][cc] + VrR[cc]) * invRm;
-    double dv = (sA[r + 1][cc] * rt[RT_SUP][r] - VrR[cc] * rt[RT_INF][r]) * idsup * invRm;
-    dv += (sB[r][cc + 1] - sB[r][cc]) * invdphi * invRm;
-    const double nu = rt[RT_NU][r];
-    sC[r][cc] = 2.0 * sS[r][cc] * nu * (drr - onethird * dv);
-    sD[r][cc] = 2.0 * sS[r][cc] * nu * (dpp - onethird * dv);
-    if (i > 0) {
-      double drp = 0.5 * (rt[RT_INF][r] * (sB[r][cc] * invRm - sB[r - 1][cc] * rt[RT_IMED][r - 1]) * rt[RT_IDMED][r] +
-                          (VrR[cc] - VrR[cc - 1]) * invdphi * rt[RT_IINF][r]);
-      sE[r][cc] = 2.0 * 0.25 * (sS[r][cc] + sS[r - 1][cc] + sS[r][cc - 1] + sS[r - 1][cc - 1]) * nu * drp;
+    // ---- S4: radial artificial pressure (Kernels.cu:409-434) of ring o ----
+    const double dvr = A3[M1] - A3[M2];
+    if constexpr (LV >= 4) QR[M2] = (IN || (o >= 0 && o < nr)) ? art_visc_q(S[M2], dvr) : 0.0;
+    // ---- ring o: the rest of S3 and S4, S5 ("kernel", Kernels.cu:438-479), damping #2, store ----
+    if constexpr (LV >= 5) {
+      const long l = (long)o * ns;
+      if (!IN && o == nr) {  // ghost ring: VradNew/VthetaNew are never written (0)
+        if (mine) {
+          at(a.odens + l, jb) = S[M2];
+          at(a.ovr + l, jb) = 0.0;
+          at(a.ovt + l, jb) = 0.0;
+        }
+        return;
+      }
+      const recip64 dr_(hr[M2], hrr[M2]), da_(ha[M2], har[M2]);
+      double b = B1[M2];
+      if (IN || (o >= 1 && o < nr - 1))
+        b += da_.div(dt * Ro[RG_IMED] *
+                     ((Ro[RG_SUP] * RP[M1] - Ro[RG_INF] * RP[M2]) * Ro[RG_IDSUP] +
+                      (PP[M2] - lane_prev(PP[M2])) * invdphi + 0.5 * (RP[M2] + RP[M1])));
+      const double dvt = lane_next(b) - b;
+      const double qt = art_visc_q(S[M2], dvt);
+      double vrnew = 0.0;
+      if (IN || o > 0) {
+        const double densint = QR[M2] - QR[C];  // (slot C: ring o - 1, not yet overwritten)
+        vrnew = A3[M2] - dr_.div(dt) * densint * Ro[RG_IDMED];
+      }
+      const double invdxtheta = Ro[RG_IDXT];
+      const double tempint = qt - lane_prev(qt);
+      double vtnew = b - da_.div(dt) * tempint * invdxtheta;
+      double s2 = S[M2];
+      double eint = 0.0;
+      if constexpr (ADI)
+        // EnergyInt ("kernel", Kernels.cu:474-477) from the energy after the
+        // first damping pass; the second pass damps Energy, which Substep3
+        // then overwrites, so it is not formed
+        eint = EN[M2] - dt * QR[M2] * dvr * Ro[RG_IDSUP] - dt * qt * dvt * invdxtheta;
+      if (zones >> (row - 2) & 1) {
+        const double *ev = evc[row - 2];
+        vrnew = ev_damp(vrnew, ev, EV_VR2);
+        vtnew = ev_damp(vtnew, ev, EV_VT2);
+        s2 = ev_damp(s2, ev, EV_S);
+      }
+      if (mine) {
+        at(a.odens + l, jb) = s2;
+        at(a.ovr + l, jb) = vrnew;
+        at(a.ovt + l, jb) = vtnew;
+        if constexpr (ADI) at(a.oeint + l, jb) = eint;
+      }
     }
-  }
-  __syncthreads();
-
-  // ---- S3: viscous velocity update (Kernels.cu:118-150), in place ----
-#pragma unroll
-  for (int kq = 0; kq < KPT; kq++) {
-    const int q = tid + kq * KTPB;
-    if (q >= KHR * KHC) break;
-    int r = q / KHC, cc = q - r * KHC;
-    int i = GI(r);
-    if (r < 2 || r >= KHR - 1 || cc < 3 || cc >= KHC - 3 || i < 1 || i >= nr) continue;
-    // (S1 covered this cell with i > 0: both halved sums' refinements are in
-    // hazi / hrad)
-    if (i < nr - 1 && r < KHR - 2)
-      sB[r][cc] += recip64(0.5 * (sS[r][cc] + sS[r][cc - 1]), hazi[kq])
-                       .div(dt * rt[RT_IMED][r] *
-                            ((rt[RT_SUP][r] * sE[r + 1][cc] - rt[RT_INF][r] * sE[r][cc]) * rt[RT_IDSUP][r] +
-                             (sD[r][cc] - sD[r][cc - 1]) * invdphi + 0.5 * (sE[r][cc] + sE[r + 1][cc])));
-    sA[r][cc] += recip64(0.5 * (sS[r][cc] + sS[r - 1][cc]), hrad[kq])
-                     .div(dt * rt[RT_IINF][r] *
-                          ((rt[RT_MED][r] * sC[r][cc] - rt[RT_MED][r - 1] * sC[r - 1][cc]) * rt[RT_IDMED][r] +
-                           (sE[r][cc + 1] - sE[r][cc]) * invdphi - 0.5 * (sD[r][cc] + sD[r - 1][cc])));
-  }
-  __syncthreads();
-
-  // ---- S4: artificial pressure (Kernels.cu:409-434) on rows [3, KHR-1), cols [3, KHC-4) ----
-#pragma unroll
-  for (int kq = 0; kq < KPT; kq++) {
-    const int q = tid + kq * KTPB;
-    if (q >= KHR * KHC) break;
-    int r = q / KHC, cc = q - r * KHC;
-    int i = GI(r);
-    if (r < 3 || r >= KHR - 1 || cc < 3 || cc >= KHC - 4 || i < 0 || i >= nr) continue;
-    sC[r][cc] = art_visc_q(sS[r][cc], sA[r + 1][cc] - sA[r][cc]);
-    sD[r][cc] = art_visc_q(sS[r][cc], sB[r][cc + 1] - sB[r][cc]);
-  }
-  __syncthreads();
-
-  // ---- S5: velocity update ("kernel", Kernels.cu:438-479), damping #2, store ----
-#pragma unroll
-  for (int kq = 0; kq < (KTH * KTW + KTPB - 1) / KTPB; kq++) {
-    const int q = tid + kq * KTPB;
-    if (q >= KTH * KTW) break;
-    int r = q / KTW + HALO_R, cc = q % KTW + HALO_C;
-    int i = GI(r), j = j0 + cc - HALO_C;
-    if (i > nr || j >= ns) continue;
-    long l = (long)i * ns + j;
-    if (i == nr) {  // ghost ring: VradNew/VthetaNew are never written (0)
-      a.odens[l] = sS[r][cc];
-      a.ovr[l] = 0.0;
-      a.ovt[l] = 0.0;
-      continue;
+  };
+  auto march = [&](auto inner) __attribute__((always_inline)) {
+    // rings i0 - 3 .. i0 + 1 fill the windows; with ring i0 + 2 in slot 2,
+    // ring i0 - 3 + x is in slot x mod 3
+    const int m0 = i0 - SRC_HT;
+    step(m0, LVL(0), LVL(0), inner);
+    step(m0 + 1, LVL(1), LVL(1), inner);
+    step(m0 + 2, LVL(2), LVL(2), inner);
+    step(m0 + 3, LVL(3), LVL(0), inner);
+    step(m0 + 4, LVL(4), LVL(1), inner);
+    int m = m0 + 5;
+    for (; m + 2 <= i1 + 1; m += 3) {
+      step(m, LVL(5), LVL(2), inner);
+      step(m + 1, LVL(5), LVL(0), inner);
+      step(m + 2, LVL(5), LVL(1), inner);
     }
-    double vrnew = 0.0;
-    if (i > 0) {
-      double d = sS[r][cc] + sS[r - 1][cc];
-      double densint = sC[r][cc] - sC[r - 1][cc];
-      vrnew = sA[r][cc] - dt * 2.0 / d * densint * rt[RT_IDMED][r];
-    }
-    const double invdxtheta = rt[RT_IDXT][r];
-    double dens2 = sS[r][cc] + sS[r][cc - 1];
-    double tempint = (sD[r][cc] - sD[r][cc - 1]);
-    double vtnew = sB[r][cc] - dt * 2.0 / dens2 * tempint * invdxtheta;
-    double s = sS[r][cc];
-    if constexpr (ADI) {
-      // EnergyInt ("kernel", Kernels.cu:474-477) from the energy after the
-      // first damping pass; the second pass damps Energy, which Substep3
-      // then overwrites, so it is not formed
-      double e = a.energy[l];
-      if (a.evanescent && rt[RT_EVZ][r] != 0.0) e = damp_toward(e, evc[r][0], rt[RT_EMED][r]);
-      a.oeint[l] = e - dt * sC[r][cc] * (sA[r + 1][cc] - sA[r][cc]) * rt[RT_IDSUP][r] -
-                   dt * sD[r][cc] * (sB[r][cc + 1] - sB[r][cc]) * invdxtheta;
-    }
-    if (a.evanescent && rt[RT_EVZ][r] != 0.0) {
-      vrnew = damp_toward(vrnew, evc[r][0], evc[r][3]);
-      vtnew = damp_toward(vtnew, evc[r][0], evc[r][4]);
-      s = damp_toward(s, evc[r][0], rt[RT_SMED][r]);
-    }
-    a.odens[l] = s;
-    a.ovr[l] = vrnew;
-    a.ovt[l] = vtnew;
-  }
-#undef GI
-#undef GJ
+    if (m <= i1 + 1) step(m, LVL(5), LVL(2), inner);
+    if (m + 1 <= i1 + 1) step(m + 1, LVL(5), LVL(0), inner);
+  };
+#undef LVL
+  if (i0 - SRC_HT >= 1 && i1 + SRC_HB <= nr)
+    march(std::true_type());
+  else
+    march(std::false_type());
 }
 
 // ----------------------------------------------------------- k_src3 ----
@@ -885,22 +919,6 @@ struct taz_args {
 // take 174-208 VGPRs and leave two)
 #define TAZW_CL64 3
 #define TAZW_P64 (64 * TAZW_CL64 - TAZW_HL - TAZW_HR)  // cells output per FP64 chunk
-
-// x of lane l-1 (lane 0 reads 0): DPP wave_shr:1 on each dword
-__device__ __forceinline__ double lane_prev(double x) {
-  const long long b = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x138, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x138, 0xf, 0xf, true);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-// x of lane l+1 (lane 63 reads 0): DPP wave_shl:1 on each dword
-__device__ __forceinline__ double lane_next(double x) {
-  const long long b = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x130, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x130, 0xf, 0xf, true);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
 
 __device__ __forceinline__ float lane_prev(float x) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xf, 0xf, true));
@@ -1790,7 +1808,6 @@ __device__ __forceinline__ void fin_ring_ov(const fin_args &a, int i, double *ri
 // Workgroups are dispatched round-robin over the 8 XCDs.  Each XCD gets a
 // contiguous band of rings, so neighbouring rings, which read each other's
 // momenta and densities, are processed side by side under one L2.
-#define FG_NXCD 8
 // ADI: adiabatic deck; S32: FP32 bulk mode (FP32 storage of k_taz's fields)
 template <bool ADI, bool S32 = false>
 __global__ __launch_bounds__(256) void k_fin(fin_args a) {
@@ -1829,6 +1846,38 @@ __global__ __launch_bounds__(256) void k_fin(fin_args a) {
 // and dispatched to a template instance; the LDS tiles are carved from dynamic
 // shared memory: six (th + 6) x HC float arrays and two th x TW
 // increment arrays.
+// per-ring tables the source stages read, staged per tile row in LDS
+enum { RT_MED, RT_IMED, RT_IDMED, RT_INF, RT_IINF, RT_IDXT, RT_SUPP, RT_IDSUP, RT_SUP, RT_NU, RT_CS, RT_SMED, RT_EVZ, RT_N };
+__device__ __forceinline__ const double *ring_table(const fg_dev_tables &t, const double *nu, int x) {
+  switch (x) {
+    case RT_MED: return t.Rmed;
+    case RT_IMED: return t.invRmed;
+    case RT_IDMED: return t.invdiffRmed;
+    case RT_INF: return t.Rinf;
+    case RT_IINF: return t.invRinf;
+    case RT_IDXT: return t.invdxtheta;
+    case RT_SUPP: return t.supp_torque;
+    case RT_IDSUP: return t.invdiffRsup;
+    case RT_SUP: return t.Rsup;
+    case RT_NU: return nu;
+    case RT_CS: return t.cs_iso;
+    default: return t.SigmaMed;
+  }
+}
+
+#define TW 64
+#define HALO_R 4  // rows above the tile (i - 4 .. )
+#define HALO_B 2  // rows below the tile ( .. i + TH + 1)
+#define HALO_C 4  // columns on each side
+#define HC (TW + 2 * HALO_C)
+// sector of a staged column j0 - HALO_C + c (j0 = the tile's first column):
+// at most one ring length outside [0, ns) once ns reaches the staged width,
+// so a compare and an add or subtract replace the two runtime modulos
+__device__ __forceinline__ int wrap_col(int x, int ns) {
+  if (x < 0) x += ns;
+  while (x >= ns) x -= ns;
+  return x;
+}
 #define SRC32_MAX_TH 32
 #define SRC32_TPB 512  // threads per FP32 source tile
 #define SRC32_PER_THREAD (((SRC32_MAX_TH + HALO_R + HALO_B) * HC + SRC32_TPB - 1) / SRC32_TPB)
@@ -2733,6 +2782,43 @@ static void fp32_pair_rings(const fg_ctx *c, const fg_planet_pot *pl, int nb, in
   *b1 = hi;
 }
 
+// whether every squared distance plus smoothing, its root and the planets'
+// quotients by it lie well inside the exponent range (planet_potential_plain)
+static int plain_potential(const fg_ctx *c, const fg_planet_pot *pl, int nb) {
+  const double lo = 1e-100, hi = 1e100;
+  bool ok = c->h_Rmed[0] > -hi && c->h_Rmed[c->nr - 1] < hi;
+  for (int k = 0; k < nb; k++) {
+    const double m = fabs(pl[k].mass);
+    ok = ok && fabs(pl[k].x) < hi && fabs(pl[k].y) < hi && pl[k].smooth > lo && pl[k].smooth < hi &&
+         (m == 0.0 || (m > lo && m < hi));
+  }
+  return ok ? 1 : 0;
+}
+
+// Rings per band of k_src: the band with the least estimated time.  A wave
+// spends about one time unit (1 us) on a step when it has its SIMD to itself
+// and shares the SIMD's issue at 0.7 units per step and wave, and a band of H
+// rings costs H + 3 steps (the first ones are partial); up to three waves per
+// SIMD are resident, so the fullest SIMD counts, beyond that the total does.
+// Measured (us, FP64 isothermal): 128x384 1 ring 11.7, 8 rings 19; 512x1536
+// 7-8 rings 24, 4 rings 28, 20 rings 36; 1024x3072 18-20 rings 50, 8 rings 57,
+// 26 rings 57; 2048x4096 18-26 rings 107, 8 rings 121.
+static int src_band(int nr, int nstrips) {
+  const int simds = 1024;
+  double best = 0.0;
+  int band = 1;
+  for (int h = 1; h <= SRC_MAX_BAND; h++) {
+    const long waves = (long)nstrips * ((nr + h) / h);
+    const double n = (double)waves / simds;
+    const double cost = (h + 3) * (n > 3.0 ? 0.7 * n : std::max(1.0, 0.7 * ceil(n)));
+    if (h == 1 || cost < best) {
+      best = cost;
+      band = h;
+    }
+  }
+  return band;
+}
+
 extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, double domega,
                                    const fg_planet_pot *planets, int nb, double ix, double iy,
                                    double DeltaT_next, int flags) {
@@ -2779,6 +2865,7 @@ extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, dou
     sa.P.smooth[k] = planets[k].smooth;
     sa.P.invd3[k] = planets[k].inv_d3;
   }
+  sa.plain = plain_potential(c, planets, nb);
   sa.P.ix = ix;
   sa.P.iy = iy;
   sa.dt = dt;
@@ -2788,7 +2875,7 @@ extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, dou
   sa.ns = ns;
   sa.indirect = c->p.indirect_term;
   sa.evanescent = c->p.evanescent;
-  sa.corotating = (domega != 0.0) ? 1 : 0;
+  const int corotating = (domega != 0.0) ? 1 : 0;
   if (c->prof_on) {
     (void)hipStreamSynchronize(c->stream);
     prof_fold(c);
@@ -2822,7 +2909,7 @@ extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, dou
     s3.ns = ns;
     s3.indirect = sa.indirect;
     s3.evanescent = sa.evanescent;
-    s3.corotating = sa.corotating;
+    s3.corotating = corotating;
     const int th = c->tile_src_th;
     FG_HIP(hipFuncSetAttribute((const void *)k_src32<32>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)src32_lds_bytes(32)));
@@ -2834,16 +2921,19 @@ extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, dou
     else
       hipLaunchKernelGGL(k_src32<16>, g32, dim3(SRC32_TPB), src32_lds_bytes(16), c->stream, s3);
   } else {
-    const dim3 gs((ns + TW - 1) / TW, (nr + 1 + TH - 1) / TH);
+    sa.nstrips = (ns + SRC_W - 1) / SRC_W;
+    sa.width = (ns + sa.nstrips - 1) / sa.nstrips;
+    sa.band = src_band(nr, sa.nstrips);
+    const dim3 gs(xcd_grid(sa.nstrips * ((nr + sa.band) / sa.band)));
     const int mode = (adi ? 1 : 0) | (sg ? 2 : 0);
     if (mode == 0)
-      hipLaunchKernelGGL((k_src<TH, TW, SRC64_TPB, 0>), gs, dim3(SRC64_TPB), 0, c->stream, sa);
+      hipLaunchKernelGGL(k_src<0>, gs, dim3(64), 0, c->stream, sa);
     else if (mode == 1)
-      hipLaunchKernelGGL((k_src<TH, TW, SRC64_TPB, 1>), gs, dim3(SRC64_TPB), 0, c->stream, sa);
+      hipLaunchKernelGGL(k_src<1>, gs, dim3(64), 0, c->stream, sa);
     else if (mode == 2)
-      hipLaunchKernelGGL((k_src<TH, TW, SRC64_TPB, 2>), gs, dim3(SRC64_TPB), 0, c->stream, sa);
+      hipLaunchKernelGGL(k_src<2>, gs, dim3(64), 0, c->stream, sa);
     else
-      hipLaunchKernelGGL((k_src<TH, TW, SRC64_TPB, 3>), gs, dim3(SRC64_TPB), 0, c->stream, sa);
+      hipLaunchKernelGGL(k_src<3>, gs, dim3(64), 0, c->stream, sa);
   }
   FG_LAUNCH_CHECK();
   if (adi) {  // Substep3 (counted with k_src by fg_profile)

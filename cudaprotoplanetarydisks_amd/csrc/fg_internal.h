@@ -95,8 +95,12 @@ struct fg_dev_tables {
   double *cos_cell, *sin_cell, *cos_pot, *sin_pot;
   double *sg_Kr, *sg_Kt;
   double *sg_norm_r, *sg_norm_t, *sg_sqrt_ratio, *sg_ratio;
+  // the ring values k_src reads, RG_NU per ring
+  double *rings;
   double dtheta, invdphi, dt1d_coef, vrad0_slope, visc_value;
 };
+// (k_src's copy holds the viscosity as well)
+enum { RG_MED, RG_IMED, RG_IDMED, RG_INF, RG_IINF, RG_IDXT, RG_IDSUP, RG_SUP, RG_CS, RG_SUPP, RG_NU, RG_N = 12 };
 
 // mixed-radix FFT plan of one transform length (fg_sg.hip)
 #define FG_FFT_MAXST 40

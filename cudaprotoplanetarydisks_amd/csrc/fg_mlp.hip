@@ -14,7 +14,7 @@
 // copies the GEMMs read are refreshed by the optimizer step.
 //
 // Networks whose widths fit in LDS (mlp_fits_rows) run two kernels per
-// training step: k_mlp_rows takes 16 batch rows per workgroup through every
+// training step: k_mlp_rows takes 4 to 16 batch rows a workgroup through every
 // layer forward and back, k_mlp_weights forms every weight gradient and
 // applies Adam to it where it stands.  Wider networks, and fg_bf16_gemm,
 // run k_gemm_bf16 layer by layer: operands addressed by (row stride, column
