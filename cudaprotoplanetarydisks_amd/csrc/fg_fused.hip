@@ -2795,20 +2795,18 @@ static int plain_potential(const fg_ctx *c, const fg_planet_pot *pl, int nb) {
   return ok ? 1 : 0;
 }
 
-// Rings per band of k_src: the band with the least estimated time.  A wave
+// Rings per band of a kernel whose waves march over `rows` rings in column
+// strips: the band with the least estimated time, up to `most`.  A wave
 // spends about one time unit (1 us) on a step when it has its SIMD to itself
 // and shares the SIMD's issue at 0.7 units per step and wave, and a band of H
 // rings costs H + 3 steps (the first ones are partial); up to three waves per
 // SIMD are resident, so the fullest SIMD counts, beyond that the total does.
-// Measured (us, FP64 isothermal): 128x384 1 ring 11.7, 8 rings 19; 512x1536
-// 7-8 rings 24, 4 rings 28, 20 rings 36; 1024x3072 18-20 rings 50, 8 rings 57,
-// 26 rings 57; 2048x4096 18-26 rings 107, 8 rings 121.
-static int src_band(int nr, int nstrips) {
+static int march_band(int rows, int nstrips, int most) {
   const int simds = 1024;
   double best = 0.0;
   int band = 1;
-  for (int h = 1; h <= SRC_MAX_BAND; h++) {
-    const long waves = (long)nstrips * ((nr + h) / h);
+  for (int h = 1; h <= most; h++) {
+    const long waves = (long)nstrips * ((rows + h - 1) / h);
     const double n = (double)waves / simds;
     const double cost = (h + 3) * (n > 3.0 ? 0.7 * n : std::max(1.0, 0.7 * ceil(n)));
     if (h == 1 || cost < best) {
@@ -2817,6 +2815,18 @@ static int src_band(int nr, int nstrips) {
     }
   }
   return band;
+}
+// Measured for k_src (us, FP64 isothermal): 128x384 1 ring 11.7, 8 rings 19;
+// 512x1536 7-8 rings 24, 4 rings 28, 20 rings 36; 1024x3072 18-20 rings 50,
+// 8 rings 57, 26 rings 57; 2048x4096 18-26 rings 107, 8 rings 121.
+static int src_band(int nr, int nstrips) { return march_band(nr + 1, nstrips, SRC_MAX_BAND); }
+// Measured for k_trad (us): 128x384 2-3 rings 11.9, 16 rings 21.5; 301x998
+// (with energy) 3-6 rings 18, 16 rings 25; 512x1536 8 rings 23, 16 rings 26;
+// from 1024x3072 on, where HBM bounds it, 10 to 16 rings are within 3 % and
+// 20 to 32 cost 5 %; k_trad32 256x768 3-4 rings 14, 16 rings 23.5.  fg_set_tiles
+// fixes the band instead.
+static int trad_band(const fg_ctx *c, int nstrips) {
+  return c->tile_trad_band ? c->tile_trad_band : march_band(c->nr, nstrips, 16);
 }
 
 extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, double domega,
@@ -2980,7 +2990,7 @@ extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, dou
   ta.ns = ns;
   ta.vmed = c->VMed;
   ta.nstrips = (ns + TRAD_TPB - 1) / TRAD_TPB;
-  ta.band = c->tile_trad_band;
+  ta.band = trad_band(c, ta.nstrips);
   ta.lob0 = lob0;
   ta.lob1 = lob1;
   prof_mark(c);
@@ -3312,6 +3322,10 @@ static fg_status upload_items(const std::vector<T> &v, T **dev) {
 }
 
 // work lists (largest disks first) and the captured graph of one substep
+// rings per radial-sweep band of a batched disk (the other disks fill the
+// chip, so a band as long as a large grid's)
+static int batch_band(const fg_ctx *c) { return c->tile_trad_band ? c->tile_trad_band : 16; }
+
 static fg_status batch_build(fg_batch_dev *b) {
   std::vector<int> order(b->n);
   for (int k = 0; k < b->n; k++) order[k] = k;
@@ -3321,7 +3335,7 @@ static fg_status batch_build(fg_batch_dev *b) {
   b->max_ns = 1;
   for (int k : order) {
     const fg_ctx *c = b->ctx[k];
-    const int nr = c->nr, ns = c->ns, th = c->tile_src_th, band = c->tile_trad_band;
+    const int nr = c->nr, ns = c->ns, th = c->tile_src_th, band = batch_band(c);
     if ((th != 8 && th != 16 && th != 32) || band < 1) {
       fg_set_error("batch: disk %d has tile shape th=%d band=%d", k, th, band);
       return FG_E_INVALID;
@@ -3467,7 +3481,7 @@ fg_status fg_batch_dev_set(fg_batch_dev *b, int k, int active, double dt, double
   ta.nr = nr;
   ta.ns = ns;
   ta.nstrips = (ns + TRAD_TPB - 1) / TRAD_TPB;
-  ta.band = c->tile_trad_band;
+  ta.band = batch_band(c);
   ta.lob0 = lob0;
   ta.lob1 = lob1;
   taz_args &za = d.taz;

@@ -159,8 +159,8 @@ struct fg_ctx {
   int prof_nev, prof_pending;
   double prof_ms[16];
   long prof_calls[16];
-  // tile shapes of the FP32 fused kernels (rings per k_src tile, rings
-  // per radial-sweep band), set by fg_set_tiles
+  // tile shapes of the fused kernels (rings per FP32 source tile, rings per
+  // radial-sweep band; 0: picked for the grid), set by fg_set_tiles
   int tile_src_th, tile_trad_band;
   // FP32 bulk mode: Sigma stored as float pairs on the rings within this
   // many Hill radii of a planet (fg_set_fp32_pairs)
