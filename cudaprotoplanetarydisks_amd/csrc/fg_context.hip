@@ -187,16 +187,10 @@ extern "C" fg_status fg_create(const fg_params *p, const fg_tables *t, int devic
     TRY(dev_alloc(&c->sg_tmp, C));
   }
   for (int k = 0; k < FG_NFIELDS; k++) TRY(dev_alloc(&c->f[k], S));
-  TRY(dev_alloc(&c->DRR, S));
-  TRY(dev_alloc(&c->DPP, S));
-  TRY(dev_alloc(&c->DRP, S));
-  TRY(dev_alloc(&c->Work, S));
-  TRY(dev_alloc(&c->QRStar, S));
-  TRY(dev_alloc(&c->DensStar, S));
-  TRY(dev_alloc(&c->dq, S));
-  TRY(dev_alloc(&c->TempShift, S));
-  TRY(dev_alloc(&c->Vradial, S));
-  TRY(dev_alloc(&c->Vazimutal, S));
+  for (int k = 0; k < 7; k++) TRY(dev_alloc(&c->sw[k], S));
+  c->shared_faces = 1;
+  for (int i = 0; i + 1 < c->nr; i++)
+    if (t->Rsup[i] != t->Rinf[i + 1]) c->shared_faces = 0;
   TRY(dev_alloc(&c->Vmoy, R));
   TRY(dev_alloc(&c->newDT, R));
   TRY(dev_alloc(&c->DT1D, R));
@@ -207,17 +201,19 @@ extern "C" fg_status fg_create(const fg_params *p, const fg_tables *t, int devic
   TRY(dev_alloc(&c->sgacc_prev, R));
   TRY(dev_alloc(&c->nu_next, R));
   TRY(dev_alloc(&c->Nshift, R));
-  TRY(dev_alloc(&c->NoSplit, R));
   TRY(dev_alloc(&c->LostByDisk, NS));
   TRY(dev_alloc(&c->red_partial, 2 * FG_RED_BLOCKS));
-  TRY(dev_alloc(&c->red_out, 8));
-  TRY(dev_alloc(&c->cfl_out, 4));
-  if (hipHostMalloc((void **)&c->h_out, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess ||
-      hipHostMalloc((void **)&c->h_cfl, 4 * sizeof(int), hipHostMallocDefault) != hipSuccess) {
+  const unsigned pin = hipHostMallocCoherent | hipHostMallocMapped;
+  if (hipHostMalloc((void **)&c->h_out, FG_OUT_SLOTS * sizeof(double), pin) != hipSuccess ||
+      hipHostGetDevicePointer((void **)&c->red_out, c->h_out, 0) != hipSuccess ||
+      hipHostMalloc((void **)&c->h_cfl, 4 * sizeof(int), pin) != hipSuccess ||
+      hipHostGetDevicePointer((void **)&c->cfl_out, c->h_cfl, 0) != hipSuccess) {
     fg_set_error("hipHostMalloc of the result mirror failed");
     fg_destroy(c);
     return FG_E_NOMEM;
   }
+  memset(c->h_out, 0, FG_OUT_SLOTS * sizeof(double));
+  memset(c->h_cfl, 0, 4 * sizeof(int));
   // initial viscosity profile (constant viscosity; alpha viscosity is
   // refreshed by fg_ring_mean_cs)
   {
@@ -253,21 +249,18 @@ extern "C" fg_status fg_destroy(fg_ctx *c) {
                   c->t.ev_zone,    c->t.ev_coef,    c->t.ev_period,   c->t.ev_vtheta_arg, c->t.visc_const,
                   c->t.visc_pow15, c->t.visc_cav,   c->t.visc_cav_on, c->t.cos_cell,     c->t.sin_cell,
                   c->t.cos_pot,    c->t.sin_pot,    c->t.sg_Kr,       c->t.sg_Kt,        c->t.sg_norm_r,
-                  c->t.sg_norm_t,  c->t.sg_sqrt_ratio, c->t.sg_ratio, c->t.rings,       c->DRR,            c->DPP,
-                  c->DRP,          c->Work,         c->QRStar,        c->DensStar,       c->dq,
-                  c->TempShift,    c->Vradial,      c->Vazimutal,     c->Vmoy,           c->newDT,
+                  c->t.sg_norm_t,  c->t.sg_sqrt_ratio, c->t.sg_ratio, c->t.rings,       c->Vmoy,           c->newDT,
                   c->DT1D,         c->VMed,         c->nu,            c->cs_mean,        c->sgacc_mean,
                   c->sgacc_prev,   c->nu_next,
-                  c->Nshift,       c->NoSplit,      c->LostByDisk,    c->red_partial,    c->red_out,
-                  c->cfl_out,      c->sg_Sr,        c->sg_St,         c->sg_Krc,         c->sg_Ktc,
+                  c->Nshift,       c->LostByDisk,    c->red_partial,    c->sg_Sr,        c->sg_St,         c->sg_Krc,         c->sg_Ktc,
                   c->sg_Gr,        c->sg_Gt,        c->sg_tmp,        c->fu_ring,        c->fu_fpart,
                   c->hill_partial, c->hill_out};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   for (int k = 0; k < FG_NFIELDS; k++)
     if (c->f[k]) (void)hipFree(c->f[k]);
-  for (int k = 0; k < 8; k++)
-    if (c->f32[k]) (void)hipFree(c->f32[k]);
+  for (int k = 0; k < 7; k++)
+    if (c->sw[k]) (void)hipFree(c->sw[k]);
   for (int k = 0; k < 4; k++)
     if (c->fu_mom[k]) (void)hipFree(c->fu_mom[k]);
   if (c->h_out) (void)hipHostFree(c->h_out);
@@ -302,8 +295,8 @@ extern "C" fg_status fg_upload_state(fg_ctx *c, const double *dens, const double
   if ((st = put(c, c->f[FG_VTHETA], vtheta))) return st;
   if ((st = put(c, c->f[FG_ENERGY], energy))) return st;
   // a new state: crash flags raised by passes over the old one no longer apply
-  FG_HIP(hipMemsetAsync(c->cfl_out + 1, 0, sizeof(int), c->stream));
   FG_HIP(hipStreamSynchronize(c->stream));
+  *(volatile int *)(c->h_cfl + 1) = 0;
   if (c->h_fused) *(volatile int *)(c->h_fused + FG_FUSED_CRASH_SLOT) = 0;
   return FG_OK;
 }

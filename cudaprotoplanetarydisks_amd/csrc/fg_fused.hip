@@ -41,7 +41,6 @@
 #include "fg_internal.h"
 #include "fg_reduce.h"
 
-fg_status fg_disk_force_async(fg_ctx *c, const double *dens, double x, double y, double rs, double *out_dev);
 
 
 
@@ -608,6 +607,7 @@ struct trad_args {
   float *fout[NQ];
   const double *sbar, *vref;  // per-ring backgrounds of Sigma and vtheta
   double *vmed;  // ring means of vtheta for the azimuthal pass
+  double *lost;  // ROUTINE: change of ring 0's Sigma per sector (open inner edge), else NULL
   fg_dev_tables t;
   double dt, omega_frame;
   int nr, ns, nstrips;
@@ -712,8 +712,11 @@ __device__ void ring_mean_wave32(const float *v, double vb, int ns, double *out)
 }
 
 // NQT transported quantities: 5, or 6 with the energy of an adiabatic deck
-// (TransportEuler.cu:60-79 sweeps it between the momenta and Sigma)
-template <int NQT>
+// (TransportEuler.cu:60-79 sweeps it between the momenta and Sigma).
+// ROUTINE: the sweep of fg_transport (the mass lost through an open edge);
+// OWN: tables whose rings' outer faces are not the next rings' inner faces, so
+// that a ring's outer flux takes its own Rsup (Kernels.cu:1039)
+template <int NQT, bool ROUTINE = false, bool OWN = false>
 __global__ __launch_bounds__(TRAD_TPB) void k_trad(trad_args a) {
   constexpr bool EN = NQT == 6;
   const int nr = a.nr, ns = a.ns;
@@ -816,6 +819,8 @@ __global__ __launch_bounds__(TRAD_TPB) void k_trad(trad_args a) {
     const double vface = (IN || k < nr) ? vr[B1] : 0.0;
     const double Rinf = lane_get(rt.Rinf, r - 1);
     for (int q = 0; q < NQT; q++) F[q][B1] = cflux * Rinf * QS[q] * DS * vface;
+    double outer = 0.0;  // radius of ring k - 1's own outer face
+    if constexpr (OWN) outer = t.Rsup[max(k - 1, 0)];
     // ring k-1 is complete: Q += (F(k-1) - F(k)) / Surf
     if (decltype(store)::value) {
       const int o = k - 1;
@@ -823,8 +828,9 @@ __global__ __launch_bounds__(TRAD_TPB) void k_trad(trad_args a) {
       const double isurf = lane_get(rt.isurf, r - 2);
       for (int q = 0; q < NQT; q++) {
         double varq = F[q][B2];
-        varq -= F[q][B1];
+        varq -= OWN ? cflux * outer * QS[q] * DS * vface : F[q][B1];
         a.out[q][lo] = Q[q][B2] + varq * isurf;
+        if (ROUTINE && q == NQT - 1 && o == 0 && a.lost) a.lost[j] = varq;
       }
     }
   };
@@ -884,6 +890,9 @@ struct taz_args {
   const double *vmed;   // its ring means
   const double *q[NQ_MAX];  // quantities after the radial sweep (Sigma last)
   double *xd, *xvt, *xrmp, *xrmm, *xe;
+  // FULL: the angular momenta, Sigma between the two sweeps (DENSINT) and the
+  // residual velocity as well
+  double *xtmp, *xtmm, *xdint, *xres;
   // FP32 bulk mode: the same fields stored in FP32 (fp32_store_bg)
   const float *fvt, *fq[NQ];
   float *fxd, *fxvt, *fxrmp, *fxrmm;
@@ -1044,7 +1053,8 @@ struct tazw_lds {
 };
 // PAIRS: a ring of the FP32 mode stored as float pairs (its own instance,
 // so that the other rings run without the residuals' loads and branches)
-template <int CL, bool F32, int NQT = 5, bool PAIRS = false>
+// FULL: the fields that fg_transport leaves besides (FP64)
+template <int CL, bool F32, int NQT = 5, bool PAIRS = false, bool FULL = false>
 __device__ __forceinline__ void tazw_body(const taz_args &a, int i, int chunk, tazw_lds<CL, NQT> &lds) {
   constexpr int N = 64 * CL, P = N - TAZW_HL - TAZW_HR;
   static_assert(NQT == 5 || !F32, "the FP32 sweeps carry five quantities");
@@ -1144,6 +1154,23 @@ __device__ __forceinline__ void tazw_body(const taz_args &a, int i, int chunk, t
     wave_sweep32<CL, true>(q, vres, (float)vuni, t, i, (float)a.dt);
   } else {
     wave_sweep<CL, false, NQT>(q, vres, 0.0, t, i, a.dt);
+    if constexpr (FULL) {  // neither is shifted
+#pragma unroll
+      for (int c = 0; c < CL; c++) {
+        ostage[0][l * CL + c] = q[NQT - 1][c];
+        ostage[1][l * CL + c] = vres[c];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < CL; m++) {
+        const int k = l + 64 * m, g = g0 + k;
+        if (k >= TAZW_HL && k < TAZW_HL + P && g < ns) {
+          a.xdint[base + g] = ostage[0][k];
+          a.xres[base + g] = ostage[1][k];
+        }
+      }
+      __syncthreads();
+    }
     wave_sweep<CL, true, NQT>(q, vres, vuni, t, i, a.dt);
   }
   // vtheta from the angular momenta (Kernels.cu:1206-1207): cells j - 1
@@ -1201,6 +1228,25 @@ __device__ __forceinline__ void tazw_body(const taz_args &a, int i, int chunk, t
       }
     }
   }
+  if constexpr (FULL) {
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < CL; c++) {
+      ostage[0][l * CL + c] = q[2][c];
+      ostage[1][l * CL + c] = q[3][c];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < CL; m++) {
+      const int k = l + 64 * m, g = g0 + k;
+      if (k >= TAZW_HL && k < TAZW_HL + P && g < ns) {
+        int jo = g + sh;
+        if (jo >= ns) jo -= ns;
+        a.xtmp[base + jo] = ostage[0][k];
+        a.xtmm[base + jo] = ostage[1][k];
+      }
+    }
+  }
 }
 
 // blockIdx.x = chunk, blockIdx.y = ring
@@ -1211,6 +1257,13 @@ __global__ __launch_bounds__(64) void k_tazw(taz_args a) {
     tazw_body<CL, F32, NQT, F32>(a, blockIdx.y, blockIdx.x, sh);
   else
     tazw_body<CL, F32, NQT, false>(a, blockIdx.y, blockIdx.x, sh);
+}
+
+// the azimuthal sweeps of fg_transport
+template <int NQT>
+__global__ __launch_bounds__(64) void k_tazw_full(taz_args a) {
+  __shared__ tazw_lds<TAZW_CL64, NQT> sh;
+  tazw_body<TAZW_CL64, false, NQT, false, true>(a, blockIdx.y, blockIdx.x, sh);
 }
 
 // the FP32 bulk mode's single-disk sweep (TAZW_CL32 cells per lane)
@@ -3115,6 +3168,101 @@ extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, dou
     if (fg_status s = fg_viscosity_into(c, c->nu_next)) return s;
     c->nu_pending = 1;
   }
+  return FG_OK;
+}
+
+// ------------------------------------------- per-routine transport ----
+// ComputeVelocities of fg_transport (Kernels.cu:1193-1210; vtheta comes from
+// the azimuthal sweep) and what the reference's whole-array copies leave in the
+// ghost ring: the shifted fields 0, DENSINT the density's ghost values.
+struct close_args {
+  double *vr, *vt, *dens, *densint, *energy, *mom[4];
+  const double *xvt;
+  int nr, ns, adiabatic;
+};
+__global__ __launch_bounds__(256) void k_transport_close(close_args a) {
+  const int i = blockIdx.y, j = blockIdx.x * 256 + threadIdx.x, ns = a.ns;
+  if (j >= ns) return;
+  const long l = (long)i * ns + j;
+  if (i == a.nr) {
+    a.densint[l] = a.dens[l];
+    a.dens[l] = 0.0;
+    for (int q = 0; q < 4; q++) a.mom[q][l] = 0.0;
+    if (a.adiabatic) a.energy[l] = 0.0;
+    return;
+  }
+  a.vr[l] = i > 0 ? (a.mom[0][l - ns] + a.mom[1][l]) / (a.dens[l] + a.dens[l - ns] + 1e-20) : 0.0;
+  a.vt[l] = a.xvt[l];
+}
+
+// Transport (TransportEuler.cu:30) with the fused path's sweeps: three
+// launches instead of one per quantity and step (86 with the copies), and the
+// fields that the routines leave.  9 + 9 + 3 us at 128 x 384, 18 + 18 + 6 us at
+// 384 x 1152; bound as the fused path's sweeps are.  A 128 x 384 substep with
+// an open edge went from 393 to 121 us with it, one wait for all of a substep's
+// reductions, and results that the kernels write to host memory.
+fg_status fg_transport_sweeps(fg_ctx *c, double dt, double omega_frame) {
+  const int nr = c->nr, ns = c->ns;
+  const bool adi = c->p.adiabatic;
+  trad_args ta{};
+  ta.dens = c->f[FG_DENS];
+  ta.vr = c->f[FG_VRAD];
+  ta.vt = c->f[FG_VTHETA];
+  ta.energy = adi ? c->f[FG_ENERGY] : nullptr;
+  for (int q = 0; q < 6; q++) ta.out[q] = c->sw[q];
+  ta.vmed = c->VMed;
+  ta.lost = c->p.open_inner ? c->LostByDisk : nullptr;
+  ta.t = c->t;
+  ta.dt = dt;
+  ta.omega_frame = omega_frame;
+  ta.nr = nr;
+  ta.ns = ns;
+  ta.nstrips = (ns + TRAD_TPB - 1) / TRAD_TPB;
+  ta.band = trad_band(c, ta.nstrips);
+  const dim3 gt(nr + ta.nstrips * ((nr + ta.band - 1) / ta.band));
+  auto trad = adi ? (c->shared_faces ? k_trad<6, true, false> : k_trad<6, true, true>)
+                  : (c->shared_faces ? k_trad<5, true, false> : k_trad<5, true, true>);
+  hipLaunchKernelGGL(trad, gt, dim3(TRAD_TPB), 0, c->stream, ta);
+  FG_LAUNCH_CHECK();
+  taz_args za{};
+  za.vt = c->f[FG_VTHETA];
+  za.vmed = c->VMed;
+  for (int q = 0; q < 6; q++) za.q[q] = c->sw[q];
+  za.xd = c->f[FG_DENS];
+  za.xvt = c->sw[6];
+  za.xrmp = c->f[FG_RADMOMP];
+  za.xrmm = c->f[FG_RADMOMM];
+  za.xtmp = c->f[FG_THETAMOMP];
+  za.xtmm = c->f[FG_THETAMOMM];
+  za.xe = c->f[FG_ENERGY];
+  za.xdint = c->f[FG_DENSINT];
+  za.xres = c->f[FG_VTHETARES];
+  za.nshift = c->Nshift;
+  za.t = c->t;
+  za.dt = dt;
+  za.omega_frame = omega_frame;
+  za.nr = nr;
+  za.ns = ns;
+  za.fast = c->p.fast_transport;
+  const dim3 gz((ns + TAZW_P64 - 1) / TAZW_P64, nr);
+  hipLaunchKernelGGL(adi ? k_tazw_full<6> : k_tazw_full<5>, gz, dim3(64), 0, c->stream, za);
+  FG_LAUNCH_CHECK();
+  close_args ca;
+  ca.vr = c->f[FG_VRAD];
+  ca.vt = c->f[FG_VTHETA];
+  ca.dens = c->f[FG_DENS];
+  ca.densint = c->f[FG_DENSINT];
+  ca.energy = c->f[FG_ENERGY];
+  ca.mom[0] = c->f[FG_RADMOMP];
+  ca.mom[1] = c->f[FG_RADMOMM];
+  ca.mom[2] = c->f[FG_THETAMOMP];
+  ca.mom[3] = c->f[FG_THETAMOMM];
+  ca.xvt = c->sw[6];
+  ca.nr = nr;
+  ca.ns = ns;
+  ca.adiabatic = adi;
+  hipLaunchKernelGGL(k_transport_close, dim3((ns + 255) / 256, nr + 1), dim3(256), 0, c->stream, ca);
+  FG_LAUNCH_CHECK();
   return FG_OK;
 }
 

@@ -28,6 +28,15 @@ void fg_set_error(const char *fmt, ...);
 // the fused results are in (fg_fused.hip)
 fg_status fg_fused_planet_force_async(fg_ctx *c, int k, double x, double y, double rs);
 void fg_fused_planet_force(const fg_ctx *c, int k, double out2[2]);
+// a per-routine substep's reductions without their waits (fg_steps.hip,
+// fg_reduce.hip): the disk force on the star (k < 0) or planet k, and the mass
+// lost in the transport
+fg_status fg_cfl_launch(fg_ctx *c, double DeltaT);
+fg_status fg_cfl_result(fg_ctx *c, int *ncfl);
+fg_status fg_disk_force_launch(fg_ctx *c, int k, double x, double y, double rs);
+void fg_disk_force_result(const fg_ctx *c, int k, double out2[2]);
+fg_status fg_transport_launch(fg_ctx *c, double dt, double omega_frame);
+double fg_lost_mass_result(const fg_ctx *c);
 
 namespace {
 
@@ -1137,31 +1146,41 @@ extern "C" fg_status fg_sim_substep(fg_sim *s, int *closed) {
   double dt = s->dt;
   s->MassTaper = s->PhysicalTime / (d.MASSTAPER * 2.0 * M_PI);
   s->MassTaper = (s->MassTaper > 1.0 ? 1.0 : pow(sin(s->MassTaper * M_PI / 2.0), 2.0));
-  if (d.IsDisk && !d.SloppyCFL) {
-    int cfl = 1;
-    CHECK(fg_cfl(c, d.DT - s->dtemp, &cfl));
-    s->last_cfl = cfl;
-    dt = (d.DT - s->dtemp) / (double)cfl;
-    s->dt = dt;
+  // the CFL count and the disk forces on the star and the planets all come from
+  // the state as it is: one wait for them together
+  Planets &p = s->ps;
+  if (d.IsDisk) {
+    if (!d.SloppyCFL) CHECK(fg_cfl_launch(c, d.DT - s->dtemp));
+    CHECK(fg_disk_force_launch(c, -1, 0.0, 0.0, 0.0));
+    for (int k = 0; k < p.nb; k++) {
+      if (!p.feeldisk[k]) continue;
+      const double x = p.x[k], y = p.y[k];
+      CHECK(fg_disk_force_launch(c, k, x, y, planet_smoothing(s, sqrt(x * x + y * y), p.mass[k], true)));
+    }
+    CHECK(fg_sync(c));
+    if (!d.SloppyCFL) {
+      int cfl = 1;
+      CHECK(fg_cfl_result(c, &cfl));
+      s->last_cfl = cfl;
+      dt = (d.DT - s->dtemp) / (double)cfl;
+      s->dt = dt;
+    }
   }
   s->dtemp += dt;
   double dopa[2] = {0.0, 0.0};
   if (d.Corotating) psys_info(s, 1);
   if (d.IsDisk) {
-    CHECK(fg_disk_force(c, 0.0, 0.0, 0.0, dopa));
+    fg_disk_force_result(c, -1, dopa);
     s->IndirectX = d.Indirect_Term ? -dopa[0] : 0.0;
     s->IndirectY = d.Indirect_Term ? -dopa[1] : 0.0;
     fg_planet_pot pl[FG_MAX_PLANETS];
     int nb = potential_planets(s, pl);
     CHECK(fg_potential(c, pl, nb, s->IndirectX, s->IndirectY));
     // AdvanceSystemFromDisk, Pframeforce.cu:97-121
-    Planets &p = s->ps;
     for (int k = 0; k < p.nb; k++) {
       if (!p.feeldisk[k]) continue;
-      double m = p.mass[k], x = p.x[k], y = p.y[k], r = sqrt(x * x + y * y);
-      double smoothing = planet_smoothing(s, r, m, true);
       double gamma[2];
-      CHECK(fg_disk_force(c, x, y, smoothing, gamma));
+      fg_disk_force_result(c, k, gamma);
       p.vx[k] += dt * gamma[0];
       p.vy[k] += dt * gamma[1];
       p.vx[k] += dt * s->IndirectX;
@@ -1177,17 +1196,19 @@ extern "C" fg_status fg_sim_substep(fg_sim *s, int *closed) {
   }
   rotate_psys(s, s->OmegaFrame * dt);
   if (d.IsDisk) {
-    double lost = 0.0;
     CHECK(fg_boundary(c, dt, s->OmegaFrame));
     CHECK(fg_pressure(c));
     CHECK(fg_substep1(c, dt, s->OmegaFrame));
     CHECK(fg_substep2(c, dt));
     CHECK(fg_boundary(c, dt, s->OmegaFrame));
     if (d.Adiabatic) CHECK(fg_substep3(c, dt));
-    CHECK(fg_transport(c, dt, s->OmegaFrame, &lost));
-    s->LostMass += lost;
+    CHECK(fg_transport_launch(c, dt, s->OmegaFrame));
     CHECK(fg_boundary(c, dt, s->OmegaFrame));
     CHECK(fg_temperature(c));
+    if (d.OpenInner) {
+      CHECK(fg_sync(c));
+      s->LostMass += fg_lost_mass_result(c);
+    }
     CHECK(substep_diagnostics(s));
   }
   s->nsub++;

@@ -26,6 +26,15 @@ fg_status fg_noalloc_setup(int device);
 fg_status fg_sg_fused(fg_ctx *c, double dt, double *kick_r, double *kick_t);
 // alpha viscosity of the current sound speed into nu_out (fg_steps.hip)
 fg_status fg_viscosity_into(fg_ctx *c, double *nu_out);
+// the sweeps of the per-routine transport (fg_fused.hip): momenta, DENSINT,
+// VTHETARES, Sigma, energy, velocities; lost mass per sector of an open edge
+fg_status fg_transport_sweeps(fg_ctx *c, double dt, double omega_frame);
+// fg_cfl, fg_disk_force and fg_transport without their waits: launched, and
+// their results read from h_out / h_cfl once the stream is idle
+fg_status fg_cfl_launch(fg_ctx *c, double DeltaT);
+fg_status fg_cfl_result(fg_ctx *c, int *ncfl);
+fg_status fg_disk_force_async(fg_ctx *c, const double *dens, double x, double y, double rs, double *out_dev);
+fg_status fg_transport_launch(fg_ctx *c, double dt, double omega_frame);
 
 // Result block of the fused path (fg_ctx::h_fused, coherent pinned host
 // memory the final kernels write straight into): [0..1] star force,
@@ -38,6 +47,9 @@ fg_status fg_viscosity_into(fg_ctx *c, double *nu_out);
 // so the host can wait for the results by watching that slot.
 #define FG_FUSED_PF_SLOT 8
 #define FG_FUSED_SEQ_SLOT 5
+// first planet slot of fg_ctx::h_out, and its size
+#define FG_OUT_PF 8
+#define FG_OUT_SLOTS (FG_OUT_PF + 2 * FG_MAX_PLANETS)
 #define FG_FUSED_SLOTS (FG_FUSED_PF_SLOT + 2 * FG_MAX_PLANETS)
 #define FG_FUSED_CFL_SLOT 6
 #define FG_FUSED_CRASH_SLOT 7
@@ -124,8 +136,9 @@ struct fg_ctx {
 
   // evolved state and per-substep fields, (nr+1)*ns doubles each
   double *f[FG_NFIELDS];
-  // remaining work arrays of the per-routine path
-  double *DRR, *DPP, *DRP, *Work, *QRStar, *DensStar, *dq, *TempShift, *Vradial, *Vazimutal;
+  // per-routine transport: the quantities between the radial and the azimuthal
+  // sweep (momenta, energy, Sigma), and vtheta before it replaces the old one
+  double *sw[7];
   // ring arrays (nr+1)
   double *Vmoy, *newDT, *DT1D, *VMed, *nu, *cs_mean, *sgacc_mean;
   // fused path: the previous self-gravity evaluation's ring means (the
@@ -134,21 +147,21 @@ struct fg_ctx {
   // takes over from nu after the next substep's first damping pass
   double *sgacc_prev, *nu_next;
   int nu_pending;
-  int *Nshift, *NoSplit;
+  int *Nshift;
+  // every ring's outer face is the next ring's inner one (Rsup[i] == Rinf[i + 1])
+  int shared_faces;
   double *LostByDisk;  // ns
   // reduction scratch
   double *red_partial;  // 2 * FG_RED_BLOCKS
-  double *red_out;      // [0..1] force, [2] lost mass, [3] circumplanetary mass, [4..5] ring means,
-                        // [6] fused path's CFL count
-  int *cfl_out;         // [0] CFL count
-  double *h_out;        // pinned host mirror of red_out (4 doubles) + CFL
-  int *h_cfl;
+  // results of the per-routine reductions, coherent pinned host memory that the
+  // final kernels write straight into (red_out / cfl_out: device aliases)
+  double *h_out, *red_out;  // [0..1] force, [2] lost mass, [3] circumplanetary mass, from FG_OUT_PF the
+                            // disk force on each planet (two per planet)
+  int *h_cfl, *cfl_out;     // [0] CFL count, [1] crash flag
   // self-gravity complex buffers: 2*nr x ns interleaved complex
   double *sg_Sr, *sg_St, *sg_Krc, *sg_Ktc, *sg_Gr, *sg_Gt, *sg_tmp;
   int sg_kernel_ready;
   fg_fft_plan *fft_row, *fft_col;  // FFT plans of the NSEC rows and 2*NRAD columns
-  // FP32 bulk mirrors (precision mode)
-  float *f32[8];
   // host copies of ring values the host-side parts of a routine need
   std::vector<double> h_Rmed, h_Rinf, h_SigmaMed, h_EnergyMed, h_vtheta_arg;
   double lr01, lr12;  // log(Rmed0/Rmed1), log(Rmed1/Rmed2), Kernels.cu:93-94

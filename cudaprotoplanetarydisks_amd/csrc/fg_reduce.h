@@ -131,16 +131,6 @@ struct cpm_src {
   }
 };
 
-struct array_src {
-  const double *a, *b;  // b may be NULL
-  static constexpr bool kRow = false;
-  template <bool NARROW = false>
-  __device__ __forceinline__ void operator()(long e, double &fx, double &fy) const {
-    fx = a[e];
-    fy = b ? b[e] : 0.0;
-  }
-};
-
 // block blk of B (a RED_TPB-thread workgroup); partial[blk] and
 // partial[B + blk] receive the x and y block sums
 // CH summand rows are staged per round (CH * 64 / RED_TPB per thread).  A

@@ -28,9 +28,37 @@ static fg_status dreduce(fg_ctx *c, Src src, long n, double *out_dev, int two, i
   return FG_OK;
 }
 
-fg_status fg_reduce_array_internal(fg_ctx *c, const double *in, int n, double *result_dev) {
-  array_src src{in, nullptr};
-  return dreduce(c, src, n, result_dev, 0, 0);
+// DeviceReduce of one ring of n <= 8192 values (global memory or LDS) by one
+// workgroup: block b of the original takes elements 64 b + t and 64 b + t + 32
+// (64 B is at least n, so one round), a half-wave each here, and thread 0 adds
+// the blocks that have elements in order.  part: LDS, n / 64 + 1 values.  The
+// result is thread 0's.
+__device__ __forceinline__ double ring_dreduce(const double *a, int n, double *part) {
+  const int t = threadIdx.x & 31, nb = (n + 63) / 64;
+  for (int b = threadIdx.x >> 5; b < nb; b += blockDim.x >> 5) {
+    const int e = 64 * b + t;
+    double acc = 0.0;
+    if (e < n) {
+      acc += a[e];
+      if (e + 32 < n) acc += a[e + 32];
+    }
+    for (int off = 16; off > 0; off >>= 1) acc += __shfl_down(acc, off, 32);
+    if (t == 0) part[b] = acc;
+  }
+  __syncthreads();
+  return threadIdx.x == 0 ? seq_sum_lds(part, nb) : 0.0;
+}
+
+__global__ __launch_bounds__(1024) void k_ring_sum(const double *ring, int n, double *out) {
+  __shared__ double part[129];
+  const double s = ring_dreduce(ring, n, part);
+  if (threadIdx.x == 0) *out = s;
+}
+
+fg_status fg_ring_sum_async(fg_ctx *c, const double *ring, double *out_dev) {
+  hipLaunchKernelGGL(k_ring_sum, dim3(1), dim3(1024), 0, c->stream, ring, c->ns, out_dev);
+  FG_LAUNCH_CHECK();
+  return FG_OK;
 }
 
 fg_status fg_disk_force_async(fg_ctx *c, const double *dens, double x, double y, double rs, double *out_dev) {
@@ -38,13 +66,24 @@ fg_status fg_disk_force_async(fg_ctx *c, const double *dens, double x, double y,
   return dreduce(c, src, (long)c->nr * c->ns, out_dev, 1, 1);
 }
 
+// the disk force on the star (k < 0) or planet k of a per-routine substep,
+// read once the stream is idle
+fg_status fg_disk_force_launch(fg_ctx *c, int k, double x, double y, double rs) {
+  return fg_disk_force_async(c, c->f[FG_DENS], x, y, rs, c->red_out + (k < 0 ? 0 : FG_OUT_PF + 2 * k));
+}
+void fg_disk_force_result(const fg_ctx *c, int k, double out2[2]) {
+  const double *h = c->h_out + (k < 0 ? 0 : FG_OUT_PF + 2 * k);
+  out2[0] = h[0];
+  out2[1] = h[1];
+}
+double fg_lost_mass_result(const fg_ctx *c) { return c->h_out[2]; }
+
 extern "C" fg_status fg_disk_force(fg_ctx *c, double x, double y, double rsmoothing, double *out2) {
   if (!c || !out2) {
     fg_set_error("fg_disk_force: NULL argument");
     return FG_E_INVALID;
   }
   if (fg_status s = fg_disk_force_async(c, c->f[FG_DENS], x, y, rsmoothing, c->red_out)) return s;
-  FG_HIP(hipMemcpyAsync(c->h_out, c->red_out, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   FG_HIP(hipStreamSynchronize(c->stream));
   out2[0] = c->h_out[0];
   out2[1] = c->h_out[1];
@@ -179,97 +218,115 @@ extern "C" fg_status fg_circumplanetary_mass(fg_ctx *c, double xpl, double ypl, 
     return FG_E_INVALID;
   }
   if (fg_status s = fg_circumplanetary_mass_async(c, xpl, ypl, hill_radius, c->red_out + 3)) return s;
-  FG_HIP(hipMemcpyAsync(c->h_out + 3, c->red_out + 3, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   FG_HIP(hipStreamSynchronize(c->stream));
   *out = c->h_out[3];
   return FG_OK;
 }
 
 // ---- non-reflecting boundary (SideEuler.cu:45-100) -------------------
-// Ring gathers and their DeviceReduce means, then the two shifted-copy
-// kernels and the mean correction.
-__global__ void k_nr_copy(double *dens, double *energy, int i_angle, int ns) {
-  int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= ns) return;
-  // ring 0 <- ring 1 shifted by i_angle (wrapped modulo NSEC)
-  long dst = ((j + i_angle) % ns + ns) % ns;
-  dens[dst] = dens[ns + j];
-  energy[dst] = energy[ns + j];
+// One workgroup per edge does all of it: the ring means of c_s (each
+// DeviceReduce(...)/NSEC of SideEuler.cu:84-99 over one ring) and the shift
+// they give, the edge ring of Sigma and energy copied shifted from its
+// neighbour (Kernels.cu:534-573, wrapped modulo NSEC) and brought to its
+// initial mean (Kernels.cu:592-607), and vrad (Kernels.cu:575-589, bounded to
+// j < NSEC).  The two edges touch different rings from NRAD = 4 on; a disk of
+// three rings runs them one after the other.  Bound: a dozen dependent
+// barriers and memory round trips.  As one launch per ring sum and copy, with
+// the host computing the shifts, a boundary pass was 22 launches and four
+// waits; this is 12 us at NSEC = 1152, and a 384 x 1152 substep with three of
+// them went from 605 to 126 us with it and fg_transport's sweeps.
+struct nr_args {
+  double *dens, *energy, *vr;
+  const double *cs;
+  // inner, outer edge: pow(Rinf, -1.5) - 1 and the ring spacing of the shift's
+  // angle, Sigma of vrad's ring, Sigma and energy means of the edge ring
+  double num[2], width[2], sigma_v[2], sigma0[2], energy0[2];
+  int nr, ns;
+};
+
+// (int)x as the host converts it: out of range and NaN give INT_MIN
+__device__ __forceinline__ int nr_to_int(double x) {
+  return (x > -2147483649.0 && x < 2147483648.0) ? (int)x : (int)0x80000000;
 }
 
-__global__ void k_nr_copy_outer(double *dens, double *energy, int i_angle2, int nr, int ns) {
-  int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= ns) return;
-  const long ii = nr - 1;
-  // ring NRAD-1 <- ring NRAD-2 shifted by -i_angle2 (wrapped modulo NSEC)
-  long src = (ii - 1) * ns + ((j - i_angle2) % ns + ns) % ns;
-  dens[ii * ns + j] = dens[src];
-  energy[ii * ns + j] = energy[src];
+__device__ __forceinline__ void nr_edge(const nr_args &a, int edge, double *ring, double *part) {
+  __shared__ double s_sum[2];
+  const int nr = a.nr, ns = a.ns, tid = threadIdx.x;
+  // rings of the edge, its neighbour, and the one whose vrad is reflected
+  const long e = edge ? nr - 1 : 0, n = edge ? nr - 2 : 1;
+  for (int q = 0; q < 2; q++) {  // c_s means, in the order of SideEuler.cu
+    const double s = ring_dreduce(a.cs + (q ? n : e) * ns, ns, part);
+    if (tid == 0) s_sum[q] = s / ns;
+    __syncthreads();
+  }
+  double dangle = a.num[edge] / (.5 * (s_sum[0] + s_sum[1]));
+  dangle *= a.width[edge];
+  const int shift = nr_to_int(dangle / 2.0 / FG_PI * (double)ns + .5);
+  for (int f = 0; f < 2; f++) {
+    double *q = f ? a.energy : a.dens;
+    __syncthreads();
+    for (int j = tid; j < ns; j += blockDim.x) {
+      if (edge == 0)
+        ring[((j + shift) % ns + ns) % ns] = q[n * ns + j];
+      else
+        ring[j] = q[n * ns + ((j - shift) % ns + ns) % ns];
+    }
+    __syncthreads();
+    const double s = ring_dreduce(ring, ns, part);
+    if (tid == 0) s_sum[0] = s / ns;
+    __syncthreads();
+    const double add = (f ? a.energy0[edge] : a.sigma0[edge]) - s_sum[0];
+    for (int j = tid; j < ns; j += blockDim.x) q[e * ns + j] = ring[j] + add;
+  }
+  const double sm = a.sigma_v[edge];
+  for (int j = tid; j < ns; j += blockDim.x) {
+    if (edge == 0) {
+      const double Vrad_med = -a.cs[ns + j] * (a.dens[ns + j] - sm) / sm;
+      a.vr[ns + j] = 2.0 * Vrad_med - a.vr[2L * ns + j];
+    } else {
+      const long i = nr - 1;
+      const double Vrad_med = a.cs[i * ns + j] * (a.dens[(i - 1) * ns + j] - sm) / sm;
+      a.vr[i * ns + j] = 2. * Vrad_med - a.vr[(i - 1) * ns + j];
+    }
+  }
 }
 
-// NonReflectingBoundaryKernel2, Kernels.cu:575-589, bounded to j < NSEC
-__global__ void k_nr_vrad(double *vr, const double *dens, const double *cs, double sm1, double sm2, int nr, int ns) {
-  int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= ns) return;
-  long i = 1;
-  double Vrad_med = -cs[i * ns + j] * (dens[i * ns + j] - sm1) / sm1;
-  vr[i * ns + j] = 2.0 * Vrad_med - vr[(i + 1) * ns + j];
-  i = nr - 1;
-  Vrad_med = cs[i * ns + j] * (dens[(i - 1) * ns + j] - sm2) / sm2;
-  vr[i * ns + j] = 2. * Vrad_med - vr[(i - 1) * ns + j];
-}
-
-// MinusMeanKernel, Kernels.cu:592-607
-__global__ void k_nr_minus_mean(double *dens, double *energy, double a0, double a1, double e0, double e1, int nr,
-                                int ns) {
-  int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= ns) return;
-  dens[j] += a0;
-  energy[j] += e0;
-  long l = (long)(nr - 1) * ns + j;
-  dens[l] += a1;
-  energy[l] += e1;
-}
-
-static fg_status ring_means(fg_ctx *c, const double *f0, const double *f1, double *m0, double *m1) {
-  // each DeviceReduce(...)/NSEC of SideEuler.cu:84-99 over one ring
-  if (fg_status s = fg_reduce_array_internal(c, f0, c->ns, c->red_out + 4)) return s;
-  if (fg_status s = fg_reduce_array_internal(c, f1, c->ns, c->red_out + 5)) return s;
-  FG_HIP(hipMemcpyAsync(c->h_out + 4, c->red_out + 4, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  FG_HIP(hipStreamSynchronize(c->stream));
-  *m0 = c->h_out[4] / c->ns;
-  *m1 = c->h_out[5] / c->ns;
-  return FG_OK;
+__global__ __launch_bounds__(1024) void k_nr_edges(nr_args a) {
+  extern __shared__ double ring[];
+  __shared__ double part[129];
+  if (gridDim.x == 2) {
+    nr_edge(a, blockIdx.x, ring, part);
+  } else {
+    nr_edge(a, 0, ring, part);
+    __syncthreads();
+    nr_edge(a, 1, ring, part);
+  }
 }
 
 fg_status fg_nonreflecting_internal(fg_ctx *c) {
   const int nr = c->nr, ns = c->ns;
-  double *cs = c->f[FG_SOUNDSPEED], *dens = c->f[FG_DENS], *en = c->f[FG_ENERGY], *vr = c->f[FG_VRAD];
-  double cs0_r, cs1_r, csnrm1_r, csnrm2_r;
-  if (fg_status s = ring_means(c, cs, cs + ns, &cs0_r, &cs1_r)) return s;
-  if (fg_status s = ring_means(c, cs + (long)(nr - 1) * ns, cs + (long)(nr - 2) * ns, &csnrm1_r, &csnrm2_r)) return s;
-  const double PI = FG_PI;
   const std::vector<double> &Rinf = c->h_Rinf, &Rmed = c->h_Rmed;
-  int i = 1;
-  double dangle = (pow(Rinf[i], -1.5) - 1.0) / (.5 * (cs0_r + cs1_r));
-  dangle *= (Rmed[i] - Rmed[i - 1]);
-  int i_angle = (int)(dangle / 2.0 / PI * (double)ns + .5);
-  i = nr - 1;
-  double dangle2 = (pow(Rinf[i - 1], -1.5) - 1.0) / (.5 * (csnrm1_r + csnrm2_r));
-  dangle2 *= (Rmed[i] - Rmed[i - 1]);
-  int i_angle2 = (int)(dangle2 / 2.0 / PI * (double)ns + .5);
-  dim3 g(fg_blocks(ns, 256)), b(256);
-  hipLaunchKernelGGL(k_nr_copy, g, b, 0, c->stream, dens, en, i_angle, ns);
-  FG_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_nr_copy_outer, g, b, 0, c->stream, dens, en, i_angle2, nr, ns);
-  FG_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_nr_vrad, g, b, 0, c->stream, vr, dens, cs, c->h_SigmaMed[1], c->h_SigmaMed[nr - 2], nr, ns);
-  FG_LAUNCH_CHECK();
-  double md0, md1, me0, me1;
-  if (fg_status s = ring_means(c, dens, dens + (long)(nr - 1) * ns, &md0, &md1)) return s;
-  if (fg_status s = ring_means(c, en, en + (long)(nr - 1) * ns, &me0, &me1)) return s;
-  hipLaunchKernelGGL(k_nr_minus_mean, g, b, 0, c->stream, dens, en, c->h_SigmaMed[0] - md0,
-                     c->h_SigmaMed[nr - 1] - md1, c->h_EnergyMed[0] - me0, c->h_EnergyMed[nr - 1] - me1, nr, ns);
+  nr_args a;
+  a.dens = c->f[FG_DENS];
+  a.energy = c->f[FG_ENERGY];
+  a.vr = c->f[FG_VRAD];
+  a.cs = c->f[FG_SOUNDSPEED];
+  a.num[0] = pow(Rinf[1], -1.5) - 1.0;
+  a.width[0] = Rmed[1] - Rmed[0];
+  a.num[1] = pow(Rinf[nr - 2], -1.5) - 1.0;
+  a.width[1] = Rmed[nr - 1] - Rmed[nr - 2];
+  a.sigma_v[0] = c->h_SigmaMed[1];
+  a.sigma_v[1] = c->h_SigmaMed[nr - 2];
+  a.sigma0[0] = c->h_SigmaMed[0];
+  a.sigma0[1] = c->h_SigmaMed[nr - 1];
+  a.energy0[0] = c->h_EnergyMed[0];
+  a.energy0[1] = c->h_EnergyMed[nr - 1];
+  a.nr = nr;
+  a.ns = ns;
+  if (ns > 7000)  // ring and partial sums beyond the 64 KB a launch gets unasked
+    FG_HIP(hipFuncSetAttribute((const void *)k_nr_edges, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               ns * (int)sizeof(double)));
+  hipLaunchKernelGGL(k_nr_edges, dim3(nr > 3 ? 2 : 1), dim3(1024), (size_t)ns * sizeof(double), c->stream, a);
   FG_LAUNCH_CHECK();
   return FG_OK;
 }

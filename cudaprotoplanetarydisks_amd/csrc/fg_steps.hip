@@ -71,9 +71,7 @@ __global__ void k_ring_mean(double *out, const double *field, int nr, int ns) {
   for (int j = threadIdx.x; j < ns; j += blockDim.x) ring[j] = field[(long)i * ns + j];
   __syncthreads();
   if (threadIdx.x == 0) {
-    double sum = 0.0;
-    for (int j = 0; j < ns; j++) sum += ring[j];
-    out[i] = sum / (double)ns;
+    out[i] = seq_sum_lds(ring, ns) / (double)ns;
   }
 }
 
@@ -192,8 +190,7 @@ __global__ void k_substep1(double *vradint, double *vthetaint, const double *P, 
 
 // ViscousTermsKernel, Kernels.cu:733-771
 __global__ void k_viscous_terms(const double *Vr, const double *Vt, const double *dens, const double *nu,
-                                double *DRR, double *DPP, double *DRP, double *divV, double *TRR, double *TPP,
-                                double *TRP, fg_dev_tables t, int nr, int ns) {
+                                double *divV, double *TRR, double *TPP, double *TRP, fg_dev_tables t, int nr, int ns) {
   CELLS(0, nr)
   const double invdphi = t.invdphi;
   const double onethird = 1.0 / 3.0;
@@ -201,15 +198,12 @@ __global__ void k_viscous_terms(const double *Vr, const double *Vt, const double
   double dpp = (Vt[JP] - Vt[l]) * invdphi * t.invRmed[i] + 0.5 * (Vr[l + ns] + Vr[l]) * t.invRmed[i];
   double dv = (Vr[l + ns] * t.Rsup[i] - Vr[l] * t.Rinf[i]) * t.invdiffRsup[i] * t.invRmed[i];
   dv += (Vt[JP] - Vt[l]) * invdphi * t.invRmed[i];
-  DRR[l] = drr;
-  DPP[l] = dpp;
   divV[l] = dv;
   TRR[l] = 2.0 * dens[l] * nu[i] * (drr - onethird * dv);
   TPP[l] = 2.0 * dens[l] * nu[i] * (dpp - onethird * dv);
   if (i > 0) {
     double drp = 0.5 * (t.Rinf[i] * (Vt[l] * t.invRmed[i] - Vt[l - ns] * t.invRmed[i - 1]) * t.invdiffRmed[i] +
                         (Vr[l] - Vr[JM]) * invdphi * t.invRinf[i]);
-    DRP[l] = drp;
     TRP[l] = 2.0 * 0.25 * (dens[l] + dens[l - ns] + dens[JM] + dens[JM - ns]) * nu[i] * drp;
   }
 }
@@ -241,19 +235,31 @@ __global__ void k_substep2(double *qr, double *qt, const double *dens, const dou
 }
 
 // "kernel", Kernels.cu:438-479
-__global__ void k_host(double *vrnew, double *vtnew, double *eint, const double *dens, const double *vri,
-                       const double *vti, const double *qr, const double *qt, const double *energy, fg_dev_tables t,
+// with ActualiseGasVrad/Vtheta (SourceEuler.cu:492-503): the new velocities,
+// rows 0 and NRAD as they were in the New fields, also into Vrad / Vtheta
+__global__ void k_host(double *vr, double *vt, double *vrnew, double *vtnew, double *eint, const double *dens,
+                       const double *vri, const double *vti, const double *qr, const double *qt, const double *energy, fg_dev_tables t,
                        double dt, int nr, int ns, int adiabatic) {
-  CELLS(0, nr)
+  CELLS(0, nr + 1)
+  if (i == nr) {
+    vr[l] = vrnew[l];
+    vt[l] = vtnew[l];
+    return;
+  }
+  double v = vrnew[l];
   if (i > 0) {
     double d = dens[l] + dens[l - ns];
     double densint = qr[l] - qr[l - ns];
-    vrnew[l] = vri[l] - dt * 2.0 / d * densint * t.invdiffRmed[i];
+    v = vri[l] - dt * 2.0 / d * densint * t.invdiffRmed[i];
+    vrnew[l] = v;
   }
+  vr[l] = v;
   const double invdxtheta = t.invdxtheta[i];
   double dens2 = dens[l] + dens[JM];
   double tempint = (qt[l] - qt[JM]);
-  vtnew[l] = vti[l] - dt * 2.0 / dens2 * tempint * invdxtheta;
+  const double w = vti[l] - dt * 2.0 / dens2 * tempint * invdxtheta;
+  vtnew[l] = w;
+  vt[l] = w;
   if (adiabatic)
     eint[l] = energy[l] - dt * qr[l] * (vri[l + ns] - vri[l]) * t.invdiffRsup[i] -
               dt * qt[l] * (vti[JP] - vti[l]) * invdxtheta;
@@ -275,10 +281,16 @@ __global__ void k_substep3a(double *qplus, const double *dens, const double *nu,
 // Substep3Kernel2, Kernels.cu:80-115.  lr01 = log(Rmed0/Rmed1),
 // lr12 = log(Rmed1/Rmed2) are host constants; the data-dependent log/exp
 // of the power-law extrapolation run on the device.
-__global__ void k_substep3b(double *enew, double *qplus, const double *dens, const double *eint, const double *divV,
-                            const double *nu, fg_dev_tables t, double dt, double gamma, double lr01, double lr12,
+// with ActualiseGasEnergy (SourceEuler.cu:362): also into Energy, the ghost row as
+// it was in EnergyNew
+__global__ void k_substep3b(double *energy, double *enew, double *qplus, const double *dens, const double *eint,
+                            const double *divV, const double *nu, fg_dev_tables t, double dt, double gamma, double lr01, double lr12,
                             int nr, int ns, int cooling) {
-  CELLS(0, nr)
+  CELLS(0, nr + 1)
+  if (i == nr) {
+    energy[l] = enew[l];
+    return;
+  }
   if (i == 0) {
     if (nu[nr - 1] != 0.0)
       qplus[l] = qplus[l + ns] * exp(log(qplus[l + ns] / qplus[l + 2 * ns]) * lr01 / lr12);
@@ -294,133 +306,9 @@ __global__ void k_substep3b(double *enew, double *qplus, const double *dens, con
           dt * t.CoolingTimeMed[i] * (qplus[l] - t.QplusMed[i] * dens[l] / t.SigmaMed[i]);
     den = dt + t.CoolingTimeMed[i] + (gamma - 1.0) * dt * t.CoolingTimeMed[i] * divV[l];
   }
-  enew[l] = num / den;
-}
-
-// --------------------------------------------------------- transport --
-// LRMomentaKernel, Kernels.cu:774-787
-__global__ void k_lr_momenta(double *rmp, double *rmm, double *tmp_, double *tmm, const double *dens,
-                             const double *vr, const double *vt, const double *Rmed, double omega_frame, int nr,
-                             int ns) {
-  CELLS(0, nr)
-  const double Rm = Rmed[i];
-  rmp[l] = dens[l] * vr[l + ns];
-  rmm[l] = dens[l] * vr[l];
-  tmp_[l] = dens[l] * (vt[JP] + Rm * omega_frame) * Rm;
-  tmm[l] = dens[l] * (vt[l] + Rm * omega_frame) * Rm;
-}
-
-// StarRadKernel, Kernels.cu:800-820
-__global__ void k_star_rad_dq(double *dq, const double *q, const double *invdiffRmed, int nr, int ns) {
-  CELLS(0, nr)
-  if (i == 0 || i == nr - 1)
-    dq[l] = 0.0;
-  else
-    dq[l] = vl_rad_slope(q[l - ns], q[l], q[l + ns], invdiffRmed[i], invdiffRmed[i + 1]);
-}
-
-// StarRadKernel2, Kernels.cu:822-838 (Rmed[nrad] is 0; it only ever
-// multiplies a zero slope)
-__global__ void k_star_rad_q(double *qstar, const double *q, const double *dq, const double *vr, const double *Rmed,
-                             double dt, int nr, int ns) {
-  CELLS(0, nr)
-  double qm = (i > 0) ? q[l - ns] : 0.0;
-  double dqm = (i > 0) ? dq[l - ns] : 0.0;
-  double rm = (i > 0) ? Rmed[i - 1] : 0.0;
-  qstar[l] = vl_rad_star(vr[l], dt, qm, q[l], dqm, dq[l], rm, Rmed[i], Rmed[i + 1], i);
-  if (i == 0) {
-    qstar[j] = 0.0;
-    qstar[(long)ns * nr + j] = 0.0;
-  }
-}
-
-// DivisePolarGridKernel, Kernels.cu:1018-1025
-__global__ void k_divise(double *work, const double *q, const double *densint, long n) {
-  long l = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (l < n) work[l] = q[l] / (densint[l] + 1e-20);
-}
-
-// VanLeerRadialKernel, Kernels.cu:1028-1046
-__global__ void k_vl_radial(double *q, double *lost, const double *qrstar, const double *densstar, const double *vr,
-                            fg_dev_tables t, double dt, int nr, int ns, int open_inner) {
-  CELLS(0, nr)
-  const double dtheta = t.dtheta;
-  double varq = dt * dtheta * t.Rinf[i] * qrstar[l] * densstar[l] * vr[l];
-  varq -= dt * dtheta * t.Rsup[i] * qrstar[l + ns] * densstar[l + ns] * vr[l + ns];
-  q[l] += varq * t.invSurf[i];
-  if (i == 0 && open_inner) lost[j] = varq;
-}
-
-// ComputeResidualsKernel, Kernels.cu:1084-1091
-__global__ void k_residual(double *vres, const double *vt, const double *vmed, int nr, int ns) {
-  CELLS(0, nr)
-  vres[l] = vt[l] - vmed[i];
-}
-
-// ComputeConstantResidualKernel, Kernels.cu:1094-1126 (Nshift written by
-// lane j == 0 of each ring only)
-__global__ void k_const_residual(double *vt, double *vres, int *nshift, int *nosplit, const double *vmed,
-                                 const double *invRmed, const double *Rmed, double dt, int nr, int ns, int fast) {
-  CELLS(0, nr)
-  double maxfrac = fast ? 1.0 : 0.0;
-  double invdt = 1.0 / dt;
-  double dpinvns = 2.0 * FG_PI / (double)ns;
-  double Ntilde = vmed[i] * invRmed[i] * dt * (double)ns / 2.0 / FG_PI;
-  double Nround = floor(Ntilde + 0.5);
-  long nitemp = (long)Nround;
-  if (j == 0) nshift[i] = (int)nitemp;
-  double v = (Ntilde - Nround) * Rmed[i] * invdt * dpinvns;
-  if (maxfrac < 0.5) {
-    if (j == 0) nosplit[i] = 1;
-    vres[l] += v;
-    v = 0.0;
-  } else if (j == 0)
-    nosplit[i] = 0;
-  vt[l] = v;
-}
-
-// StarThetaKernel, Kernels.cu:1129-1148
-__global__ void k_star_theta_dq(double *dq, const double *q, const double *invdxtheta, int nr, int ns) {
-  CELLS(0, nr)
-  dq[l] = vl_theta_slope(q[JM], q[l], q[JP], invdxtheta[i]);
-}
-
-// StarThetaKernel2, Kernels.cu:1151-1170
-__global__ void k_star_theta_q(double *qstar, const double *q, const double *dq, const double *v,
-                               const double *dxtheta, double dt, int nr, int ns) {
-  CELLS(0, nr)
-  qstar[l] = vl_theta_star(v[l], dt, q[JM], q[l], dq[JM], dq[l], dxtheta[i]);
-}
-
-// VanLeerThetaKernel, Kernels.cu:1049-1066
-__global__ void k_vl_theta(double *q, const double *qrstar, const double *densstar, const double *v,
-                           fg_dev_tables t, double dt, int nr, int ns) {
-  CELLS(0, nr)
-  double dxrad = (t.Rsup[i] - t.Rinf[i]) * dt;
-  double invsurf = t.invSurf[i];
-  double varq = dxrad * qrstar[l] * densstar[l] * v[l];
-  varq -= dxrad * qrstar[JP] * densstar[JP] * v[JP];
-  q[l] += varq * invsurf;
-}
-
-// AdvectSHIFTKernel, Kernels.cu:1173-1190
-__global__ void k_advect_shift(double *out, const double *in, const int *nshift, int nr, int ns) {
-  CELLS(0, nr)
-  int ji = (j - nshift[i]) % ns;
-  if (ji < 0) ji += ns;
-  out[l] = in[(long)i * ns + ji];
-}
-
-// ComputeVelocitiesKernel, Kernels.cu:1193-1210
-__global__ void k_compute_velocities(double *vr, double *vt, const double *dens, const double *Rmed,
-                                     const double *tmp_, const double *tmm, const double *rmp, const double *rmm,
-                                     double omega_frame, int nr, int ns) {
-  CELLS(0, nr)
-  if (i == 0)
-    vr[l] = 0.0;
-  else
-    vr[l] = (rmp[l - ns] + rmm[l]) / (dens[l] + dens[l - ns] + 1e-20);
-  vt[l] = (tmp_[JM] + tmm[l]) / (dens[l] + dens[JM] + 1e-15) / Rmed[i] - Rmed[i] * omega_frame;
+  const double e = num / den;
+  enew[l] = e;
+  energy[l] = e;
 }
 
 // ------------------------------------------------------------------ CFL --
@@ -454,8 +342,7 @@ __global__ void k_cfl_ring(double *vmoy, double *newdt, const double *vr, const 
   if (bad) *crash = 1;
   __syncthreads();
   if (threadIdx.x == 0) {
-    double m = 0.0;
-    for (int j = 0; j < ns; j++) m += ring[j];
+    double m = seq_sum_lds(ring, ns);
     m /= (double)ns;
     vmoy[i] = m;
     s_vmoy = m;
@@ -557,9 +444,7 @@ fg_status fg_viscosity_into(fg_ctx *c, double *nu_out) {
   return refresh_viscosity(c, nu_out);
 }
 
-extern "C" fg_status fg_cfl(fg_ctx *c, double DeltaT, int *ncfl) {
-  if (fg_status s = check(c)) return s;
-  if (!ncfl) return FG_E_INVALID;
+fg_status fg_cfl_launch(fg_ctx *c, double DeltaT) {
   const int nr = c->nr, ns = c->ns;
   size_t shm = (size_t)(ns + 256) * sizeof(double);
   hipLaunchKernelGGL(k_cfl_ring, dim3(nr), dim3(256), shm, c->stream, c->Vmoy, c->newDT, F(c, FG_VRAD),
@@ -570,16 +455,27 @@ extern "C" fg_status fg_cfl(fg_ctx *c, double DeltaT, int *ncfl) {
   hipLaunchKernelGGL(k_cfl_final, dim3(1), dim3(256), 0, c->stream, c->cfl_out, c->DT1D, c->Vmoy, c->newDT,
                      c->t.invRmed, c->t.dt1d_coef, DeltaT, nr);
   FG_LAUNCH_CHECK();
-  FG_HIP(hipMemcpyAsync(c->h_cfl, c->cfl_out, 2 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  FG_HIP(hipStreamSynchronize(c->stream));
-  if (c->h_cfl[1]) {  // reported once; the next pass over a bad state flags it again
-    FG_HIP(hipMemsetAsync(c->cfl_out + 1, 0, sizeof(int), c->stream));
+  return FG_OK;
+}
+
+fg_status fg_cfl_result(fg_ctx *c, int *ncfl) {
+  volatile int *h = c->h_cfl;
+  if (h[1]) {  // reported once; the next pass over a bad state flags it again
+    h[1] = 0;
     fg_set_error("crash: negative or non-finite density or energy");
     return FG_E_CRASH;
   }
-  if (fg_status s = fg_check_substep_results((double)c->h_cfl[0], nullptr)) return s;
-  *ncfl = c->h_cfl[0];
+  if (fg_status s = fg_check_substep_results((double)h[0], nullptr)) return s;
+  *ncfl = h[0];
   return FG_OK;
+}
+
+extern "C" fg_status fg_cfl(fg_ctx *c, double DeltaT, int *ncfl) {
+  if (fg_status s = check(c)) return s;
+  if (!ncfl) return FG_E_INVALID;
+  if (fg_status s = fg_cfl_launch(c, DeltaT)) return s;
+  FG_HIP(hipStreamSynchronize(c->stream));
+  return fg_cfl_result(c, ncfl);
 }
 
 static fg_status pack_planets(fg_planets_arg *P, const fg_planet_pot *pl, int nb, double ix, double iy) {
@@ -645,8 +541,8 @@ static fg_status viscous_terms(fg_ctx *c, const double *vr, const double *vt) {
   const int nr = c->nr, ns = c->ns;
   if (c->p.viscosity_alpha)
     if (fg_status s = fg_ring_mean_cs(c)) return s;
-  LAUNCH(k_viscous_terms, 0, nr, vr, vt, F(c, FG_DENS), c->nu, c->DRR, c->DPP, c->DRP, F(c, FG_DIVV),
-         F(c, FG_TAURR), F(c, FG_TAUPP), F(c, FG_TAURP), c->t, nr, ns);
+  LAUNCH(k_viscous_terms, 0, nr, vr, vt, F(c, FG_DENS), c->nu, F(c, FG_DIVV), F(c, FG_TAURR),
+         F(c, FG_TAUPP), F(c, FG_TAURP), c->t, nr, ns);
   return FG_OK;
 }
 
@@ -678,15 +574,11 @@ extern "C" fg_status fg_substep2(fg_ctx *c, double dt) {
   const int nr = c->nr, ns = c->ns;
   LAUNCH(k_substep2, 0, nr, F(c, FG_DENSINT), F(c, FG_TEMPERINT), F(c, FG_DENS), F(c, FG_VRADINT),
          F(c, FG_VTHETAINT), nr, ns);
-  LAUNCH(k_host, 0, nr, F(c, FG_VRADNEW), F(c, FG_VTHETANEW), F(c, FG_ENERGYINT), F(c, FG_DENS), F(c, FG_VRADINT),
-         F(c, FG_VTHETAINT), F(c, FG_DENSINT), F(c, FG_TEMPERINT), F(c, FG_ENERGY), c->t, dt, nr, ns,
-         c->p.adiabatic);
-  const size_t bytes = c->S * sizeof(double);
-  FG_HIP(hipMemcpyAsync(F(c, FG_VRAD), F(c, FG_VRADNEW), bytes, hipMemcpyDeviceToDevice, c->stream));
-  FG_HIP(hipMemcpyAsync(F(c, FG_VTHETA), F(c, FG_VTHETANEW), bytes, hipMemcpyDeviceToDevice, c->stream));
+  LAUNCH(k_host, 0, nr + 1, F(c, FG_VRAD), F(c, FG_VTHETA), F(c, FG_VRADNEW), F(c, FG_VTHETANEW),
+         F(c, FG_ENERGYINT), F(c, FG_DENS), F(c, FG_VRADINT), F(c, FG_VTHETAINT), F(c, FG_DENSINT),
+         F(c, FG_TEMPERINT), F(c, FG_ENERGY), c->t, dt, nr, ns, c->p.adiabatic);
   return FG_OK;
 }
-
 
 extern "C" fg_status fg_substep3(fg_ctx *c, double dt) {
   if (fg_status s = check(c)) return s;
@@ -696,108 +588,27 @@ extern "C" fg_status fg_substep3(fg_ctx *c, double dt) {
   LAUNCH(k_substep3a, 1, nr, F(c, FG_QPLUS), F(c, FG_DENS), c->nu, F(c, FG_TAURR), F(c, FG_TAURP), F(c, FG_TAUPP),
          F(c, FG_DIVV), nr, ns);
   const double lr01 = c->lr01, lr12 = c->lr12;
-  LAUNCH(k_substep3b, 0, nr, F(c, FG_ENERGYNEW), F(c, FG_QPLUS), F(c, FG_DENS), F(c, FG_ENERGYINT), F(c, FG_DIVV),
-         c->nu, c->t, dt, c->p.adiabatic_index, lr01, lr12, nr, ns, c->p.cooling);
-  FG_HIP(hipMemcpyAsync(F(c, FG_ENERGY), F(c, FG_ENERGYNEW), c->S * sizeof(double), hipMemcpyDeviceToDevice,
-                        c->stream));
+  LAUNCH(k_substep3b, 0, nr + 1, F(c, FG_ENERGY), F(c, FG_ENERGYNEW), F(c, FG_QPLUS), F(c, FG_DENS),
+         F(c, FG_ENERGYINT), F(c, FG_DIVV), c->nu, c->t, dt, c->p.adiabatic_index, lr01, lr12, nr, ns, c->p.cooling);
   return FG_OK;
 }
 
-fg_status fg_reduce_array_internal(fg_ctx *c, const double *in, int n, double *result_dev);
+fg_status fg_ring_sum_async(fg_ctx *c, const double *ring, double *out_dev);
 
-// ComputeStarRad (TransportEuler.cu:81-95) of q into qstar
-static fg_status star_rad(fg_ctx *c, const double *q, double *qstar, double dt) {
-  const int nr = c->nr, ns = c->ns;
-  LAUNCH(k_star_rad_dq, 0, nr, c->dq, q, c->t.invdiffRmed, nr, ns);
-  LAUNCH(k_star_rad_q, 0, nr, qstar, q, c->dq, F(c, FG_VRAD), c->t.Rmed, dt, nr, ns);
-  return FG_OK;
-}
-
-// VanLeerRadial (TransportEuler.cu:106-156)
-static fg_status van_leer_radial(fg_ctx *c, double *q, double dt) {
-  const int nr = c->nr, ns = c->ns;
-  long n = (long)nr * ns;
-  hipLaunchKernelGGL(k_divise, dim3(fg_blocks(n, TPB)), dim3(TPB), 0, c->stream, c->Work, q, F(c, FG_DENSINT), n);
-  FG_LAUNCH_CHECK();
-  if (fg_status s = star_rad(c, c->Work, c->QRStar, dt)) return s;
-  LAUNCH(k_vl_radial, 0, nr, q, c->LostByDisk, c->QRStar, c->DensStar, F(c, FG_VRAD), c->t, dt, nr, ns,
-         c->p.open_inner);
-  return FG_OK;
-}
-
-// ComputeStarTheta (TransportEuler.cu:261-269)
-static fg_status star_theta(fg_ctx *c, const double *q, const double *v, double *qstar, double dt) {
-  const int nr = c->nr, ns = c->ns;
-  LAUNCH(k_star_theta_dq, 0, nr, c->dq, q, c->t.invdxtheta, nr, ns);
-  LAUNCH(k_star_theta_q, 0, nr, qstar, q, c->dq, v, c->t.dxtheta, dt, nr, ns);
-  return FG_OK;
-}
-
-// VanLeerTheta (TransportEuler.cu:249-257)
-static fg_status van_leer_theta(fg_ctx *c, const double *v, double *q, double dt) {
-  const int nr = c->nr, ns = c->ns;
-  long n = (long)nr * ns;
-  hipLaunchKernelGGL(k_divise, dim3(fg_blocks(n, TPB)), dim3(TPB), 0, c->stream, c->Work, q, F(c, FG_DENSINT), n);
-  FG_LAUNCH_CHECK();
-  if (fg_status s = star_theta(c, c->Work, v, c->QRStar, dt)) return s;
-  LAUNCH(k_vl_theta, 0, nr, q, c->QRStar, c->DensStar, v, c->t, dt, nr, ns);
-  return FG_OK;
-}
-
-// QuantitiesAdvection (TransportEuler.cu:229-245)
-static fg_status quantities_advection(fg_ctx *c, const double *v, double dt) {
-  if (fg_status s = star_theta(c, F(c, FG_DENS), v, c->DensStar, dt)) return s;
-  FG_HIP(hipMemcpyAsync(F(c, FG_DENSINT), F(c, FG_DENS), c->S * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-  const int order[4] = {FG_RADMOMP, FG_RADMOMM, FG_THETAMOMP, FG_THETAMOMM};
-  for (int k = 0; k < 4; k++)
-    if (fg_status s = van_leer_theta(c, v, F(c, order[k]), dt)) return s;
-  if (c->p.adiabatic)
-    if (fg_status s = van_leer_theta(c, v, F(c, FG_ENERGY), dt)) return s;
-  return van_leer_theta(c, v, F(c, FG_DENS), dt);
-}
-
-static fg_status advect_shift(fg_ctx *c, double *q) {
-  const int nr = c->nr, ns = c->ns;
-  LAUNCH(k_advect_shift, 0, nr, c->TempShift, q, c->Nshift, nr, ns);
-  FG_HIP(hipMemcpyAsync(q, c->TempShift, c->S * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+fg_status fg_transport_launch(fg_ctx *c, double dt, double omega_frame) {
+  if (fg_status s = fg_transport_sweeps(c, dt, omega_frame)) return s;
+  // the mass that left through an open inner edge (TransportEuler.cu:77); the
+  // other edges' faces carry no flux
+  if (c->p.open_inner) return fg_ring_sum_async(c, c->LostByDisk, c->red_out + 2);
   return FG_OK;
 }
 
 extern "C" fg_status fg_transport(fg_ctx *c, double dt, double omega_frame, double *lost_mass) {
   if (fg_status s = check(c)) return s;
-  const int nr = c->nr, ns = c->ns;
-  LAUNCH(k_lr_momenta, 0, nr, F(c, FG_RADMOMP), F(c, FG_RADMOMM), F(c, FG_THETAMOMP), F(c, FG_THETAMOMM),
-         F(c, FG_DENS), F(c, FG_VRAD), F(c, FG_VTHETA), c->t.Rmed, omega_frame, nr, ns);
-  // OneWindRad
-  if (fg_status s = star_rad(c, F(c, FG_DENS), c->DensStar, dt)) return s;
-  FG_HIP(hipMemcpyAsync(F(c, FG_DENSINT), F(c, FG_DENS), c->S * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-  const int order[4] = {FG_RADMOMP, FG_RADMOMM, FG_THETAMOMP, FG_THETAMOMM};
-  for (int k = 0; k < 4; k++)
-    if (fg_status s = van_leer_radial(c, F(c, order[k]), dt)) return s;
-  if (c->p.adiabatic)
-    if (fg_status s = van_leer_radial(c, F(c, FG_ENERGY), dt)) return s;
-  if (fg_status s = van_leer_radial(c, F(c, FG_DENS), dt)) return s;
-  if (fg_status s = fg_reduce_array_internal(c, c->LostByDisk, ns, c->red_out + 2)) return s;
-  // OneWindTheta
-  hipLaunchKernelGGL(k_ring_mean, dim3(nr), dim3(256), ns * sizeof(double), c->stream, c->VMed, F(c, FG_VTHETA), nr,
-                     ns);
-  FG_LAUNCH_CHECK();
-  LAUNCH(k_residual, 0, nr, F(c, FG_VTHETARES), F(c, FG_VTHETA), c->VMed, nr, ns);
-  LAUNCH(k_const_residual, 0, nr, F(c, FG_VTHETA), F(c, FG_VTHETARES), c->Nshift, c->NoSplit, c->VMed,
-         c->t.invRmed, c->t.Rmed, dt, nr, ns, c->p.fast_transport);
-  if (fg_status s = quantities_advection(c, F(c, FG_VTHETARES), dt)) return s;
-  if (fg_status s = quantities_advection(c, F(c, FG_VTHETA), dt)) return s;
-  for (int k = 0; k < 4; k++)
-    if (fg_status s = advect_shift(c, F(c, order[k]))) return s;
-  if (c->p.adiabatic)
-    if (fg_status s = advect_shift(c, F(c, FG_ENERGY))) return s;
-  if (fg_status s = advect_shift(c, F(c, FG_DENS))) return s;
-  LAUNCH(k_compute_velocities, 0, nr, F(c, FG_VRAD), F(c, FG_VTHETA), F(c, FG_DENS), c->t.Rmed, F(c, FG_THETAMOMP),
-         F(c, FG_THETAMOMM), F(c, FG_RADMOMP), F(c, FG_RADMOMM), omega_frame, nr, ns);
+  if (fg_status s = fg_transport_launch(c, dt, omega_frame)) return s;
   if (lost_mass) {
-    FG_HIP(hipMemcpyAsync(c->h_out + 2, c->red_out + 2, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    FG_HIP(hipStreamSynchronize(c->stream));
-    *lost_mass = c->h_out[2];
+    if (c->p.open_inner) FG_HIP(hipStreamSynchronize(c->stream));
+    *lost_mass = c->p.open_inner ? c->h_out[2] : 0.0;
   }
   return FG_OK;
 }

@@ -1,0 +1,100 @@
+"""fg_transport's strip sweeps and the one-kernel non-reflecting edges where
+they can go wrong, against the FP64 oracle bit for bit (1e-12 for adiabatic
+decks, whose exp/log differ): rings narrower than a wave, of one azimuthal
+chunk (183 cells) and one cell more, the longest rings, disks of three and
+four rings (the two edges share rings), every edge with energy, and the full
+rotation swept at once."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from test_gpu_parity import run_pair
+
+pytestmark = pytest.mark.gpu
+
+OPEN, NONREF = dict(InnerBoundary="OPEN"), dict(InnerBoundary="NONREFLECTING")
+
+
+@pytest.mark.parametrize("nrad, nsec", [(5, 3), (9, 63), (7, 183), (6, 184), (131, 130), (4, 4100), (3, 8192)])
+@pytest.mark.parametrize("kw", [OPEN, NONREF, dict(OPEN, Transport="STANDARD")], ids=["open", "nonref", "standard"])
+def test_edges(deck, nrad, nsec, kw):
+    run_pair(deck(Nrad=nrad, Nsec=nsec, DT=0.01, **kw), 3, 0.0)
+
+
+@pytest.mark.parametrize("kw", [OPEN, NONREF], ids=["open", "nonref"])
+@pytest.mark.parametrize("nrad, nsec", [(4, 65), (33, 182)])
+def test_edges_energy(deck, nrad, nsec, kw):
+    run_pair(deck(Nrad=nrad, Nsec=nsec, Adiabatic="YES", AdiabaticIndex=1.4, **kw), 4, 1e-12, adiabatic=True)
+
+
+class Params(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int) for n in ("nrad nsec precision adiabatic cooling self_gravity viscosity_alpha "
+                                            "fast_transport open_inner non_reflecting evanescent indirect_term "
+                                            "exclude_hill").split()]
+    _fields_ += [(n, ctypes.c_double) for n in ("adiabatic_index alphaviscosity sigmaslope flaringindex sg_eps "
+                                                "sg_rstep sg_tstep").split()]
+
+
+RING = ("Radii Rinf Rsup Rmed Surf invRinf invSurf invRmed invdiffRsup invdiffRmed SigmaMed SigmaInf EnergyMed "
+        "CoolingTimeMed QplusMed cs_iso supp_torque dxtheta invdxtheta dxtheta_cfl ev_zone ev_coef ev_period "
+        "ev_vtheta_arg visc_const visc_pow15 visc_cav_on visc_cav").split()
+SECTOR = "cos_cell sin_cell cos_pot sin_pot".split()
+
+
+class Tables(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in RING + SECTOR + ["sg_Kr", "sg_Kt"]]
+    _fields_ += [(n, ctypes.c_double) for n in "dtheta invdphi dt1d_coef vrad0_slope visc_value".split()]
+
+
+def axisymmetric_sweep(stretch):
+    """Sigma of 20 axisymmetric rings before and after fg_transport, and what
+    one ring's flux is multiplied with; outer faces at stretch * Rinf[i + 1]."""
+    from cudaprotoplanetarydisks_amd import native
+    from cudaprotoplanetarydisks_amd.sim import Context
+    nr, ns = 20, 70
+    edge = np.linspace(0.5, 2.5, nr + 2)
+    tab = {n: np.ones(nr + 1) for n in RING}
+    tab["Radii"], tab["Rinf"], tab["Rsup"] = edge[:-1], edge[:-1], edge[1:] * stretch
+    tab["Rmed"] = 0.5 * (edge[:-1] + edge[1:])
+    tab["Surf"] = np.pi * (edge[1:]**2 - edge[:-1]**2) / ns
+    for n in ("Rinf", "Surf", "Rmed"):
+        tab["inv" + n] = 1.0 / tab[n]
+    tab["invdiffRmed"] = np.concatenate([[0.0], 1.0 / np.diff(tab["Rmed"])])
+    tab["dxtheta"] = 2 * np.pi / ns * tab["Rmed"]
+    tab["invdxtheta"] = 1.0 / tab["dxtheta"]
+    for n in ("ev_zone", "visc_cav_on"):
+        tab[n] = np.zeros(nr + 1, dtype=np.int32)
+    for n in SECTOR:
+        tab[n] = np.ones(ns)
+    tab = {n: np.ascontiguousarray(a) for n, a in tab.items()}
+    T = Tables(**{n: a.ctypes.data for n, a in tab.items()}, dtheta=2 * np.pi / ns, invdphi=ns / (2 * np.pi))
+    P = Params(nrad=nr, nsec=ns, fast_transport=1, open_inner=1, adiabatic_index=1.4)
+    h = ctypes.c_void_p()
+    native.call("fg_create", ctypes.byref(P), ctypes.byref(T), 0, ctypes.byref(h))
+    try:
+        ctx = Context(h, (nr + 1, ns))
+        rng = np.random.default_rng(3)
+        dens = np.repeat(rng.uniform(1.0, 2.0, (nr + 1, 1)), ns, axis=1)
+        ctx.set_field("DENS", dens)
+        ctx.set_field("VRAD", np.repeat(rng.uniform(-0.2, 0.2, (nr + 1, 1)), ns, axis=1))
+        ctx.set_field("VTHETA", np.repeat(tab["Rmed"][:, None] ** -0.5, ns, axis=1))
+        lost = ctypes.c_double()
+        native.call("fg_transport", h, 0.01, 1.0, ctypes.byref(lost))
+        return dens[:-1, 0], ctx.field("DENS")[:-1, 0], tab["invSurf"][:-1], lost.value / ns
+    finally:
+        native.call("fg_destroy", h)
+
+
+def test_own_outer_faces():
+    """Tables whose rings end elsewhere than the next ring begins: a ring's
+    outer flux carries its own radius, its inner flux the inner one.  The
+    faces' fluxes follow from a sweep with shared faces; ~20 roundings of
+    values near 1 separate the two sides."""
+    old, new, isurf, lost = axisymmetric_sweep(1.0)
+    out = -np.cumsum((new - old) / isurf)  # flux through each ring's outer face
+    assert abs(lost + out[0]) < 1e-14
+    stretch = 1.25
+    _, got, _, lost2 = axisymmetric_sweep(stretch)
+    assert np.abs(got - (new - (stretch - 1.0) * out * isurf)).max() < 1e-13 * isurf.max()
+    assert abs(lost2 - stretch * lost) < 1e-14
