@@ -4,10 +4,11 @@ For each (NRAD, NSEC) it builds a batch of `copies` disks of that grid (an
 ensemble's worth of parallel work: with one small disk the GPU is mostly
 idle and small tiles win for the wrong reason) and times batch substeps
 (the whole captured graph: every phase and reduction) for every candidate
-(rings per source tile) x (rings per radial-sweep band), keeping the
+(rings per source band) x (rings per radial-sweep band), keeping the
 fastest.  Results go to a JSON cache keyed "NRADxNSEC" that
-Ensemble reads.  Tile shapes change only the work decomposition: results
-are identical for every candidate.
+Ensemble and Simulation read; none ships with the package, since the bands
+picked without one are within 1 to 2 % of the best.  Tile shapes change only
+the work decomposition: results are identical for every candidate.
 
     python -m cudaprotoplanetarydisks_amd.autotune --grids 128x384 256x768
 """

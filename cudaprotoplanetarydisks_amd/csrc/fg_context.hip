@@ -78,7 +78,7 @@ extern "C" fg_status fg_create(const fg_params *p, const fg_tables *t, int devic
   // the context itself does not need it
   (void)fg_noalloc_setup(device);
   fg_ctx *c = new fg_ctx();
-  c->tile_src_th = 16;
+  c->tile_src_th = 0;   // picked for the grid
   c->tile_trad_band = 0;  // picked for the grid
   c->fp32_pair_hill = 1.0;
   c->p = *p;

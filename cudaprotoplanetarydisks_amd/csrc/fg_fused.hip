@@ -156,6 +156,13 @@ __device__ __forceinline__ double lane_next(double x) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+// p as the global pointer it is: read from a struct in memory it would be a
+// generic one, and its accesses flat ones, which wait for LDS and memory alike
+template <class T>
+__device__ __forceinline__ T *global(T *p) {
+  return (T *)(__attribute__((address_space(1))) T *)(unsigned long)p;
+}
+
 // Workgroups are dispatched round-robin over the 8 XCDs.  The block of a list
 // of n that this workgroup of a grid of 8 ceil(n / 8) takes, each XCD a
 // contiguous run, so that neighbouring blocks, which read each other's halos,
@@ -190,8 +197,14 @@ __device__ __forceinline__ double ev_damp(double q, const double *ev, int which)
 
 // element at byte offset `off` of a row: the scalar row address plus a 32-bit
 // lane offset is the memory instructions' own form, no vector arithmetic
-__device__ __forceinline__ double &at(double *row, unsigned off) { return *(double *)((char *)row + off); }
-__device__ __forceinline__ double at(const double *row, unsigned off) { return *(const double *)((const char *)row + off); }
+template <class T>
+__device__ __forceinline__ T &at(T *row, unsigned off) {
+  return *(T *)((char *)row + off);
+}
+template <class T>
+__device__ __forceinline__ T at(const T *row, unsigned off) {
+  return *(const T *)((const char *)row + off);
+}
 
 // MODE bit 1: adiabatic (energy damped, P = (gamma - 1) e, EnergyInt out);
 // bit 2: self-gravity kick after Substep1
@@ -1895,48 +1908,6 @@ __global__ __launch_bounds__(256) void k_fin(fin_args a) {
 //   - cell-planet separations are differenced in FP64;
 //   - the FARGO ring mean, Ntilde/Nshift and the uniform residual, the CFL
 //     count and the disk force are the FP64 code of the exact path.
-// The tile height th (rings per tile: 8, 16 or 32) is chosen per grid size
-// and dispatched to a template instance; the LDS tiles are carved from dynamic
-// shared memory: six (th + 6) x HC float arrays and two th x TW
-// increment arrays.
-// per-ring tables the source stages read, staged per tile row in LDS
-enum { RT_MED, RT_IMED, RT_IDMED, RT_INF, RT_IINF, RT_IDXT, RT_SUPP, RT_IDSUP, RT_SUP, RT_NU, RT_CS, RT_SMED, RT_EVZ, RT_N };
-__device__ __forceinline__ const double *ring_table(const fg_dev_tables &t, const double *nu, int x) {
-  switch (x) {
-    case RT_MED: return t.Rmed;
-    case RT_IMED: return t.invRmed;
-    case RT_IDMED: return t.invdiffRmed;
-    case RT_INF: return t.Rinf;
-    case RT_IINF: return t.invRinf;
-    case RT_IDXT: return t.invdxtheta;
-    case RT_SUPP: return t.supp_torque;
-    case RT_IDSUP: return t.invdiffRsup;
-    case RT_SUP: return t.Rsup;
-    case RT_NU: return nu;
-    case RT_CS: return t.cs_iso;
-    default: return t.SigmaMed;
-  }
-}
-
-#define TW 64
-#define HALO_R 4  // rows above the tile (i - 4 .. )
-#define HALO_B 2  // rows below the tile ( .. i + TH + 1)
-#define HALO_C 4  // columns on each side
-#define HC (TW + 2 * HALO_C)
-// sector of a staged column j0 - HALO_C + c (j0 = the tile's first column):
-// at most one ring length outside [0, ns) once ns reaches the staged width,
-// so a compare and an add or subtract replace the two runtime modulos
-__device__ __forceinline__ int wrap_col(int x, int ns) {
-  if (x < 0) x += ns;
-  while (x >= ns) x -= ns;
-  return x;
-}
-#define SRC32_MAX_TH 32
-#define SRC32_TPB 512  // threads per FP32 source tile
-#define SRC32_PER_THREAD (((SRC32_MAX_TH + HALO_R + HALO_B) * HC + SRC32_TPB - 1) / SRC32_TPB)
-
-static size_t src32_lds_bytes(int th) { return (size_t)(6 * (th + HALO_R + HALO_B) * HC + 2 * th * TW) * sizeof(float); }
-
 struct src32_args {
   const double *dens, *vr, *vt;
   const double *vref;  // per-ring reference vtheta
@@ -1947,378 +1918,314 @@ struct src32_args {
   fg_dev_tables t;
   fg_planets_arg P;
   double dt, omega_frame, domega;
-  int nr, ns, indirect, evanescent, corotating;
-  int lob0, lob1;  // FP32 storage: rings stored as float pairs
+  int nr, ns, indirect, evanescent;
+  int lob0, lob1;            // FP32 storage: rings stored as float pairs
+  int nstrips, width, band;  // strips of `width` columns, bands of `band` rings
 };
 
-// planet part of the potential at one cell (the star's -1/r is applied per
-// ring by the caller); Kernels.cu:1234-1252 with the separation in FP64
-__device__ __forceinline__ float cell_potential_planets_f(const fg_planets_arg &P, double Rm, double cosp,
-                                                          double sinp, int indirect) {
-  const double x = Rm * cosp, y = Rm * sinp;
-  float acc = 0.0f;
-  for (int k = 0; k < P.nb; k++) {
-    const float dx = (float)(x - P.x[k]), dy = (float)(y - P.y[k]);
-    const float m = (float)P.m[k];
-    float pv = -m * __builtin_amdgcn_rsqf(dx * dx + dy * dy + (float)P.smooth[k]);
-    if (indirect) pv += m * (float)P.invd3[k] * (float)(x * P.x[k] + y * P.y[k]);
-    acc += pv;
-    if (k == 0) acc -= (float)(P.ix * x + P.iy * y);
-  }
-  return acc;
+// a planet's part of the potential at (x, y) (the star's -1/r is applied per
+// ring); Kernels.cu:1234-1252 with the separation in FP64
+__device__ __forceinline__ float planet_potential_f(double x, double y, double xp, double yp, double m, double smooth,
+                                                    double invd3, int indirect) {
+  const float dx = (float)(x - xp), dy = (float)(y - yp);
+  const float mf = (float)m;
+  float pv = -mf * __builtin_amdgcn_rsqf(dx * dx + dy * dy + (float)smooth);
+  if (indirect) pv += mf * (float)invd3 * (float)(x * xp + y * yp);
+  return pv;
 }
 
-// CorrectVtheta and the first damping pass of one cell's state (FP64);
-// rt = the ring's tables (RT_* layout, one value per ring), ev = its
-// damping constants (lambda, vrad0, vtheta0)
-__device__ __forceinline__ void src32_adjust(const src32_args &a, int i, double rmed, double evz, double smed,
-                                             const double *ev, double &s, double &vr, double &vt) {
-  if (i < a.nr) {
-    if (a.corotating) vt = vt - a.domega * rmed;
-    if (a.evanescent && evz != 0.0) {
-      vr = damp_toward(vr, ev[0], ev[1]);
-      vt = damp_toward(vt, ev[0], ev[2]);
-      s = damp_toward(s, ev[0], smed);
-    }
-  }
-}
+// k_src's march in the FP32 bulk mode: the same strips, halos, stages and
+// windows (there), in single precision, with the ring's FP64 state of
+// step m kept until ring m is complete; block `block` of the disk's strips
+// and bands.  Per-ring values: in FP64 S3_*, rounded to FP32 S3F_*; VB the
+// ring part of the azimuthal velocity at the ring's inner face, STAR the
+// star's gravity there, DREF the reference part of the shear.
+// Bound: VALU issue (~300 instructions a cell) and latency on small grids; as
+// 16 x 64 LDS tiles it evaluated 1.55 cells per cell and 590 instructions.
+// 1024 x 3072: 66 -> 42 us; 64 disks of 128 to 384 rings: 216 -> 106 us.
+#define SRC32_WAVES 4  // per SIMD
+enum { S3_MED, S3_CS, S3_VB, S3_IINF, S3_STAR, S3_VREF, S3_SBAR, S3_N };
+enum { S3F_IDMED, S3F_IDXT, S3F_SUPP, S3F_IMED, S3F_IDSUP, S3F_SUP, S3F_INF, S3F_NU, S3F_IINF, S3F_MED, S3F_DREF, S3F_N = 12 };
+struct src32_lds {
+  double tab[SRC_ROWS][S3_N], evc[SRC_ROWS][EV_N];
+  float ftab[SRC_ROWS][S3F_N];
+};
 
-#define SRC32_OWN_MAX (SRC32_MAX_TH * TW / SRC32_TPB)  // own cells per thread
-
-// staged position (row r, column cc of the TH+6 x HC stage) of halo cell h
-// of a tile of TH rows: the HALO_R rows above, the HALO_B rows below, then
-// the HALO_C columns on either side of each tile row
-template <int TH_>
-__device__ __forceinline__ void halo_cell(int h, int &r, int &cc) {
-  constexpr int NTOP = HALO_R * HC, NBOT = HALO_B * HC;
-  if (h < NTOP) {
-    r = h / HC;
-    cc = h % HC;
-  } else if (h < NTOP + NBOT) {
-    h -= NTOP;
-    r = HALO_R + TH_ + h / HC;
-    cc = h % HC;
-  } else {
-    h -= NTOP + NBOT;
-    const int c = h % (2 * HALO_C);
-    r = HALO_R + h / (2 * HALO_C);
-    cc = c < HALO_C ? c : c + TW;
-  }
-}
-
-// the damping constants of the tile's rings are computed once per ring
-// into LDS
-// ROWS (rings per tile) is a template parameter so that the LDS array offsets
-// and the per-thread trip counts are constants
-template <int ROWS>
-__device__ __forceinline__ void src32_tile(const src32_args &a, int bx, int by, float *lds) {
-  constexpr int th = ROWS, hr = th + HALO_R + HALO_B;
-  float(*sS)[HC] = (float(*)[HC])(lds);           // Sigma after the first damping
-  float(*sA)[HC] = (float(*)[HC])(lds + hr * HC);  // pressure, then VradInt
-  float(*sB)[HC] = (float(*)[HC])(lds + 2 * hr * HC);  // planet potential, then VthetaInt - vref
-  float(*sC)[HC] = (float(*)[HC])(lds + 3 * hr * HC);  // vtheta - vref, then TAURR, then Qr
-  float(*sD)[HC] = (float(*)[HC])(lds + 4 * hr * HC);  // vrad, then TAUPP, then Qtheta
-  float(*sE)[HC] = (float(*)[HC])(lds + 5 * hr * HC);  // TAURP
-  float(*incR)[TW] = (float(*)[TW])(lds + 6 * hr * HC);  // own-cell velocity increments
-  float(*incT)[TW] = (float(*)[TW])(lds + 6 * hr * HC + th * TW);
-  __shared__ double evc[SRC32_MAX_TH + HALO_R + HALO_B][3];  // damping constants per tile row
-  const int nr = a.nr, ns = a.ns;
-  const int i0 = by * th, j0 = bx * TW;
-  const int tid = threadIdx.x;
+// PL: where the planets behind the first one are read (indexed by a loop, a
+// by-value copy would live in scratch)
+template <class PL>
+__device__ __forceinline__ void src32_march(const src32_args &a, const PL &more, int block, src32_lds &lds) {
+  constexpr int AHEAD = 2;  // rings whose loads are in flight
+  auto &tab = lds.tab;
+  auto &evc = lds.evc;
+  auto &ftab = lds.ftab;
+  const int nr = a.nr, ns = a.ns, lane = threadIdx.x, band = a.band, nstrips = a.nstrips, width = a.width;
+  const int strip = block % nstrips, i0 = block / nstrips * band;
+  const int i1 = min(i0 + band, nr + 1);
   const fg_dev_tables &t = a.t;
-  const double dt = a.dt;
+  const double *dens = global(a.dens), *vrad = global(a.vr), *vtheta = global(a.vt);
+  float *odens = global(a.odens), *ovr = global(a.ovr), *ovt = global(a.ovt);
+  double *opress = global(a.opress);
+  const double dt = a.dt, OF = a.omega_frame, domega = a.domega;
   const float dtf = (float)dt;
-#define GI(r) (i0 - HALO_R + (r))
-#define GJ(c) wrap_col(j0 - HALO_C + (c), ns)
-  // per-ring tables of the tile's rows as in k_src, plus the reference
-  // vtheta (0 outside the disk), and the potential's cos/sin per column
-  constexpr int RT_VREF = RT_N, RT_SBAR = RT_N + 1, MAXR = SRC32_MAX_TH + HALO_R + HALO_B;
-  __shared__ double rt[RT_N + 2][MAXR];
-  __shared__ double ct[2][HC];
-
-  // ---- S0: load, CorrectVtheta, damping #1 (FP64), pressure, potential ----
-  // all of a thread's loads are issued before any of them is used.  The
-  // tile's own cells are loaded in the mapping of the final stage (S5) and
-  // their adjusted FP64 state stays in registers until then; the halo
-  // cells (rows above and below, columns on either side) separately
-  constexpr int NH = hr * HC - th * TW, HPT = (NH + SRC32_TPB - 1) / SRC32_TPB;
-  double os[SRC32_OWN_MAX], ovr[SRC32_OWN_MAX], ovt[SRC32_OWN_MAX];
-  {
-    double ls[HPT], lvr[HPT], lvt[HPT];
+  const int lob0 = a.lob0, lob1 = a.lob1, indirect = a.indirect, nb = a.P.nb;
+  const int g = strip * width - SRC_HL + lane;
+  const int j = (g % ns + ns) % ns;
+  unsigned jb = 8u * j, jf = 4u * j;
+  const bool mine = lane >= SRC_HL && lane < SRC_HL + width && g < ns;
+  const double cosp = global(t.cos_pot)[j], sinp = global(t.sin_pot)[j];
+  double n_s[3], n_vr[3], n_vt[3];
+  auto fetch = [&](int m, auto phase) __attribute__((always_inline)) {
+    constexpr int X = decltype(phase)::value % 3;
+    const long l = (long)min(max(m, 0), nr) * ns;
+    n_s[X] = at(dens + l, jb);
+    n_vr[X] = at(vrad + l, jb);
+    n_vt[X] = at(vtheta + l, jb);
+  };
+#define LVL(n) std::integral_constant<int, n>()
+  fetch(i0 - SRC_HT, LVL(0));
+  if (AHEAD > 1) fetch(i0 - SRC_HT + 1, LVL(1));
+  bool damped = false;
+  if (lane < i1 - i0 + SRC_HT + SRC_HB) {
+    const int i = i0 - SRC_HT + lane, ic = min(max(i, 0), nr - 1), il = max(ic - 1, 0);
+    const double *rings = global(t.rings), *vrefs = global(a.vref);
+    double r[RG_NU];
 #pragma unroll
-    for (int k = 0; k < SRC32_OWN_MAX; k++) {
-      const int q = tid + k * SRC32_TPB;
-      os[k] = ovr[k] = ovt[k] = 0.0;
-      if (q < th * TW) {
-        const int r = q / TW + HALO_R, cc = q % TW + HALO_C, i = GI(r);
-        if (i >= 0 && i <= nr) {
-          const long l = (long)i * ns + GJ(cc);
-          os[k] = a.dens[l];
-          ovr[k] = a.vr[l];
-          ovt[k] = a.vt[l];
-        }
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < HPT; k++) {
-      const int h = tid + k * SRC32_TPB;
-      ls[k] = lvr[k] = lvt[k] = 0.0;
-      if (h < NH) {
-        int r, cc;
-        halo_cell<th>(h, r, cc);
-        const int i = GI(r);
-        if (i >= 0 && i <= nr) {
-          const long l = (long)i * ns + GJ(cc);
-          ls[k] = a.dens[l];
-          lvr[k] = a.vr[l];
-          lvt[k] = a.vt[l];
-        }
-      }
-    }
-    // tables staged while the loads above are in flight: wave w loads
-    // tables w, w + 4, w + 8 (wave 0 also the ev_zone flags, wave 1 the
-    // reference vtheta) of rows ln and ln + 64
-    {
-      const int w = tid >> 6, ln = tid & 63;
-      for (int r = ln; w < 4 && r < hr; r += 64) {
-        const int gi = GI(r), i = min(max(gi, 0), nr - 1);
-        const double v0 = ring_table(t, a.nu, w)[i], v1 = ring_table(t, a.nu, w + 4)[i];
-        const double v2 = ring_table(t, a.nu, w + 8)[i];
-        const int ez = t.ev_zone[i];
-        const double vref = (gi >= 0 && gi < nr) ? a.vref[gi] : 0.0;
-        const double sbar = (gi >= 0 && gi < nr) ? a.sbar[gi] : 0.0;
-        rt[w][r] = v0;
-        rt[w + 4][r] = v1;
-        rt[w + 8][r] = v2;
-        if (w == 0) rt[RT_EVZ][r] = (double)ez;
-        if (w == 1) rt[RT_VREF][r] = vref;
-        if (w == 2) rt[RT_SBAR][r] = sbar;
-      }
-      for (int c = tid; c < HC; c += SRC32_TPB) {
-        const int j = GJ(c);
-        ct[0][c] = t.cos_pot[j];
-        ct[1][c] = t.sin_pot[j];
-      }
-    }
-    // damping constants of the tile's rings, once per ring (Kernels.cu:978-1004)
-    if (a.evanescent) {
-      for (int r = tid; r < hr; r += SRC32_TPB) {
-        const int i = GI(r);
-        if (i >= 0 && i < nr && t.ev_zone[i]) ev_consts(t, a.nu, i, dt, a.omega_frame, evc[r][0], evc[r][1], evc[r][2]);
-      }
-    }
-    __syncthreads();
-    // CorrectVtheta and damping #1 of a staged cell (the FP64 values in
-    // place), then its FP32 stage values
-    auto stage = [&](int r, int cc, double &sd, double &vrd, double &vtd) {
-      const int i = GI(r);
-      float s = 0.f, vr = 0.f, vt = 0.f, p = 0.f, phi = 0.f;
-      if (i >= 0 && i <= nr) {
-        src32_adjust(a, i, rt[RT_MED][r], rt[RT_EVZ][r], rt[RT_SMED][r], evc[r], sd, vrd, vtd);
-        s = (float)sd;
-        vr = (float)vrd;
-        vt = (float)(vtd - rt[RT_VREF][r]);
-        if (i < nr) {
-          const double cs = rt[RT_CS][r];
-          p = (float)(sd * cs * cs);
-          phi = cell_potential_planets_f(a.P, rt[RT_MED][r], ct[0][cc], ct[1][cc], a.indirect);
-        }
-      }
-      sS[r][cc] = s;
-      sA[r][cc] = p;
-      sB[r][cc] = phi;
-      sC[r][cc] = vt;
-      sD[r][cc] = vr;
-    };
-#pragma unroll
-    for (int k = 0; k < SRC32_OWN_MAX; k++) {
-      const int q = tid + k * SRC32_TPB;
-      if (q >= th * TW) break;
-      stage(q / TW + HALO_R, q % TW + HALO_C, os[k], ovr[k], ovt[k]);
-    }
-#pragma unroll
-    for (int k = 0; k < HPT; k++) {
-      const int h = tid + k * SRC32_TPB;
-      if (h >= NH) break;
-      int r, cc;
-      halo_cell<th>(h, r, cc);
-      stage(r, cc, ls[k], lvr[k], lvt[k]);
+    for (int x = 0; x < RG_NU; x++) r[x] = rings[(long)ic * RG_NU + x];
+    const double v = global(a.nu)[ic], imed_l = rings[(long)il * RG_NU + RG_IMED];
+    // the reference velocity and Sigma's background are 0 outside the disk
+    const double vref = i == ic ? vrefs[ic] : 0.0, vref_l = vrefs[il];
+    const double sbar = i == ic ? global(a.sbar)[ic] : 0.0;
+    damped = a.evanescent && i == ic && global(t.ev_zone)[ic];
+    tab[lane][S3_MED] = r[RG_MED];
+    tab[lane][S3_CS] = r[RG_CS];
+    tab[lane][S3_VB] = 0.5 * (vref + vref_l) + OF * r[RG_INF];
+    tab[lane][S3_IINF] = r[RG_IINF];
+    tab[lane][S3_STAR] = (imed_l - r[RG_IMED]) * r[RG_IDMED];
+    tab[lane][S3_VREF] = vref;
+    tab[lane][S3_SBAR] = sbar;
+    ftab[lane][S3F_IDMED] = (float)r[RG_IDMED];
+    ftab[lane][S3F_IDXT] = (float)r[RG_IDXT];
+    ftab[lane][S3F_SUPP] = (float)r[RG_SUPP];
+    ftab[lane][S3F_IMED] = (float)r[RG_IMED];
+    ftab[lane][S3F_IDSUP] = (float)r[RG_IDSUP];
+    ftab[lane][S3F_SUP] = (float)r[RG_SUP];
+    ftab[lane][S3F_INF] = (float)r[RG_INF];
+    ftab[lane][S3F_NU] = (float)v;
+    ftab[lane][S3F_IINF] = (float)r[RG_IINF];
+    ftab[lane][S3F_MED] = (float)r[RG_MED];
+    ftab[lane][S3F_DREF] = (float)(vref * r[RG_IMED] - vref_l * imed_l);
+    if (damped) {
+      // (Kernels.cu:978-1004; one viscosity: the two passes damp alike)
+      const double Rm = r[RG_MED], lambda = global(t.ev_coef)[ic] * dt / global(t.ev_period)[ic];
+      const double vt0 = sqrt(global(t.ev_vtheta_arg)[ic]) - Rm * OF, vr0 = -3.0 * v / Rm * t.vrad0_slope;
+      const recip64 d(1.0 + lambda);
+      double *ev = evc[lane];
+      ev[EV_D] = d.d;
+      ev[EV_R] = d.r;
+      ev[EV_S] = lambda * global(t.SigmaMed)[ic];
+      ev[EV_VR1] = lambda * vr0;
+      ev[EV_VT1] = lambda * vt0;
     }
   }
+  const unsigned zones = (unsigned)__ballot(damped);  // bit r: ring i0 - SRC_HT + r is damped
   __syncthreads();
-
-  // ---- S1: Substep1 (Kernels.cu:13-53) ----
-  const bool star = a.P.nb > 0;  // the star's -1/r enters with the first planet
-  float regA[SRC32_PER_THREAD], regB[SRC32_PER_THREAD];
-  {
-#pragma unroll
-    for (int k = 0; k < SRC32_PER_THREAD; k++) {
-      const int q = tid + k * SRC32_TPB;
-      if (q >= hr * HC) break;
-      int r = q / HC, cc = q - r * HC;
-      int i = GI(r);
+  double px = a.P.x[0], py = a.P.y[0], pm = a.P.m[0], ps = a.P.smooth[0], pi3 = a.P.invd3[0], ix = a.P.ix, iy = a.P.iy;
+  asm volatile("" : "+s"(px), "+s"(py), "+s"(pm), "+s"(ps), "+s"(pi3), "+s"(ix), "+s"(iy));
+  const bool star = nb > 0;  // the star's -1/r enters with the first planet
+  const float invdphi = (float)t.invdphi, onethird = 1.0f / 3.0f;
+  // windows as in k_src (T: vtheta - vref); IR, IT: the velocity increments;
+  // Ds, Dvr, Dvt: the state in FP64 after the first damping pass
+  double Ds[3] = {}, Dvr[3] = {}, Dvt[3] = {};
+  float S[3] = {}, Sl[3] = {}, P[3] = {}, F[3] = {}, T[3] = {}, Tn[3] = {};
+  float A1[3] = {}, B1[3] = {}, A3[3] = {}, RR[3] = {}, PP[3] = {}, RP[3] = {}, QR[3] = {}, IR[3] = {}, IT[3] = {};
+  float hr[3] = {}, ha[3] = {};  // reciprocals of Sigma_i + Sigma_i-1, Sigma_j + Sigma_j-1
+  auto step = [&](int m, auto level, auto phase, auto inner) __attribute__((always_inline)) {
+    constexpr int LV = decltype(level)::value, C = decltype(phase)::value, M1 = (C + 2) % 3, M2 = (C + 1) % 3;
+    constexpr bool IN = decltype(inner)::value;
+    double s = n_s[C], vr = n_vr[C], vt = n_vt[C];
+    fetch(m + AHEAD, LVL(C + AHEAD));
+    asm volatile("" : "+v"(jb), "+v"(jf));
+    const int row = m - i0 + SRC_HT;  // rings m, k, o in the tables
+    const double *Dm = tab[row], *Do = tab[max(row - 2, 0)];
+    const float *Rm = ftab[row], *Rk = ftab[max(row - 1, 0)], *Ro = ftab[max(row - 2, 0)];
+    const int k = m - 1, o = m - 2;
+    // ---- S0: CorrectVtheta, damping #1 (FP64), pressure, potential of ring m ----
+    float fs = 0.f, fvr = 0.f, fvt = 0.f, p = 0.f, phi = 0.f;
+    if (IN || (m >= 0 && m < nr)) {
+      vt = vt - domega * Dm[S3_MED];
+      if (zones >> row & 1) {
+        const double *ev = evc[row];
+        vr = ev_damp(vr, ev, EV_VR1);
+        vt = ev_damp(vt, ev, EV_VT1);
+        s = ev_damp(s, ev, EV_S);
+      }
+      const double cs = Dm[S3_CS], pd = s * cs * cs;
+      p = (float)pd;
+      if (opress && mine && m >= i0 && m < i1) at(opress + (long)m * ns, jb) = pd;  // for the temperature output
+      const double x = Dm[S3_MED] * cosp, y = Dm[S3_MED] * sinp;
+      if (nb > 0) {
+        phi = 0.0f + planet_potential_f(x, y, px, py, pm, ps, pi3, indirect);
+        phi -= (float)(ix * x + iy * y);
+      }
+      for (int q = 1; q < nb; q++)
+        phi += planet_potential_f(x, y, more.x[q], more.y[q], more.m[q], more.smooth[q], more.invd3[q], indirect);
+      fs = (float)s;
+      fvr = (float)vr;
+      fvt = (float)(vt - Dm[S3_VREF]);
+    } else if (m == nr) {
+      fs = (float)s;
+      fvr = (float)vr;
+      fvt = (float)vt;
+    }
+    Ds[C] = s;
+    Dvr[C] = vr;
+    Dvt[C] = vt;
+    S[C] = fs;
+    P[C] = p;
+    F[C] = phi;
+    T[C] = fvt;
+    Tn[C] = lane_next(fvt);
+    Sl[C] = lane_prev(fs);
+    // ---- S1: Substep1 (Kernels.cu:13-53) of ring m ----
+    if constexpr (LV >= 1) {
       float vri = 0.f, vti = 0.f, dvr = 0.f, dvt = 0.f;
-      if (r >= 1 && cc >= 1 && cc < HC - 1 && i >= 0 && i < nr) {
-        if (i > 0) {
-          const float idr = (float)rt[RT_IDMED][r];
-          float gradp = (sA[r][cc] - sA[r - 1][cc]) * 2.0f * rcp_f(sS[r][cc] + sS[r - 1][cc]) * idr;
-          float gradphi = (sB[r][cc] - sB[r - 1][cc]) * idr;
+      if (IN || (m >= 0 && m < nr)) {
+        if (IN || m > 0) {
+          const float idr = Rm[S3F_IDMED];
+          hr[C] = rcp_f(fs + S[M1]);
+          const float gradp = (p - P[M1]) * 2.0f * hr[C] * idr;
+          const float gradphi = (phi - F[M1]) * idr;
           // centrifugal minus star gravity in FP64: vbar = ring part + offset
-          double vbar = 0.5 * (rt[RT_VREF][r] + rt[RT_VREF][r - 1]) + a.omega_frame * rt[RT_INF][r];
-          vbar += (double)((sC[r][cc] + sC[r][cc + 1] + sC[r - 1][cc] + sC[r - 1][cc + 1]) * 0.25f);
-          double bal = vbar * vbar * rt[RT_IINF][r];
-          if (star) bal -= (rt[RT_IMED][r - 1] - rt[RT_IMED][r]) * rt[RT_IDMED][r];
+          double vbar = Dm[S3_VB];
+          vbar += (double)((T[C] + Tn[C] + T[M1] + Tn[M1]) * 0.25f);
+          double bal = vbar * vbar * Dm[S3_IINF];
+          if (star) bal -= Dm[S3_STAR];
           dvr = dtf * (-gradp - gradphi + (float)bal);
-          vri = sD[r][cc] + dvr;
+          vri = fvr + dvr;
         }
-        const float invdxtheta = (float)rt[RT_IDXT][r];
-        float gradp = (sA[r][cc] - sA[r][cc - 1]) * 2.0f * rcp_f(sS[r][cc] + sS[r][cc - 1]) * invdxtheta;
-        float gradphi = (sB[r][cc] - sB[r][cc - 1]) * invdxtheta;
-        dvt = dtf * ((float)rt[RT_SUPP][r] - (gradp + gradphi));
-        vti = sC[r][cc] + dvt;
+        const float invdxtheta = Rm[S3F_IDXT];
+        ha[C] = rcp_f(fs + Sl[C]);
+        const float gradp = (p - lane_prev(p)) * 2.0f * ha[C] * invdxtheta;
+        const float gradphi = (phi - lane_prev(phi)) * invdxtheta;
+        dvt = dtf * (Rm[S3F_SUPP] - (gradp + gradphi));
+        vti = fvt + dvt;
       }
-      regA[k] = vri;
-      regB[k] = vti;
-      const int ro = r - HALO_R, co = cc - HALO_C;
-      if (ro >= 0 && ro < th && co >= 0 && co < TW) {
-        incR[ro][co] = dvr;
-        incT[ro][co] = dvt;
+      A1[C] = vri;
+      B1[C] = vti;
+      IR[C] = dvr;
+      IT[C] = dvt;
+    }
+    // ---- S2: viscous stress (Kernels.cu:733-771) of ring k ----
+    if constexpr (LV >= 2) {
+      if (IN || (k >= 0 && k < nr)) {
+        const float iRm = Rk[S3F_IMED], idRs = Rk[S3F_IDSUP], v = Rk[S3F_NU];
+        const float vr0 = A1[M1], vr1 = A1[C], b = B1[M1];
+        const float dv_t = lane_next(b) - b;
+        const float drr = (vr1 - vr0) * idRs;
+        const float dpp = dv_t * invdphi * iRm + 0.5f * (vr1 + vr0) * iRm;
+        float dv = (vr1 * Rk[S3F_SUP] - vr0 * Rk[S3F_INF]) * idRs * iRm;
+        dv += dv_t * invdphi * iRm;
+        const float nu2s = 2.0f * S[M1] * v;
+        RR[M1] = nu2s * (drr - onethird * dv);
+        PP[M1] = nu2s * (dpp - onethird * dv);
+        if (LV >= 3 && (IN || k > 0)) {
+          // d(vtheta/r)/dr with the reference part of vtheta differenced in FP64
+          const float dom = Rk[S3F_DREF] + (b * iRm - B1[M2] * Ro[S3F_IMED]);
+          const float drp = 0.5f * (Rk[S3F_INF] * dom * Rk[S3F_IDMED] +
+                                    (vr0 - lane_prev(vr0)) * invdphi * Rk[S3F_IINF]);
+          RP[M1] = 0.5f * (S[M1] + S[M2] + Sl[M1] + Sl[M2]) * v * drp;
+        }
       }
     }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < SRC32_PER_THREAD; k++) {
-      const int q = tid + k * SRC32_TPB;
-      if (q >= hr * HC) break;
-      int r = q / HC, cc = q - r * HC;
-      sA[r][cc] = regA[k];
-      sB[r][cc] = regB[k];
+    // ---- S3: viscous velocity update (Kernels.cu:118-150): VradInt of ring k ----
+    if constexpr (LV >= 3) {
+      A3[M1] = A1[M1];
+      if (IN || (k >= 1 && k < nr)) {
+        const float d = dtf * Rk[S3F_IINF] *
+                        ((Rk[S3F_MED] * RR[M1] - Ro[S3F_MED] * RR[M2]) * Rk[S3F_IDMED] +
+                         (lane_next(RP[M1]) - RP[M1]) * invdphi - 0.5f * (PP[M1] + PP[M2])) *
+                        rcp_f(0.5f * (S[M1] + S[M2]));
+        A3[M1] += d;
+        IR[M1] += d;
+      }
     }
-  }
-  __syncthreads();
-
-  // ---- S2: viscous stress (Kernels.cu:733-771) ----
-  const float invdphi = (float)t.invdphi;
-  const float onethird = 1.0f / 3.0f;
-#pragma unroll
-  for (int kq = 0; kq < SRC32_PER_THREAD; kq++) {
-    const int q = tid + kq * SRC32_TPB;
-    if (q >= hr * HC) break;
-    int r = q / HC, cc = q - r * HC;
-    int i = GI(r);
-    if (r < 1 || r >= hr - 1 || cc < 2 || cc >= HC - 2 || i < 0 || i >= nr) continue;
-    const float iRm = (float)rt[RT_IMED][r], idRs = (float)rt[RT_IDSUP][r];
-    const float vr0 = sA[r][cc], vr1 = sA[r + 1][cc];
-    const float dvt = sB[r][cc + 1] - sB[r][cc];
-    float drr = (vr1 - vr0) * idRs;
-    float dpp = dvt * invdphi * iRm + 0.5f * (vr1 + vr0) * iRm;
-    float dv = (vr1 * (float)rt[RT_SUP][r] - vr0 * (float)rt[RT_INF][r]) * idRs * iRm;
-    dv += dvt * invdphi * iRm;
-    const float nu2s = 2.0f * sS[r][cc] * (float)rt[RT_NU][r];
-    sC[r][cc] = nu2s * (drr - onethird * dv);
-    sD[r][cc] = nu2s * (dpp - onethird * dv);
-    if (i > 0) {
-      // d(vtheta/r)/dr with the reference part of vtheta differenced in FP64
-      const double dref = (rt[RT_VREF][r] * rt[RT_IMED][r] - rt[RT_VREF][r - 1] * rt[RT_IMED][r - 1]);
-      const float dom = (float)dref + (sB[r][cc] * iRm - sB[r - 1][cc] * (float)rt[RT_IMED][r - 1]);
-      float drp = 0.5f * ((float)rt[RT_INF][r] * dom * (float)rt[RT_IDMED][r] +
-                          (sA[r][cc] - sA[r][cc - 1]) * invdphi * (float)rt[RT_IINF][r]);
-      sE[r][cc] = 0.5f * (sS[r][cc] + sS[r - 1][cc] + sS[r][cc - 1] + sS[r - 1][cc - 1]) * (float)rt[RT_NU][r] * drp;
+    // ---- S4: radial artificial pressure (Kernels.cu:409-434) of ring o ----
+    if constexpr (LV >= 4) QR[M2] = (IN || (o >= 0 && o < nr)) ? art_visc_q_f(S[M2], A3[M1] - A3[M2]) : 0.f;
+    // ---- ring o: the rest of S3 and S4, S5 ("kernel", Kernels.cu:438-479), damping #2, store ----
+    if constexpr (LV >= 5) {
+      const long l = (long)o * ns;
+      if (!IN && o == nr) {  // ghost ring (never read)
+        if (mine) {
+          at(odens + l, jf) = 0.0f;
+          at(ovr + l, jf) = 0.0f;
+          at(ovt + l, jf) = 0.0f;
+        }
+        return;
+      }
+      float b = B1[M2], it = IT[M2];
+      if (IN || (o >= 1 && o < nr - 1)) {
+        const float d = dtf * Ro[S3F_IMED] *
+                        ((Ro[S3F_SUP] * RP[M1] - Ro[S3F_INF] * RP[M2]) * Ro[S3F_IDSUP] +
+                         (PP[M2] - lane_prev(PP[M2])) * invdphi + 0.5f * (RP[M2] + RP[M1])) *
+                        rcp_f(0.5f * (S[M2] + Sl[M2]));
+        b += d;
+        it += d;
+      }
+      const float qt = art_visc_q_f(S[M2], lane_next(b) - b);
+      double s2 = Ds[M2], vrnew = 0.0;
+      if (IN || o > 0) {
+        const float dq = (QR[M2] - QR[C]) * 2.0f * hr[M2] * Ro[S3F_IDMED];  // (slot C: ring o - 1)
+        vrnew = Dvr[M2] + (double)(IR[M2] - dtf * dq);
+      }
+      const float dq = (qt - lane_prev(qt)) * 2.0f * ha[M2] * Ro[S3F_IDXT];
+      double vtnew = Dvt[M2] + (double)(it - dtf * dq);
+      if (zones >> (row - 2) & 1) {
+        const double *ev = evc[row - 2];
+        vrnew = ev_damp(vrnew, ev, EV_VR1);
+        vtnew = ev_damp(vtnew, ev, EV_VT1);
+        s2 = ev_damp(s2, ev, EV_S);
+      }
+      if (mine) {
+        const double xs = s2 - Do[S3_SBAR];
+        const float hs = (float)xs;
+        at(odens + l, jf) = hs;
+        at(ovr + l, jf) = (float)vrnew;
+        at(ovt + l, jf) = (float)(vtnew - Do[S3_VREF]);
+        if (in_lob(o, lob0, lob1))  // Sigma as a float pair near the planets
+          at(odens + (long)(nr + 1) * ns + l, jf) = (float)(xs - (double)hs);
+      }
     }
-  }
-  __syncthreads();
-
-  // ---- S3: viscous velocity update (Kernels.cu:118-150) ----
-#pragma unroll
-  for (int kq = 0; kq < SRC32_PER_THREAD; kq++) {
-    const int q = tid + kq * SRC32_TPB;
-    if (q >= hr * HC) break;
-    int r = q / HC, cc = q - r * HC;
-    int i = GI(r);
-    if (r < 2 || r >= hr - 1 || cc < 3 || cc >= HC - 3 || i < 1 || i >= nr) continue;
-    const float iRm = (float)rt[RT_IMED][r];
-    const int ro = r - HALO_R, co = cc - HALO_C;
-    const bool own = ro >= 0 && ro < th && co >= 0 && co < TW;
-    if (i < nr - 1 && r < hr - 2) {
-      float d = dtf * iRm *
-                (((float)rt[RT_SUP][r] * sE[r + 1][cc] - (float)rt[RT_INF][r] * sE[r][cc]) * (float)rt[RT_IDSUP][r] +
-                 (sD[r][cc] - sD[r][cc - 1]) * invdphi + 0.5f * (sE[r][cc] + sE[r + 1][cc])) *
-                rcp_f(0.5f * (sS[r][cc] + sS[r][cc - 1]));
-      sB[r][cc] += d;
-      if (own) incT[ro][co] += d;
+  };
+  auto march = [&](auto inner) __attribute__((always_inline)) {
+    const int m0 = i0 - SRC_HT;  // (as k_src)
+    step(m0, LVL(0), LVL(0), inner);
+    step(m0 + 1, LVL(1), LVL(1), inner);
+    step(m0 + 2, LVL(2), LVL(2), inner);
+    step(m0 + 3, LVL(3), LVL(0), inner);
+    step(m0 + 4, LVL(4), LVL(1), inner);
+    int m = m0 + 5;
+    for (; m + 2 <= i1 + 1; m += 3) {
+      step(m, LVL(5), LVL(2), inner);
+      step(m + 1, LVL(5), LVL(0), inner);
+      step(m + 2, LVL(5), LVL(1), inner);
     }
-    float d = dtf * (float)rt[RT_IINF][r] *
-              (((float)rt[RT_MED][r] * sC[r][cc] - (float)rt[RT_MED][r - 1] * sC[r - 1][cc]) * (float)rt[RT_IDMED][r] +
-               (sE[r][cc + 1] - sE[r][cc]) * invdphi - 0.5f * (sD[r][cc] + sD[r - 1][cc])) *
-              rcp_f(0.5f * (sS[r][cc] + sS[r - 1][cc]));
-    sA[r][cc] += d;
-    if (own) incR[ro][co] += d;
-  }
-  __syncthreads();
-
-  // ---- S4: artificial pressure (Kernels.cu:409-434) ----
-#pragma unroll
-  for (int kq = 0; kq < SRC32_PER_THREAD; kq++) {
-    const int q = tid + kq * SRC32_TPB;
-    if (q >= hr * HC) break;
-    int r = q / HC, cc = q - r * HC;
-    int i = GI(r);
-    if (r < 3 || r >= hr - 1 || cc < 3 || cc >= HC - 4 || i < 0 || i >= nr) continue;
-    sC[r][cc] = art_visc_q_f(sS[r][cc], sA[r + 1][cc] - sA[r][cc]);
-    sD[r][cc] = art_visc_q_f(sS[r][cc], sB[r][cc + 1] - sB[r][cc]);
-  }
-  __syncthreads();
-
-  // ---- S5: velocity update ("kernel", Kernels.cu:438-479), damping #2 ----
-  // (the own cells' state as adjusted by S0 is still in os, ovr, ovt)
-#pragma unroll
-  for (int k = 0; k < SRC32_OWN_MAX; k++) {
-    const int q = tid + k * SRC32_TPB;
-    if (q >= th * TW) break;
-    int ro = q / TW, co = q % TW;
-    int r = ro + HALO_R, cc = co + HALO_C;
-    int i = GI(r), j = j0 + co;
-    if (i > nr || j >= ns) continue;
-    long l = (long)i * ns + j;
-    double s = os[k], vr = ovr[k], vt = ovt[k];
-    const double *ev = evc[r];
-    if (a.opress && i < nr) a.opress[l] = s * rt[RT_CS][r] * rt[RT_CS][r];
-    if (i == nr) {  // ghost ring (never read)
-      a.odens[l] = 0.0f;
-      a.ovr[l] = 0.0f;
-      a.ovt[l] = 0.0f;
-      continue;
-    }
-    double vrnew = 0.0;
-    if (i > 0) {
-      float dq = (sC[r][cc] - sC[r - 1][cc]) * 2.0f * rcp_f(sS[r][cc] + sS[r - 1][cc]) * (float)rt[RT_IDMED][r];
-      vrnew = vr + (double)(incR[ro][co] - dtf * dq);
-    }
-    float dq = (sD[r][cc] - sD[r][cc - 1]) * 2.0f * rcp_f(sS[r][cc] + sS[r][cc - 1]) * (float)rt[RT_IDXT][r];
-    double vtnew = vt + (double)(incT[ro][co] - dtf * dq);
-    if (a.evanescent && rt[RT_EVZ][r] != 0.0) {
-      vrnew = damp_toward(vrnew, ev[0], ev[1]);
-      vtnew = damp_toward(vtnew, ev[0], ev[2]);
-      s = damp_toward(s, ev[0], rt[RT_SMED][r]);
-    }
-    const double xs = s - rt[RT_SBAR][r], xv = vtnew - rt[RT_VREF][r];
-    const float hs = (float)xs, hv = (float)vrnew, ht = (float)xv;
-    a.odens[l] = hs;
-    a.ovr[l] = hv;
-    a.ovt[l] = ht;
-    if (in_lob(i, a.lob0, a.lob1))  // Sigma as a float pair near the planets
-      a.odens[(long)(nr + 1) * ns + l] = (float)(xs - (double)hs);
-  }
-#undef GI
-#undef GJ
+    if (m <= i1 + 1) step(m, LVL(5), LVL(2), inner);
+    if (m + 1 <= i1 + 1) step(m + 1, LVL(5), LVL(0), inner);
+  };
+#undef LVL
+  if (i0 - SRC_HT >= 1 && i1 + SRC_HB <= nr)
+    march(std::true_type());
+  else
+    march(std::false_type());
 }
 
-// one kernel per tile height (8, 16 or 32, the heights fg_set_tiles
-// accepts): each instance needs only its own registers
-template <int ROWS>
-__global__ __launch_bounds__(SRC32_TPB) void k_src32(src32_args a) {
-  extern __shared__ float lds_src32[];
-  src32_tile<ROWS>(a, blockIdx.x, blockIdx.y, lds_src32);
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SRC32_WAVES))) void k_src32(src32_args a) {
+  __shared__ src32_lds lds;
+  const int block = xcd_block(a.nstrips * ((a.nr + a.band) / a.band));
+  if (block < 0) return;
+  const auto &more = ((__attribute__((address_space(4))) const src32_args *)__builtin_amdgcn_kernarg_segment_ptr())->P;
+  src32_march(a, more, block, lds);
 }
 
 // Radial sweep in FP32 (k_trad above): Q of each ring is formed in FP64,
@@ -2851,17 +2758,20 @@ static int plain_potential(const fg_ctx *c, const fg_planet_pot *pl, int nb) {
 // Rings per band of a kernel whose waves march over `rows` rings in column
 // strips: the band with the least estimated time, up to `most`.  A wave
 // spends about one time unit (1 us) on a step when it has its SIMD to itself
-// and shares the SIMD's issue at 0.7 units per step and wave, and a band of H
-// rings costs H + 3 steps (the first ones are partial); up to three waves per
-// SIMD are resident, so the fullest SIMD counts, beyond that the total does.
-static int march_band(int rows, int nstrips, int most) {
+// and shares the SIMD's issue at `share` units per step and wave, and a band of
+// H rings costs H + 3 steps (the first ones are partial); up to `resident` waves
+// per SIMD are there at once, so the fullest SIMD counts, beyond that the total
+// does.  A batch's disks share the SIMDs.
+// disks: rows, strips of each
+static int march_band(const std::vector<int2> &disks, int most, int resident = 3, double share = 0.7) {
   const int simds = 1024;
   double best = 0.0;
   int band = 1;
   for (int h = 1; h <= most; h++) {
-    const long waves = (long)nstrips * ((rows + h - 1) / h);
+    long waves = 0;
+    for (const int2 &d : disks) waves += (long)d.y * ((d.x + h - 1) / h);
     const double n = (double)waves / simds;
-    const double cost = (h + 3) * (n > 3.0 ? 0.7 * n : std::max(1.0, 0.7 * ceil(n)));
+    const double cost = (h + 3) * (n > resident ? share * n : std::max(1.0, share * ceil(n)));
     if (h == 1 || cost < best) {
       best = cost;
       band = h;
@@ -2872,14 +2782,19 @@ static int march_band(int rows, int nstrips, int most) {
 // Measured for k_src (us, FP64 isothermal): 128x384 1 ring 11.7, 8 rings 19;
 // 512x1536 7-8 rings 24, 4 rings 28, 20 rings 36; 1024x3072 18-20 rings 50,
 // 8 rings 57, 26 rings 57; 2048x4096 18-26 rings 107, 8 rings 121.
-static int src_band(int nr, int nstrips) { return march_band(nr + 1, nstrips, SRC_MAX_BAND); }
+static int src_band(int nr, int nstrips) { return march_band({make_int2(nr + 1, nstrips)}, SRC_MAX_BAND); }
+// Measured for k_src32, four waves per SIMD at 1.4 us a step (us with 3 of
+// launch): 128x384 1 ring 12.7, 8 rings 19, 16 rings 29; 256x768 2 rings 14.8, 8
+// rings 20; 512x1536 6 rings 21.9, 13 rings 27.6; 1024x3072 20 rings 42, 10
+// rings 44, 27 rings 53.  fg_set_tiles fixes the band instead.
+static int src32_band(const std::vector<int2> &disks) { return march_band(disks, SRC_MAX_BAND, SRC32_WAVES, 0.44); }
 // Measured for k_trad (us): 128x384 2-3 rings 11.9, 16 rings 21.5; 301x998
 // (with energy) 3-6 rings 18, 16 rings 25; 512x1536 8 rings 23, 16 rings 26;
 // from 1024x3072 on, where HBM bounds it, 10 to 16 rings are within 3 % and
 // 20 to 32 cost 5 %; k_trad32 256x768 3-4 rings 14, 16 rings 23.5.  fg_set_tiles
 // fixes the band instead.
 static int trad_band(const fg_ctx *c, int nstrips) {
-  return c->tile_trad_band ? c->tile_trad_band : march_band(c->nr, nstrips, 16);
+  return c->tile_trad_band ? c->tile_trad_band : march_band({make_int2(c->nr, nstrips)}, 16);
 }
 
 extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, double domega,
@@ -2938,7 +2853,6 @@ extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, dou
   sa.ns = ns;
   sa.indirect = c->p.indirect_term;
   sa.evanescent = c->p.evanescent;
-  const int corotating = (domega != 0.0) ? 1 : 0;
   if (c->prof_on) {
     (void)hipStreamSynchronize(c->stream);
     prof_fold(c);
@@ -2972,17 +2886,11 @@ extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, dou
     s3.ns = ns;
     s3.indirect = sa.indirect;
     s3.evanescent = sa.evanescent;
-    s3.corotating = corotating;
-    const int th = c->tile_src_th;
-    FG_HIP(hipFuncSetAttribute((const void *)k_src32<32>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)src32_lds_bytes(32)));
-    const dim3 g32((ns + TW - 1) / TW, (nr + 1 + th - 1) / th);
-    if (th == 8)
-      hipLaunchKernelGGL(k_src32<8>, g32, dim3(SRC32_TPB), src32_lds_bytes(8), c->stream, s3);
-    else if (th == 32)
-      hipLaunchKernelGGL(k_src32<32>, g32, dim3(SRC32_TPB), src32_lds_bytes(32), c->stream, s3);
-    else
-      hipLaunchKernelGGL(k_src32<16>, g32, dim3(SRC32_TPB), src32_lds_bytes(16), c->stream, s3);
+    s3.nstrips = (ns + SRC_W - 1) / SRC_W;
+    s3.width = (ns + s3.nstrips - 1) / s3.nstrips;
+    s3.band = c->tile_src_th ? std::min(c->tile_src_th, SRC_MAX_BAND)
+                             : src32_band({make_int2(nr + 1, s3.nstrips)});
+    hipLaunchKernelGGL(k_src32, dim3(xcd_grid(s3.nstrips * ((nr + s3.band) / s3.band))), dim3(64), 0, c->stream, s3);
   } else {
     sa.nstrips = (ns + SRC_W - 1) / SRC_W;
     sa.width = (ns + sa.nstrips - 1) / sa.nstrips;
@@ -3282,10 +3190,6 @@ struct batch_disk {
   trad_args trad;
   taz_args taz;
   fin_args fin;
-  force_src force;
-  long ncell;      // NRAD * NSEC
-  int B;           // DeviceReduce blocks of the force sum
-  double *partial; // block sums (the context's reduction scratch)
   double *DT1D, *Vmoy, *newDT;
   const double *invRmed;
   double coef, DeltaT;  // CFL coefficient and the next substep's DeltaT
@@ -3297,80 +3201,103 @@ struct batch_result {
   int cfl, pad;
 };
 
-// Each phase launch covers its whole work list, one workgroup per item (the
-// kernels keep a grid-stride loop, so any grid is correct).  Measured on
-// 64 disks: 1.83 ms per batch substep with 4096 looping workgroups per
-// phase, 1.61 ms with one item per workgroup.
-#define BATCH_CAP_BLOCKS (1 << 20)
+// Each phase launch covers its whole work list, one workgroup per item.
+// Measured on 64 disks: 1.83 ms per batch substep with 4096 looping workgroups
+// per phase, 1.61 ms with one item per workgroup.
 
 // work items are the same for the whole workgroup: keep them (and every
 // address derived from them) in scalar registers
-__device__ __forceinline__ int4 uniform4(int4 w) {
-  return make_int4(__builtin_amdgcn_readfirstlane(w.x), __builtin_amdgcn_readfirstlane(w.y),
-                   __builtin_amdgcn_readfirstlane(w.z), __builtin_amdgcn_readfirstlane(w.w));
-}
 __device__ __forceinline__ int2 uniform2(int2 w) {
   return make_int2(__builtin_amdgcn_readfirstlane(w.x), __builtin_amdgcn_readfirstlane(w.y));
 }
 
-// one work item per workgroup: without a loop's carried scalars the tile's
-// uniform arguments fit the SGPRs instead of spilling into VGPR lanes
-// (253 -> 112 VGPRs)
-template <int ROWS>
-__global__ __launch_bounds__(SRC32_TPB) void k_batch_src(const batch_disk *__restrict__ D, const int4 *__restrict__ items, int n) {
-  extern __shared__ float lds_bsrc[];
-  if ((int)blockIdx.x >= n) return;
-  const int4 w = uniform4(items[blockIdx.x]);
-  if (D[w.x].active) src32_tile<ROWS>(D[w.x].src, w.y, w.z, lds_bsrc);
+// a phase's arguments with their pointers as global ones
+__device__ __forceinline__ fg_dev_tables global_tables(const fg_dev_tables &t) {
+  fg_dev_tables g = t;
+  for (double **p : {&g.Radii, &g.Rinf, &g.Rsup, &g.Rmed, &g.Surf, &g.invRinf, &g.invSurf, &g.invRmed, &g.invdiffRsup,
+                     &g.invdiffRmed, &g.SigmaMed, &g.cs_iso, &g.dxtheta, &g.invdxtheta, &g.dxtheta_cfl, &g.ev_coef,
+                     &g.ev_period, &g.ev_vtheta_arg, &g.cos_cell, &g.sin_cell})
+    *p = global(*p);
+  g.ev_zone = global(g.ev_zone);
+  return g;
+}
+
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SRC32_WAVES))) void k_batch_src(
+    const batch_disk *__restrict__ D, const int2 *__restrict__ items, int n) {
+  __shared__ src32_lds lds;
+  const int it = xcd_block(n);
+  if (it < 0) return;
+  const int2 w = uniform2(items[it]);
+  if (D[w.x].active) src32_march(D[w.x].src, D[w.x].src.P, w.y, lds);
 }
 
 __global__ __launch_bounds__(TRAD_TPB) void k_batch_trad(const batch_disk *__restrict__ D, const int2 *__restrict__ items, int n) {
-  for (int it = blockIdx.x; it < n; it += gridDim.x) {
-    const int2 w = uniform2(items[it]);
-    if (D[w.x].active) trad32_block(D[w.x].trad, w.y);
-    __syncthreads();
-  }
+  if ((int)blockIdx.x >= n) return;
+  const int2 w = uniform2(items[blockIdx.x]);
+  if (!D[w.x].active) return;
+  trad_args a = D[w.x].trad;
+  a.t = global_tables(a.t);
+  a.fdens = global(a.fdens);
+  a.fvr = global(a.fvr);
+  a.fvt = global(a.fvt);
+  for (int q = 0; q < NQ; q++) a.fout[q] = global(a.fout[q]);
+  a.sbar = global(a.sbar);
+  a.vref = global(a.vref);
+  a.vmed = global(a.vmed);
+  trad32_block(a, w.y);
 }
 
 // one chunk of one ring per item: y = ring * chunks + chunk
 __global__ __launch_bounds__(64) void k_batch_taz(const batch_disk *__restrict__ D, const int2 *__restrict__ items, int n) {
   __shared__ tazw_lds<4, 5> sh;
-  for (int it = blockIdx.x; it < n; it += gridDim.x) {
-    const int2 w = uniform2(items[it]);
-    if (D[w.x].active) {
-      const int nch = (D[w.x].taz.ns + TAZW_P32 - 1) / TAZW_P32;
-      const int i = w.y / nch;
-      if (in_lob(i, D[w.x].taz.lob0, D[w.x].taz.lob1))
-        tazw_body<4, true, 5, true>(D[w.x].taz, i, w.y % nch, sh);
-      else
-        tazw_body<4, true, 5, false>(D[w.x].taz, i, w.y % nch, sh);
-    }
-    __syncthreads();
-  }
+  if ((int)blockIdx.x >= n) return;
+  const int2 w = uniform2(items[blockIdx.x]);
+  if (!D[w.x].active) return;
+  taz_args a = D[w.x].taz;
+  a.t = global_tables(a.t);
+  a.vmed = global(a.vmed);
+  a.fvt = global(a.fvt);
+  for (int q = 0; q < NQ; q++) a.fq[q] = global(a.fq[q]);
+  a.fxd = global(a.fxd);
+  a.fxvt = global(a.fxvt);
+  a.fxrmp = global(a.fxrmp);
+  a.fxrmm = global(a.fxrmm);
+  a.sbar = global(a.sbar);
+  a.vref = global(a.vref);
+  a.nshift = global(a.nshift);
+  const int nch = (a.ns + TAZW_P32 - 1) / TAZW_P32;
+  const int i = w.y / nch;
+  if (in_lob(i, a.lob0, a.lob1))
+    tazw_body<4, true, 5, true>(a, i, w.y % nch, sh);
+  else
+    tazw_body<4, true, 5, false>(a, i, w.y % nch, sh);
 }
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_batch_fin(const batch_disk *__restrict__ D, const int2 *__restrict__ items, int n) {
   extern __shared__ double lds_bfin[];
-  for (int it = blockIdx.x; it < n; it += gridDim.x) {
-    const int2 w = uniform2(items[it]);
-    if (D[w.x].active) {
-      const fin_args &fa = D[w.x].fin;
-      if (in_lob(w.y, fa.lob0 - 1, fa.lob1 + 1))
-        fin_ring<1, false, true, true>(fa, w.y, lds_bfin);
-      else
-        fin_ring<1, false, true, false>(fa, w.y, lds_bfin);
-    }
-    __syncthreads();
-  }
-}
-
-__global__ __launch_bounds__(RED_TPB) void k_batch_force(const batch_disk *__restrict__ D, const int2 *__restrict__ items, int n) {
-  for (int it = blockIdx.x; it < n; it += gridDim.x) {
-    const int2 w = uniform2(items[it]);
-    const batch_disk &d = D[w.x];
-    if (d.active) dreduce_block(d.force, d.ncell, d.B, w.y, d.partial);
-    __syncthreads();
-  }
+  if ((int)blockIdx.x >= n) return;
+  const int2 w = uniform2(items[blockIdx.x]);
+  if (!D[w.x].active) return;
+  fin_args a = D[w.x].fin;
+  a.t = global_tables(a.t);
+  a.dens = global(a.dens);
+  a.vr = global(a.vr);
+  a.vt = global(a.vt);
+  a.fxd = global(a.fxd);
+  a.fxvt = global(a.fxvt);
+  a.fxrmp = global(a.fxrmp);
+  a.fxrmm = global(a.fxrmm);
+  a.sbar = global(a.sbar);
+  a.sbar_next = global(a.sbar_next);
+  a.vmoy = global(a.vmoy);
+  a.newdt = global(a.newdt);
+  a.fpart = global(a.fpart);
+  a.crash = global(a.crash);
+  a.nu = global(a.nu);
+  if (in_lob(w.y, a.lob0 - 1, a.lob1 + 1))
+    fin_ring<1, false, true, true>(a, w.y, lds_bfin);
+  else
+    fin_ring<1, false, true, false>(a, w.y, lds_bfin);
 }
 
 // per disk: the force's final sum and the CFL count of the next substep
@@ -3397,10 +3324,9 @@ struct fg_batch_dev {
   hipStream_t stream;
   batch_disk *h_disk, *d_disk;  // pinned host block and its device copy
   batch_result *h_res, *d_res;
-  int4 *it_src;
-  int2 *it_trad, *it_taz, *it_fin, *it_force;
-  int n_src, n_trad, n_taz, n_fin, n_force;
-  int n_src_rows[3];  // source items of tile height 8, 16, 32 (in that order in it_src)
+  int2 *it_src, *it_trad, *it_taz, *it_fin;
+  int n_src, n_trad, n_taz, n_fin;
+  int src_band, trad_band;  // of the disks without fixed ones
   int max_ns;
   hipGraph_t graph;
   hipGraphExec_t exec;
@@ -3410,7 +3336,7 @@ struct fg_batch_dev {
 static void batch_free(fg_batch_dev *b) {
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
-  void *dev[] = {b->d_disk, b->d_res, b->it_src, b->it_trad, b->it_taz, b->it_fin, b->it_force};
+  void *dev[] = {b->d_disk, b->d_res, b->it_src, b->it_trad, b->it_taz, b->it_fin};
   for (void *q : dev)
     if (q) (void)hipFree(q);
   if (b->h_disk) (void)hipHostFree(b->h_disk);
@@ -3446,6 +3372,13 @@ fg_status fg_batch_dev_create(fg_ctx *const *ctx, int n, fg_batch_dev **out) {
   fg_batch_dev *b = new fg_batch_dev();
   b->n = n;
   b->ctx.assign(ctx, ctx + n);
+  std::vector<int2> src, trad;
+  for (int k = 0; k < n; k++) {
+    src.push_back(make_int2(ctx[k]->nr + 1, (ctx[k]->ns + SRC_W - 1) / SRC_W));
+    trad.push_back(make_int2(ctx[k]->nr, (ctx[k]->ns + TRAD_TPB - 1) / TRAD_TPB));
+  }
+  b->src_band = src32_band(src);
+  b->trad_band = march_band(trad, 16);
   hipError_t e = hipStreamCreate(&b->stream);
   if (e == hipSuccess) e = hipHostMalloc((void **)&b->h_disk, n * sizeof(batch_disk), hipHostMallocDefault);
   if (e == hipSuccess) e = hipHostMalloc((void **)&b->h_res, n * sizeof(batch_result), hipHostMallocDefault);
@@ -3469,29 +3402,29 @@ static fg_status upload_items(const std::vector<T> &v, T **dev) {
   return FG_OK;
 }
 
-// work lists (largest disks first) and the captured graph of one substep
-// rings per radial-sweep band of a batched disk (the other disks fill the
-// chip, so a band as long as a large grid's)
-static int batch_band(const fg_ctx *c) { return c->tile_trad_band ? c->tile_trad_band : 16; }
+// rings per band of a batched disk's source march and radial sweep: those that
+// suit all the disks together (8 disks of 128 to 384 rings: 8 rings of the radial
+// sweep 187 us per substep, 16 rings 194; 64 disks 891 and 879)
+static int batch_src_band(const fg_batch_dev *b, const fg_ctx *c) {
+  return c->tile_src_th ? std::min(c->tile_src_th, SRC_MAX_BAND) : b->src_band;
+}
+static int batch_trad_band(const fg_batch_dev *b, const fg_ctx *c) {
+  return c->tile_trad_band ? c->tile_trad_band : b->trad_band;
+}
 
+// work lists (largest disks first) and the captured graph of one substep
 static fg_status batch_build(fg_batch_dev *b) {
   std::vector<int> order(b->n);
   for (int k = 0; k < b->n; k++) order[k] = k;
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return b->ctx[x]->S > b->ctx[y]->S; });
-  std::vector<int4> src_rows[3];  // by tile height 8, 16, 32
-  std::vector<int2> trad, taz, fin, force;
+  std::vector<int2> src, trad, taz, fin;
   b->max_ns = 1;
   for (int k : order) {
     const fg_ctx *c = b->ctx[k];
-    const int nr = c->nr, ns = c->ns, th = c->tile_src_th, band = batch_band(c);
-    if ((th != 8 && th != 16 && th != 32) || band < 1) {
-      fg_set_error("batch: disk %d has tile shape th=%d band=%d", k, th, band);
-      return FG_E_INVALID;
-    }
+    const int nr = c->nr, ns = c->ns, band = batch_trad_band(b, c), sband = batch_src_band(b, c);
     b->max_ns = std::max(b->max_ns, ns);
-    std::vector<int4> &src = src_rows[th == 8 ? 0 : th == 16 ? 1 : 2];
-    for (int by = 0; by < (nr + 1 + th - 1) / th; by++)
-      for (int bx = 0; bx < (ns + TW - 1) / TW; bx++) src.push_back(make_int4(k, bx, by, th));
+    const int nsrc = (ns + SRC_W - 1) / SRC_W * ((nr + sband) / sband);
+    for (int q = 0; q < nsrc; q++) src.push_back(make_int2(k, q));
     const int nstrips = (ns + TRAD_TPB - 1) / TRAD_TPB;
     const int nblk = nr + nstrips * ((nr + band - 1) / band);
     for (int q = 0; q < nblk; q++) trad.push_back(make_int2(k, q));
@@ -3500,48 +3433,25 @@ static fg_status batch_build(fg_batch_dev *b) {
       for (int ch = 0; ch < nch; ch++) taz.push_back(make_int2(k, i * nch + ch));
       fin.push_back(make_int2(k, i));
     }
-    const int B = red_blocks((long)nr * ns);
-    for (int q = 0; q < B; q++) force.push_back(make_int2(k, q));
-  }
-  std::vector<int4> src;
-  for (int h = 0; h < 3; h++) {
-    b->n_src_rows[h] = (int)src_rows[h].size();
-    src.insert(src.end(), src_rows[h].begin(), src_rows[h].end());
   }
   b->n_src = (int)src.size();
   b->n_trad = (int)trad.size();
   b->n_taz = (int)taz.size();
   b->n_fin = (int)fin.size();
-  b->n_force = (int)force.size();
   if (fg_status s = upload_items(src, &b->it_src)) return s;
   if (fg_status s = upload_items(trad, &b->it_trad)) return s;
   if (fg_status s = upload_items(taz, &b->it_taz)) return s;
   if (fg_status s = upload_items(fin, &b->it_fin)) return s;
-  if (fg_status s = upload_items(force, &b->it_force)) return s;
-  FG_HIP(hipFuncSetAttribute((const void *)k_batch_src<32>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)src32_lds_bytes(32)));
   // capture: arguments in, five phases, two reductions, results out
   hipStream_t st = b->stream;
   FG_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-  auto grid = [](int n) { return dim3(n < BATCH_CAP_BLOCKS ? (n > 0 ? n : 1) : BATCH_CAP_BLOCKS); };
   (void)hipMemcpyAsync(b->d_disk, b->h_disk, b->n * sizeof(batch_disk), hipMemcpyHostToDevice, st);
-  // one source launch per tile height present (the work list holds them
-  // in order 8, 16, 32)
-  {
-    const int4 *it = b->it_src;
-    const int n8 = b->n_src_rows[0], n16 = b->n_src_rows[1], n32 = b->n_src_rows[2];
-    if (n8) hipLaunchKernelGGL(k_batch_src<8>, dim3(n8), dim3(SRC32_TPB), src32_lds_bytes(8), st, b->d_disk, it, n8);
-    if (n16)
-      hipLaunchKernelGGL(k_batch_src<16>, dim3(n16), dim3(SRC32_TPB), src32_lds_bytes(16), st, b->d_disk, it + n8, n16);
-    if (n32)
-      hipLaunchKernelGGL(k_batch_src<32>, dim3(n32), dim3(SRC32_TPB), src32_lds_bytes(32), st, b->d_disk,
-                         it + n8 + n16, n32);
-  }
-  hipLaunchKernelGGL(k_batch_trad, grid(b->n_trad), dim3(TRAD_TPB), 0, st, b->d_disk, b->it_trad, b->n_trad);
-  hipLaunchKernelGGL(k_batch_taz, grid(b->n_taz), dim3(64), 0, st, b->d_disk, b->it_taz, b->n_taz);
-  hipLaunchKernelGGL(k_batch_fin, grid(b->n_fin), dim3(256), (size_t)b->max_ns * sizeof(double), st, b->d_disk,
+  hipLaunchKernelGGL(k_batch_src, dim3(xcd_grid(b->n_src)), dim3(64), 0, st, b->d_disk, b->it_src, b->n_src);
+  hipLaunchKernelGGL(k_batch_trad, dim3(b->n_trad), dim3(TRAD_TPB), 0, st, b->d_disk, b->it_trad, b->n_trad);
+  hipLaunchKernelGGL(k_batch_taz, dim3(b->n_taz), dim3(64), 0, st, b->d_disk, b->it_taz, b->n_taz);
+  hipLaunchKernelGGL(k_batch_fin, dim3(b->n_fin), dim3(256), (size_t)b->max_ns * sizeof(double), st, b->d_disk,
                      b->it_fin, b->n_fin);
-  hipLaunchKernelGGL(k_batch_close, grid(b->n), dim3(256), 0, st, b->d_disk, b->d_res, b->n);
+  hipLaunchKernelGGL(k_batch_close, dim3(b->n), dim3(256), 0, st, b->d_disk, b->d_res, b->n);
   (void)hipMemcpyAsync(b->h_res, b->d_res, b->n * sizeof(batch_result), hipMemcpyDeviceToHost, st);
   hipError_t ce = hipStreamEndCapture(st, &b->graph);
   if (ce != hipSuccess) {
@@ -3606,7 +3516,9 @@ fg_status fg_batch_dev_set(fg_batch_dev *b, int k, int active, double dt, double
   s.ns = ns;
   s.indirect = c->p.indirect_term;
   s.evanescent = c->p.evanescent;
-  s.corotating = (domega != 0.0) ? 1 : 0;
+  s.nstrips = (ns + SRC_W - 1) / SRC_W;
+  s.width = (ns + s.nstrips - 1) / s.nstrips;
+  s.band = batch_src_band(b, c);
   trad_args &ta = d.trad;
   ta.dens = fb.Bd;
   ta.vr = fb.Bvr;
@@ -3629,7 +3541,7 @@ fg_status fg_batch_dev_set(fg_batch_dev *b, int k, int active, double dt, double
   ta.nr = nr;
   ta.ns = ns;
   ta.nstrips = (ns + TRAD_TPB - 1) / TRAD_TPB;
-  ta.band = batch_band(c);
+  ta.band = batch_trad_band(b, c);
   ta.lob0 = lob0;
   ta.lob1 = lob1;
   taz_args &za = d.taz;
@@ -3696,10 +3608,6 @@ fg_status fg_batch_dev_set(fg_batch_dev *b, int k, int active, double dt, double
   fa.sbar_next = sbar_next;
   fa.lob0 = lob0;
   fa.lob1 = lob1;
-  d.force = force_src{c->f[FG_DENS], c->t.Surf, c->t.Rmed, c->t.cos_cell, c->t.sin_cell, 0.0, 0.0, 0.0, ns};
-  d.ncell = (long)nr * ns;
-  d.B = red_blocks(d.ncell);
-  d.partial = c->red_partial;
   d.DT1D = c->DT1D;
   d.Vmoy = c->Vmoy;
   d.newDT = c->newDT;
@@ -3738,8 +3646,7 @@ void fg_batch_dev_invalidate(fg_batch_dev *b) {
   if (b->graph) (void)hipGraphDestroy(b->graph);
   b->exec = nullptr;
   b->graph = nullptr;
-  for (void **q : {(void **)&b->it_src, (void **)&b->it_trad, (void **)&b->it_taz, (void **)&b->it_fin,
-                   (void **)&b->it_force}) {
+  for (void **q : {(void **)&b->it_src, (void **)&b->it_trad, (void **)&b->it_taz, (void **)&b->it_fin}) {
     if (*q) (void)hipFree(*q);
     *q = nullptr;
   }

@@ -237,9 +237,9 @@ fg_status fg_step_fused(fg_ctx *ctx, double dt, double omega_frame, double domeg
 /* CFL count and star force of the current state (fused reductions) */
 fg_status fg_fused_prepare(fg_ctx *ctx, double DeltaT);
 fg_status fg_fused_results(fg_ctx *ctx, int *ncfl, double *force2, double *lost_mass);
-/* Tile shapes of the fused kernels: rings per FP32 source tile (8, 16
- * or 32) and rings per radial-sweep band (without a call 16, and a band picked
- * for the grid).  Results do not depend on them; the
+/* Tile shapes of the fused kernels: rings per band of the FP32 source march (8,
+ * 16 or 32, held to 27) and of the radial sweep (without a call, bands picked for
+ * the grid, in a batch for all its disks together).  Results do not depend on them; the
  * autotuner (cudaprotoplanetarydisks_amd/autotune.py) picks them per grid.
  * No reference counterpart (the reference's launch shape is fixed,
  * Main.cu:204-226). */
