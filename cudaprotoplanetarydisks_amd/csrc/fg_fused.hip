@@ -633,7 +633,9 @@ struct trad_args {
 // (the next 512 loaded into registers meanwhile) and lane 0 adds them in j
 // order with its LDS reads issued ahead of the dependent adds.  One wave:
 // the barrier only orders the LDS accesses, and lane 0 has finished a
-// round's sum before the next round's stores in program order.
+// round's sum before the next round's stores in program order.  (The sum by the
+// whole wave's lanes, as ring_seq_sum, was no faster here: 512 x 1536 28.8
+// against 25.7 us for the kernel, 1024 x 3072 the same, 2048 x 4096 131 and 137.)
 #define RMW_CH 8  // sectors per lane per round
 __device__ void ring_mean_wave(const double *v, int ns, double *out) {
   __shared__ double buf[64 * RMW_CH];
@@ -654,14 +656,6 @@ __device__ void ring_mean_wave(const double *v, int ns, double *out) {
     __syncthreads();
   }
   if (lane == 0) *out = sum / (double)ns;
-}
-
-// x of lane `lane` (uniform), as scalars
-__device__ __forceinline__ double lane_get(double x, int lane) {
-  const long long b = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_readlane((int)b, lane);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
 // Ring tables of the rings a column strip marches over, one ring per lane
@@ -1441,9 +1435,6 @@ __global__ __launch_bounds__(256) void k_force_rings_cfl(const double *fpart, in
   seq_store(out2, seq);
 }
 
-// one ring; ring holds NSEC doubles (the ring's final vtheta).  FIN_B
-// cells per thread have their loads issued together (4 for the single-disk
-// kernel; 1 in the batched one, which would otherwise lose a wave per SIMD)
 // minimum over the workgroup's 256 threads into *out (thread 0): within
 // each wave by shuffles, then the four wave minima (a minimum does not
 // depend on the order of its comparisons)
@@ -1463,155 +1454,227 @@ __device__ __forceinline__ void ring_min_store(double best, double *red, double 
   }
 }
 
-#define FIN_OV_K 16  // cells per thread of the overlapped CFL pass (rings up to 3072 cells)
-// PAIRS: FP32 mode, ring i - 1, i or i + 1 stored as float pairs (its own
-// instance, so that the other rings run without the residuals' loads)
-template <int FIN_B, bool ADI = false, bool S32 = false, bool PAIRS = false>
+// One ring by 256 threads, thread t its cells t, t + 256, ...; ring: NSEC doubles
+// of LDS.  First the final vtheta of every cell goes to LDS and its ring mean
+// is formed (FP64: ring_seq_sum; the FP32 mode, which does not
+// replay the reference's summation order, from the threads' own sums), then one
+// pass over the cells does the rest: ComputeVelocities (Kernels.cu:1200-1205)
+// with the energy, sound speed and temperature of an adiabatic deck, and the
+// cell's CFL time step (Kernels.cu:1284-1329).  Every cell issues the same memory
+// operations, its loads one cell ahead, so that the waits for them count past
+// the stores: threads without a cell left repeat the last one's.
+// The ring minimum of dt = 0.5 / sqrt(S) over the cells is taken as one
+// quotient at the largest S: rounded sqrt and rounded division are both
+// monotone, so 0.5 / sqrt(max S) is the smallest rounded dt bit for bit
+// (a NaN S is skipped by both comparisons; the 1e30 start caps both).
+// ADI: adiabatic deck; S32: FP32 bulk mode (FP32 storage of k_taz's fields);
+// PAIRS: ring i - 1, i or i + 1 stored as float pairs (its own instance, so that
+// the other rings run without the residuals' loads).
+// Bound: HBM on large grids (2048 x 4096: 454 MB in 112 us), latency on small
+// ones.  Was one lane's sum of the ring beside a pass that kept its terms in
+// registers (and two passes over rings beyond 3072 cells): 1024 x 3072 58 -> 51
+// us, 2048 x 4096 201 -> 112, 512 x 1536 24 -> 17; FP32 1024 x 3072 43 -> 34.
+// Keeping that pass's terms unrolled over 12 or 16 cells was slower than the loop,
+// 512 threads a ring too (two rounds of workgroups).
+template <bool ADI, bool S32, bool PAIRS>
 __device__ __forceinline__ void fin_ring(const fin_args &a, int i, double *ring) {
+  using real = typename std::conditional<S32, float, double>::type;
+  struct cell {
+    real rpm, rm, dm, d, rp, rn, dn;  // momenta and Sigma of rings i - 1, i and i + 1
+    float ym, y, yn;                  // PAIRS: Sigma's residuals
+    double e, c, cosj, sinj;          // energy, sound speed; S32: the cell's direction
+  };
   __shared__ double red[4];
-  __shared__ double s_vmoy;
   const int ns = a.ns, nr = a.nr, tid = threadIdx.x;
   const fg_dev_tables &t = a.t;
-  const long base = (long)i * ns;
+  const long row = (long)i * ns, rowm = (long)max(i - 1, 0) * ns, rown = row + ns, S2 = (long)(nr + 1) * ns;
   double lam_i = 0, vr0_i = 0, vt0_i = 0, lam_n = 0, vr0_n = 0, vt0_n = 0;
   const bool damp_i = a.evanescent && t.ev_zone[i];
   const bool damp_n = a.evanescent && (i + 1 < nr) && t.ev_zone[i + 1];
   if (damp_i) ev_consts(t, a.nu, i, a.dt, a.omega_frame, lam_i, vr0_i, vt0_i, a.sgacc);
   if (damp_n) ev_consts(t, a.nu, i + 1, a.dt, a.omega_frame, lam_n, vr0_n, vt0_n, a.sgacc);
-  constexpr bool adi = ADI;  // an adiabatic deck (a.adiabatic): energy and per-cell sound speed
-  double fsx = 0.0, fcx = 0.0, fsy = 0.0, fcy = 0.0;
+  const bool radial = i > 0, radial_n = i + 1 < nr;  // vrad is 0 on ring 0 and the ghost ring
+  const bool cfl = i > 0;                            // ring 0 has no CFL term (Kernels.cu:1286)
+  // FP32 storage: backgrounds of rings i-1, i, i+1 and of vtheta on ring i
+  const double sb_m = S32 && radial ? a.sbar[i - 1] : 0.0, sb_i = S32 ? a.sbar[i] : 0.0;
+  const double sb_n = S32 && radial_n ? a.sbar[i + 1] : 0.0, vb_i = S32 ? a.vmoy[i] : 0.0;
+  const bool lob_m = PAIRS && in_lob(i - 1, a.lob0, a.lob1), lob_i = PAIRS && in_lob(i, a.lob0, a.lob1);
+  const bool lob_n = PAIRS && in_lob(i + 1, a.lob0, a.lob1);
+  auto fetch = [&](int jc, cell &x) __attribute__((always_inline)) {
+    unsigned o = min(jc, ns - 1) * (unsigned)sizeof(real);
+    asm volatile("" : "+v"(o));  // (the rows' addresses stay scalar)
+    if constexpr (S32) {
+      x.rpm = at(a.fxrmp + rowm, o);
+      x.rm = at(a.fxrmm + row, o);
+      x.dm = at(a.fxd + rowm, o);
+      x.d = at(a.fxd + row, o);
+      x.rp = at(a.fxrmp + row, o);
+      x.rn = at(a.fxrmm + rown, o);
+      x.dn = at(a.fxd + rown, o);
+      x.cosj = at(t.cos_cell, 2 * o);
+      x.sinj = at(t.sin_cell, 2 * o);
+      x.ym = x.y = x.yn = 0.f;
+      if constexpr (PAIRS) {
+        x.ym = at(a.fxd + S2 + rowm, o);
+        x.y = at(a.fxd + S2 + row, o);
+        x.yn = at(a.fxd + S2 + rown, o);
+      }
+    } else {
+      x.rpm = at(a.xrmp + rowm, o);
+      x.rm = at(a.xrmm + row, o);
+      x.dm = at(a.xd + rowm, o);
+      x.d = at(a.xd + row, o);
+      x.rp = at(a.xrmp + row, o);
+      x.rn = at(a.xrmm + rown, o);
+      x.dn = at(a.xd + rown, o);
+      if constexpr (ADI) {
+        x.e = at(a.xe + row, o);
+        x.c = at((const double *)a.cs + row, o);
+      }
+    }
+  };
+  double vsum = 0.0;
+  for (int j0 = tid; j0 < ns; j0 += 256 * 4) {
+    real v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int j = min(j0 + 256 * u, ns - 1);
+      if constexpr (S32)
+        v[u] = a.fxvt[row + j];
+      else
+        v[u] = a.xvt[row + j];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int j = j0 + 256 * u;
+      double vt = S32 ? vb_i + (double)v[u] : v[u];
+      if (damp_i) vt = damp_toward(vt, lam_i, vt0_i);
+      if (j < ns) {
+        ring[j] = vt;
+        if (S32) vsum += vt;
+      }
+    }
+  }
+  cell c0, c1;
+  fetch(tid, c0);
+  __shared__ double fw[S32 ? 4 : 1][5];
+  double vm;
+  if constexpr (S32) {  // per wave by a shuffle tree, the waves in order
+    for (int off = 32; off > 0; off >>= 1) vsum += __shfl_down(vsum, off);
+    if ((tid & 63) == 0) red[tid >> 6] = vsum;
+    __syncthreads();
+    vm = (((red[0] + red[1]) + red[2]) + red[3]) / (double)ns;
+  } else {
+    __syncthreads();
+    vm = ring_seq_sum(ring, ns) / (double)ns;
+  }
+  if (tid == 0) a.vmoy[i] = vm;
   const double Rm = t.Rmed[i], surf = t.Surf[i];
   // star at the origin (x = y = 0, no smoothing): the cell's distance is
   // Rmed, so 1/d^3 is one value per ring (FP32 mode only; the FP64 path
   // sums the reference's per-cell expression in DeviceReduce order)
   const double inv3 = 1.0 / (Rm * Rm) / Rm;
-  const bool radial = i > 0 && i < nr;  // vrad recovery reads rings i-1 and i
-  bool bad = false;                      // a density below 0, infinite or NaN
-  // FP32 storage backgrounds of rings i-1, i, i+1 and of vtheta on ring i
-  const double sb_m = S32 && i > 0 ? a.sbar[i - 1] : 0.0, sb_i = S32 ? a.sbar[i] : 0.0;
-  const double vb_i = S32 ? a.vmoy[i] : 0.0;
-  double vsum = 0.0, ssum = 0.0;  // FP32 mode: this thread's sums of vtheta and Sigma
-  // FP32 storage: Sigma of rings i - 1, i and i + 1 stored as float pairs
-  const bool lob_m = PAIRS && in_lob(i - 1, a.lob0, a.lob1), lob_i = PAIRS && in_lob(i, a.lob0, a.lob1);
-  const bool lob_p = PAIRS && in_lob(i + 1, a.lob0, a.lob1);
-  const long S2 = (long)(nr + 1) * ns;
-  // FIN_B cells per thread per batch: all their loads first, then the math
-  for (int j0 = tid; j0 < ns; j0 += FIN_B * 256) {
-    double lrp[FIN_B], lrm[FIN_B], ld[FIN_B], ldm[FIN_B], lvt[FIN_B], lp[FIN_B], lcs[FIN_B], lsn[FIN_B];
-#pragma unroll
-    for (int u = 0; u < FIN_B; u++) {
-      const int j = j0 + u * 256;
-      lrp[u] = lrm[u] = ld[u] = ldm[u] = lvt[u] = lp[u] = lcs[u] = lsn[u] = 0.0;
-      if (j < ns) {
-        const long l = base + j;
-        if constexpr (S32) {
-          lcs[u] = t.cos_cell[j];
-          lsn[u] = t.sin_cell[j];
-          float hdm = 0.f, ydm = 0.f, yd = 0.f;
-          if (radial) {
-            lrp[u] = (double)a.fxrmp[l - ns];
-            lrm[u] = (double)a.fxrmm[l];
-            hdm = a.fxd[l - ns];
-          }
-          const float hd = a.fxd[l];
-          lvt[u] = vb_i + (double)a.fxvt[l];
-          if (radial && lob_m) ydm = a.fxd[S2 + l - ns];  // Sigma residuals of float-pair rings
-          if (lob_i) yd = a.fxd[S2 + l];
-          if (radial) ldm[u] = rec32(sb_m, hdm, ydm);
-          ld[u] = rec32(sb_i, hd, yd);
-        } else {
-          if (radial) {
-            lrp[u] = a.xrmp[l - ns];
-            lrm[u] = a.xrmm[l];
-            ldm[u] = a.xd[l - ns];
-          }
-          ld[u] = a.xd[l];
-          lvt[u] = a.xvt[l];
-        }
-        if (adi)
-          lp[u] = a.xe[l];
-        else if (a.temp)
-          lp[u] = a.press[l];
-      }
+  double fsx = 0.0, fcx = 0.0, fsy = 0.0, fcy = 0.0, ssum = 0.0;
+  const double dxrad = t.Rsup[i] - t.Rinf[i], dxtheta = t.dxtheta_cfl[i];
+  const double mindx = (dxtheta < dxrad) ? dxtheta : dxrad;
+  const double invdt1r = t.cs_iso[i] / mindx;
+  const recip64 rdr(dxrad), rdt(dxtheta);
+  const double sigma0 = t.SigmaMed[i], energy0 = ADI ? t.EnergyMed[i] : 0.0;
+  bool bad = false;  // a density below 0, infinite or NaN
+  double smax = -1.0;
+  auto pass = [&](int jc, const cell &x) __attribute__((always_inline)) {
+    const bool mine = jc < ns;
+    const int j = min(jc, ns - 1);
+    unsigned o = 8u * j;
+    asm volatile("" : "+v"(o));
+    double ld = x.d, ldm = x.dm, ldn = x.dn;
+    if constexpr (S32) {
+      ld = rec32(sb_i, x.d, lob_i ? x.y : 0.f);
+      ldm = rec32(sb_m, x.dm, lob_m ? x.ym : 0.f);
+      ldn = rec32(sb_n, x.dn, lob_n ? x.yn : 0.f);
     }
-#pragma unroll
-  for (int u = 0; u < FIN_B; u++) {
-    const int j = j0 + u * 256;
-    if (j >= ns) break;
-    const long l = base + j;
-    // ComputeVelocities, Kernels.cu:1200-1205 (0 on ring 0 and the ghost ring)
-    double vr = radial ? (lrp[u] + lrm[u]) / (ld[u] + ldm[u] + 1e-20) : 0.0, vt = lvt[u], s = ld[u];
+    double vr = radial ? ((double)x.rpm + (double)x.rm) / (ld + ldm + 1e-20) : 0.0;
+    const double vt = ring[j];
+    double s = ld;
     if (damp_i) {
       vr = damp_toward(vr, lam_i, vr0_i);
-      vt = damp_toward(vt, lam_i, vt0_i);
-      s = damp_toward(s, lam_i, t.SigmaMed[i]);
+      s = damp_toward(s, lam_i, sigma0);
     }
-    a.dens[l] = s;
+    at(a.dens + row, o) = s;
     bad |= !(s >= 0.0 && s < HUGE_VAL);
-    a.vr[l] = vr;
-    a.vt[l] = vt;
-    ring[j] = vt;
+    at(a.vr + row, o) = vr;
+    at(a.vt + row, o) = vt;
     if constexpr (S32) {
-      vsum += vt;
-      ssum += s;
-      const double cm = surf * s;
-      kadd(fsx, fcx, cm * (Rm * lcs[u]) * inv3);
-      kadd(fsy, fcy, cm * (Rm * lsn[u]) * inv3);
+      if (mine) {
+        ssum += s;
+        const double cm = surf * s;
+        kadd(fsx, fcx, cm * (Rm * x.cosj) * inv3);
+        kadd(fsy, fcy, cm * (Rm * x.sinj) * inv3);
+      }
     }
-    if (adi) {
-      double e = lp[u];
-      if (damp_i) e = damp_toward(e, lam_i, t.EnergyMed[i]);
-      a.energy[l] = e;
+    double csv = x.c;
+    if (ADI) {
+      double e = x.e;
+      if (damp_i) e = damp_toward(e, lam_i, energy0);
+      at(a.energy + row, o) = e;
       bad |= !(e >= 0.0 && e < HUGE_VAL);
-      if (a.temp) a.temp[l] = (a.gamma - 1.0) * e / s;              // Kernels.cu:211
-      if (a.cs_refresh) a.cs[l] = sqrt(a.gamma * (a.gamma - 1.0) * e / s);  // Kernels.cu:181
+      if (a.temp) at(a.temp + row, o) = (a.gamma - 1.0) * e / s;  // Kernels.cu:211
+      if (a.cs_refresh) {
+        csv = sqrt(a.gamma * (a.gamma - 1.0) * e / s);  // Kernels.cu:181
+        at(a.cs + row, o) = csv;
+      }
     } else if (a.temp) {
-      a.temp[l] = lp[u] / s;
+      at(a.temp + row, o) = at(a.press + row, o) / s;
     }
-    if (i == nr - 1) {  // ghost ring after transport: all zero
-      a.dens[l + ns] = 0.0;
-      a.vr[l + ns] = 0.0;
-      a.vt[l + ns] = 0.0;
-      if (adi) a.energy[l + ns] = 0.0;
+    if (cfl) {
+      double vrn = radial_n ? ((double)x.rp + (double)x.rn) / (ldn + ld + 1e-20) : 0.0;
+      if (damp_n) vrn = damp_toward(vrn, lam_n, vr0_n);
+      const double invdt1 = ADI ? csv / mindx : invdt1r;
+      const double invdt2 = rdr.div(fabs(vr));
+      double dvr = vrn - vr;
+      const double vres = a.fast ? vt - vm : vt;
+      const double invdt3 = rdt.div(fabs(vres));
+      double dvt = ring[j + 1 == ns ? 0 : j + 1] - vt;
+      dvr = (dvr >= 0.0) ? 1e-10 : -dvr;
+      dvt = (dvt >= 0.0) ? 1e-10 : -dvt;
+      const double xx = rdr.div(dvr), y = rdt.div(dvt);
+      double invdt4 = (y > xx) ? y : xx;
+      invdt4 *= 4.0 * 1.41 * 1.41;
+      const double sq = invdt1 * invdt1 + invdt2 * invdt2 + invdt3 * invdt3 + invdt4 * invdt4;
+      if (sq > smax) smax = sq;
     }
-  }
+  };
+  for (int j = tid; j - tid < ns; j += 512) {
+    fetch(j + 256, c1);
+    pass(j, c0);
+    if (j - tid + 256 >= ns) break;
+    fetch(j + 512, c0);
+    pass(j + 256, c1);
   }
   if (bad) *a.crash = 1;
-  __syncthreads();
-  // ConditionCFLKernel2D1 + 2D2 for ring i (Kernels.cu:1284-1329)
-  const double dxrad = t.Rsup[i] - t.Rinf[i];
-  const double dxtheta = t.dxtheta_cfl[i];
-  const double mindx = (dxtheta < dxrad) ? dxtheta : dxrad;
-  const double cs = t.cs_iso[i];
-  const bool radial_n = i + 1 < nr;  // vrad of ring i+1 (0 on the ghost ring)
-  double best = 1e30;
-  double vm;
+  if (i == nr - 1) {  // ghost ring after transport: all zero
+    for (int j = tid; j < ns; j += 256) {
+      a.dens[rown + j] = a.vr[rown + j] = a.vt[rown + j] = 0.0;
+      if (ADI) a.energy[rown + j] = 0.0;
+    }
+  }
   if constexpr (S32) {
-    // FP32 mode, which does not replay the reference's summation order: the
-    // ring mean of vtheta, the gravity of the ring's cells on the star
-    // (Kernels.cu:703-727 at x = y = 0: the star sits at the origin with no
-    // smoothing, so 1/d^3 is one value per ring) and the ring's Sigma sum
-    // (the next substep's background) come from the per-thread partials of
-    // the pass above, reduced per wave by a shuffle tree and over the waves
-    // in order; the force as one compensated partial per ring
-    __shared__ double fw[4][6];
+    // the gravity of the ring's cells on the star (Kernels.cu:703-727 at x = y =
+    // 0: the star sits at the origin with no smoothing, so 1/d^3 is one value
+    // per ring) and the ring's Sigma sum (the next substep's background),
+    // reduced as above; the force as one compensated partial per ring
     kwave(fsx, fcx);
     kwave(fsy, fcy);
-    for (int off = 32; off > 0; off >>= 1) {
-      vsum += __shfl_down(vsum, off);
-      ssum += __shfl_down(ssum, off);
-    }
+    for (int off = 32; off > 0; off >>= 1) ssum += __shfl_down(ssum, off);
     if ((tid & 63) == 0) {
       double *w = fw[tid >> 6];
       w[0] = fsx;
       w[1] = fcx;
       w[2] = fsy;
       w[3] = fcy;
-      w[4] = vsum;
-      w[5] = ssum;
+      w[4] = ssum;
     }
     __syncthreads();
-    vm = (((fw[0][4] + fw[1][4]) + fw[2][4]) + fw[3][4]) / (double)ns;
     if (tid == 0) {
       double sx = fw[0][0], cx = fw[0][1], sy = fw[0][2], cy = fw[0][3];
       for (int w = 1; w < 4; w++) {
@@ -1622,77 +1685,11 @@ __device__ __forceinline__ void fin_ring(const fin_args &a, int i, double *ring)
       a.fpart[4 * i + 1] = cx;
       a.fpart[4 * i + 2] = sy;
       a.fpart[4 * i + 3] = cy;
-      a.sbar_next[i] = (((fw[0][5] + fw[1][5]) + fw[2][5]) + fw[3][5]) / (double)ns;
-      a.vmoy[i] = vm;
+      a.sbar_next[i] = (((fw[0][4] + fw[1][4]) + fw[2][4]) + fw[3][4]) / (double)ns;
     }
-    if (i == 0) return;
-  } else {
-  if (tid == 0) {
-    double m = seq_sum_lds(ring, ns);
-    m /= (double)ns;
-    a.vmoy[i] = m;
-    s_vmoy = m;
   }
-  __syncthreads();
-  if (i == 0) return;
-  vm = s_vmoy;
-  }
-  const recip64 rdr(dxrad), rdt(dxtheta);
-  double smax = -1.0;
-  for (int j0 = tid; j0 < ns; j0 += FIN_B * 256) {
-    double pvr[FIN_B], prp[FIN_B], prm[FIN_B], pd0[FIN_B], pd1[FIN_B], pcs[FIN_B];
-#pragma unroll
-    for (int u = 0; u < FIN_B; u++) {
-      const int j = j0 + u * 256;
-      pvr[u] = prp[u] = prm[u] = pd0[u] = pd1[u] = pcs[u] = 0.0;
-      if (j < ns) {
-        const long l = base + j;
-        pvr[u] = a.vr[l];  // written above by this thread
-        if (adi) pcs[u] = a.cs[l];
-        if (radial_n) {
-          if constexpr (S32) {
-            const double sb_p = a.sbar[i + 1];
-            prp[u] = (double)a.fxrmp[l];
-            prm[u] = (double)a.fxrmm[l + ns];
-            const float hd1 = a.fxd[l + ns], hd0 = a.fxd[l];
-            float yd1 = 0.f, yd0 = 0.f;
-            if (lob_i) yd0 = a.fxd[S2 + l];  // Sigma residuals of float-pair rings
-            if (lob_p) yd1 = a.fxd[S2 + l + ns];
-            pd1[u] = rec32(sb_p, hd1, yd1);
-            pd0[u] = rec32(sb_i, hd0, yd0);
-          } else {
-            prp[u] = a.xrmp[l];
-            prm[u] = a.xrmm[l + ns];
-            pd1[u] = a.xd[l + ns];
-            pd0[u] = a.xd[l];
-          }
-        }
-      }
-    }
-#pragma unroll
-  for (int u = 0; u < FIN_B; u++) {
-    const int j = j0 + u * 256;
-    if (j >= ns) break;
-    double vr = pvr[u];
-    double vrn = radial_n ? (prp[u] + prm[u]) / (pd1[u] + pd0[u] + 1e-20) : 0.0;
-    if (damp_n) vrn = damp_toward(vrn, lam_n, vr0_n);
-    double vres = a.fast ? (ring[j] - vm) : ring[j];
-    double invdt1 = (adi ? pcs[u] : cs) / mindx;
-    double invdt2 = rdr.div(fabs(vr));
-    double invdt3 = rdt.div(fabs(vres));
-    double dvr = vrn - vr;
-    double dvt = ring[j + 1 == ns ? 0 : j + 1] - ring[j];
-    dvr = (dvr >= 0.0) ? 1e-10 : -dvr;
-    dvt = (dvt >= 0.0) ? 1e-10 : -dvt;
-    double x = rdr.div(dvr), y = rdt.div(dvt);
-    double invdt4 = (y > x) ? y : x;
-    invdt4 *= 4.0 * 1.41 * 1.41;
-    const double sq = invdt1 * invdt1 + invdt2 * invdt2 + invdt3 * invdt3 + invdt4 * invdt4;
-    if (sq > smax) smax = sq;
-  }
-  }
-  // the smallest rounded 0.5 / sqrt(sq) is the one at the largest sq (both
-  // roundings are monotone; a NaN sq is skipped by both comparisons)
+  if (!cfl) return;
+  double best = 1e30;
   if (smax >= 0.0) {
     const double dtc = 0.5 / sqrt(smax);
     if (dtc < best) best = dtc;
@@ -1700,197 +1697,18 @@ __device__ __forceinline__ void fin_ring(const fin_args &a, int i, double *ring)
   ring_min_store(best, red, a.newdt + i);
 }
 
-// FP64 rings of up to FIN_OV_K * 192 cells.  The ring mean of vtheta is a
-// left-to-right sum in one lane (3072 dependent adds at 1024 x 3072), so it
-// starts at once: wave 0 loads the ring's transported vtheta, damps it as
-// the pass below does, stages it in LDS and lane 0 adds it up, while waves
-// 1-3 do everything else in one pass over their cells: ComputeVelocities
-// (Kernels.cu:1200-1205) with the energy, sound speed and temperature of an
-// adiabatic deck, and every term of the cell's CFL time step
-// (Kernels.cu:1284-1329) that does not need the mean.  Only the
-// vtheta-residual and shear terms wait for the workgroup barrier.
-// The ring minimum of dt = 0.5 / sqrt(S) over the cells is taken as one
-// quotient at the largest S: rounded sqrt and rounded division are both
-// monotone, so 0.5 / sqrt(max S) is the smallest rounded dt bit for bit
-// (a NaN S is skipped by both comparisons; the 1e30 start caps both).
-template <bool ADI>
-__device__ __forceinline__ void fin_ring_ov(const fin_args &a, int i, double *ring) {
-  constexpr int U = 2;  // cells per thread whose loads are issued together
-  __shared__ double red[4];
-  __shared__ double s_vmoy;
-  const int ns = a.ns, nr = a.nr, tid = threadIdx.x;
-  const fg_dev_tables &t = a.t;
-  const long base = (long)i * ns;
-  double lam_i = 0, vr0_i = 0, vt0_i = 0;
-  const bool damp_i = a.evanescent && t.ev_zone[i];
-  if (damp_i) ev_consts(t, a.nu, i, a.dt, a.omega_frame, lam_i, vr0_i, vt0_i, a.sgacc);
-  const bool cfl = i > 0;  // ring 0 has no CFL term (Kernels.cu:1286)
-  double A[FIN_OV_K], X[FIN_OV_K];
-  if (tid < 64) {
-    // the damped vtheta of every cell, which the pass below also stores
-    for (int j0 = 0; j0 < ns; j0 += 64 * 16) {
-      double v[16];
-#pragma unroll
-      for (int u = 0; u < 16; u++) {
-        const int j = j0 + u * 64 + tid;
-        v[u] = j < ns ? a.xvt[base + j] : 0.0;
-      }
-#pragma unroll
-      for (int u = 0; u < 16; u++) {
-        const int j = j0 + u * 64 + tid;
-        if (j < ns) ring[j] = damp_i ? damp_toward(v[u], lam_i, vt0_i) : v[u];
-      }
-    }
-    // one wave: its LDS stores complete in order before lane 0's loads
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (tid == 0) {
-      double m = seq_sum_lds(ring, ns);
-      m /= (double)ns;
-      a.vmoy[i] = m;
-      s_vmoy = m;
-    }
-  } else {
-    double lam_n = 0, vr0_n = 0, vt0_n = 0;
-    const bool damp_n = a.evanescent && (i + 1 < nr) && t.ev_zone[i + 1];
-    if (damp_n) ev_consts(t, a.nu, i + 1, a.dt, a.omega_frame, lam_n, vr0_n, vt0_n, a.sgacc);
-    const bool radial = i > 0;          // vrad recovery reads rings i-1 and i
-    const bool radial_n = i + 1 < nr;  // vrad of ring i+1 (0 on the ghost ring)
-    const double dxrad = t.Rsup[i] - t.Rinf[i];
-    const double dxtheta = t.dxtheta_cfl[i];
-    const double mindx = (dxtheta < dxrad) ? dxtheta : dxrad;
-    const double invdt1r = t.cs_iso[i] / mindx;
-    const recip64 rdr(dxrad);
-    bool bad = false;
-    const int t0 = tid - 64;
-#pragma unroll
-    for (int u0 = 0; u0 < FIN_OV_K; u0 += U) {
-      double lrp[U], lrm[U], ld[U], ldm[U], lvt[U], lp[U], prp[U], prm[U], pd1[U], pcs[U];
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int j = t0 + (u0 + u) * 192;
-        lrp[u] = lrm[u] = ld[u] = ldm[u] = lvt[u] = lp[u] = prp[u] = prm[u] = pd1[u] = pcs[u] = 0.0;
-        if (j < ns) {
-          const long l = base + j;
-          if (radial) {
-            lrp[u] = a.xrmp[l - ns];
-            lrm[u] = a.xrmm[l];
-            ldm[u] = a.xd[l - ns];
-          }
-          ld[u] = a.xd[l];
-          lvt[u] = a.xvt[l];
-          if (ADI)
-            lp[u] = a.xe[l];
-          else if (a.temp)
-            lp[u] = a.press[l];
-          if (cfl && radial_n) {
-            prp[u] = a.xrmp[l];
-            prm[u] = a.xrmm[l + ns];
-            pd1[u] = a.xd[l + ns];
-          }
-          if (ADI && cfl && !a.cs_refresh) pcs[u] = a.cs[l];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int j = t0 + (u0 + u) * 192;
-        if (j >= ns) break;
-        const long l = base + j;
-        // ComputeVelocities, Kernels.cu:1200-1205 (0 on ring 0)
-        double vr = radial ? (lrp[u] + lrm[u]) / (ld[u] + ldm[u] + 1e-20) : 0.0, vt = lvt[u], s = ld[u];
-        if (damp_i) {
-          vr = damp_toward(vr, lam_i, vr0_i);
-          vt = damp_toward(vt, lam_i, vt0_i);
-          s = damp_toward(s, lam_i, t.SigmaMed[i]);
-        }
-        a.dens[l] = s;
-        bad |= !(s >= 0.0 && s < HUGE_VAL);
-        a.vr[l] = vr;
-        a.vt[l] = vt;
-        double csv = pcs[u];
-        if (ADI) {
-          double e = lp[u];
-          if (damp_i) e = damp_toward(e, lam_i, t.EnergyMed[i]);
-          a.energy[l] = e;
-          bad |= !(e >= 0.0 && e < HUGE_VAL);
-          if (a.temp) a.temp[l] = (a.gamma - 1.0) * e / s;  // Kernels.cu:211
-          if (a.cs_refresh) {
-            csv = sqrt(a.gamma * (a.gamma - 1.0) * e / s);  // Kernels.cu:181
-            a.cs[l] = csv;
-          }
-        } else if (a.temp) {
-          a.temp[l] = lp[u] / s;
-        }
-        if (i == nr - 1) {  // ghost ring after transport: all zero
-          a.dens[l + ns] = 0.0;
-          a.vr[l + ns] = 0.0;
-          a.vt[l + ns] = 0.0;
-          if (ADI) a.energy[l + ns] = 0.0;
-        }
-        if (cfl) {
-          double vrn = radial_n ? (prp[u] + prm[u]) / (pd1[u] + ld[u] + 1e-20) : 0.0;
-          if (damp_n) vrn = damp_toward(vrn, lam_n, vr0_n);
-          const double invdt1 = ADI ? csv / mindx : invdt1r;
-          const double invdt2 = rdr.div(fabs(vr));
-          double dvr = vrn - vr;
-          dvr = (dvr >= 0.0) ? 1e-10 : -dvr;
-          A[u0 + u] = invdt1 * invdt1 + invdt2 * invdt2;
-          X[u0 + u] = rdr.div(dvr);
-        }
-      }
-    }
-    if (bad) *a.crash = 1;
-  }
-  __syncthreads();
-  if (i == 0) return;
-  double best = 1e30;
-  if (tid >= 64) {
-    const double vm = s_vmoy;
-    const recip64 rdt(t.dxtheta_cfl[i]);
-    double smax = -1.0;
-#pragma unroll
-    for (int u = 0; u < FIN_OV_K; u++) {
-      const int j = tid - 64 + u * 192;
-      if (j >= ns) break;
-      const double vres = a.fast ? (ring[j] - vm) : ring[j];
-      const double invdt3 = rdt.div(fabs(vres));
-      double dvt = ring[j + 1 == ns ? 0 : j + 1] - ring[j];
-      dvt = (dvt >= 0.0) ? 1e-10 : -dvt;
-      const double y = rdt.div(dvt);
-      double invdt4 = (y > X[u]) ? y : X[u];
-      invdt4 *= 4.0 * 1.41 * 1.41;
-      const double sq = (A[u] + invdt3 * invdt3) + invdt4 * invdt4;
-      if (sq > smax) smax = sq;
-    }
-    if (smax >= 0.0) {
-      const double dtc = 0.5 / sqrt(smax);
-      if (dtc < best) best = dtc;
-    }
-  }
-  ring_min_store(best, red, a.newdt + i);
-}
-
 // Workgroups are dispatched round-robin over the 8 XCDs.  Each XCD gets a
 // contiguous band of rings, so neighbouring rings, which read each other's
 // momenta and densities, are processed side by side under one L2.
-// ADI: adiabatic deck; S32: FP32 bulk mode (FP32 storage of k_taz's fields)
-template <bool ADI, bool S32 = false>
-__global__ __launch_bounds__(256) void k_fin(fin_args a) {
+template <bool ADI, bool S32>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_fin(fin_args a) {
   extern __shared__ double lds_fin[];
-  const int band = (a.nr + FG_NXCD - 1) / FG_NXCD;
-  const int i = (int)(blockIdx.x % FG_NXCD) * band + (int)(blockIdx.x / FG_NXCD);
-  if (i >= a.nr) return;
-  if constexpr (S32) {
-    if (in_lob(i, a.lob0 - 1, a.lob1 + 1))
-      fin_ring<2, ADI, true, true>(a, i, lds_fin);
-    else
-      fin_ring<2, ADI, true, false>(a, i, lds_fin);
-  } else if (a.ns <= 192 * FIN_OV_K) {
-    fin_ring_ov<ADI>(a, i, lds_fin);
-  } else {
-    fin_ring<4, ADI, false>(a, i, lds_fin);
-  }
+  const int i = xcd_block(a.nr);
+  if (i < 0) return;
+  if (S32 && in_lob(i, a.lob0 - 1, a.lob1 + 1))
+    fin_ring<ADI, S32, true>(a, i, lds_fin);
+  else
+    fin_ring<ADI, S32, false>(a, i, lds_fin);
 }
 
 // ================================================== FP32 bulk mode ====
@@ -3054,13 +2872,8 @@ extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, dou
   fa.lob0 = lob0;
   fa.lob1 = lob1;
   prof_mark(c);
-  const dim3 gfin(FG_NXCD * ((nr + FG_NXCD - 1) / FG_NXCD));
-  if (adi)
-    hipLaunchKernelGGL(k_fin<true>, gfin, dim3(256), (size_t)ns * sizeof(double), c->stream, fa);
-  else if (fp32)
-    hipLaunchKernelGGL((k_fin<false, true>), gfin, dim3(256), (size_t)ns * sizeof(double), c->stream, fa);
-  else
-    hipLaunchKernelGGL(k_fin<false>, gfin, dim3(256), (size_t)ns * sizeof(double), c->stream, fa);
+  auto fin = adi ? k_fin<true, false> : fp32 ? k_fin<false, true> : k_fin<false, false>;
+  hipLaunchKernelGGL(fin, dim3(xcd_grid(nr)), dim3(256), (size_t)ns * sizeof(double), c->stream, fa);
   FG_LAUNCH_CHECK();
   if (fp32) c->fu_sbar_cur ^= 1;  // k_fin wrote the next substep's Sigma background
   prof_mark(c);
@@ -3273,7 +3086,8 @@ __global__ __launch_bounds__(64) void k_batch_taz(const batch_disk *__restrict__
     tazw_body<4, true, 5, false>(a, i, w.y % nch, sh);
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_batch_fin(const batch_disk *__restrict__ D, const int2 *__restrict__ items, int n) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_batch_fin(
+    const batch_disk *__restrict__ D, const int2 *__restrict__ items, int n) {
   extern __shared__ double lds_bfin[];
   if ((int)blockIdx.x >= n) return;
   const int2 w = uniform2(items[blockIdx.x]);
@@ -3294,10 +3108,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   a.fpart = global(a.fpart);
   a.crash = global(a.crash);
   a.nu = global(a.nu);
+  a.temp = nullptr;
+  a.sgacc = nullptr;
   if (in_lob(w.y, a.lob0 - 1, a.lob1 + 1))
-    fin_ring<1, false, true, true>(a, w.y, lds_bfin);
+    fin_ring<false, true, true>(a, w.y, lds_bfin);
   else
-    fin_ring<1, false, true, false>(a, w.y, lds_bfin);
+    fin_ring<false, true, false>(a, w.y, lds_bfin);
 }
 
 // per disk: the force's final sum and the CFL count of the next substep
@@ -3449,8 +3265,8 @@ static fg_status batch_build(fg_batch_dev *b) {
   hipLaunchKernelGGL(k_batch_src, dim3(xcd_grid(b->n_src)), dim3(64), 0, st, b->d_disk, b->it_src, b->n_src);
   hipLaunchKernelGGL(k_batch_trad, dim3(b->n_trad), dim3(TRAD_TPB), 0, st, b->d_disk, b->it_trad, b->n_trad);
   hipLaunchKernelGGL(k_batch_taz, dim3(b->n_taz), dim3(64), 0, st, b->d_disk, b->it_taz, b->n_taz);
-  hipLaunchKernelGGL(k_batch_fin, dim3(b->n_fin), dim3(256), (size_t)b->max_ns * sizeof(double), st, b->d_disk,
-                     b->it_fin, b->n_fin);
+  hipLaunchKernelGGL(k_batch_fin, dim3(b->n_fin), dim3(256), (size_t)b->max_ns * sizeof(double), st, b->d_disk, b->it_fin,
+                     b->n_fin);
   hipLaunchKernelGGL(k_batch_close, dim3(b->n), dim3(256), 0, st, b->d_disk, b->d_res, b->n);
   (void)hipMemcpyAsync(b->h_res, b->d_res, b->n * sizeof(batch_result), hipMemcpyDeviceToHost, st);
   hipError_t ce = hipStreamEndCapture(st, &b->graph);

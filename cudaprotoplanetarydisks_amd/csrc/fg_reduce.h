@@ -286,6 +286,173 @@ __device__ __forceinline__ double seq_sum_lds(const double *ring, int n, double 
   return m;
 }
 
+// x moved between the lanes of a wave by DPP (CTRL, rows of MASK; 0 elsewhere)
+template <int CTRL, int MASK>
+__device__ __forceinline__ int dpp_move(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, MASK, 0xf, true);
+}
+template <int CTRL, int MASK>
+__device__ __forceinline__ double dpp_move(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = dpp_move<CTRL, MASK>((int)b), hi = dpp_move<CTRL, MASK>((int)(b >> 32));
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+// f(x.lane(l - n)) of the six steps of an inclusive scan over 64 lanes: by 1, 2,
+// 4 and 8 lanes within rows of 16, then the rows' last lanes to the rows behind
+#define WAVE_SCAN_STEPS(STEP) \
+  STEP(0x111, 0xf) STEP(0x112, 0xf) STEP(0x114, 0xf) STEP(0x118, 0xf) STEP(0x142, 0xa) STEP(0x143, 0xc)
+
+// m + x[0] + x[1] + ... + x[n-1] added up left to right, every addition
+// rounded, as by the reference's one-thread ring loops: the same bits from a
+// whole workgroup (ring_seq_sum).  Lane k takes the L elements k L, k L + 1, ...
+//
+// While the running sum stays within one binade it is a multiple of one ulp,
+// and what an element adds to it, rounded to even, depends on nothing but the
+// element and the sum's last bit.  So a lane adds its elements to a stand-in for
+// the sum before them, once for either last bit: the parallel prefix sum, whose
+// distance from the rounded sequential one is bounded by T = |m| + sum |x| (n
+// additions of at most half an ulp of T each, below 2^-39 T for n <= 2^13).  If
+// the stand-ins stay that far within a binade throughout, so does the sequential
+// sum, and the lane's two exact differences and last bits are all that is
+// needed of it; such maps are composed by a scan.  Lanes whose elements may cross
+// a binade (about log2 n of them in a sum of one sign), and sums with infinities
+// and NaN, are added up one by one.
+// Rings shorter than RING_SEQ_MIN are added up by one lane (k_fin with the one and
+// the other, us: 384 cells 10.8 and 12.0, 576 12.7 and 12.8, 768 14.7 and 13.8,
+// 1536 26.8 and 19.7).
+#define RING_SEQ_MIN 640
+struct seq_map {
+  double d0, d1;  // what the lanes up to this one, from the last single one on, add to an even, odd sum
+  int f;          // bits: the even sum becomes odd, the odd one even, a single lane before
+  unsigned long long single;  // the wave's lanes that are added up one by one
+};
+
+// inclusive prefix sums over a wave of the lanes' sums and of their absolute values
+__device__ __forceinline__ void seq_prefix(int k0, int n, int L, const double *x, double &s, double &t) {
+  s = t = 0.0;
+#pragma unroll 4
+  for (int q = 0; q < L; q++) {
+    const double v = k0 + q < n ? x[k0 + q] : 0.0;
+    s += v;
+    t += fabs(v);
+  }
+#define STEP(C, M)        \
+  s += dpp_move<C, M>(s); \
+  t += dpp_move<C, M>(t);
+  WAVE_SCAN_STEPS(STEP)
+#undef STEP
+}
+
+// the wave's maps; before: about the sum before this lane's elements
+__device__ __forceinline__ seq_map seq_maps(int k0, int n, int L, const double *x, double before, double T) {
+  const double margin = T * 0x1p-37;
+  const long long p = __double_as_longlong(before);
+  const double b0 = __longlong_as_double(p & ~1ll), b1 = __longlong_as_double(p | 1ll);
+  double t0 = b0, t1 = b1, lo = b0, hi = b0;
+#pragma unroll 4
+  for (int q = 0; q < L; q++) {
+    const double v = k0 + q < n ? x[k0 + q] : 0.0;
+    t0 += v;
+    t1 += v;
+    lo = fmin(lo, t0);
+    hi = fmax(hi, t0);
+  }
+  // sign and exponent of both ends (NaN and infinity have the largest exponent,
+  // and the smallest ones leave the margin no room)
+  const int el = (int)(__double_as_longlong(lo - margin) >> 52), eh = (int)(__double_as_longlong(hi + margin) >> 52);
+  const bool alone = el != eh || (el & 0x7ff) < 128 || (el & 0x7ff) > 2000;
+  seq_map r;
+  r.single = __ballot(alone);
+  r.d0 = alone ? 0.0 : t0 - b0;
+  r.d1 = alone ? 0.0 : t1 - b1;
+  r.f = alone ? 4 : (int)(__double_as_longlong(t0) & 1) | (int)(~__double_as_longlong(t1) & 1) << 1;
+#define STEP(C, M)                                                                            \
+  {                                                                                           \
+    const double l0 = dpp_move<C, M>(r.d0), l1 = dpp_move<C, M>(r.d1);                        \
+    const int lf = dpp_move<C, M>(r.f);                                                       \
+    if (!(r.f & 4)) {                                                                         \
+      const double e0 = l0 + (lf & 1 ? r.d1 : r.d0), e1 = l1 + (lf & 2 ? r.d0 : r.d1);        \
+      const int g0 = lf & 1 ? ~r.f >> 1 & 1 : r.f & 1, g1 = lf & 2 ? ~r.f & 1 : r.f >> 1 & 1; \
+      r.d0 = e0;                                                                              \
+      r.d1 = e1;                                                                              \
+      r.f = g0 | g1 << 1 | (lf & 4);                                                          \
+    }                                                                                         \
+  }
+  WAVE_SCAN_STEPS(STEP)
+#undef STEP
+  return r;
+}
+
+// x of lane `lane` (uniform), as scalars
+__device__ __forceinline__ double lane_get(double x, int lane) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_readlane((int)b, lane);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// the wave's elements added to m; lane 0's are first, first + 1, ... (L <= 64: a
+// single lane's elements come one to a lane, the next one's while it is added up)
+__device__ __forceinline__ double seq_apply(const seq_map &r, double m, int first, int n, int L, const double *x) {
+  unsigned long long single = r.single;
+  auto run = [&](int end) {  // the run of lanes that ends at `end`
+    const double a0 = lane_get(r.d0, end), a1 = lane_get(r.d1, end);
+    m += __double_as_longlong(m) & 1 ? a1 : a0;
+  };
+  const int lane = threadIdx.x & 63;
+  int at = 0;
+  double next = single ? x[min(first + __builtin_ctzll(single) * L + lane, n - 1)] : 0.0;
+  while (single) {
+    const int k = __builtin_ctzll(single);
+    const double mine = next;
+    single &= single - 1;
+    if (single) next = x[min(first + __builtin_ctzll(single) * L + lane, n - 1)];
+    if (k > at) run(k - 1);
+    const int count = min(L, n - first - k * L);
+#pragma unroll 4
+    for (int q = 0; q < count; q++) m += lane_get(mine, q);
+    at = k + 1;
+  }
+  if (at < 64) run(63);
+  return m;
+}
+
+// of a ring in LDS by a workgroup of 256 threads, which all call it behind the
+// ring's barrier and get the sum (an odd number of elements a lane keeps the
+// lanes on different banks).  Four waves' lanes have a quarter of the elements
+// to add one by one at a binade: about 4 us from 768 to 3072 elements, where one
+// lane's chain of additions takes 3 to 12 alone and up to 40 beside other waves.
+__device__ __forceinline__ double ring_seq_sum(const double *ring, int n) {
+  __shared__ double s_s[4], s_t[4], s_m[4];
+  if (n < RING_SEQ_MIN) {
+    if (threadIdx.x == 0) s_m[3] = seq_sum_lds(ring, n);
+    __syncthreads();
+    return s_m[3];
+  }
+  const int L = ((n + 255) / 256) | 1, w = threadIdx.x >> 6, k0 = threadIdx.x * L;
+  double s, t;
+  seq_prefix(k0, n, L, ring, s, t);
+  if ((threadIdx.x & 63) == 63) {
+    s_s[w] = s;
+    s_t[w] = t;
+  }
+  __syncthreads();
+  double before = 0.0, T = 0.0;
+  for (int q = 0; q < 4; q++) {
+    if (q < w) before += s_s[q];
+    T += s_t[q];
+  }
+  const seq_map r = seq_maps(k0, n, L, ring, before + dpp_move<0x138, 0xf>(s), T);
+  for (int q = 0; q < 4; q++) {
+    if (q == w) {
+      const double m = seq_apply(r, q ? s_m[q - 1] : 0.0, 64 * q * L, n, L, ring);
+      if ((threadIdx.x & 63) == 0) s_m[q] = m;
+    }
+    __syncthreads();
+  }
+  return s_m[3];
+}
+
 // host loop of DeviceReduce (Kernels.cu:385-390).  With add_inner, the
 // result is fx_inner + fx_outer of SideEuler.cu:144 where the inner sum
 // is the DeviceReduce of an all-zero array (+0.0).

@@ -70,9 +70,8 @@ __global__ void k_ring_mean(double *out, const double *field, int nr, int ns) {
   const int i = blockIdx.x;
   for (int j = threadIdx.x; j < ns; j += blockDim.x) ring[j] = field[(long)i * ns + j];
   __syncthreads();
-  if (threadIdx.x == 0) {
-    out[i] = seq_sum_lds(ring, ns) / (double)ns;
-  }
+  const double m = ring_seq_sum(ring, ns) / (double)ns;
+  if (threadIdx.x == 0) out[i] = m;
 }
 
 // FViscosity (Viscosity.cu:33-50) from the ring mean of c_s
@@ -326,7 +325,6 @@ __global__ void k_cfl_ring(double *vmoy, double *newdt, const double *vr, const 
   extern __shared__ double sh[];
   double *ring = sh;               // ns
   double *red = sh + ns;           // blockDim
-  __shared__ double s_vmoy;
   const int i = blockIdx.x;
   bool bad = false;
   for (int j = threadIdx.x; j < ns; j += blockDim.x) {
@@ -341,18 +339,12 @@ __global__ void k_cfl_ring(double *vmoy, double *newdt, const double *vr, const 
   }
   if (bad) *crash = 1;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double m = seq_sum_lds(ring, ns);
-    m /= (double)ns;
-    vmoy[i] = m;
-    s_vmoy = m;
-  }
-  __syncthreads();
+  const double vm = ring_seq_sum(ring, ns) / (double)ns;
+  if (threadIdx.x == 0) vmoy[i] = vm;
   if (i == 0) return;
   const double dxrad = t.Rsup[i] - t.Rinf[i];
   const double dxtheta = t.dxtheta_cfl[i];
   const double mindx = (dxtheta < dxrad) ? dxtheta : dxrad;  // min2
-  const double vm = s_vmoy;
   double best = 1e30;
   for (int j = threadIdx.x; j < ns; j += blockDim.x) {
     long l = (long)i * ns + j;
