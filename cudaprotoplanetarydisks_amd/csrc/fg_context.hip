@@ -81,6 +81,7 @@ extern "C" fg_status fg_create(const fg_params *p, const fg_tables *t, int devic
   c->tile_src_th = 0;   // picked for the grid
   c->tile_trad_band = 0;  // picked for the grid
   c->fp32_pair_hill = 1.0;
+  c->fu_waits = -1;
   c->p = *p;
   c->nr = p->nrad;
   c->ns = p->nsec;
@@ -202,7 +203,7 @@ extern "C" fg_status fg_create(const fg_params *p, const fg_tables *t, int devic
   TRY(dev_alloc(&c->nu_next, R));
   TRY(dev_alloc(&c->Nshift, R));
   TRY(dev_alloc(&c->LostByDisk, NS));
-  TRY(dev_alloc(&c->red_partial, 2 * FG_RED_BLOCKS));
+  TRY(dev_alloc(&c->red_partial, 2 * FG_RED_BLOCKS * (1 + FG_MAX_PLANETS)));
   const unsigned pin = hipHostMallocCoherent | hipHostMallocMapped;
   if (hipHostMalloc((void **)&c->h_out, FG_OUT_SLOTS * sizeof(double), pin) != hipSuccess ||
       hipHostGetDevicePointer((void **)&c->red_out, c->h_out, 0) != hipSuccess ||

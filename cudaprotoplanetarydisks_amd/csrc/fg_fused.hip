@@ -20,7 +20,7 @@
 //           X -> state A
 //   force   DeviceReduce-order disk force on the star (partials as in
 //           fg_reduce.hip) and the CFL count in one final kernel
-//           (k_force_cfl_final; FP32 mode: k_force_rings_cfl)
+//           (k_results)
 //
 // Adiabatic decks add Substep3 (k_src3) between k_src and k_trad and carry
 // the energy through the sweeps and k_fin; self-gravitating decks run the
@@ -1377,22 +1377,20 @@ __device__ __forceinline__ void force_rings_final(const double *fpart, int nr, d
 // result block out (behind a system-scope fence: every result above is
 // visible to the host first; thread 0 and the lanes that wrote them are in
 // wave 0).
-__device__ __forceinline__ void seq_store(double *out, double seq) {
+__device__ __forceinline__ void seq_store(double *slot, double seq) {
   if (threadIdx.x == 0) {
     __threadfence_system();
-    out[FG_FUSED_SEQ_SLOT] = seq;
+    *slot = seq;
   }
 }
 
-__global__ __launch_bounds__(256) void k_force_rings_cfl(const double *fpart, int nr, double *out2, double *cfl,
-                                                         double *dt1d, const double *vmoy, const double *newdt,
-                                                         const double *invRmed, double coef, double DeltaT,
-                                                         double seq) {
+__device__ __forceinline__ void force_rings_cfl(const double *fpart, int nr, double *out2, double *cfl, double *dt1d,
+                                                const double *vmoy, const double *newdt, const double *invRmed,
+                                                double coef, double DeltaT) {
   if (nr > 4 * 256) {
     force_rings_final(fpart, nr, out2);
     __syncthreads();
     cfl_final(cfl, dt1d, vmoy, newdt, invRmed, coef, DeltaT, nr);
-    seq_store(out2, seq);
     return;
   }
   __shared__ double ws[4][4];
@@ -1432,7 +1430,6 @@ __global__ __launch_bounds__(256) void k_force_rings_cfl(const double *fpart, in
     out2[1] = c + d;
   }
   cfl_count_store(cfl, m, DeltaT);
-  seq_store(out2, seq);
 }
 
 // minimum over the workgroup's 256 threads into *out (thread 0): within
@@ -2348,26 +2345,73 @@ static fg_status fused_supported(fg_ctx *c) {
   return FG_OK;
 }
 
-// The host loop of DeviceReduce for the star force (dreduce_final: lanes 0
-// and 1 add the B block sums of x and y in order, then +0.0 for the inner
-// sum, SideEuler.cu:144) and, in waves 1-3 meanwhile, the CFL count of the
-// same substep (DT1D of every ring, Kernels.cu:1331-1337, and the minimum
-// with the ring minima, Kernels.cu:1337-1359; a minimum does not depend on
-// the order its candidates are compared in), then the result block's
-// sequence slot.  p: LDS for the 2B block sums; every thread of a
-// 256-thread block calls it.
-__device__ __forceinline__ void force_cfl_final(const double *partial, int B, double *out, double *cfl, double *dt1d,
-                                                const double *vmoy, const double *newdt, const double *invRmed,
-                                                double coef, double DeltaT, int nr, double seq, double *p) {
+// DeviceReduce of the disk force on several points at once (dreduce_block):
+// blockIdx.y takes point y, whose block sums go to its part of `partial`.  The
+// star, if it is among them, is point 0.
+struct forces_args {
+  force_src src;  // (position and smoothing of the star)
+  long n;
+  int B, star;
+  double *partial;
+  fg_force_list list;
+};
+__global__ __launch_bounds__(RED_TPB) void k_forces_partial(forces_args a) {
+  force_src src = a.src;
+  const int q = (int)blockIdx.y - a.star;
+  if (q >= 0) {  // (read where the launch put them: indexed, a by-value copy would live in scratch)
+    const auto &list = ((__attribute__((address_space(4))) const forces_args *)__builtin_amdgcn_kernarg_segment_ptr())->list;
+    src.x = list.x[q];
+    src.y = list.y[q];
+    src.rs = list.rs[q];
+  }
+  dreduce_block<force_src, RED_CH>(src, a.n, a.B, blockIdx.x, a.partial + 2l * FG_RED_BLOCKS * blockIdx.y);
+}
+
+// Their final sums, the host loop of DeviceReduce (dreduce_final: lanes 0 and 1
+// add the B block sums of x and y in order, then +0.0 for the inner sum,
+// SideEuler.cu:144), one workgroup a point, and beside the star's, in waves 1-3
+// of workgroup 0, the CFL count of the same state (DT1D of every ring,
+// Kernels.cu:1331-1337, and the minimum with the ring minima,
+// Kernels.cu:1337-1359; a minimum does not depend on the order its candidates
+// are compared in); then the result block's sequence slots.  RINGS: the star's
+// force from k_fin's ring partials (FP32 mode).
+// Bound: latency, the chain of B = 1024 additions and the write to host memory:
+// 10.5 us however many planets there are, where two planets' own pairs of
+// launches took 36 (301 x 998 with two planets: 135 us per substep, now 104).
+struct results_args {
+  const double *partial;
+  int B, star;
+  double *out;     // result block
+  double *cfl;     // CFL count, as a double or an int (neither: not wanted)
+  int *icfl;
+  double *dt1d;
+  const double *vmoy, *newdt, *invRmed, *fpart;
+  double coef, DeltaT;
+  int nr;
+  double seq;      // > 0: into the sequence slots
+  fg_force_list list;
+};
+template <bool RINGS>
+__global__ __launch_bounds__(256) void k_results(results_args a) {
+  __shared__ double p[2 * FG_RED_BLOCKS];
   __shared__ double wmin[4];
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, q = (int)blockIdx.x - 1, B = a.B;
+  if (RINGS && q < 0) {
+    force_rings_cfl(a.fpart, a.nr, a.out, a.cfl, a.dt1d, a.vmoy, a.newdt, a.invRmed, a.coef, a.DeltaT);
+    seq_store(a.out + FG_FUSED_SEQ_SLOT, a.seq);
+    return;
+  }
+  const double *partial = a.partial + 2l * FG_RED_BLOCKS * (q + a.star);
   for (int k = tid; k < 2 * B; k += 256) p[k] = partial[k];
   __syncthreads();
+  int slot = 0;
+  if (q >= 0)
+    slot = ((__attribute__((address_space(4))) const results_args *)__builtin_amdgcn_kernarg_segment_ptr())->list.slot[q];
   if (tid < 2) {
     double s = seq_sum_lds(p + tid * B, B);
-    out[tid] = 0.0 + s;
-  } else if (tid >= 64) {
-    double best = cfl_ring_min(dt1d, vmoy, newdt, invRmed, coef, nr, tid - 64, 192);
+    a.out[slot + tid] = 0.0 + s;
+  } else if (tid >= 64 && q < 0 && (a.cfl || a.icfl)) {
+    double best = cfl_ring_min(a.dt1d, a.vmoy, a.newdt, a.invRmed, a.coef, a.nr, tid - 64, 192);
     for (int off = 32; off > 0; off >>= 1) {
       const double o = __shfl_down(best, off, 64);
       if (o < best) best = o;
@@ -2375,58 +2419,100 @@ __device__ __forceinline__ void force_cfl_final(const double *partial, int B, do
     if ((tid & 63) == 0) wmin[tid >> 6] = best;
   }
   __syncthreads();
-  if (tid == 0) {
+  if (tid == 0 && q < 0 && (a.cfl || a.icfl)) {
     double newdt_ = wmin[1];
     if (wmin[2] < newdt_) newdt_ = wmin[2];
     if (wmin[3] < newdt_) newdt_ = wmin[3];
-    if (DeltaT < newdt_) newdt_ = DeltaT;
-    cfl[0] = (double)(int)(ceil(DeltaT / newdt_));
+    if (a.DeltaT < newdt_) newdt_ = a.DeltaT;
+    const int count = (int)(ceil(a.DeltaT / newdt_));
+    if (a.cfl)
+      a.cfl[0] = (double)count;
+    else
+      a.icfl[0] = count;
   }
-  seq_store(out, seq);
+  if (a.seq > 0.0) seq_store(a.out + (q < 0 ? FG_FUSED_SEQ_SLOT : FG_FUSED_PFSEQ_SLOT + q), a.seq);
 }
 
-// the DeviceReduce-order partials of the star force (dreduce_block)
-template <int CH>
-__global__ __launch_bounds__(RED_TPB) void k_dreduce_partial_f(force_src src, long n, int B, double *partial) {
-  dreduce_block<force_src, CH>(src, n, B, blockIdx.x, partial);
+// the block sums of the star, unless its ring partials serve, and of the points
+// of c->pf, which are no longer pending then
+static fg_status forces_partial(fg_ctx *c, bool star, results_args &r) {
+  const long n = (long)c->nr * c->ns;
+  const int B = red_blocks(n), points = (star ? 1 : 0) + c->pf.n;
+  r.partial = c->red_partial;
+  r.B = B;
+  r.star = star;
+  r.list = c->pf;
+  r.dt1d = c->DT1D;
+  r.vmoy = c->Vmoy;
+  r.newdt = c->newDT;
+  r.invRmed = c->t.invRmed;
+  r.fpart = c->fu_fpart;
+  r.coef = c->t.dt1d_coef;
+  r.nr = c->nr;
+  if (points > 0) {
+    forces_args a;
+    a.src = force_src{c->f[FG_DENS], c->t.Surf, c->t.Rmed, c->t.cos_cell, c->t.sin_cell, 0.0, 0.0, 0.0, c->ns};
+    a.n = n;
+    a.B = B;
+    a.star = star;
+    a.partial = c->red_partial;
+    a.list = c->pf;
+    hipLaunchKernelGGL(k_forces_partial, dim3(B, points), dim3(RED_TPB), 0, c->stream, a);
+    FG_LAUNCH_CHECK();
+  }
+  c->pf.n = 0;
+  return FG_OK;
 }
 
-__global__ __launch_bounds__(256) void k_force_cfl_final(const double *partial, int B, double *out, double *cfl,
-                                                         double *dt1d, const double *vmoy, const double *newdt,
-                                                         const double *invRmed, double coef, double DeltaT,
-                                                         int nr, double seq) {
-  __shared__ double p[2 * FG_RED_BLOCKS];
-  force_cfl_final(partial, B, out, cfl, dt1d, vmoy, newdt, invRmed, coef, DeltaT, nr, seq, p);
+static void set_forces(fg_force_list &f, int n, const int *k, const double *x, const double *y, const double *rs,
+                       int slot0) {
+  f.n = n;
+  for (int q = 0; q < n; q++) {
+    f.x[q] = x[q];
+    f.y[q] = y[q];
+    f.rs[q] = rs[q];
+    f.slot[q] = slot0 + 2 * k[q];
+  }
+}
+
+void fg_fused_planet_forces(fg_ctx *c, int n, const int *k, const double *x, const double *y, const double *rs) {
+  set_forces(c->pf, n, k, x, y, rs, FG_FUSED_PF_SLOT);
+}
+
+fg_status fg_routine_results(fg_ctx *c, bool cfl, double DeltaT, int n, const int *k, const double *x, const double *y,
+                             const double *rs) {
+  if (cfl)
+    if (fg_status s = fg_cfl_ring_launch(c)) return s;
+  set_forces(c->pf, n, k, x, y, rs, FG_OUT_PF);
+  results_args r;
+  if (fg_status s = forces_partial(c, true, r)) return s;
+  r.out = c->red_out;
+  r.cfl = nullptr;
+  r.icfl = cfl ? c->cfl_out : nullptr;
+  r.DeltaT = DeltaT;
+  r.seq = 0.0;
+  hipLaunchKernelGGL(k_results<false>, dim3(1 + n), dim3(256), 0, c->stream, r);
+  FG_LAUNCH_CHECK();
+  return FG_OK;
 }
 
 // results of the reductions for the next substep: CFL count and the disk
-// force on the star; copied to pinned memory behind an event
+// force on the star and on the planets of c->pf.
 // ring_partials: the star force comes from k_fin's per-ring compensated
 // partials (FP32 mode) instead of the DeviceReduce-order sum
 static fg_status fused_reductions(fg_ctx *c, double DeltaT, bool ring_partials = false) {
-  const double seq = (double)++c->fu_seq;
-  c->fu_seq_last = 1;
-  if (ring_partials) {
-    prof_mark(c);  // (no separate force phase)
-    hipLaunchKernelGGL(k_force_rings_cfl, dim3(1), dim3(256), 0, c->stream, c->fu_fpart, c->nr, c->d_fused,
-                       c->d_fused + FG_FUSED_CFL_SLOT, c->DT1D, c->Vmoy, c->newDT, c->t.invRmed, c->t.dt1d_coef, DeltaT,
-                       seq);
-    FG_LAUNCH_CHECK();
-  } else {
-    // DeviceReduce partials, then one kernel for their final sum and the
-    // CFL count
-    const long n = (long)c->nr * c->ns;
-    const int B = red_blocks(n);
-    force_src src{c->f[FG_DENS], c->t.Surf, c->t.Rmed, c->t.cos_cell, c->t.sin_cell, 0.0, 0.0, 0.0, c->ns};
-    hipLaunchKernelGGL((k_dreduce_partial_f<RED_CH>), dim3(B), dim3(RED_TPB), 0, c->stream, src, n, B,
-                       c->red_partial);
-    FG_LAUNCH_CHECK();
-    prof_mark(c);
-    hipLaunchKernelGGL(k_force_cfl_final, dim3(1), dim3(256), 0, c->stream, c->red_partial, B, c->d_fused,
-                       c->d_fused + FG_FUSED_CFL_SLOT, c->DT1D, c->Vmoy, c->newDT, c->t.invRmed, c->t.dt1d_coef,
-                       DeltaT, c->nr, seq);
-    FG_LAUNCH_CHECK();
-  }
+  results_args r;
+  const int n = c->pf.n;
+  if (fg_status s = forces_partial(c, !ring_partials, r)) return s;
+  prof_mark(c);
+  r.out = c->d_fused;
+  r.cfl = c->d_fused + FG_FUSED_CFL_SLOT;
+  r.icfl = nullptr;
+  r.DeltaT = DeltaT;
+  r.seq = (double)++c->fu_seq;
+  c->fu_waits = n;
+  hipLaunchKernelGGL(ring_partials ? k_results<true> : k_results<false>, dim3(1 + n), dim3(256), 0, c->stream, r);
+  FG_LAUNCH_CHECK();
   prof_mark(c);
   return FG_OK;
 }
@@ -2482,15 +2568,6 @@ fg_status fg_fused_check(fg_ctx *c, double cfl, const double *force2) {
   return fg_check_substep_results(cfl, force2);
 }
 
-fg_status fg_fused_planet_force_async(fg_ctx *c, int k, double x, double y, double rs) {
-  if (!c->d_fused || k < 0 || k >= FG_MAX_PLANETS) {
-    fg_set_error("fused planet force: no result block or planet %d", k);
-    return FG_E_INVALID;
-  }
-  c->fu_seq_last = 0;  // the results now wait for this reduction too
-  return fg_disk_force_async(c, c->f[FG_DENS], x, y, rs, c->d_fused + FG_FUSED_PF_SLOT + 2 * k);
-}
-
 void fg_fused_planet_force(const fg_ctx *c, int k, double out2[2]) {
   out2[0] = c->h_fused[FG_FUSED_PF_SLOT + 2 * k];
   out2[1] = c->h_fused[FG_FUSED_PF_SLOT + 2 * k + 1];
@@ -2502,22 +2579,24 @@ extern "C" fg_status fg_fused_results(fg_ctx *c, int *ncfl, double *force2, doub
     fg_set_error("fg_fused_results: no fused reductions were launched (fg_fused_prepare or fg_step_fused first)");
     return FG_E_INVALID;
   }
-  if (c->fu_seq_last && !c->prof_on) {
-    // only the final kernel is awaited: watch the slot it writes last
-    // (quicker than the stream's completion signal), asking the stream
+  if (c->fu_waits >= 0 && !c->prof_on) {
+    // only the final kernel is awaited: watch the slots its workgroups write
+    // last (quicker than the stream's completion signal), asking the stream
     // every 1024 polls so that a failed launch still ends the wait
-    volatile double *slot = c->h_fused + FG_FUSED_SEQ_SLOT;
     const double want = (double)c->fu_seq;
-    for (unsigned n = 1; *slot != want; n++) {
-      if ((n & 1023) == 0) {
-        const hipError_t e = hipStreamQuery(c->stream);
-        if (e == hipErrorNotReady) continue;
-        FG_HIP(e);
-        if (*slot != want) {
-          fg_set_error("fg_fused_results: the final reduction finished without reporting");
-          return FG_E_HIP;
+    for (int q = -1; q < c->fu_waits; q++) {
+      volatile double *slot = c->h_fused + (q < 0 ? FG_FUSED_SEQ_SLOT : FG_FUSED_PFSEQ_SLOT + q);
+      for (unsigned n = 1; *slot != want; n++) {
+        if ((n & 1023) == 0) {
+          const hipError_t e = hipStreamQuery(c->stream);
+          if (e == hipErrorNotReady) continue;
+          FG_HIP(e);
+          if (*slot != want) {
+            fg_set_error("fg_fused_results: the final reduction finished without reporting");
+            return FG_E_HIP;
+          }
+          break;
         }
-        break;
       }
     }
     std::atomic_thread_fence(std::memory_order_acquire);

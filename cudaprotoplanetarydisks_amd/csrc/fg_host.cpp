@@ -26,14 +26,14 @@ void fg_set_error(const char *fmt, ...);
 #define host_error fg_set_error
 // a planet's disk force queued behind a fused substep, and its result once
 // the fused results are in (fg_fused.hip)
-fg_status fg_fused_planet_force_async(fg_ctx *c, int k, double x, double y, double rs);
+void fg_fused_planet_forces(fg_ctx *c, int n, const int *k, const double *x, const double *y, const double *rs);
 void fg_fused_planet_force(const fg_ctx *c, int k, double out2[2]);
-// a per-routine substep's reductions without their waits (fg_steps.hip,
-// fg_reduce.hip): the disk force on the star (k < 0) or planet k, and the mass
-// lost in the transport
-fg_status fg_cfl_launch(fg_ctx *c, double DeltaT);
+// a per-routine substep's reductions without their waits (fg_fused.hip, fg_steps.hip,
+// fg_reduce.hip): the CFL count (if cfl), the disk force on the star (k < 0)
+// and the planets, and the mass lost in the transport
+fg_status fg_routine_results(fg_ctx *c, bool cfl, double DeltaT, int n, const int *k, const double *x, const double *y,
+                             const double *rs);
 fg_status fg_cfl_result(fg_ctx *c, int *ncfl);
-fg_status fg_disk_force_launch(fg_ctx *c, int k, double x, double y, double rs);
 void fg_disk_force_result(const fg_ctx *c, int k, double out2[2]);
 fg_status fg_transport_launch(fg_ctx *c, double dt, double omega_frame);
 double fg_lost_mass_result(const fg_ctx *c);
@@ -1098,6 +1098,23 @@ static void fused_close(fg_sim *s, const fused_launch &L, int *closed) {
   if (closed) *closed = L.done;
 }
 
+// the planets that feel the disk, where they are
+struct feeling_planets {
+  int n = 0, k[FG_MAX_PLANETS];
+  double x[FG_MAX_PLANETS], y[FG_MAX_PLANETS], rs[FG_MAX_PLANETS];
+  explicit feeling_planets(fg_sim *s) {
+    const Planets &p = s->ps;
+    for (int q = 0; q < p.nb; q++) {
+      if (!p.feeldisk[q]) continue;
+      k[n] = q;
+      x[n] = p.x[q];
+      y[n] = p.y[q];
+      rs[n] = planet_smoothing(s, sqrt(x[n] * x[n] + y[n] * y[n]), p.mass[q], true);
+      n++;
+    }
+  }
+};
+
 static fg_status fused_substep(fg_sim *s, int *closed) {
   const Deck &d = s->d;
   fg_ctx *c = s->ctx;
@@ -1113,23 +1130,15 @@ static fg_status fused_substep(fg_sim *s, int *closed) {
   CHECK(fg_fused_results(c, &cfl, force, nullptr));
   fused_launch L;
   CHECK(fused_plan(s, cfl, force, L));
+  // the next substep's AdvanceSystemFromDisk reads the density this one
+  // leaves at the planets' positions now (fused_plan moved them): their
+  // sums go with the star's and come back with its results, so the next
+  // substep waits for the GPU once
+  const feeling_planets f(s);
+  fg_fused_planet_forces(c, f.n, f.k, f.x, f.y, f.rs);
   CHECK(fg_step_fused(c, L.dt, s->OmegaFrame, L.domega, L.pl, L.nb, s->IndirectX, s->IndirectY, L.DeltaT_next,
                       (d.Write_Temperature ? FG_STEP_TEMPERATURE : 0) | (L.done ? FG_STEP_CLOSES_DT : 0)));
-  // the next substep's AdvanceSystemFromDisk reads the density this one
-  // leaves at the planets' positions now (fused_plan moved them): its
-  // reductions queue behind this substep and come back with its results,
-  // so the next substep waits for the GPU once
-  {
-    const Planets &p = s->ps;
-    int any = 0;
-    for (int k = 0; k < p.nb; k++) {
-      if (!p.feeldisk[k]) continue;
-      const double m = p.mass[k], x = p.x[k], y = p.y[k], r = sqrt(x * x + y * y);
-      CHECK(fg_fused_planet_force_async(c, k, x, y, planet_smoothing(s, r, m, true)));
-      any = 1;
-    }
-    s->pf_ready = any;
-  }
+  s->pf_ready = f.n > 0;
   CHECK(substep_diagnostics(s));
   fused_close(s, L, closed);
   return FG_OK;
@@ -1150,13 +1159,8 @@ extern "C" fg_status fg_sim_substep(fg_sim *s, int *closed) {
   // the state as it is: one wait for them together
   Planets &p = s->ps;
   if (d.IsDisk) {
-    if (!d.SloppyCFL) CHECK(fg_cfl_launch(c, d.DT - s->dtemp));
-    CHECK(fg_disk_force_launch(c, -1, 0.0, 0.0, 0.0));
-    for (int k = 0; k < p.nb; k++) {
-      if (!p.feeldisk[k]) continue;
-      const double x = p.x[k], y = p.y[k];
-      CHECK(fg_disk_force_launch(c, k, x, y, planet_smoothing(s, sqrt(x * x + y * y), p.mass[k], true)));
-    }
+    const feeling_planets f(s);
+    CHECK(fg_routine_results(c, !d.SloppyCFL, d.DT - s->dtemp, f.n, f.k, f.x, f.y, f.rs));
     CHECK(fg_sync(c));
     if (!d.SloppyCFL) {
       int cfl = 1;

@@ -31,9 +31,8 @@ fg_status fg_viscosity_into(fg_ctx *c, double *nu_out);
 fg_status fg_transport_sweeps(fg_ctx *c, double dt, double omega_frame);
 // fg_cfl, fg_disk_force and fg_transport without their waits: launched, and
 // their results read from h_out / h_cfl once the stream is idle
-fg_status fg_cfl_launch(fg_ctx *c, double DeltaT);
+fg_status fg_cfl_ring_launch(fg_ctx *c);
 fg_status fg_cfl_result(fg_ctx *c, int *ncfl);
-fg_status fg_disk_force_async(fg_ctx *c, const double *dens, double x, double y, double rs, double *out_dev);
 fg_status fg_transport_launch(fg_ctx *c, double dt, double omega_frame);
 
 // Result block of the fused path (fg_ctx::h_fused, coherent pinned host
@@ -41,23 +40,35 @@ fg_status fg_transport_launch(fg_ctx *c, double dt, double omega_frame);
 // FG_FUSED_CFL_SLOT the CFL count (as a double), FG_FUSED_CRASH_SLOT an int
 // that k_fin and the CFL ring pass set to 1 when they meet a negative or
 // non-finite density, and from FG_FUSED_PF_SLOT the disk force on each
-// planet that feels the disk (two doubles per planet), launched behind a
-// substep for the next one.  FG_FUSED_SEQ_SLOT: the final kernel writes the
+// planet that feels the disk (two doubles per planet), summed at the end of a
+// substep for the next one.  FG_FUSED_SEQ_SLOT, and from FG_FUSED_PFSEQ_SLOT
+// one slot per requested planet: the final kernel's workgroups write the
 // sequence number of its launch there last, after a system-scope fence,
-// so the host can wait for the results by watching that slot.
+// so the host can wait for the results by watching those slots.
 #define FG_FUSED_PF_SLOT 8
 #define FG_FUSED_SEQ_SLOT 5
 // first planet slot of fg_ctx::h_out, and its size
 #define FG_OUT_PF 8
 #define FG_OUT_SLOTS (FG_OUT_PF + 2 * FG_MAX_PLANETS)
-#define FG_FUSED_SLOTS (FG_FUSED_PF_SLOT + 2 * FG_MAX_PLANETS)
+#define FG_FUSED_PFSEQ_SLOT (FG_FUSED_PF_SLOT + 2 * FG_MAX_PLANETS)
+#define FG_FUSED_SLOTS (FG_FUSED_PFSEQ_SLOT + FG_MAX_PLANETS)
 #define FG_FUSED_CFL_SLOT 6
 #define FG_FUSED_CRASH_SLOT 7
-// disk force on planet k at (x, y) with smoothing rs from the current
-// density into the result block (fg_fused.hip), read once the fused
-// results are in (fg_fused_results)
-fg_status fg_fused_planet_force_async(fg_ctx *c, int k, double x, double y, double rs);
+// Points whose disk force the next reductions sum besides the star's: their
+// position and smoothing, and where the two results go in the result block
+struct fg_force_list {
+  int n;
+  double x[FG_MAX_PLANETS], y[FG_MAX_PLANETS], rs[FG_MAX_PLANETS];
+  int slot[FG_MAX_PLANETS];
+};
+// the planets at (x, y) of the next fused substep's end (fg_fused.hip; planet
+// k's results are read with fg_fused_planet_force once the fused results are in)
+void fg_fused_planet_forces(fg_ctx *c, int n, const int *k, const double *x, const double *y, const double *rs);
 void fg_fused_planet_force(const fg_ctx *c, int k, double out2[2]);
+// a per-routine substep's reductions of the state as it is, to h_out and h_cfl:
+// the disk force on the star and the listed planets and, if cfl, the CFL count
+fg_status fg_routine_results(fg_ctx *c, bool cfl, double DeltaT, int n, const int *k, const double *x, const double *y,
+                             const double *rs);
 
 // Largest CFL sub-cycle count accepted per DT.  The count is
 // ceil(DeltaT / dt) (SourceEuler.cu:228); a count outside 1..FG_CFL_MAX
@@ -152,7 +163,7 @@ struct fg_ctx {
   int shared_faces;
   double *LostByDisk;  // ns
   // reduction scratch
-  double *red_partial;  // 2 * FG_RED_BLOCKS
+  double *red_partial;  // 2 * FG_RED_BLOCKS for the star and each planet
   // results of the per-routine reductions, coherent pinned host memory that the
   // final kernels write straight into (red_out / cfl_out: device aliases)
   double *h_out, *red_out;  // [0..1] force, [2] lost mass, [3] circumplanetary mass, from FG_OUT_PF the
@@ -191,7 +202,8 @@ struct fg_ctx {
   // straight into coherent pinned host memory (no copy); device alias
   double *h_fused, *d_fused;
   unsigned long long fu_seq;  // sequence number of the last final-kernel launch
-  int fu_seq_last;            // nothing the results depend on is queued behind it
+  fg_force_list pf;           // planets of the next fused reductions
+  int fu_waits;               // of the last ones (-1: none were launched)
   // Hill-cut force variants (fg_disk_force_hill), allocated on first use
   double *hill_partial;  // 4 * FG_HILL_MAX * FG_RED_BLOCKS block sums
   double *hill_out;      // 4 * FG_HILL_MAX results

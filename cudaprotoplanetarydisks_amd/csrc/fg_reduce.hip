@@ -61,29 +61,21 @@ fg_status fg_ring_sum_async(fg_ctx *c, const double *ring, double *out_dev) {
   return FG_OK;
 }
 
-fg_status fg_disk_force_async(fg_ctx *c, const double *dens, double x, double y, double rs, double *out_dev) {
-  force_src src{dens, c->t.Surf, c->t.Rmed, c->t.cos_cell, c->t.sin_cell, x, y, rs, c->ns};
-  return dreduce(c, src, (long)c->nr * c->ns, out_dev, 1, 1);
-}
-
-// the disk force on the star (k < 0) or planet k of a per-routine substep,
-// read once the stream is idle
-fg_status fg_disk_force_launch(fg_ctx *c, int k, double x, double y, double rs) {
-  return fg_disk_force_async(c, c->f[FG_DENS], x, y, rs, c->red_out + (k < 0 ? 0 : FG_OUT_PF + 2 * k));
-}
+double fg_lost_mass_result(const fg_ctx *c) { return c->h_out[2]; }
+// of fg_routine_results: the disk force on the star (k < 0) or planet k
 void fg_disk_force_result(const fg_ctx *c, int k, double out2[2]) {
   const double *h = c->h_out + (k < 0 ? 0 : FG_OUT_PF + 2 * k);
   out2[0] = h[0];
   out2[1] = h[1];
 }
-double fg_lost_mass_result(const fg_ctx *c) { return c->h_out[2]; }
 
 extern "C" fg_status fg_disk_force(fg_ctx *c, double x, double y, double rsmoothing, double *out2) {
   if (!c || !out2) {
     fg_set_error("fg_disk_force: NULL argument");
     return FG_E_INVALID;
   }
-  if (fg_status s = fg_disk_force_async(c, c->f[FG_DENS], x, y, rsmoothing, c->red_out)) return s;
+  force_src src{c->f[FG_DENS], c->t.Surf, c->t.Rmed, c->t.cos_cell, c->t.sin_cell, x, y, rsmoothing, c->ns};
+  if (fg_status s = dreduce(c, src, (long)c->nr * c->ns, c->red_out, 1, 1)) return s;
   FG_HIP(hipStreamSynchronize(c->stream));
   out2[0] = c->h_out[0];
   out2[1] = c->h_out[1];

@@ -436,16 +436,13 @@ fg_status fg_viscosity_into(fg_ctx *c, double *nu_out) {
   return refresh_viscosity(c, nu_out);
 }
 
-fg_status fg_cfl_launch(fg_ctx *c, double DeltaT) {
+fg_status fg_cfl_ring_launch(fg_ctx *c) {
   const int nr = c->nr, ns = c->ns;
   size_t shm = (size_t)(ns + 256) * sizeof(double);
   hipLaunchKernelGGL(k_cfl_ring, dim3(nr), dim3(256), shm, c->stream, c->Vmoy, c->newDT, F(c, FG_VRAD),
                      F(c, FG_VTHETA), F(c, FG_SOUNDSPEED), F(c, FG_DENS),
                      c->p.adiabatic ? (const double *)F(c, FG_ENERGY) : (const double *)nullptr, c->cfl_out + 1, c->t,
                      nr, ns, c->p.fast_transport);
-  FG_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_cfl_final, dim3(1), dim3(256), 0, c->stream, c->cfl_out, c->DT1D, c->Vmoy, c->newDT,
-                     c->t.invRmed, c->t.dt1d_coef, DeltaT, nr);
   FG_LAUNCH_CHECK();
   return FG_OK;
 }
@@ -465,7 +462,10 @@ fg_status fg_cfl_result(fg_ctx *c, int *ncfl) {
 extern "C" fg_status fg_cfl(fg_ctx *c, double DeltaT, int *ncfl) {
   if (fg_status s = check(c)) return s;
   if (!ncfl) return FG_E_INVALID;
-  if (fg_status s = fg_cfl_launch(c, DeltaT)) return s;
+  if (fg_status s = fg_cfl_ring_launch(c)) return s;
+  hipLaunchKernelGGL(k_cfl_final, dim3(1), dim3(256), 0, c->stream, c->cfl_out, c->DT1D, c->Vmoy, c->newDT,
+                     c->t.invRmed, c->t.dt1d_coef, DeltaT, c->nr);
+  FG_LAUNCH_CHECK();
   FG_HIP(hipStreamSynchronize(c->stream));
   return fg_cfl_result(c, ncfl);
 }
