@@ -2972,33 +2972,10 @@ extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, dou
 }
 
 // ------------------------------------------- per-routine transport ----
-// ComputeVelocities of fg_transport (Kernels.cu:1193-1210; vtheta comes from
-// the azimuthal sweep) and what the reference's whole-array copies leave in the
-// ghost ring: the shifted fields 0, DENSINT the density's ghost values.
-struct close_args {
-  double *vr, *vt, *dens, *densint, *energy, *mom[4];
-  const double *xvt;
-  int nr, ns, adiabatic;
-};
-__global__ __launch_bounds__(256) void k_transport_close(close_args a) {
-  const int i = blockIdx.y, j = blockIdx.x * 256 + threadIdx.x, ns = a.ns;
-  if (j >= ns) return;
-  const long l = (long)i * ns + j;
-  if (i == a.nr) {
-    a.densint[l] = a.dens[l];
-    a.dens[l] = 0.0;
-    for (int q = 0; q < 4; q++) a.mom[q][l] = 0.0;
-    if (a.adiabatic) a.energy[l] = 0.0;
-    return;
-  }
-  a.vr[l] = i > 0 ? (a.mom[0][l - ns] + a.mom[1][l]) / (a.dens[l] + a.dens[l - ns] + 1e-20) : 0.0;
-  a.vt[l] = a.xvt[l];
-}
-
-// Transport (TransportEuler.cu:30) with the fused path's sweeps: three
+// Transport (TransportEuler.cu:30) with the fused path's sweeps: two
 // launches instead of one per quantity and step (86 with the copies), and the
-// fields that the routines leave.  9 + 9 + 3 us at 128 x 384, 18 + 18 + 6 us at
-// 384 x 1152; bound as the fused path's sweeps are.  A 128 x 384 substep with
+// fields that the routines leave (k_cells forms the velocities).  9 + 9 us at
+// 128 x 384, 18 + 18 us at 384 x 1152; bound as the fused path's sweeps are.  A 128 x 384 substep with
 // an open edge went from 393 to 121 us with it, one wait for all of a substep's
 // reductions, and results that the kernels write to host memory.
 fg_status fg_transport_sweeps(fg_ctx *c, double dt, double omega_frame) {
@@ -3046,22 +3023,6 @@ fg_status fg_transport_sweeps(fg_ctx *c, double dt, double omega_frame) {
   za.fast = c->p.fast_transport;
   const dim3 gz((ns + TAZW_P64 - 1) / TAZW_P64, nr);
   hipLaunchKernelGGL(adi ? k_tazw_full<6> : k_tazw_full<5>, gz, dim3(64), 0, c->stream, za);
-  FG_LAUNCH_CHECK();
-  close_args ca;
-  ca.vr = c->f[FG_VRAD];
-  ca.vt = c->f[FG_VTHETA];
-  ca.dens = c->f[FG_DENS];
-  ca.densint = c->f[FG_DENSINT];
-  ca.energy = c->f[FG_ENERGY];
-  ca.mom[0] = c->f[FG_RADMOMP];
-  ca.mom[1] = c->f[FG_RADMOMM];
-  ca.mom[2] = c->f[FG_THETAMOMP];
-  ca.mom[3] = c->f[FG_THETAMOMM];
-  ca.xvt = c->sw[6];
-  ca.nr = nr;
-  ca.ns = ns;
-  ca.adiabatic = adi;
-  hipLaunchKernelGGL(k_transport_close, dim3((ns + 255) / 256, nr + 1), dim3(256), 0, c->stream, ca);
   FG_LAUNCH_CHECK();
   return FG_OK;
 }

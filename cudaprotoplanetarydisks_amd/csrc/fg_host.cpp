@@ -35,7 +35,10 @@ fg_status fg_routine_results(fg_ctx *c, bool cfl, double DeltaT, int n, const in
                              const double *rs);
 fg_status fg_cfl_result(fg_ctx *c, int *ncfl);
 void fg_disk_force_result(const fg_ctx *c, int k, double out2[2]);
-fg_status fg_transport_launch(fg_ctx *c, double dt, double omega_frame);
+// a substep's routines up to the pressure and from the transport on
+fg_status fg_routine_begin(fg_ctx *c, const fg_planet_pot *planets, int nb, double ix, double iy, bool corotating,
+                           double domega, double dt, double omega_frame);
+fg_status fg_routine_end(fg_ctx *c, double dt, double omega_frame);
 double fg_lost_mass_result(const fg_ctx *c);
 
 namespace {
@@ -1172,14 +1175,14 @@ extern "C" fg_status fg_sim_substep(fg_sim *s, int *closed) {
   }
   s->dtemp += dt;
   double dopa[2] = {0.0, 0.0};
+  fg_planet_pot pl[FG_MAX_PLANETS];
+  int nb = 0;
   if (d.Corotating) psys_info(s, 1);
   if (d.IsDisk) {
     fg_disk_force_result(c, -1, dopa);
     s->IndirectX = d.Indirect_Term ? -dopa[0] : 0.0;
     s->IndirectY = d.Indirect_Term ? -dopa[1] : 0.0;
-    fg_planet_pot pl[FG_MAX_PLANETS];
-    int nb = potential_planets(s, pl);
-    CHECK(fg_potential(c, pl, nb, s->IndirectX, s->IndirectY));
+    nb = potential_planets(s, pl);
     // AdvanceSystemFromDisk, Pframeforce.cu:97-121
     for (int k = 0; k < p.nb; k++) {
       if (!p.feeldisk[k]) continue;
@@ -1192,23 +1195,20 @@ extern "C" fg_status fg_sim_substep(fg_sim *s, int *closed) {
     }
   }
   advance_rk5(s, dt);
+  double domega = 0.0;
   if (d.Corotating) {
     double OmegaNew = psys_info(s, 0) / dt;
-    double domega = OmegaNew - s->OmegaFrame;
-    if (d.IsDisk) CHECK(fg_correct_vtheta(c, domega));
+    domega = OmegaNew - s->OmegaFrame;
     s->OmegaFrame = OmegaNew;
   }
   rotate_psys(s, s->OmegaFrame * dt);
   if (d.IsDisk) {
-    CHECK(fg_boundary(c, dt, s->OmegaFrame));
-    CHECK(fg_pressure(c));
+    CHECK(fg_routine_begin(c, pl, nb, s->IndirectX, s->IndirectY, d.Corotating, domega, dt, s->OmegaFrame));
     CHECK(fg_substep1(c, dt, s->OmegaFrame));
     CHECK(fg_substep2(c, dt));
     CHECK(fg_boundary(c, dt, s->OmegaFrame));
     if (d.Adiabatic) CHECK(fg_substep3(c, dt));
-    CHECK(fg_transport_launch(c, dt, s->OmegaFrame));
-    CHECK(fg_boundary(c, dt, s->OmegaFrame));
-    CHECK(fg_temperature(c));
+    CHECK(fg_routine_end(c, dt, s->OmegaFrame));
     if (d.OpenInner) {
       CHECK(fg_sync(c));
       s->LostMass += fg_lost_mass_result(c);

@@ -33,7 +33,7 @@ fg_status fg_transport_sweeps(fg_ctx *c, double dt, double omega_frame);
 // their results read from h_out / h_cfl once the stream is idle
 fg_status fg_cfl_ring_launch(fg_ctx *c);
 fg_status fg_cfl_result(fg_ctx *c, int *ncfl);
-fg_status fg_transport_launch(fg_ctx *c, double dt, double omega_frame);
+fg_status fg_nonreflecting_internal(fg_ctx *c, double *press, double *temp);
 
 // Result block of the fused path (fg_ctx::h_fused, coherent pinned host
 // memory the final kernels write straight into): [0..1] star force,

@@ -228,12 +228,13 @@ extern "C" fg_status fg_circumplanetary_mass(fg_ctx *c, double xpl, double ypl, 
 // waits; this is 12 us at NSEC = 1152, and a 384 x 1152 substep with three of
 // them went from 605 to 126 us with it and fg_transport's sweeps.
 struct nr_args {
-  double *dens, *energy, *vr;
-  const double *cs;
+  double *dens, *energy, *vr, *press, *temp;  // press, temp: NULL or formed anew on the edge rings
+  const double *cs, *fpress;
   // inner, outer edge: pow(Rinf, -1.5) - 1 and the ring spacing of the shift's
   // angle, Sigma of vrad's ring, Sigma and energy means of the edge ring
   double num[2], width[2], sigma_v[2], sigma0[2], energy0[2];
-  int nr, ns;
+  double gamma;
+  int nr, ns, adiabatic;
 };
 
 // (int)x as the host converts it: out of range and NaN give INT_MIN
@@ -270,6 +271,14 @@ __device__ __forceinline__ void nr_edge(const nr_args &a, int edge, double *ring
     const double add = (f ? a.energy0[edge] : a.sigma0[edge]) - s_sum[0];
     for (int j = tid; j < ns; j += blockDim.x) q[e * ns + j] = ring[j] + add;
   }
+  if (a.press || a.temp) {
+    for (int j = tid; j < ns; j += blockDim.x) {  // as k_cells, of the cells that this thread wrote
+      const long l = e * ns + j;
+      if (a.press) a.press[l] = a.adiabatic ? (a.gamma - 1.0) * a.energy[l] : a.dens[l] * a.cs[l] * a.cs[l];
+      if (a.temp)
+        a.temp[l] = a.adiabatic ? (a.gamma - 1.0) * a.energy[l] / a.dens[l] : a.fpress[l] / a.dens[l];
+    }
+  }
   const double sm = a.sigma_v[edge];
   for (int j = tid; j < ns; j += blockDim.x) {
     if (edge == 0) {
@@ -295,7 +304,7 @@ __global__ __launch_bounds__(1024) void k_nr_edges(nr_args a) {
   }
 }
 
-fg_status fg_nonreflecting_internal(fg_ctx *c) {
+fg_status fg_nonreflecting_internal(fg_ctx *c, double *press, double *temp) {
   const int nr = c->nr, ns = c->ns;
   const std::vector<double> &Rinf = c->h_Rinf, &Rmed = c->h_Rmed;
   nr_args a;
@@ -303,6 +312,11 @@ fg_status fg_nonreflecting_internal(fg_ctx *c) {
   a.energy = c->f[FG_ENERGY];
   a.vr = c->f[FG_VRAD];
   a.cs = c->f[FG_SOUNDSPEED];
+  a.press = press;
+  a.temp = temp;
+  a.fpress = c->f[FG_PRESSURE];
+  a.gamma = c->p.adiabatic_index;
+  a.adiabatic = c->p.adiabatic;
   a.num[0] = pow(Rinf[1], -1.5) - 1.0;
   a.width[0] = Rmed[1] - Rmed[0];
   a.num[1] = pow(Rinf[nr - 2], -1.5) - 1.0;

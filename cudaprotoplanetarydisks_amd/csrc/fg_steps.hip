@@ -41,26 +41,6 @@ __global__ void k_sound_speed(double *cs, const double *dens, const double *ener
     cs[l] = sqrt(gamma * (gamma - 1.0) * energy[l] / dens[l]);
 }
 
-// Kernels.cu:187-200
-__global__ void k_pressure(double *P, const double *dens, const double *cs, const double *energy, int nr, int ns,
-                           int adiabatic, double gamma) {
-  CELLS(0, nr)
-  if (!adiabatic)
-    P[l] = dens[l] * cs[l] * cs[l];
-  else
-    P[l] = (gamma - 1.0) * energy[l];
-}
-
-// Kernels.cu:203-213 (MU/R = 1)
-__global__ void k_temperature(double *T, const double *dens, const double *P, const double *energy, int nr, int ns,
-                              int adiabatic, double gamma) {
-  CELLS(0, nr)
-  if (!adiabatic)
-    T[l] = P[l] / dens[l];
-  else
-    T[l] = (gamma - 1.0) * energy[l] / dens[l];
-}
-
 // Make1DprofileKernel, Kernels.cu:610-623: one ring per block, the ring is
 // staged in LDS and summed sequentially by one lane (the reference's j
 // order) so the mean is bit-identical.
@@ -85,82 +65,101 @@ __global__ void k_viscosity(double *nu, const double *cs_mean, const double *pow
   nu[i] = v;
 }
 
-// ---------------------------------------------------------- potential --
-// FillForcesArraysKernel, Kernels.cu:1226-1253, all planets in one pass
-// (the additions keep the reference's order: planet k, then the star
-// after planet 0).
-__global__ void k_potential(double *pot, const double *Rmed, const double *cosp, const double *sinp,
-                            fg_planets_arg P, int nr, int ns, int indirect) {
-  CELLS(0, nr)
-  const double Rm = Rmed[i];
-  const double InvDistance = 1.0 / Rm;
-  const double x = Rm * cosp[j];
-  const double y = Rm * sinp[j];
-  double acc = 0.0;
-  for (int k = 0; k < P.nb; k++) {
-    double xp = P.x[k], yp = P.y[k], m = P.m[k];
-    double distance = (x - xp) * (x - xp) + (y - yp) * (y - yp);
-    double distancesmooth = sqrt(distance + P.smooth[k]);
-    double pv = -1.0 * m / distancesmooth;
-    if (indirect) pv += 1.0 * m * P.invd3[k] * (x * xp + y * yp);
-    acc += pv;
-    if (k == 0) {
-      pv = -1.0 * 1.0 * InvDistance;
-      pv -= P.ix * x + P.iy * y;
+// ------------------------------------------------- cell by cell --
+// The routines that take each cell by itself, those of `flags` in this order:
+// a public routine launches its own, a substep of the simulation the ones that
+// follow each other, since at 128x384 each takes about 2 us and the next launch
+// as much again (a substep with an open edge: 20 launches 116 us, 13 launches
+// 100 us; 384x1152 with non-reflecting edges 20 launches 120, 14 launches 115 us).
+enum {
+  CELL_POTENTIAL = 1,    // FillForcesArraysKernel, Kernels.cu:1226-1253
+  CELL_CLOSE = 2,        // end of the transport, below
+  CELL_CORRECT = 4,      // CorrectVthetaKernel, Kernels.cu:1256-1263
+  CELL_OPEN = 8,         // OpenBoundaryKernel, Kernels.cu:482-495
+  CELL_EVANESCENT = 16,  // EvanescentBoundaryKernel, Kernels.cu:967-1015
+  CELL_PRESSURE = 32,    // Kernels.cu:187-200
+  CELL_TEMPERATURE = 64  // Kernels.cu:203-213 (MU/R = 1)
+};
+struct cells_args {
+  double *vr, *vt, *dens, *energy, *press, *temp, *pot, *densint, *mom[4];
+  const double *xvt, *cs, *nu, *sgacc;
+  fg_dev_tables t;
+  fg_planets_arg P;
+  double domega, dt, omega_frame, sigma0, gamma;
+  int flags, nr, ns, adiabatic, sg, indirect;
+};
+__global__ __launch_bounds__(TPB) void k_cells(cells_args a) {
+  const int nr = a.nr, ns = a.ns, flags = a.flags;
+  CELLS(0, nr + 1)
+  const fg_dev_tables &t = a.t;
+  if (i == nr) {
+    // what the reference's whole-array copies leave in the ghost ring: the
+    // shifted fields 0, DENSINT the density's ghost values
+    if (flags & CELL_CLOSE) {
+      a.densint[l] = a.dens[l];
+      a.dens[l] = 0.0;
+      for (int q = 0; q < 4; q++) a.mom[q][l] = 0.0;
+      if (a.adiabatic) a.energy[l] = 0.0;
+    }
+    return;
+  }
+  const double Rm = t.Rmed[i];
+  if (flags & CELL_POTENTIAL) {
+    // all planets in one pass (the additions keep the reference's order:
+    // planet k, then the star after planet 0)
+    const auto &P = ((__attribute__((address_space(4))) const cells_args *)__builtin_amdgcn_kernarg_segment_ptr())->P;
+    const double InvDistance = 1.0 / Rm;
+    const double x = Rm * t.cos_pot[j];
+    const double y = Rm * t.sin_pot[j];
+    double acc = 0.0;
+    for (int k = 0; k < P.nb; k++) {
+      const double xp = P.x[k], yp = P.y[k], m = P.m[k];
+      const double distance = (x - xp) * (x - xp) + (y - yp) * (y - yp);
+      const double distancesmooth = sqrt(distance + P.smooth[k]);
+      double pv = -1.0 * m / distancesmooth;
+      if (a.indirect) pv += 1.0 * m * P.invd3[k] * (x * xp + y * yp);
       acc += pv;
+      if (k == 0) {
+        pv = -1.0 * 1.0 * InvDistance;
+        pv -= P.ix * x + P.iy * y;
+        acc += pv;
+      }
+    }
+    a.pot[l] = acc;
+  }
+  // vrad of ring i >= 1 after the transport (Kernels.cu:1193-1210; vtheta
+  // comes from the azimuthal sweep)
+  auto closed_vr = [&](long m) { return (a.mom[0][m - ns] + a.mom[1][m]) / (a.dens[m] + a.dens[m - ns] + 1e-20); };
+  if (flags & CELL_CLOSE) {
+    if (!(flags & CELL_OPEN) || i != 1) a.vr[l] = i > 0 ? closed_vr(l) : 0.0;
+    a.vt[l] = a.xvt[l];
+  }
+  if (flags & CELL_CORRECT) a.vt[l] = a.vt[l] - a.domega * Rm;
+  if (flags & CELL_OPEN) {  // (rings 1 and 2 keep their density, ring 2 its vrad)
+    if (i == 0) {
+      a.dens[l] = a.dens[l + ns];
+      a.energy[l] = a.energy[l + ns];
+    } else if (i == 1) {
+      const double next = flags & CELL_CLOSE ? closed_vr(l + ns) : a.vr[l + ns];
+      a.vr[l] = (next > 0.0 || a.dens[l] < a.sigma0) ? 0.0 : next;
     }
   }
-  pot[l] = acc;
-}
-
-// ---------------------------------------------------------- boundaries --
-// CorrectVthetaKernel, Kernels.cu:1256-1263
-__global__ void k_correct_vtheta(double *vt, const double *Rmed, double domega, int nr, int ns) {
-  CELLS(0, nr)
-  vt[l] = vt[l] - domega * Rmed[i];
-}
-
-// EvanescentBoundaryKernel, Kernels.cu:967-1015 (per-ring constants from
-// host tables; lambda, vtheta0 and vrad0 evaluated as in the kernel)
-__global__ void k_evanescent(double *vr, double *vt, double *dens, double *energy, fg_dev_tables t, const double *nu,
-                             const double *sgacc, double step, double omega_frame, int nr, int ns, int adiabatic,
-                             int sg) {
-  CELLS(0, nr)
-  if (!t.ev_zone[i]) return;
-  const double Rm = t.Rmed[i];
-  double lambda = t.ev_coef[i] * step / t.ev_period[i];
-  double vtheta0 = sg ? sqrt(t.ev_vtheta_arg[i] - Rm * sgacc[i]) : sqrt(t.ev_vtheta_arg[i]);
-  vtheta0 -= Rm * omega_frame;
-  double vrad0 = -3.0 * nu[i] / Rm * t.vrad0_slope;
-  vr[l] = damp_toward(vr[l], lambda, vrad0);
-  vt[l] = damp_toward(vt[l], lambda, vtheta0);
-  dens[l] = damp_toward(dens[l], lambda, t.SigmaMed[i]);
-  if (adiabatic) energy[l] = damp_toward(energy[l], lambda, t.EnergyMed[i]);
-}
-
-// OpenBoundaryKernel, Kernels.cu:482-495
-__global__ void k_open_boundary(double *vr, double *dens, double *energy, int ns, double sigmamed0) {
-  int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= ns) return;
-  const int i = 1;
-  dens[(i - 1) * ns + j] = dens[i * ns + j];
-  energy[(i - 1) * ns + j] = energy[i * ns + j];
-  if (vr[(i + 1) * ns + j] > 0.0 || (dens[i * ns + j] < sigmamed0))
-    vr[i * ns + j] = 0.0;
-  else
-    vr[i * ns + j] = vr[(i + 1) * ns + j];
-}
-
-// ApplySubKeplerianBoundaryKernel, Kernels.cu:1416-1430 (host passes the
-// sqrt arguments; with self-gravity the ring mean of g_r enters)
-__global__ void k_sub_keplerian(double *vti, const double *Rmed, const double *sgacc, double arg_in,
-                                double arg_out, double omega_frame, int nr, int ns, int sg) {
-  int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= ns) return;
-  double vin = sg ? sqrt(arg_in - Rmed[0] * sgacc[0]) : sqrt(arg_in);
-  double vout = sg ? sqrt(arg_out - Rmed[nr - 1] * sgacc[nr - 1]) : sqrt(arg_out);
-  vti[j] = vin - Rmed[0] * omega_frame;
-  vti[(long)(nr - 1) * ns + j] = vout - Rmed[nr - 1] * omega_frame;
+  if ((flags & CELL_EVANESCENT) && t.ev_zone[i]) {
+    // per-ring constants from host tables; lambda, vtheta0 and vrad0
+    // evaluated as in the kernel
+    const double lambda = t.ev_coef[i] * a.dt / t.ev_period[i];
+    double vtheta0 = a.sg ? sqrt(t.ev_vtheta_arg[i] - Rm * a.sgacc[i]) : sqrt(t.ev_vtheta_arg[i]);
+    vtheta0 -= Rm * a.omega_frame;
+    const double vrad0 = -3.0 * a.nu[i] / Rm * t.vrad0_slope;
+    a.vr[l] = damp_toward(a.vr[l], lambda, vrad0);
+    a.vt[l] = damp_toward(a.vt[l], lambda, vtheta0);
+    a.dens[l] = damp_toward(a.dens[l], lambda, t.SigmaMed[i]);
+    if (a.adiabatic) a.energy[l] = damp_toward(a.energy[l], lambda, t.EnergyMed[i]);
+  }
+  if (flags & CELL_PRESSURE)
+    a.press[l] = a.adiabatic ? (a.gamma - 1.0) * a.energy[l] : a.dens[l] * a.cs[l] * a.cs[l];
+  if (flags & CELL_TEMPERATURE)
+    a.temp[l] = a.adiabatic ? (a.gamma - 1.0) * a.energy[l] / a.dens[l] : a.press[l] / a.dens[l];
 }
 
 // --------------------------------------------------------- Substep 1 --
@@ -208,16 +207,26 @@ __global__ void k_viscous_terms(const double *Vr, const double *Vt, const double
 }
 
 // UpdateVelocitiesKernel, Kernels.cu:118-150
+// and then, unless the edges damp (kepler), ApplySubKeplerianBoundaryKernel
+// (Kernels.cu:1416-1430; the sqrt arguments come from the host; with
+// self-gravity the ring mean of g_r enters)
 __global__ void k_update_velocities(double *vti, double *vri, const double *dens, const double *TRR,
                                     const double *TPP, const double *TRP, fg_dev_tables t, double DeltaT, int nr,
-                                    int ns) {
-  CELLS(1, nr)
+                                    int ns, int kepler, const double *sgacc, double arg_in, double arg_out,
+                                    double omega_frame, int sg) {
+  CELLS(0, nr)
   const double invdphi = t.invdphi;
-  if (i < nr - 1)
+  if (kepler && (i == 0 || i == nr - 1)) {
+    const double arg = i == 0 ? arg_in : arg_out;
+    const double v = sg ? sqrt(arg - t.Rmed[i] * sgacc[i]) : sqrt(arg);
+    vti[l] = v - t.Rmed[i] * omega_frame;
+  } else if (i > 0 && i < nr - 1) {
     vti[l] += DeltaT * t.invRmed[i] *
               ((t.Rsup[i] * TRP[l + ns] - t.Rinf[i] * TRP[l]) * t.invdiffRsup[i] + (TPP[l] - TPP[JM]) * invdphi +
                0.5 * (TRP[l] + TRP[l + ns])) /
               (0.5 * (dens[l] + dens[JM]));
+  }
+  if (i == 0) return;
   vri[l] += DeltaT * t.invRinf[i] *
             ((t.Rmed[i] * TRR[l] - t.Rmed[i - 1] * TRR[l - ns]) * t.invdiffRmed[i] + (TRP[JP] - TRP[l]) * invdphi -
              0.5 * (TPP[l] + TPP[l - ns])) /
@@ -225,43 +234,39 @@ __global__ void k_update_velocities(double *vti, double *vri, const double *dens
 }
 
 // --------------------------------------------------------- Substep 2 --
-// Substep2Kernel, Kernels.cu:409-434
-__global__ void k_substep2(double *qr, double *qt, const double *dens, const double *vri, const double *vti, int nr,
-                           int ns) {
-  CELLS(0, nr)
-  qr[l] = art_visc_q(dens[l], vri[l + ns] - vri[l]);
-  qt[l] = art_visc_q(dens[l], vti[JP] - vti[l]);
-}
-
-// "kernel", Kernels.cu:438-479
-// with ActualiseGasVrad/Vtheta (SourceEuler.cu:492-503): the new velocities,
-// rows 0 and NRAD as they were in the New fields, also into Vrad / Vtheta
-__global__ void k_host(double *vr, double *vt, double *vrnew, double *vtnew, double *eint, const double *dens,
-                       const double *vri, const double *vti, const double *qr, const double *qt, const double *energy, fg_dev_tables t,
-                       double dt, int nr, int ns, int adiabatic) {
+// Substep 2: the artificial pressure (Kernels.cu:409-434) into qr and qt, and
+// "kernel", Kernels.cu:438-479, which takes the neighbours' formed again, with
+// ActualiseGasVrad/Vtheta (SourceEuler.cu:492-503): the new velocities, rows 0
+// and NRAD as they were in the New fields, also into Vrad / Vtheta
+__global__ void k_substep2(double *vr, double *vt, double *vrnew, double *vtnew, double *eint, double *qr, double *qt,
+                           const double *dens, const double *vri, const double *vti, const double *energy,
+                           fg_dev_tables t, double dt, int nr, int ns, int adiabatic) {
   CELLS(0, nr + 1)
   if (i == nr) {
     vr[l] = vrnew[l];
     vt[l] = vtnew[l];
     return;
   }
+  const double dvr = vri[l + ns] - vri[l], dvt = vti[JP] - vti[l];
+  const double q = art_visc_q(dens[l], dvr), w = art_visc_q(dens[l], dvt);
+  qr[l] = q;
+  qt[l] = w;
   double v = vrnew[l];
   if (i > 0) {
     double d = dens[l] + dens[l - ns];
-    double densint = qr[l] - qr[l - ns];
+    double densint = q - art_visc_q(dens[l - ns], vri[l] - vri[l - ns]);
     v = vri[l] - dt * 2.0 / d * densint * t.invdiffRmed[i];
     vrnew[l] = v;
   }
   vr[l] = v;
   const double invdxtheta = t.invdxtheta[i];
   double dens2 = dens[l] + dens[JM];
-  double tempint = (qt[l] - qt[JM]);
-  const double w = vti[l] - dt * 2.0 / dens2 * tempint * invdxtheta;
-  vtnew[l] = w;
-  vt[l] = w;
+  double tempint = w - art_visc_q(dens[JM], vti[l] - vti[JM]);
+  const double u = vti[l] - dt * 2.0 / dens2 * tempint * invdxtheta;
+  vtnew[l] = u;
+  vt[l] = u;
   if (adiabatic)
-    eint[l] = energy[l] - dt * qr[l] * (vri[l + ns] - vri[l]) * t.invdiffRsup[i] -
-              dt * qt[l] * (vti[JP] - vti[l]) * invdxtheta;
+    eint[l] = energy[l] - dt * q * dvr * t.invdiffRsup[i] - dt * w * dvt * invdxtheta;
 }
 
 // --------------------------------------------------------- Substep 3 --
@@ -394,20 +399,67 @@ extern "C" fg_status fg_sound_speed(fg_ctx *c) {
   return FG_OK;
 }
 
+static fg_status pack_planets(fg_planets_arg *P, const fg_planet_pot *pl, int nb, double ix, double iy) {
+  if (nb < 0 || nb > FG_MAX_PLANETS || (nb > 0 && !pl)) {
+    fg_set_error("planet count %d outside 0..%d", nb, FG_MAX_PLANETS);
+    return FG_E_INVALID;
+  }
+  P->nb = nb;
+  for (int k = 0; k < nb; k++) {
+    P->x[k] = pl[k].x;
+    P->y[k] = pl[k].y;
+    P->m[k] = pl[k].mass;
+    P->smooth[k] = pl[k].smooth;
+    P->invd3[k] = pl[k].inv_d3;
+  }
+  P->ix = ix;
+  P->iy = iy;
+  return FG_OK;
+}
+
+// k_cells with the context's fields; the caller adds what its flags read besides
+static cells_args cells(fg_ctx *c, int flags) {
+  cells_args a{};
+  a.vr = F(c, FG_VRAD);
+  a.vt = F(c, FG_VTHETA);
+  a.dens = F(c, FG_DENS);
+  a.energy = F(c, FG_ENERGY);
+  a.press = F(c, FG_PRESSURE);
+  a.temp = F(c, FG_TEMPERATURE);
+  a.pot = F(c, FG_POTENTIAL);
+  a.densint = F(c, FG_DENSINT);
+  a.mom[0] = F(c, FG_RADMOMP);
+  a.mom[1] = F(c, FG_RADMOMM);
+  a.mom[2] = F(c, FG_THETAMOMP);
+  a.mom[3] = F(c, FG_THETAMOMM);
+  a.xvt = c->sw[6];
+  a.cs = F(c, FG_SOUNDSPEED);
+  a.nu = c->nu;
+  a.sgacc = c->sgacc_mean;
+  a.t = c->t;
+  a.sigma0 = c->h_SigmaMed[0];
+  a.gamma = c->p.adiabatic_index;
+  a.flags = flags;
+  a.nr = c->nr;
+  a.ns = c->ns;
+  a.adiabatic = c->p.adiabatic;
+  a.sg = c->p.self_gravity;
+  a.indirect = c->p.indirect_term;
+  return a;
+}
+static fg_status launch_cells(fg_ctx *c, const cells_args &a) {
+  LAUNCH(k_cells, 0, c->nr + 1, a);
+  return FG_OK;
+}
+
 extern "C" fg_status fg_pressure(fg_ctx *c) {
   if (fg_status s = check(c)) return s;
-  const int nr = c->nr, ns = c->ns;
-  LAUNCH(k_pressure, 0, nr, F(c, FG_PRESSURE), F(c, FG_DENS), F(c, FG_SOUNDSPEED), F(c, FG_ENERGY), nr, ns,
-         c->p.adiabatic, c->p.adiabatic_index);
-  return FG_OK;
+  return launch_cells(c, cells(c, CELL_PRESSURE));
 }
 
 extern "C" fg_status fg_temperature(fg_ctx *c) {
   if (fg_status s = check(c)) return s;
-  const int nr = c->nr, ns = c->ns;
-  LAUNCH(k_temperature, 0, nr, F(c, FG_TEMPERATURE), F(c, FG_DENS), F(c, FG_PRESSURE), F(c, FG_ENERGY), nr, ns,
-         c->p.adiabatic, c->p.adiabatic_index);
-  return FG_OK;
+  return launch_cells(c, cells(c, CELL_TEMPERATURE));
 }
 
 static fg_status refresh_viscosity(fg_ctx *c, double *nu_out) {
@@ -470,61 +522,68 @@ extern "C" fg_status fg_cfl(fg_ctx *c, double DeltaT, int *ncfl) {
   return fg_cfl_result(c, ncfl);
 }
 
-static fg_status pack_planets(fg_planets_arg *P, const fg_planet_pot *pl, int nb, double ix, double iy) {
-  if (nb < 0 || nb > FG_MAX_PLANETS || (nb > 0 && !pl)) {
-    fg_set_error("planet count %d outside 0..%d", nb, FG_MAX_PLANETS);
-    return FG_E_INVALID;
-  }
-  P->nb = nb;
-  for (int k = 0; k < nb; k++) {
-    P->x[k] = pl[k].x;
-    P->y[k] = pl[k].y;
-    P->m[k] = pl[k].mass;
-    P->smooth[k] = pl[k].smooth;
-    P->invd3[k] = pl[k].inv_d3;
-  }
-  P->ix = ix;
-  P->iy = iy;
-  return FG_OK;
-}
-
 extern "C" fg_status fg_potential(fg_ctx *c, const fg_planet_pot *planets, int nb, double ix, double iy) {
   if (fg_status s = check(c)) return s;
-  fg_planets_arg P;
-  if (fg_status s = pack_planets(&P, planets, nb, ix, iy)) return s;
-  const int nr = c->nr, ns = c->ns;
-  LAUNCH(k_potential, 0, nr, F(c, FG_POTENTIAL), c->t.Rmed, c->t.cos_pot, c->t.sin_pot, P, nr, ns,
-         c->p.indirect_term);
-  return FG_OK;
+  cells_args a = cells(c, CELL_POTENTIAL);
+  if (fg_status s = pack_planets(&a.P, planets, nb, ix, iy)) return s;
+  return launch_cells(c, a);
 }
 
 extern "C" fg_status fg_correct_vtheta(fg_ctx *c, double domega) {
   if (fg_status s = check(c)) return s;
-  const int nr = c->nr, ns = c->ns;
-  LAUNCH(k_correct_vtheta, 0, nr, F(c, FG_VTHETA), c->t.Rmed, domega, nr, ns);
-  return FG_OK;
+  cells_args a = cells(c, CELL_CORRECT);
+  a.domega = domega;
+  return launch_cells(c, a);
 }
 
-fg_status fg_nonreflecting_internal(fg_ctx *c);
+// the edges' routines behind the cells' (before) and before them (after: the
+// pressure or temperature), in as few launches as their order allows: an open or
+// an evanescent edge goes with the cells, the non-reflecting ones, which take ring
+// means, behind them, and form the edge rings' pressure or temperature anew.  With
+// several kinds of edges at once each has its own launch, and so has the end of the
+// transport, which reads the neighbours' densities, before the damping
+static fg_status with_boundary(fg_ctx *c, cells_args a, int after, double dt, double omega_frame) {
+  const fg_params &p = c->p;
+  a.dt = dt;
+  a.omega_frame = omega_frame;
+  const bool one = (p.open_inner != 0) + (p.non_reflecting != 0) + (p.evanescent != 0) <= 1 &&
+                   !(p.evanescent && a.flags & CELL_CLOSE);
+  if (one) {
+    a.flags |= after | (p.open_inner ? CELL_OPEN : 0) | (p.evanescent ? CELL_EVANESCENT : 0);
+    if (a.flags)
+      if (fg_status s = launch_cells(c, a)) return s;
+    if (!p.non_reflecting) return FG_OK;
+    if (p.adiabatic)
+      if (fg_status s = fg_sound_speed(c)) return s;
+    return fg_nonreflecting_internal(c, after & CELL_PRESSURE ? F(c, FG_PRESSURE) : nullptr,
+                                     after & CELL_TEMPERATURE ? F(c, FG_TEMPERATURE) : nullptr);
+  }
+  auto cells_of = [&](int flags) {
+    a.flags = flags;
+    return flags ? launch_cells(c, a) : FG_OK;
+  };
+  if (fg_status s = cells_of(a.flags)) return s;
+  if (fg_status s = cells_of(p.open_inner ? CELL_OPEN : 0)) return s;
+  if (p.non_reflecting) {
+    if (p.adiabatic)
+      if (fg_status s = fg_sound_speed(c)) return s;
+    if (fg_status s = fg_nonreflecting_internal(c, nullptr, nullptr)) return s;
+  }
+  return cells_of((p.evanescent ? CELL_EVANESCENT : 0) | after);
+}
 
 extern "C" fg_status fg_boundary(fg_ctx *c, double dt, double omega_frame) {
   if (fg_status s = check(c)) return s;
-  const int nr = c->nr, ns = c->ns;
-  if (c->p.open_inner) {
-    double sm0 = c->h_SigmaMed[0];
-    hipLaunchKernelGGL(k_open_boundary, dim3(fg_blocks(ns, 256)), dim3(256), 0, c->stream, F(c, FG_VRAD),
-                       F(c, FG_DENS), F(c, FG_ENERGY), ns, sm0);
-    FG_LAUNCH_CHECK();
-  }
-  if (c->p.non_reflecting) {
-    if (c->p.adiabatic)
-      if (fg_status s = fg_sound_speed(c)) return s;
-    if (fg_status s = fg_nonreflecting_internal(c)) return s;
-  }
-  if (c->p.evanescent)
-    LAUNCH(k_evanescent, 0, nr, F(c, FG_VRAD), F(c, FG_VTHETA), F(c, FG_DENS), F(c, FG_ENERGY), c->t, c->nu,
-           c->sgacc_mean, dt, omega_frame, nr, ns, c->p.adiabatic, c->p.self_gravity);
-  return FG_OK;
+  return with_boundary(c, cells(c, 0), 0, dt, omega_frame);
+}
+
+// fg_potential, fg_correct_vtheta (if corotating), fg_boundary and fg_pressure
+fg_status fg_routine_begin(fg_ctx *c, const fg_planet_pot *planets, int nb, double ix, double iy, bool corotating,
+                           double domega, double dt, double omega_frame) {
+  cells_args a = cells(c, CELL_POTENTIAL | (corotating ? CELL_CORRECT : 0));
+  a.domega = domega;
+  if (fg_status s = pack_planets(&a.P, planets, nb, ix, iy)) return s;
+  return with_boundary(c, a, CELL_PRESSURE, dt, omega_frame);
 }
 
 // Viscous stress of (vr, vt) into the TAU fields (Viscosity.cu:52-67).
@@ -548,27 +607,20 @@ extern "C" fg_status fg_substep1(fg_ctx *c, double dt, double omega_frame) {
   if (c->p.self_gravity)
     if (fg_status s = fg_selfgravity_kick(c, dt)) return s;
   if (fg_status s = viscous_terms(c, F(c, FG_VRADINT), F(c, FG_VTHETAINT))) return s;
-  LAUNCH(k_update_velocities, 1, nr, F(c, FG_VTHETAINT), F(c, FG_VRADINT), F(c, FG_DENS), F(c, FG_TAURR),
-         F(c, FG_TAUPP), F(c, FG_TAURP), c->t, dt, nr, ns);
-  if (!c->p.evanescent) {
-    // SideEuler.cu:194-206: the sqrt arguments are the evanescent
-    // vtheta0 arguments of the edge rings (same expression)
-    double ain = c->h_vtheta_arg[0], aout = c->h_vtheta_arg[nr - 1];
-    hipLaunchKernelGGL(k_sub_keplerian, dim3(fg_blocks(ns, 256)), dim3(256), 0, c->stream, F(c, FG_VTHETAINT),
-                       c->t.Rmed, c->sgacc_mean, ain, aout, omega_frame, nr, ns, c->p.self_gravity);
-    FG_LAUNCH_CHECK();
-  }
+  // SideEuler.cu:194-206: the sqrt arguments are the evanescent vtheta0
+  // arguments of the edge rings (same expression)
+  LAUNCH(k_update_velocities, 0, nr, F(c, FG_VTHETAINT), F(c, FG_VRADINT), F(c, FG_DENS), F(c, FG_TAURR),
+         F(c, FG_TAUPP), F(c, FG_TAURP), c->t, dt, nr, ns, !c->p.evanescent, c->sgacc_mean, c->h_vtheta_arg[0],
+         c->h_vtheta_arg[nr - 1], omega_frame, c->p.self_gravity);
   return FG_OK;
 }
 
 extern "C" fg_status fg_substep2(fg_ctx *c, double dt) {
   if (fg_status s = check(c)) return s;
   const int nr = c->nr, ns = c->ns;
-  LAUNCH(k_substep2, 0, nr, F(c, FG_DENSINT), F(c, FG_TEMPERINT), F(c, FG_DENS), F(c, FG_VRADINT),
-         F(c, FG_VTHETAINT), nr, ns);
-  LAUNCH(k_host, 0, nr + 1, F(c, FG_VRAD), F(c, FG_VTHETA), F(c, FG_VRADNEW), F(c, FG_VTHETANEW),
-         F(c, FG_ENERGYINT), F(c, FG_DENS), F(c, FG_VRADINT), F(c, FG_VTHETAINT), F(c, FG_DENSINT),
-         F(c, FG_TEMPERINT), F(c, FG_ENERGY), c->t, dt, nr, ns, c->p.adiabatic);
+  LAUNCH(k_substep2, 0, nr + 1, F(c, FG_VRAD), F(c, FG_VTHETA), F(c, FG_VRADNEW), F(c, FG_VTHETANEW),
+         F(c, FG_ENERGYINT), F(c, FG_DENSINT), F(c, FG_TEMPERINT), F(c, FG_DENS), F(c, FG_VRADINT),
+         F(c, FG_VTHETAINT), F(c, FG_ENERGY), c->t, dt, nr, ns, c->p.adiabatic);
   return FG_OK;
 }
 
@@ -587,17 +639,24 @@ extern "C" fg_status fg_substep3(fg_ctx *c, double dt) {
 
 fg_status fg_ring_sum_async(fg_ctx *c, const double *ring, double *out_dev);
 
-fg_status fg_transport_launch(fg_ctx *c, double dt, double omega_frame) {
+// the mass that left through an open inner edge (TransportEuler.cu:77); the
+// other edges' faces carry no flux
+static fg_status sum_lost_mass(fg_ctx *c) {
+  return c->p.open_inner ? fg_ring_sum_async(c, c->LostByDisk, c->red_out + 2) : FG_OK;
+}
+
+// fg_transport, fg_boundary and fg_temperature
+fg_status fg_routine_end(fg_ctx *c, double dt, double omega_frame) {
   if (fg_status s = fg_transport_sweeps(c, dt, omega_frame)) return s;
-  // the mass that left through an open inner edge (TransportEuler.cu:77); the
-  // other edges' faces carry no flux
-  if (c->p.open_inner) return fg_ring_sum_async(c, c->LostByDisk, c->red_out + 2);
-  return FG_OK;
+  if (fg_status s = with_boundary(c, cells(c, CELL_CLOSE), CELL_TEMPERATURE, dt, omega_frame)) return s;
+  return sum_lost_mass(c);
 }
 
 extern "C" fg_status fg_transport(fg_ctx *c, double dt, double omega_frame, double *lost_mass) {
   if (fg_status s = check(c)) return s;
-  if (fg_status s = fg_transport_launch(c, dt, omega_frame)) return s;
+  if (fg_status s = fg_transport_sweeps(c, dt, omega_frame)) return s;
+  if (fg_status s = launch_cells(c, cells(c, CELL_CLOSE))) return s;
+  if (fg_status s = sum_lost_mass(c)) return s;
   if (lost_mass) {
     if (c->p.open_inner) FG_HIP(hipStreamSynchronize(c->stream));
     *lost_mass = c->p.open_inner ? c->h_out[2] : 0.0;

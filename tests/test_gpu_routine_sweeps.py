@@ -2,13 +2,17 @@
 they can go wrong, against the FP64 oracle bit for bit (1e-12 for adiabatic
 decks, whose exp/log differ): rings narrower than a wave, of one azimuthal
 chunk (183 cells) and one cell more, the longest rings, disks of three and
-four rings (the two edges share rings), every edge with energy, and the full
-rotation swept at once."""
+four rings (the two edges share rings), every edge with energy, the full
+rotation swept at once, and several kinds of edges at once."""
+import contextlib
 import ctypes
+import itertools
 
 import numpy as np
 import pytest
 
+from cudaprotoplanetarydisks_amd import native
+from cudaprotoplanetarydisks_amd.sim import Context
 from test_gpu_parity import run_pair
 
 pytestmark = pytest.mark.gpu
@@ -47,43 +51,75 @@ class Tables(ctypes.Structure):
     _fields_ += [(n, ctypes.c_double) for n in "dtheta invdphi dt1d_coef vrad0_slope visc_value".split()]
 
 
-def axisymmetric_sweep(stretch):
-    """Sigma of 20 axisymmetric rings before and after fg_transport, and what
-    one ring's flux is multiplied with; outer faces at stretch * Rinf[i + 1]."""
-    from cudaprotoplanetarydisks_amd import native
-    from cudaprotoplanetarydisks_amd.sim import Context
-    nr, ns = 20, 70
-    edge = np.linspace(0.5, 2.5, nr + 2)
-    tab = {n: np.ones(nr + 1) for n in RING}
+NR, NS = 20, 70
+
+
+@contextlib.contextmanager
+def context(stretch=1.0, **params):
+    """A context of 20 rings of 70 cells on tables of its own, outer faces at
+    stretch * Rinf[i + 1], the three innermost rings in the damping zone."""
+    edge = np.linspace(0.5, 2.5, NR + 2)
+    tab = {n: np.ones(NR + 1) for n in RING}
     tab["Radii"], tab["Rinf"], tab["Rsup"] = edge[:-1], edge[:-1], edge[1:] * stretch
     tab["Rmed"] = 0.5 * (edge[:-1] + edge[1:])
-    tab["Surf"] = np.pi * (edge[1:]**2 - edge[:-1]**2) / ns
+    tab["Surf"] = np.pi * (edge[1:]**2 - edge[:-1]**2) / NS
     for n in ("Rinf", "Surf", "Rmed"):
         tab["inv" + n] = 1.0 / tab[n]
     tab["invdiffRmed"] = np.concatenate([[0.0], 1.0 / np.diff(tab["Rmed"])])
-    tab["dxtheta"] = 2 * np.pi / ns * tab["Rmed"]
+    tab["dxtheta"] = 2 * np.pi / NS * tab["Rmed"]
     tab["invdxtheta"] = 1.0 / tab["dxtheta"]
-    for n in ("ev_zone", "visc_cav_on"):
-        tab[n] = np.zeros(nr + 1, dtype=np.int32)
+    tab["visc_cav_on"] = np.zeros(NR + 1, dtype=np.int32)
+    tab["ev_zone"] = (np.arange(NR + 1) < 3).astype(np.int32)
     for n in SECTOR:
-        tab[n] = np.ones(ns)
+        tab[n] = np.ones(NS)
     tab = {n: np.ascontiguousarray(a) for n, a in tab.items()}
-    T = Tables(**{n: a.ctypes.data for n, a in tab.items()}, dtheta=2 * np.pi / ns, invdphi=ns / (2 * np.pi))
-    P = Params(nrad=nr, nsec=ns, fast_transport=1, open_inner=1, adiabatic_index=1.4)
+    T = Tables(**{n: a.ctypes.data for n, a in tab.items()}, dtheta=2 * np.pi / NS, invdphi=NS / (2 * np.pi))
+    P = Params(nrad=NR, nsec=NS, fast_transport=1, adiabatic_index=1.4, **params)
     h = ctypes.c_void_p()
     native.call("fg_create", ctypes.byref(P), ctypes.byref(T), 0, ctypes.byref(h))
     try:
-        ctx = Context(h, (nr + 1, ns))
-        rng = np.random.default_rng(3)
-        dens = np.repeat(rng.uniform(1.0, 2.0, (nr + 1, 1)), ns, axis=1)
-        ctx.set_field("DENS", dens)
-        ctx.set_field("VRAD", np.repeat(rng.uniform(-0.2, 0.2, (nr + 1, 1)), ns, axis=1))
-        ctx.set_field("VTHETA", np.repeat(tab["Rmed"][:, None] ** -0.5, ns, axis=1))
-        lost = ctypes.c_double()
-        native.call("fg_transport", h, 0.01, 1.0, ctypes.byref(lost))
-        return dens[:-1, 0], ctx.field("DENS")[:-1, 0], tab["invSurf"][:-1], lost.value / ns
+        yield Context(h, (NR + 1, NS)), h, tab
     finally:
         native.call("fg_destroy", h)
+
+
+def axisymmetric_sweep(stretch):
+    """Sigma of axisymmetric rings before and after fg_transport, what a ring's
+    flux is multiplied with, and the mass lost per sector."""
+    with context(stretch, open_inner=1) as (ctx, h, tab):
+        rng = np.random.default_rng(3)
+        dens = np.repeat(rng.uniform(1.0, 2.0, (NR + 1, 1)), NS, axis=1)
+        ctx.set_field("DENS", dens)
+        ctx.set_field("VRAD", np.repeat(rng.uniform(-0.2, 0.2, (NR + 1, 1)), NS, axis=1))
+        ctx.set_field("VTHETA", np.repeat(tab["Rmed"][:, None] ** -0.5, NS, axis=1))
+        lost = ctypes.c_double()
+        native.call("fg_transport", h, 0.01, 1.0, ctypes.byref(lost))
+        return dens[:-1, 0], ctx.field("DENS")[:-1, 0], tab["invSurf"][:-1], lost.value / NS
+
+
+EDGES = ("open_inner", "non_reflecting", "evanescent")
+
+
+@pytest.mark.parametrize("kinds", [c for n in (1, 2, 3) for c in itertools.combinations(EDGES, n)], ids="-".join)
+@pytest.mark.parametrize("adiabatic", [0, 1])
+def test_edges_one_after_the_other(kinds, adiabatic):
+    """Several kinds of edges at once: as one after the other, bit for bit."""
+    rng = np.random.default_rng(5)
+    names = ("DENS", "VRAD", "VTHETA", "ENERGY", "SOUNDSPEED")
+    state = [rng.uniform(0.5, 1.5, (NR + 1, NS)) for _ in names]
+
+    def boundary(state, kinds):
+        with context(adiabatic=adiabatic, **{k: 1 for k in kinds}) as (ctx, h, _):
+            for n, a in zip(names, state):
+                ctx.set_field(n, a)
+            native.call("fg_boundary", h, 0.01, 1.0)
+            return [ctx.field(n) for n in names]
+
+    want = state
+    for k in kinds:
+        want = boundary(want, [k])
+    for n, a, b in zip(names, boundary(state, kinds), want):
+        assert np.array_equal(a, b), n
 
 
 def test_own_outer_faces():
