@@ -925,16 +925,15 @@ struct taz_args {
 // overlap by those halos; each cell is output by exactly one chunk.
 #define TAZW_HL 5
 #define TAZW_HR 4
-#define TAZW_P32 (64 * 4 - TAZW_HL - TAZW_HR)  // cells output per batched FP32 chunk (CL = 4)
-// single-disk FP32 chunks: three cells per lane in their own kernel held to
-// 96 VGPRs, five waves per SIMD (seven dwords go to scratch)
-#define TAZW_CL32 3
-#define TAZW_P32S (64 * TAZW_CL32 - TAZW_HL - TAZW_HR)
-// FP64 chunks: three cells per lane (the five- and six-quantity sweeps fit
-// in 142 and 164 VGPRs, three waves per SIMD; four or five cells per lane
-// take 174-208 VGPRs and leave two)
-#define TAZW_CL64 3
-#define TAZW_P64 (64 * TAZW_CL64 - TAZW_HL - TAZW_HR)  // cells output per FP64 chunk
+// Cells per lane: two on grids below 2^20 cells and in batches, where more and
+// shorter chunks fill the chip (k_tazw, us with two and three: 128 x 384 9.0 and
+// 10.4, 512 x 1536 27.8 and 29.3; FP32 128 x 384 7.9 and 9.1, 512 x 1536 18.3 and
+// 19.0; 8 batched disks 177 and 180 per substep), three beyond, where the halo's
+// bytes count (FP32 1024 x 3072 41.8 and 41.0, FP64 the same within 1 %).  Three
+// FP64 cells take 142 or 164 VGPRs and leave three waves per SIMD, four or five
+// cells two; three FP32 cells are held to 96 VGPRs, five waves.
+#define TAZW_P(CL) (64 * (CL) - TAZW_HL - TAZW_HR)  // cells that a chunk outputs
+static int tazw_cells(const fg_ctx *c) { return (long)c->nr * c->ns < (1L << 20) ? 2 : 3; }
 
 __device__ __forceinline__ float lane_prev(float x) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xf, 0xf, true));
@@ -1257,29 +1256,27 @@ __device__ __forceinline__ void tazw_body(const taz_args &a, int i, int chunk, t
 }
 
 // blockIdx.x = chunk, blockIdx.y = ring
-template <int CL, bool F32, int NQT = 5>
+template <int CL, int NQT>
 __global__ __launch_bounds__(64) void k_tazw(taz_args a) {
   __shared__ tazw_lds<CL, NQT> sh;
-  if (F32 && in_lob(blockIdx.y, a.lob0, a.lob1))
-    tazw_body<CL, F32, NQT, F32>(a, blockIdx.y, blockIdx.x, sh);
-  else
-    tazw_body<CL, F32, NQT, false>(a, blockIdx.y, blockIdx.x, sh);
+  tazw_body<CL, false, NQT>(a, blockIdx.y, blockIdx.x, sh);
 }
 
 // the azimuthal sweeps of fg_transport
-template <int NQT>
+template <int CL, int NQT>
 __global__ __launch_bounds__(64) void k_tazw_full(taz_args a) {
-  __shared__ tazw_lds<TAZW_CL64, NQT> sh;
-  tazw_body<TAZW_CL64, false, NQT, false, true>(a, blockIdx.y, blockIdx.x, sh);
+  __shared__ tazw_lds<CL, NQT> sh;
+  tazw_body<CL, false, NQT, false, true>(a, blockIdx.y, blockIdx.x, sh);
 }
 
-// the FP32 bulk mode's single-disk sweep (TAZW_CL32 cells per lane)
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_tazw32(taz_args a) {
-  __shared__ tazw_lds<TAZW_CL32, 5> sh;
+// the FP32 bulk mode's single-disk sweep
+template <int CL>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CL == 2 ? 7 : 5))) void k_tazw32(taz_args a) {
+  __shared__ tazw_lds<CL, 5> sh;
   if (in_lob(blockIdx.y, a.lob0, a.lob1))
-    tazw_body<TAZW_CL32, true, 5, true>(a, blockIdx.y, blockIdx.x, sh);
+    tazw_body<CL, true, 5, true>(a, blockIdx.y, blockIdx.x, sh);
   else
-    tazw_body<TAZW_CL32, true, 5, false>(a, blockIdx.y, blockIdx.x, sh);
+    tazw_body<CL, true, 5, false>(a, blockIdx.y, blockIdx.x, sh);
 }
 
 // ------------------------------------------------------------ k_fin ----
@@ -2893,22 +2890,13 @@ extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, dou
   za.lob0 = lob0;
   za.lob1 = lob1;
   prof_mark(c);
-  if (!fp32) {
-    // FP64, five quantities or six with the energy: at 1024 x 3072, 17
-    // chunks a ring (6 % halo cells) at three waves per SIMD run 65 us
-    // against 72 us for 10 chunks of five cells per lane at two waves (the
-    // ring as one 256-thread workgroup took 143 us)
-    const dim3 gw((ns + TAZW_P64 - 1) / TAZW_P64, nr);
-    if (adi)
-      hipLaunchKernelGGL((k_tazw<TAZW_CL64, false, 6>), gw, dim3(64), 0, c->stream, za);
-    else
-      hipLaunchKernelGGL((k_tazw<TAZW_CL64, false>), gw, dim3(64), 0, c->stream, za);
-  } else {
-    // FP32: three cells per lane at five waves per SIMD, 40.7 -> 38.4 us at
-    // 1024 x 3072 against four cells per lane at four (113 us as one
-    // 256-thread workgroup per ring)
-    const dim3 gw((ns + TAZW_P32S - 1) / TAZW_P32S, nr);
-    hipLaunchKernelGGL(k_tazw32, gw, dim3(64), 0, c->stream, za);
+  {
+    const int cl = tazw_cells(c);
+    const dim3 gw((ns + TAZW_P(cl) - 1) / TAZW_P(cl), nr);
+    auto taz = fp32 ? (cl == 2 ? k_tazw32<2> : k_tazw32<3>)
+               : adi ? (cl == 2 ? k_tazw<2, 6> : k_tazw<3, 6>)
+                     : (cl == 2 ? k_tazw<2, 5> : k_tazw<3, 5>);
+    hipLaunchKernelGGL(taz, gw, dim3(64), 0, c->stream, za);
   }
   FG_LAUNCH_CHECK();
   // k_fin
@@ -3021,8 +3009,10 @@ fg_status fg_transport_sweeps(fg_ctx *c, double dt, double omega_frame) {
   za.nr = nr;
   za.ns = ns;
   za.fast = c->p.fast_transport;
-  const dim3 gz((ns + TAZW_P64 - 1) / TAZW_P64, nr);
-  hipLaunchKernelGGL(adi ? k_tazw_full<6> : k_tazw_full<5>, gz, dim3(64), 0, c->stream, za);
+  const int cl = tazw_cells(c);
+  const dim3 gz((ns + TAZW_P(cl) - 1) / TAZW_P(cl), nr);
+  auto taz = adi ? (cl == 2 ? k_tazw_full<2, 6> : k_tazw_full<3, 6>) : (cl == 2 ? k_tazw_full<2, 5> : k_tazw_full<3, 5>);
+  hipLaunchKernelGGL(taz, gz, dim3(64), 0, c->stream, za);
   FG_LAUNCH_CHECK();
   return FG_OK;
 }
@@ -3102,7 +3092,7 @@ __global__ __launch_bounds__(TRAD_TPB) void k_batch_trad(const batch_disk *__res
 
 // one chunk of one ring per item: y = ring * chunks + chunk
 __global__ __launch_bounds__(64) void k_batch_taz(const batch_disk *__restrict__ D, const int2 *__restrict__ items, int n) {
-  __shared__ tazw_lds<4, 5> sh;
+  __shared__ tazw_lds<2, 5> sh;
   if ((int)blockIdx.x >= n) return;
   const int2 w = uniform2(items[blockIdx.x]);
   if (!D[w.x].active) return;
@@ -3118,12 +3108,12 @@ __global__ __launch_bounds__(64) void k_batch_taz(const batch_disk *__restrict__
   a.sbar = global(a.sbar);
   a.vref = global(a.vref);
   a.nshift = global(a.nshift);
-  const int nch = (a.ns + TAZW_P32 - 1) / TAZW_P32;
+  const int nch = (a.ns + TAZW_P(2) - 1) / TAZW_P(2);
   const int i = w.y / nch;
   if (in_lob(i, a.lob0, a.lob1))
-    tazw_body<4, true, 5, true>(a, i, w.y % nch, sh);
+    tazw_body<2, true, 5, true>(a, i, w.y % nch, sh);
   else
-    tazw_body<4, true, 5, false>(a, i, w.y % nch, sh);
+    tazw_body<2, true, 5, false>(a, i, w.y % nch, sh);
 }
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_batch_fin(
@@ -3284,7 +3274,7 @@ static fg_status batch_build(fg_batch_dev *b) {
     const int nstrips = (ns + TRAD_TPB - 1) / TRAD_TPB;
     const int nblk = nr + nstrips * ((nr + band - 1) / band);
     for (int q = 0; q < nblk; q++) trad.push_back(make_int2(k, q));
-    const int nch = (ns + TAZW_P32 - 1) / TAZW_P32;
+    const int nch = (ns + TAZW_P(2) - 1) / TAZW_P(2);
     for (int i = 0; i < nr; i++) {
       for (int ch = 0; ch < nch; ch++) taz.push_back(make_int2(k, i * nch + ch));
       fin.push_back(make_int2(k, i));

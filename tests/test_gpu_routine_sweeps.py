@@ -1,7 +1,7 @@
 """fg_transport's strip sweeps and the one-kernel non-reflecting edges where
 they can go wrong, against the FP64 oracle bit for bit (1e-12 for adiabatic
 decks, whose exp/log differ): rings narrower than a wave, of one azimuthal
-chunk (183 cells) and one cell more, the longest rings, disks of three and
+chunk (119 cells) and one cell more, the longest rings, disks of three and
 four rings (the two edges share rings), every edge with energy, the full
 rotation swept at once, and several kinds of edges at once."""
 import contextlib
@@ -20,7 +20,7 @@ pytestmark = pytest.mark.gpu
 OPEN, NONREF = dict(InnerBoundary="OPEN"), dict(InnerBoundary="NONREFLECTING")
 
 
-@pytest.mark.parametrize("nrad, nsec", [(5, 3), (9, 63), (7, 183), (6, 184), (131, 130), (4, 4100), (3, 8192)])
+@pytest.mark.parametrize("nrad, nsec", [(5, 3), (9, 63), (7, 119), (6, 120), (7, 183), (6, 184), (131, 130), (4, 4100), (3, 8192)])
 @pytest.mark.parametrize("kw", [OPEN, NONREF, dict(OPEN, Transport="STANDARD")], ids=["open", "nonref", "standard"])
 def test_edges(deck, nrad, nsec, kw):
     run_pair(deck(Nrad=nrad, Nsec=nsec, DT=0.01, **kw), 3, 0.0)
