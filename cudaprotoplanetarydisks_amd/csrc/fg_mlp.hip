@@ -322,12 +322,13 @@ __device__ __forceinline__ void mlp_store_rows(mlp_b *t, const bf16_t (&h)[V]) {
 // through one L2 (with neighbouring rows on different XCDs, k_mlp_weights
 // read the partly written lines 55 us slower).
 // The last workgroup of a launch with loss != NULL reduces the previous
-// step's loss partials instead.
+// step's loss partials instead.  Y: where a forward pass's output goes (NULL:
+// Z of the last layer).
 template <int V, bool TRAIN>
 __global__ __launch_bounds__(MLP_ROWS_TPB) void k_mlp_rows(const mlp_layer *__restrict__ net, int L,
                                                            const float *__restrict__ X, const float *__restrict__ T,
                                                            int batch, int ldb, int ld, const float *lossp,
-                                                           float *loss) {
+                                                           float *loss, float *Y) {
   extern __shared__ __attribute__((aligned(16))) bf16_t lds_mlp[];
   if (TRAIN && loss && blockIdx.x == gridDim.x - 1) {
     mlp_loss_tree(lossp, (long)batch * net[L - 1].N, (float *)lds_mlp, loss);
@@ -404,7 +405,7 @@ __global__ __launch_bounds__(MLP_ROWS_TPB) void k_mlp_rows(const mlp_layer *__re
             if (TRAIN) n.Z[o] = d;
           }
         } else if (in) {
-          n.Z[o] = x;
+          (!TRAIN && Y ? (mlp_f *)Y : n.Z)[o] = x;
           if (TRAIN) {  // dY = 2 (Y - T) / n
             const float d = x - t[v];
             const float gd = scale * d;
@@ -658,7 +659,14 @@ struct fg_mlp {
   int ld, ldb;                   // LDS row length of k_mlp_rows, row length of the transposes
   float *Xall, *Tall;
   size_t all_cap;                // samples they hold
+  // small forward passes: pinned host memory that k_mlp_rows reads its rows from
+  // and writes its output to, and its device alias
+  float *h_io, *d_io;
 };
+// Bytes of it at most.  The two copies cost the call more than the kernel's own
+// way over the bus (us per fg_mlp_forward of 5-256x4-512 with and without them:
+// 1 row 39 and 27, 128 rows 50 and 37, 1024 rows, 2.1 MB, 161 and 135).
+#define MLP_IO_BYTES (4 << 20)
 
 // Rows per workgroup of k_mlp_rows, 4 V: few, so that the chip's CUs share
 // the GELUs, until every CU has a workgroup; then more rows for each passage
@@ -706,6 +714,7 @@ extern "C" fg_status fg_mlp_destroy(fg_mlp *m) {
     for (void *x : q)
       if (x) (void)hipFree(x);
   }
+  if (m->h_io) (void)hipHostFree(m->h_io);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
   return FG_OK;
@@ -870,30 +879,31 @@ extern "C" fg_status fg_mlp_get_params(fg_mlp *m, float *params) {
 }
 
 // networks in LDS: forward pass of `batch` rows of x (device); output in
-// Z[L-1].  With t (device targets) also the gradients of the
+// y, or Z[L-1] without it.  With t (device targets) also the gradients of the
 // pre-activations; *prev_loss, when not NULL, takes the loss of the step
 // before this one.
 template <int V>
-static fg_status mlp_rows_launch(fg_mlp *m, const float *x, const float *t, int batch, float *prev_loss) {
+static fg_status mlp_rows_launch(fg_mlp *m, const float *x, const float *t, int batch, float *prev_loss, float *y) {
   const size_t lds = mlp_rows_lds(m->ld, V);
   if (t) {
     // rows up to the next multiple of 32 are written (as zeros), which the
     // weight gradients' last step over the batch reads
     const int blocks = fg_blocks((batch + 31) / 32 * (32 / (4 * V)), 8) * 8 + (prev_loss ? 1 : 0);
     hipLaunchKernelGGL((k_mlp_rows<V, true>), dim3(blocks), dim3(MLP_ROWS_TPB), lds, m->stream, m->net, m->L, x, t,
-                       batch, m->ldb, m->ld, m->lossp, prev_loss);
+                       batch, m->ldb, m->ld, m->lossp, prev_loss, nullptr);
   } else {
     hipLaunchKernelGGL((k_mlp_rows<V, false>), dim3(fg_blocks(fg_blocks(batch, 4 * V), 8) * 8), dim3(MLP_ROWS_TPB), lds,
-                       m->stream, m->net, m->L, x, nullptr, batch, m->ldb, m->ld, nullptr, nullptr);
+                       m->stream, m->net, m->L, x, nullptr, batch, m->ldb, m->ld, nullptr, nullptr, y);
   }
   FG_LAUNCH_CHECK();
   return FG_OK;
 }
-static fg_status mlp_rows(fg_mlp *m, const float *x, const float *t, int batch, float *prev_loss) {
+static fg_status mlp_rows(fg_mlp *m, const float *x, const float *t, int batch, float *prev_loss,
+                          float *y = nullptr) {
   switch (mlp_rows_v(batch)) {
-    case 1: return mlp_rows_launch<1>(m, x, t, batch, prev_loss);
-    case 2: return mlp_rows_launch<2>(m, x, t, batch, prev_loss);
-    default: return mlp_rows_launch<4>(m, x, t, batch, prev_loss);
+    case 1: return mlp_rows_launch<1>(m, x, t, batch, prev_loss, y);
+    case 2: return mlp_rows_launch<2>(m, x, t, batch, prev_loss, y);
+    default: return mlp_rows_launch<4>(m, x, t, batch, prev_loss, y);
   }
 }
 
@@ -1009,6 +1019,26 @@ static fg_status check_batch(fg_mlp *m, int batch) {
 // y[batch x outputs] = MLP(x[batch x inputs]), row-major FP32
 extern "C" fg_status fg_mlp_forward(fg_mlp *m, const float *x, int batch, float *y) {
   if (fg_status s = check_batch(m, batch)) return s;
+  const size_t nx = (size_t)batch * m->width[0], ny = (size_t)batch * m->width[m->L];
+  if (m->net && (nx + ny) * 4 <= MLP_IO_BYTES) {
+    if (!m->h_io) {
+      void *h = nullptr, *d = nullptr;
+      const size_t most = (size_t)m->max_batch * (m->width[0] + m->width[m->L]) * 4;
+      FG_HIP(hipHostMalloc(&h, std::min(most, (size_t)MLP_IO_BYTES), hipHostMallocCoherent | hipHostMallocMapped));
+      if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
+        (void)hipHostFree(h);
+        fg_set_error("mlp: no device address of pinned memory");
+        return FG_E_HIP;
+      }
+      m->h_io = (float *)h;
+      m->d_io = (float *)d;
+    }
+    std::memcpy(m->h_io, x, nx * 4);
+    if (fg_status s = mlp_rows(m, m->d_io, nullptr, batch, nullptr, m->d_io + nx)) return s;
+    FG_HIP(hipStreamSynchronize(m->stream));
+    std::memcpy(y, m->h_io + nx, ny * 4);
+    return FG_OK;
+  }
   FG_HIP(hipMemcpyAsync(m->X, x, (size_t)batch * m->width[0] * 4, hipMemcpyHostToDevice, m->stream));
   if (fg_status s = mlp_forward(m, batch)) return s;
   FG_HIP(hipMemcpyAsync(y, m->Z[m->L - 1], (size_t)batch * m->width[m->L] * 4, hipMemcpyDeviceToHost, m->stream));

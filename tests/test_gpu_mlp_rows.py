@@ -58,3 +58,16 @@ def test_rows_do_not_depend_on_the_batch():
         for n in (1, 6, 1000, 1030, 2049):
             assert np.array_equal(net.forward(x[:n]), whole[:n]), n
         assert np.array_equal(net.forward(x[1000:1007]), whole[1000:1007])
+
+
+def test_forward_without_copies():
+    """Batches that go over pinned memory (to 4 MB) and beyond: a row's output
+    does not depend on its batch, bit for bit."""
+    rng = np.random.default_rng(8)
+    x = rng.normal(size=(2100, 5))
+    edge = (4 << 20) // (4 * (5 + 512))
+    with MLP([5, 256, 256, 256, 256, 512], max_batch=2100) as m:
+        want = m.forward(x)
+        for batch in (1, 3, 128, edge, edge + 1):
+            assert np.array_equal(m.forward(x[:batch]), want[:batch]), batch
+        assert np.array_equal(m.forward(x[::-1][:77]), want[::-1][:77])  # a new batch in the same memory
