@@ -1464,7 +1464,8 @@ __device__ __forceinline__ void ring_min_store(double best, double *red, double 
 // ADI: adiabatic deck; S32: FP32 bulk mode (FP32 storage of k_taz's fields);
 // PAIRS: ring i - 1, i or i + 1 stored as float pairs (its own instance, so that
 // the other rings run without the residuals' loads).
-// Bound: HBM on large grids (2048 x 4096: 454 MB in 112 us), latency on small
+// Bound: HBM on large grids (2048 x 4096: 478 MB by the counters, 470 of them
+// compulsory, in 112 us), latency on small
 // ones.  Was one lane's sum of the ring beside a pass that kept its terms in
 // registers (and two passes over rings beyond 3072 cells): 1024 x 3072 58 -> 51
 // us, 2048 x 4096 201 -> 112, 512 x 1536 24 -> 17; FP32 1024 x 3072 43 -> 34.
@@ -2665,7 +2666,7 @@ static int march_band(const std::vector<int2> &disks, int most, int resident = 3
     long waves = 0;
     for (const int2 &d : disks) waves += (long)d.y * ((d.x + h - 1) / h);
     const double n = (double)waves / simds;
-    const double cost = (h + 3) * (n > resident ? share * n : std::max(1.0, share * ceil(n)));
+    const double cost = (h + 3) * std::max(1.0, share * (n > resident ? n : ceil(n)));
     if (h == 1 || cost < best) {
       best = cost;
       band = h;
