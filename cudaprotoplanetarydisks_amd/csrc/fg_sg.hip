@@ -207,8 +207,13 @@ __device__ __forceinline__ double2 bfly2(double2 x0, double2 x1, double2 w0, dou
 // same radix-2 expression of the same operands as when the levels run one
 // after the other through LDS, so both give the same bits (as does
 // k_fft_lines), with half the LDS round trips and barriers.
+// Bound: the levels' chain of LDS round trips, 112 FP64 operations a group and
+// barriers, at eight waves per SIMD (62 VGPRs, which the attribute keeps).
+// 512 x 1536 (us): columns with the product 51 -> 46, inverse columns 39 -> 33, rows
+// 39 and 23 as before, since a pair's twiddles are loaded before the barriers in
+// front of it and a deepest factor of 2 is a radix-2 level like the others.
 template <int CB, int MODE, int TPB>
-__global__ __launch_bounds__(TPB) void k_fft_pow2(fft_args a) {
+__global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(8))) void k_fft_pow2(fft_args a) {
   extern __shared__ double2 buf[];
   constexpr int LCB = CB == 1 ? 0 : CB == 2 ? 1 : CB == 4 ? 2 : 3;
   const int N = a.n, tid = threadIdx.x;
@@ -222,11 +227,31 @@ __global__ __launch_bounds__(TPB) void k_fft_pow2(fft_args a) {
   } else {
     for (int e = tid; e < E; e += TPB) buf[e] = fft_load<MODE>(a, g, line0 + (e & (CB - 1)), e >> LCB);
   }
+  // Pairs of levels: lower d (L/2, 2S), upper d - 1 (L, S); one group of four per
+  // thread (E / 4 <= TPB).  Its six twiddles are loaded in front of the barriers
+  // that precede it, so that no level begins with a round trip to the table
+  // (r = 0 has the same w[0] on every level).
+  const double2 w0 = a.tw[a.off[0]];
+  const bool live = tid < (E >> 2);
+  const int cb4 = tid & (CB - 1), rest = tid >> LCB;  // group: line cb4, sub-problem s, k2
+  double2 ta, tb, u0, u1, u2, u3;
+  auto twiddles = [&](int d) __attribute__((always_inline)) {
+    if (d < 1 || !live) return;
+    const int q = a.L[d - 1] >> 2, k2 = rest >> a.sh[d - 1];
+    const double2 *wl = a.tw + a.off[d], *wu = a.tw + a.off[d - 1];
+    ta = wl[k2];
+    tb = wl[k2 + q];
+    u0 = wu[k2];
+    u1 = wu[k2 + q];
+    u2 = wu[k2 + 2 * q];
+    u3 = wu[k2 + 3 * q];
+  };
+  int d = a.nst - 1;
+  if (a.p[d] == 2 && (d & 1)) twiddles(d);
   __syncthreads();
   double2 out[FFT2_U];
-  {
+  if (a.p[d] != 2) {
     // deepest level: L = p (any factor), S = N / p, m = 1, k = 0
-    const int d = a.nst - 1;
     const int p = a.p[d], L = a.L[d], sh = a.sh[d], S = 1 << sh;
     const double2 *w = a.tw + a.off[d];
 #pragma unroll
@@ -255,16 +280,16 @@ __global__ __launch_bounds__(TPB) void k_fft_pow2(fft_args a) {
       const int e = tid + u * TPB;
       if (e < E) buf[e] = out[u];
     }
+    d--;
+    if (d & 1) twiddles(d);
     __syncthreads();
   }
-  int d = a.nst - 2;
   if (d >= 0 && (d & 1) == 0) {
     // an odd number of radix-2 levels: the lowest one alone (r = 0 with
     // w[0], r = 1 with w[kk])
     const int L = a.L[d], sh = a.sh[d], m = L >> 1;
     const int S = 1 << sh;
     const double2 *w = a.tw + a.off[d];
-    const double2 w0 = w[0];
 #pragma unroll
     for (int u = 0; u < FFT2_U; u++) {
       const int e = tid + u * TPB;
@@ -282,41 +307,36 @@ __global__ __launch_bounds__(TPB) void k_fft_pow2(fft_args a) {
       const int e = tid + u * TPB;
       if (e < E) buf[e] = out[u];
     }
-    __syncthreads();
     d--;
+    twiddles(d);
+    __syncthreads();
   }
-  // pairs of levels: lower d (L/2, 2S), upper d - 1 (L, S); one group of
-  // four per thread (E / 4 <= TPB)
   for (; d >= 1; d -= 2) {
-    const int L = a.L[d - 1], sh = a.sh[d - 1], q = L >> 2;  // q = L/4
+    const int sh = a.sh[d - 1], q = a.L[d - 1] >> 2;  // q = L/4
     const int S = 1 << sh;
-    const double2 *wl = a.tw + a.off[d], *wu = a.tw + a.off[d - 1];
-    const double2 wl0 = wl[0], wu0 = wu[0];
-    const bool live = tid < (E >> 2);
-    const int cb = tid & (CB - 1), rest = tid >> LCB;  // group: line cb, sub-problem s, k2
     const int s = rest & (S - 1), k2 = rest >> sh;
     double2 z0 = make_double2(0.0, 0.0), z1 = z0, z2 = z0, z3 = z0;
     if (live) {
       const int b = s + 4 * S * k2;
-      const double2 x0 = buf[b * CB + cb], x1 = buf[(b + S) * CB + cb];
-      const double2 x2 = buf[(b + 2 * S) * CB + cb], x3 = buf[(b + 3 * S) * CB + cb];
+      const double2 x0 = buf[b * CB + cb4], x1 = buf[(b + S) * CB + cb4];
+      const double2 x2 = buf[(b + 2 * S) * CB + cb4], x3 = buf[(b + 3 * S) * CB + cb4];
       // lower level: sub-problem s (x0, x2) and s + S (x1, x3) at k2, k2 + L/4
-      const double2 ta = wl[k2], tb = wl[k2 + q];
-      const double2 y0 = bfly2(x0, x2, wl0, ta), y1 = bfly2(x0, x2, wl0, tb);
-      const double2 y2 = bfly2(x1, x3, wl0, ta), y3 = bfly2(x1, x3, wl0, tb);
+      const double2 y0 = bfly2(x0, x2, w0, ta), y1 = bfly2(x0, x2, w0, tb);
+      const double2 y2 = bfly2(x1, x3, w0, ta), y3 = bfly2(x1, x3, w0, tb);
       // upper level: outputs k2 + i L/4 of sub-problem s
-      z0 = bfly2(y0, y2, wu0, wu[k2]);
-      z1 = bfly2(y1, y3, wu0, wu[k2 + q]);
-      z2 = bfly2(y0, y2, wu0, wu[k2 + 2 * q]);
-      z3 = bfly2(y1, y3, wu0, wu[k2 + 3 * q]);
+      z0 = bfly2(y0, y2, w0, u0);
+      z1 = bfly2(y1, y3, w0, u1);
+      z2 = bfly2(y0, y2, w0, u2);
+      z3 = bfly2(y1, y3, w0, u3);
     }
+    twiddles(d - 2);
     __syncthreads();
     if (live) {
       const int o = s + S * k2;
-      buf[o * CB + cb] = z0;
-      buf[(o + S * q) * CB + cb] = z1;
-      buf[(o + 2 * S * q) * CB + cb] = z2;
-      buf[(o + 3 * S * q) * CB + cb] = z3;
+      buf[o * CB + cb4] = z0;
+      buf[(o + S * q) * CB + cb4] = z1;
+      buf[(o + 2 * S * q) * CB + cb4] = z2;
+      buf[(o + 3 * S * q) * CB + cb4] = z3;
     }
     __syncthreads();
   }
