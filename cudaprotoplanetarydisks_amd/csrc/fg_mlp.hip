@@ -660,12 +660,16 @@ struct fg_mlp {
   float *Xall, *Tall;
   size_t all_cap;                // samples they hold
   // small forward passes: pinned host memory that k_mlp_rows reads its rows from
-  // and writes its output to, and its device alias
+  // and writes its output to, and its device alias.  Allocated with the network,
+  // while its device is the current one; NULL where it could not be: rows are copied
   float *h_io, *d_io;
 };
-// Bytes of it at most.  The two copies cost the call more than the kernel's own
-// way over the bus (us per fg_mlp_forward of 5-256x4-512 with and without them:
-// 1 row 39 and 27, 128 rows 50 and 37, 1024 rows, 2.1 MB, 161 and 135).
+// Bytes of it at most, as it stays pinned while the network lives.  The two copies
+// cost a call more than the kernel's own way over the bus (us per fg_mlp_forward of
+// 5-256x4-512 with and without them: 1 row 39 and 27, 128 rows 50 and 38, 512 rows 97
+// and 82, 1024 rows 158 and 136, 2000 rows, 4.1 MB, 266 and 245; beyond the bound the
+// gain is 6 to 8 %: 3000 rows 386 and 370).  A network's first call: 128 rows 52
+// and 43, 2000 rows 270 and 275; fg_mlp_create takes 1.13 ms with it, 1.10 without.
 #define MLP_IO_BYTES (4 << 20)
 
 // Rows per workgroup of k_mlp_rows, 4 V: few, so that the chip's CUs share
@@ -831,6 +835,17 @@ extern "C" fg_status fg_mlp_create(const int *widths, int nlayers, int max_batch
     MLP_TRY(hipMemcpy(m->net, net, sizeof net, hipMemcpyHostToDevice));
     MLP_TRY(hipMalloc((void **)&m->jobs, jobs.size() * sizeof(mlp_job)));
     MLP_TRY(hipMemcpy(m->jobs, jobs.data(), jobs.size() * sizeof(mlp_job), hipMemcpyHostToDevice));
+    const size_t most = (size_t)max_batch * (widths[0] + widths[nlayers]) * 4;
+    void *h = nullptr, *d = nullptr;
+    if (hipHostMalloc(&h, std::min(most, (size_t)MLP_IO_BYTES), hipHostMallocCoherent | hipHostMallocMapped) !=
+            hipSuccess ||
+        hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
+      if (h) (void)hipHostFree(h);
+      h = d = nullptr;
+      (void)hipGetLastError();  // (a later launch's check would report it)
+    }
+    m->h_io = (float *)h;
+    m->d_io = (float *)d;
   }
   MLP_TRY(hipMalloc((void **)&m->X, (size_t)max_batch * widths[0] * 4));
   MLP_TRY(hipMalloc((void **)&m->T, (size_t)max_batch * widths[nlayers] * 4));
@@ -1020,19 +1035,7 @@ static fg_status check_batch(fg_mlp *m, int batch) {
 extern "C" fg_status fg_mlp_forward(fg_mlp *m, const float *x, int batch, float *y) {
   if (fg_status s = check_batch(m, batch)) return s;
   const size_t nx = (size_t)batch * m->width[0], ny = (size_t)batch * m->width[m->L];
-  if (m->net && (nx + ny) * 4 <= MLP_IO_BYTES) {
-    if (!m->h_io) {
-      void *h = nullptr, *d = nullptr;
-      const size_t most = (size_t)m->max_batch * (m->width[0] + m->width[m->L]) * 4;
-      FG_HIP(hipHostMalloc(&h, std::min(most, (size_t)MLP_IO_BYTES), hipHostMallocCoherent | hipHostMallocMapped));
-      if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
-        (void)hipHostFree(h);
-        fg_set_error("mlp: no device address of pinned memory");
-        return FG_E_HIP;
-      }
-      m->h_io = (float *)h;
-      m->d_io = (float *)d;
-    }
+  if (m->h_io && (nx + ny) * 4 <= MLP_IO_BYTES) {
     std::memcpy(m->h_io, x, nx * 4);
     if (fg_status s = mlp_rows(m, m->d_io, nullptr, batch, nullptr, m->d_io + nx)) return s;
     FG_HIP(hipStreamSynchronize(m->stream));

@@ -1,0 +1,67 @@
+"""The library's host code over a HIP runtime that runs no kernels
+(hip_host_stub.cpp): what it does when memory or launches are refused, and
+what it asks the runtime for.  Each case is a process of its own, in which
+the stub's symbols stand before the real runtime's."""
+import os
+import shutil
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+from conftest import ROOT
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes, sys
+import numpy as np
+sys.path[:0] = [{root!r}, {here!r}]
+stub = ctypes.CDLL({stub!r}, mode=ctypes.RTLD_GLOBAL)
+stub.stub_device_bytes.restype = ctypes.c_size_t
+stub.stub_pinned_device.argtypes = [ctypes.c_uint64]
+from cudaprotoplanetarydisks_amd import native
+from cudaprotoplanetarydisks_amd.mlp import MLP
+from cudaprotoplanetarydisks_amd.native import lib
+lib()
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    if not shutil.which("g++"):
+        pytest.skip("g++ not available")
+    so = str(tmp_path_factory.mktemp("stub") / "hip_host_stub.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", os.path.join(HERE, "hip_host_stub.cpp"), "-o", so],
+                   check=True)
+
+    def go(code):
+        text = PRELUDE.format(root=ROOT, here=HERE, stub=so) + textwrap.dedent(code)
+        r = subprocess.run([sys.executable, "-c", text], capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, (r.returncode, r.stdout[-2000:], r.stderr[-3000:])
+    return go
+
+
+def test_forward_without_pinned_memory_copies(run):
+    """A prediction needs no pinned memory: without it the rows are copied."""
+    run("""
+    stub.stub_fail_pinned(1)
+    with MLP([5, 16, 8], max_batch=4) as net:
+        for _ in range(2):
+            assert net.forward(np.ones((4, 5))).shape == (4, 8)
+        net.train(np.ones((4, 5)), np.ones((4, 8)), batch=4, steps=1, lr=1e-3)
+    """)
+
+
+def test_pinned_rows_belong_to_the_networks_device(run):
+    """Whatever device is current when a network predicts, the memory its
+    kernel reads the rows from is mapped for the network's own."""
+    run("""
+    stub.stub_watch(b"k_mlp_rows", 2, 8)
+    with MLP([5, 16, 8], max_batch=4, device=1) as net, MLP([5, 16, 8], max_batch=4, device=0):
+        net.forward(np.ones((4, 5)))
+        rows = ctypes.c_uint64()
+        stub.stub_watched(ctypes.byref(rows))
+        assert stub.stub_pinned_device(rows) == 1, stub.stub_pinned_device(rows)
+    """)
