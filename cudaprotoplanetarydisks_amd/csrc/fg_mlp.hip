@@ -1035,7 +1035,8 @@ static fg_status check_batch(fg_mlp *m, int batch) {
 extern "C" fg_status fg_mlp_forward(fg_mlp *m, const float *x, int batch, float *y) {
   if (fg_status s = check_batch(m, batch)) return s;
   const size_t nx = (size_t)batch * m->width[0], ny = (size_t)batch * m->width[m->L];
-  if (m->h_io && (nx + ny) * 4 <= MLP_IO_BYTES) {
+  // (NULL goes the way of the copies, which refuse it)
+  if (m->h_io && x && y && (nx + ny) * 4 <= MLP_IO_BYTES) {
     std::memcpy(m->h_io, x, nx * 4);
     if (fg_status s = mlp_rows(m, m->d_io, nullptr, batch, nullptr, m->d_io + nx)) return s;
     FG_HIP(hipStreamSynchronize(m->stream));

@@ -65,3 +65,17 @@ def test_pinned_rows_belong_to_the_networks_device(run):
         stub.stub_watched(ctypes.byref(rows))
         assert stub.stub_pinned_device(rows) == 1, stub.stub_pinned_device(rows)
     """)
+
+
+def test_forward_refuses_null(run):
+    """A NULL input or output is an error of the call, with the rows in pinned
+    memory as with the copies."""
+    run("""
+    y = np.zeros((2, 8), np.float32)
+    p = y.ctypes.data_as(ctypes.POINTER(ctypes.c_float))
+    for pinned in (1, 0):
+        stub.stub_fail_pinned(1 - pinned)
+        with MLP([5, 16, 8], max_batch=4) as net:
+            assert lib().fg_mlp_forward(net.h, None, 2, p) == native.FG_E_HIP
+            assert lib().fg_mlp_forward(net.h, p, 1, None) == native.FG_E_HIP
+    """)
