@@ -650,7 +650,8 @@ struct fg_mlp {
   long step;                     // Adam steps taken
   // networks in LDS (mlp_fits_rows): the kernels' view of the arrays, the
   // padded arrays it points to in one allocation, and fg_mlp_train's
-  // samples (kept for the next call, grown when a larger set comes)
+  // samples (kept for the next call, grown when a larger set comes, given back
+  // after a call whose set takes more than MLP_KEEP_BYTES)
   mlp_layer *net;                // device copy; NULL: layer by layer
   mlp_job *jobs;                 // k_mlp_weights's work list, njobs entries
   int njobs;
@@ -671,6 +672,8 @@ struct fg_mlp {
 // gain is 6 to 8 %: 3000 rows 386 and 370).  A network's first call: 128 rows 52
 // and 43, 2000 rows 270 and 275; fg_mlp_create takes 1.13 ms with it, 1.10 without.
 #define MLP_IO_BYTES (4 << 20)
+// Bytes of fg_mlp_train's samples that a network keeps between calls
+#define MLP_KEEP_BYTES (64 << 20)
 
 // Rows per workgroup of k_mlp_rows, 4 V: few, so that the chip's CUs share
 // the GELUs, until every CU has a workgroup; then more rows for each passage
@@ -1075,6 +1078,13 @@ extern "C" fg_status fg_mlp_gradient(fg_mlp *m, const float *x, const float *t, 
   return FG_OK;
 }
 
+static void mlp_free_samples(fg_mlp *m) {
+  if (m->Xall) (void)hipFree(m->Xall);
+  if (m->Tall) (void)hipFree(m->Tall);
+  m->Xall = m->Tall = nullptr;
+  m->all_cap = 0;
+}
+
 // `steps` Adam steps on the n samples (x: n x inputs, t: n x outputs),
 // cycling through consecutive batches of `batch` rows (n a multiple of
 // batch); losses[s] = the loss of step s before its update
@@ -1088,12 +1098,11 @@ extern "C" fg_status fg_mlp_train(fg_mlp *m, const float *x, const float *t, int
   const int din = m->width[0], dout = m->width[m->L];
   fg_status st = FG_OK;
   if (m->all_cap < (size_t)n) {
-    if (m->Xall) (void)hipFree(m->Xall);
-    if (m->Tall) (void)hipFree(m->Tall);
-    m->Xall = m->Tall = nullptr;
-    m->all_cap = 0;
-    FG_HIP(hipMalloc((void **)&m->Xall, (size_t)n * din * 4));
-    FG_HIP(hipMalloc((void **)&m->Tall, (size_t)n * dout * 4));
+    mlp_free_samples(m);
+    hipError_t e = hipMalloc((void **)&m->Xall, (size_t)n * din * 4);
+    if (e == hipSuccess) e = hipMalloc((void **)&m->Tall, (size_t)n * dout * 4);
+    if (e != hipSuccess) mlp_free_samples(m);
+    FG_HIP(e);
     m->all_cap = (size_t)n;
   }
   if (m->loss_cap < steps) {
@@ -1137,6 +1146,7 @@ extern "C" fg_status fg_mlp_train(fg_mlp *m, const float *x, const float *t, int
       hipMemcpyAsync(losses, m->loss, (size_t)steps * 4, hipMemcpyDeviceToHost, m->stream) != hipSuccess)
     st = FG_E_HIP;
   (void)hipStreamSynchronize(m->stream);
+  if (m->all_cap * (size_t)(din + dout) * 4 > MLP_KEEP_BYTES) mlp_free_samples(m);
   if (st && st != FG_E_NOMEM) fg_set_error("fg_mlp_train: HIP error");
   return st;
 }

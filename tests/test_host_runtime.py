@@ -79,3 +79,22 @@ def test_forward_refuses_null(run):
             assert lib().fg_mlp_forward(net.h, None, 2, p) == native.FG_E_HIP
             assert lib().fg_mlp_forward(net.h, p, 1, None) == native.FG_E_HIP
     """)
+
+
+def test_training_gives_large_sample_sets_back(run):
+    """What a network holds between training calls is bounded: a sample set
+    beyond the bound (64 MB) is freed when the call returns."""
+    run("""
+    widths, bound = [1024, 8, 1024], 64 << 20
+    rows = 2 * bound // (4 * 2048)
+    with MLP(widths, max_batch=16) as net:
+        held = stub.stub_device_bytes()
+        small = np.zeros((16, 1024), np.float32)
+        net.train(small, small, batch=16, steps=2, lr=1e-3)
+        large = np.zeros((rows, 1024), np.float32)
+        for _ in range(2):
+            net.train(large, large, batch=16, steps=2, lr=1e-3)
+            assert stub.stub_device_bytes() - held < bound, stub.stub_device_bytes() - held
+        net.train(small, small, batch=16, steps=2, lr=1e-3)
+    assert stub.stub_device_bytes() == 0
+    """)
