@@ -1122,12 +1122,12 @@ extern "C" fg_status fg_mlp_train(fg_mlp *m, const float *x, const float *t, int
   for (int s = 0; s < steps && !st; s++) {
     const int q = s % nb;
     const float *xs = m->Xall + (size_t)q * batch * din, *ts = m->Tall + (size_t)q * batch * dout;
-    m->step++;
-    const float c1 = 1.0f - powf(b1, (float)m->step), c2 = 1.0f - powf(b2, (float)m->step);
+    // (counted once its gradients stand, or, with both in one, its update)
+    const float taken = (float)(m->step + 1), c1 = 1.0f - powf(b1, taken), c2 = 1.0f - powf(b2, taken);
     if (m->net) {
       const adam_args adam = {lr, b1, b2, eps, c1, c2};
       if ((st = mlp_rows(m, xs, ts, batch, s > 0 ? m->loss + s - 1 : nullptr))) break;
-      st = mlp_weights(m, ts, batch, &adam);
+      if (!(st = mlp_weights(m, ts, batch, &adam))) m->step++;
       continue;
     }
     if (hipMemcpyAsync(m->X, xs, (size_t)batch * din * 4, hipMemcpyDeviceToDevice, m->stream) != hipSuccess ||
@@ -1137,6 +1137,7 @@ extern "C" fg_status fg_mlp_train(fg_mlp *m, const float *x, const float *t, int
     }
     if ((st = mlp_forward(m, batch))) break;
     if ((st = mlp_backward(m, batch, m->loss + s))) break;
+    m->step++;
     hipLaunchKernelGGL(k_adam, dim3(fg_blocks(m->nparam, 256)), dim3(256), 0, m->stream, m->p, m->g, m->m, m->v,
                        m->pb, m->nparam, lr, b1, b2, eps, c1, c2);
     if (hipGetLastError() != hipSuccess) st = FG_E_HIP;

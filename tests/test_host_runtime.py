@@ -98,3 +98,29 @@ def test_training_gives_large_sample_sets_back(run):
         net.train(small, small, batch=16, steps=2, lr=1e-3)
     assert stub.stub_device_bytes() == 0
     """)
+
+
+@pytest.mark.parametrize("widths", [[5, 16, 8], [5, 1000, 8]], ids=["rows", "layers"])
+@pytest.mark.parametrize("kernel", ["forward", "weights"])
+def test_failed_training_step_is_not_counted(run, widths, kernel):
+    """The bias corrections of Adam take the steps that were taken: a step
+    whose launches failed before its update is none of them."""
+    rows = len(widths) == 3 and widths[1] <= 896
+    fail = {"forward": "k_mlp_rows" if rows else "k_gemm", "weights": "k_mlp_weights" if rows else "k_colsum"}[kernel]
+    # 1 - 0.9: the last but one of adam_args' six floats, or k_adam's argument
+    watch, index, size, at = ("k_mlp_weights", 11, 24, 4) if rows else ("k_adam", 10, 4, 0)
+    run(f"""
+    stub.stub_watch({watch.encode()!r}, {index}, {size})
+    x, t = np.ones((4, 5), np.float32), np.ones((4, 8), np.float32)
+    with MLP({widths!r}, max_batch=4) as net:
+        stub.stub_fail_launches({fail.encode()!r}, 1)
+        try:
+            net.train(x, t, batch=4, steps=1, lr=1e-3)
+            raise SystemExit("the step did not fail")
+        except native.FargoError:
+            pass
+        net.train(x, t, batch=4, steps=1, lr=1e-3)
+        arg = (ctypes.c_float * {size // 4})()
+        stub.stub_watched(arg)
+        assert arg[{at}] == np.float32(1) - np.float32(0.9), list(arg)
+    """)
