@@ -2657,16 +2657,16 @@ static int plain_potential(const fg_ctx *c, const fg_planet_pot *pl, int nb) {
 // H rings costs H + 3 steps (the first ones are partial); up to `resident` waves
 // per SIMD are there at once, so the fullest SIMD counts, beyond that the total
 // does.  A batch's disks share the SIMDs.
-// disks: rows, strips of each
-static int march_band(const std::vector<int2> &disks, int most, int resident = 3, double share = 0.7) {
+// disks: rows, strips of each of n
+static int march_band(const int2 *disks, int n, int most, int resident = 3, double share = 0.7) {
   const int simds = 1024;
   double best = 0.0;
   int band = 1;
   for (int h = 1; h <= most; h++) {
     long waves = 0;
-    for (const int2 &d : disks) waves += (long)d.y * ((d.x + h - 1) / h);
-    const double n = (double)waves / simds;
-    const double cost = (h + 3) * std::max(1.0, share * (n > resident ? n : ceil(n)));
+    for (int k = 0; k < n; k++) waves += (long)disks[k].y * ((disks[k].x + h - 1) / h);
+    const double each = (double)waves / simds;
+    const double cost = (h + 3) * std::max(1.0, share * (each > resident ? each : ceil(each)));
     if (h == 1 || cost < best) {
       best = cost;
       band = h;
@@ -2677,19 +2677,23 @@ static int march_band(const std::vector<int2> &disks, int most, int resident = 3
 // Measured for k_src (us, FP64 isothermal): 128x384 1 ring 11.7, 8 rings 19;
 // 512x1536 7-8 rings 24, 4 rings 28, 20 rings 36; 1024x3072 18-20 rings 50,
 // 8 rings 57, 26 rings 57; 2048x4096 18-26 rings 107, 8 rings 121.
-static int src_band(int nr, int nstrips) { return march_band({make_int2(nr + 1, nstrips)}, SRC_MAX_BAND); }
+static int src_band(int nr, int nstrips) {
+  const int2 disk = make_int2(nr + 1, nstrips);
+  return march_band(&disk, 1, SRC_MAX_BAND);
+}
 // Measured for k_src32, four waves per SIMD at 1.4 us a step (us with 3 of
 // launch): 128x384 1 ring 12.7, 8 rings 19, 16 rings 29; 256x768 2 rings 14.8, 8
 // rings 20; 512x1536 6 rings 21.9, 13 rings 27.6; 1024x3072 20 rings 42, 10
 // rings 44, 27 rings 53.  fg_set_tiles fixes the band instead.
-static int src32_band(const std::vector<int2> &disks) { return march_band(disks, SRC_MAX_BAND, SRC32_WAVES, 0.44); }
+static int src32_band(const int2 *disks, int n) { return march_band(disks, n, SRC_MAX_BAND, SRC32_WAVES, 0.44); }
 // Measured for k_trad (us): 128x384 2-3 rings 11.9, 16 rings 21.5; 301x998
 // (with energy) 3-6 rings 18, 16 rings 25; 512x1536 8 rings 23, 16 rings 26;
 // from 1024x3072 on, where HBM bounds it, 10 to 16 rings are within 3 % and
 // 20 to 32 cost 5 %; k_trad32 256x768 3-4 rings 14, 16 rings 23.5.  fg_set_tiles
 // fixes the band instead.
 static int trad_band(const fg_ctx *c, int nstrips) {
-  return c->tile_trad_band ? c->tile_trad_band : march_band({make_int2(c->nr, nstrips)}, 16);
+  const int2 disk = make_int2(c->nr, nstrips);
+  return c->tile_trad_band ? c->tile_trad_band : march_band(&disk, 1, 16);
 }
 
 extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, double domega,
@@ -2783,8 +2787,8 @@ extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, dou
     s3.evanescent = sa.evanescent;
     s3.nstrips = (ns + SRC_W - 1) / SRC_W;
     s3.width = (ns + s3.nstrips - 1) / s3.nstrips;
-    s3.band = c->tile_src_th ? std::min(c->tile_src_th, SRC_MAX_BAND)
-                             : src32_band({make_int2(nr + 1, s3.nstrips)});
+    const int2 disk = make_int2(nr + 1, s3.nstrips);
+    s3.band = c->tile_src_th ? std::min(c->tile_src_th, SRC_MAX_BAND) : src32_band(&disk, 1);
     hipLaunchKernelGGL(k_src32, dim3(xcd_grid(s3.nstrips * ((nr + s3.band) / s3.band))), dim3(64), 0, c->stream, s3);
   } else {
     sa.nstrips = (ns + SRC_W - 1) / SRC_W;
@@ -3224,8 +3228,8 @@ fg_status fg_batch_dev_create(fg_ctx *const *ctx, int n, fg_batch_dev **out) {
     src.push_back(make_int2(ctx[k]->nr + 1, (ctx[k]->ns + SRC_W - 1) / SRC_W));
     trad.push_back(make_int2(ctx[k]->nr, (ctx[k]->ns + TRAD_TPB - 1) / TRAD_TPB));
   }
-  b->src_band = src32_band(src);
-  b->trad_band = march_band(trad, 16);
+  b->src_band = src32_band(src.data(), n);
+  b->trad_band = march_band(trad.data(), n, 16);
   hipError_t e = hipStreamCreate(&b->stream);
   if (e == hipSuccess) e = hipHostMalloc((void **)&b->h_disk, n * sizeof(batch_disk), hipHostMallocDefault);
   if (e == hipSuccess) e = hipHostMalloc((void **)&b->h_res, n * sizeof(batch_result), hipHostMallocDefault);

@@ -124,3 +124,21 @@ def test_failed_training_step_is_not_counted(run, widths, kernel):
         stub.stub_watched(arg)
         assert arg[{at}] == np.float32(1) - np.float32(0.9), list(arg)
     """)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_substep_entries_allocate_no_host_memory(run, deck, precision):
+    """A substep's C entries take no memory from the C++ heap, whose failure
+    would be an exception that no C caller can catch."""
+    path = deck(Nrad=16, Nsec=32)
+    run(f"""
+    from cudaprotoplanetarydisks_amd import Simulation
+    sim = Simulation({path!r}, precision={precision!r}, fused=True)
+    planet = native.FgPlanetPot(1.0, 0.0, 1e-3, 1e-4, 1.0)
+    for fail in (0, 1):
+        stub.stub_fail_new(fail)
+        status = [lib().fg_step_fused(sim.ctx.h, 1e-3, 1.0, 0.0, ctypes.byref(planet), 1, 0.0, 0.0, 0.1, 0)]
+        status.append(lib().fg_transport(sim.ctx.h, 1e-3, 1.0, None))
+        stub.stub_fail_new(0)
+        assert status == [0, 0], (status, lib().fg_last_error())
+    """)
