@@ -62,8 +62,8 @@ extern "C" fg_status fg_create(const fg_params *p, const fg_tables *t, int devic
     fg_set_error("fg_create: grid %d x %d too small (NRAD >= 3, NSEC >= 2)", p->nrad, p->nsec);
     return FG_E_INVALID;
   }
-  if (p->nsec > 8192) {
-    fg_set_error("fg_create: NSEC = %d exceeds the 8192 sectors a ring kernel stages in LDS", p->nsec);
+  if (p->nsec > FG_NSEC_MAX) {
+    fg_set_error("fg_create: NSEC = %d exceeds the %d sectors a ring kernel stages in LDS", p->nsec, FG_NSEC_MAX);
     return FG_E_UNSUPPORTED;
   }
   int ndev = 0;
@@ -77,6 +77,11 @@ extern "C" fg_status fg_create(const fg_params *p, const fg_tables *t, int devic
   // a failure is reported by that entry point (fg_disk_force_hill_noalloc),
   // the context itself does not need it
   (void)fg_noalloc_setup(device);
+  if (p->nsec > FG_RING_UNASKED) {  // (a refusal shows in the launches)
+    fg_ask_ring_lds();
+    fg_ask_edge_lds();
+    (void)hipGetLastError();
+  }
   fg_ctx *c = new fg_ctx();
   c->tile_src_th = 0;   // picked for the grid
   c->tile_trad_band = 0;  // picked for the grid

@@ -34,6 +34,14 @@ fg_status fg_transport_sweeps(fg_ctx *c, double dt, double omega_frame);
 fg_status fg_cfl_ring_launch(fg_ctx *c);
 fg_status fg_cfl_result(fg_ctx *c, int *ncfl);
 fg_status fg_nonreflecting_internal(fg_ctx *c, double *press, double *temp);
+// The kernels that stage a whole ring in LDS, and what they keep beside it, take
+// more than the 64 KB that a launch gets unasked on rings wider than
+// FG_RING_UNASKED: fg_create asks for it, for its device (fg_steps.hip, fg_reduce.hip)
+#define FG_NSEC_MAX 8192
+#define FG_RING_UNASKED 7000
+#define FG_RING_LDS ((FG_NSEC_MAX + 256) * (int)sizeof(double))
+void fg_ask_ring_lds();
+void fg_ask_edge_lds();
 
 // Result block of the fused path (fg_ctx::h_fused, coherent pinned host
 // memory the final kernels write straight into): [0..1] star force,

@@ -304,6 +304,10 @@ __global__ __launch_bounds__(1024) void k_nr_edges(nr_args a) {
   }
 }
 
+void fg_ask_edge_lds() {
+  (void)hipFuncSetAttribute((const void *)k_nr_edges, hipFuncAttributeMaxDynamicSharedMemorySize, FG_RING_LDS);
+}
+
 fg_status fg_nonreflecting_internal(fg_ctx *c, double *press, double *temp) {
   const int nr = c->nr, ns = c->ns;
   const std::vector<double> &Rinf = c->h_Rinf, &Rmed = c->h_Rmed;
@@ -329,9 +333,6 @@ fg_status fg_nonreflecting_internal(fg_ctx *c, double *press, double *temp) {
   a.energy0[1] = c->h_EnergyMed[nr - 1];
   a.nr = nr;
   a.ns = ns;
-  if (ns > 7000)  // ring and partial sums beyond the 64 KB a launch gets unasked
-    FG_HIP(hipFuncSetAttribute((const void *)k_nr_edges, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               ns * (int)sizeof(double)));
   hipLaunchKernelGGL(k_nr_edges, dim3(nr > 3 ? 2 : 1), dim3(1024), (size_t)ns * sizeof(double), c->stream, a);
   FG_LAUNCH_CHECK();
   return FG_OK;

@@ -383,6 +383,11 @@ __global__ void k_cfl_final(int *cfl, double *dt1d, const double *vmoy, const do
 }
 
 // ----------------------------------------------------- entry points --
+void fg_ask_ring_lds() {
+  for (const void *k : {(const void *)k_ring_mean, (const void *)k_cfl_ring})
+    (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, FG_RING_LDS);
+}
+
 static fg_status check(fg_ctx *c) {
   if (!c) {
     fg_set_error("NULL context");

@@ -142,3 +142,22 @@ def test_substep_entries_allocate_no_host_memory(run, deck, precision):
         stub.stub_fail_new(0)
         assert status == [0, 0], (status, lib().fg_last_error())
     """)
+
+
+def test_wide_rings_ask_for_their_lds(run, deck):
+    """A launch beyond 64 KB of LDS, dynamic and static together, asks for it
+    first: the kernels that stage a ring, at the widest grid."""
+    path = deck(Nrad=8, Nsec=8192, InnerBoundary="NONREFLECTING", Viscosity=None, AlphaViscosity=1e-3)
+    run(f"""
+    from cudaprotoplanetarydisks_amd import Simulation
+    sim = Simulation({path!r})
+    n, c = ctypes.c_int(), sim.ctx.h
+    lib().fg_cfl(c, 0.1, ctypes.byref(n))
+    lib().fg_ring_mean_cs(c)
+    lib().fg_boundary(c, 1e-3, 1.0)
+    for kernel in (b"k_cfl_ring", b"k_ring_mean", b"k_nr_edges"):
+        asked, granted = ctypes.c_size_t(), ctypes.c_size_t()
+        stub.stub_lds(kernel, ctypes.byref(asked), ctypes.byref(granted))
+        assert asked.value >= 8192 * 8, kernel
+        assert granted.value >= asked.value, (kernel, asked.value, granted.value)
+    """)
