@@ -7,10 +7,11 @@ idle and small tiles win for the wrong reason) and times batch substeps
 (rings per source band; 32 stands for the widest, 27) x (rings per
 radial-sweep band), and, before and after them, with the bands that the
 library picks when nothing is set.  The fastest candidate goes to a JSON cache
-keyed "NRADxNSEC" that Ensemble and Simulation read, if it beats the picked
-bands at their better time; otherwise the grid has no entry.  No cache ships
-with the package.  Tile shapes change only the work decomposition: results
-are identical for every candidate.
+keyed "NRADxNSEC" that Ensemble reads, if it beats the picked bands at their
+better time; otherwise the grid has no entry.  No cache ships with the
+package, and a lone disk (Simulation) keeps the bands picked for its grid,
+which are narrower than a batch's.  Tile shapes change only the work
+decomposition: results are identical for every candidate.
 
     python -m cudaprotoplanetarydisks_amd.autotune --grids 128x384 256x768
 """

@@ -40,13 +40,8 @@ class Simulation:
         self.h = h
         self.nrad = int(self.get("NRAD"))
         self.nsec = int(self.get("NSEC"))
-        if precision == "fp32":  # autotuned tile shapes of this grid, if any
-            from .ensemble import load_tiles
-            t = load_tiles().get(f"{self.nrad}x{self.nsec}")
-            if t:
-                call("fg_set_tiles", lib().fg_sim_ctx(self.h), int(t["src_rows"]), int(t["trad_band"]))
-            if fp32_pairs is not None:  # Hill radii of float-pair Sigma storage (default 1)
-                call("fg_set_fp32_pairs", lib().fg_sim_ctx(self.h), float(fp32_pairs))
+        if precision == "fp32" and fp32_pairs is not None:  # Hill radii of float-pair Sigma storage (default 1)
+            call("fg_set_fp32_pairs", lib().fg_sim_ctx(self.h), float(fp32_pairs))
 
     def close(self):
         if getattr(self, "h", None):

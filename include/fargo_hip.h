@@ -240,7 +240,7 @@ fg_status fg_fused_results(fg_ctx *ctx, int *ncfl, double *force2, double *lost_
 /* Tile shapes of the fused kernels: rings per band of the FP32 source march (8,
  * 16 or 32, held to 27) and of the radial sweep (without a call, bands picked for
  * the grid, in a batch for all its disks together).  Results do not depend on them; the
- * autotuner (cudaprotoplanetarydisks_amd/autotune.py) picks them per grid.
+ * autotuner (cudaprotoplanetarydisks_amd/autotune.py) times them for batches.
  * No reference counterpart (the reference's launch shape is fixed,
  * Main.cu:204-226). */
 fg_status fg_set_tiles(fg_ctx *ctx, int src_rows, int trad_band);

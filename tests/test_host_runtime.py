@@ -161,3 +161,23 @@ def test_wide_rings_ask_for_their_lds(run, deck):
         assert asked.value >= 8192 * 8, kernel
         assert granted.value >= asked.value, (kernel, asked.value, granted.value)
     """)
+
+
+def test_single_disks_take_no_batch_tuned_shapes(run, deck):
+    """The autotuner times batches; a lone FP32 disk keeps the bands picked for
+    its grid, and a batch takes the entry."""
+    path = deck(Nrad=16, Nsec=32)
+    run(f"""
+    from cudaprotoplanetarydisks_amd import Simulation, ensemble, sim
+    entry = dict([("16x32", dict(src_rows=16, trad_band=8))])
+    ensemble.load_tiles = lambda path=None: entry
+    calls = []
+    def call(name, *args):
+        calls.append(name)
+        return native.call(name, *args)
+    sim.call = ensemble.call = call
+    Simulation({path!r}, precision="fp32").close()
+    assert "fg_set_tiles" not in calls
+    ensemble.Ensemble([{path!r}]).close()
+    assert "fg_batch_set_tiles" in calls
+    """)
