@@ -6,7 +6,8 @@
 //
 // Every dense layer is one GEMM C = A B (M x K times K x N) with a fused
 // epilogue:
-//   forward hidden   Z = H W^T + b,  H' = bf16(GELU(Z))      (Z kept, FP32)
+//   forward hidden   Z = H W^T + b,  H' = bf16(GELU(Z))
+//   (kept in FP32 for the way back: GELU'(Z) by k_mlp_rows, Z by k_gemm_bf16)
 //   forward output   Y = H W^T + b                          (FP32)
 //   backward         dZ_below = (dZ W) * GELU'(Z_below)     (FP32 + BF16)
 //   weight gradient  dW = dZ^T H                            (FP32)
@@ -20,8 +21,8 @@
 // run k_gemm_bf16 layer by layer: operands addressed by (row stride, column
 // stride), a 256-thread workgroup per 64 x 64 tile as four waves of 2 x 2
 // MFMA blocks, 64 x 32 slices of A and B^T staged in LDS.  Both accumulate
-// every output over k in the same 32-wide MFMA steps, so they give the same
-// bits.
+// every output over k in the same 32-wide MFMA steps, so their products are the
+// same bits.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -641,7 +642,10 @@ struct fg_mlp {
   float *p, *g, *m, *v;  // parameters, gradients, Adam moments (FP32)
   bf16_t *pb;            // BF16 parameters
   bf16_t *H[MLP_MAX_LAYERS];     // BF16 layer inputs (H[0] = x)
-  float *Z[MLP_MAX_LAYERS];      // pre-activations (Z[L-1] = output)
+  // Z[L-1]: the output.  Below it what the way back needs: with net (networks in
+  // LDS) GELU' of the pre-activations, left by a training pass alone; without it
+  // the pre-activations
+  float *Z[MLP_MAX_LAYERS];
   float *dZ[MLP_MAX_LAYERS];     // FP32 gradients of the pre-activations
   bf16_t *dZb[MLP_MAX_LAYERS];   // and their BF16 copies
   float *X, *T;                  // FP32 batch inputs and targets
