@@ -26,6 +26,10 @@
 // the energy through the sweeps and k_fin; self-gravitating decks run the
 // SG field (fg_sg_fused) first and add its kick in k_src.
 //
+// Kernel times in the comments are means per launch of a rocprofv3 kernel trace,
+// before and after on one card; "by events": HIP events around the launch
+// (fg_profile), which add 1 to 5 us.
+//
 // Supported decks: evanescent boundaries, per-substep CFL; isothermal or
 // adiabatic, with or without self-gravity (FP32 bulk mode: isothermal
 // without self-gravity).  Everything else uses the per-routine path.
@@ -218,12 +222,13 @@ __device__ __forceinline__ T at(const T *row, unsigned off) {
 // (H + 5) / H x 64 / 59 cells per cell, where the 16 x 64 LDS tile with its
 // halo of four evaluated 1.55.
 // Bound: HBM on large grids (2048 x 4096: 442 MB by the counters, of which
-// 403 are the fields read and written once, in 104 us, was 238 us; 1024 x 3072:
-// 47 us, was 89), the waves' own issue on small ones (a dependent FP64
-// operation every nine cycles; 128 x 384: 9 us, was 13).  Three waves per SIMD
+// 403 are the fields read and written once, in 119 us, was 222 us; 1024 x 3072:
+// 61 us, was 91, and 50 us by events with the band that suits it, src_band), the
+// waves' own issue on small ones (a dependent FP64 operation every nine cycles;
+// 512 x 1536: 23 us, was 30; 128 x 384: 9 us, was 13).  Three waves per SIMD
 // (168 VGPRs) and two rings in flight without energy and self-gravity; with
 // them two waves and one ring (177 to 191 VGPRs), since the third wave would
-// spill (512 x 1536 with both 29 us, was 34; 37 with three).
+// spill (512 x 1536 with both 26 us, was 35; by events 29, and 37 with three).
 template <int MODE>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE ? 2 : 3))) void k_src(src_args a) {
   constexpr int AHEAD = MODE ? 1 : 2;  // rings whose loads are in flight
@@ -635,7 +640,8 @@ struct trad_args {
 // the barrier only orders the LDS accesses, and lane 0 has finished a
 // round's sum before the next round's stores in program order.  (The sum by the
 // whole wave's lanes, as ring_seq_sum, was no faster here: 512 x 1536 28.8
-// against 25.7 us for the kernel, 1024 x 3072 the same, 2048 x 4096 131 and 137.)
+// against 25.7 us by events for the kernel, 1024 x 3072 the same, 2048 x 4096 131 and
+// 137.)
 #define RMW_CH 8  // sectors per lane per round
 __device__ void ring_mean_wave(const double *v, int ns, double *out) {
   __shared__ double buf[64 * RMW_CH];
@@ -926,9 +932,9 @@ struct taz_args {
 #define TAZW_HL 5
 #define TAZW_HR 4
 // Cells per lane: two on grids below 2^20 cells and in batches, where more and
-// shorter chunks fill the chip (k_tazw, us with two and three: 128 x 384 9.0 and
-// 10.4, 512 x 1536 27.8 and 29.3; FP32 128 x 384 7.9 and 9.1, 512 x 1536 18.3 and
-// 19.0; 8 batched disks 177 and 180 per substep), three beyond, where the halo's
+// shorter chunks fill the chip (k_tazw, us by events with two and three: 128 x 384
+// 9.0 and 10.4, 512 x 1536 27.8 and 29.3; FP32 128 x 384 7.9 and 9.1, 512 x 1536 18.3
+// and 19.0; 8 batched disks 177 and 180 per substep), three beyond, where the halo's
 // bytes count (FP32 1024 x 3072 41.8 and 41.0, FP64 the same within 1 %).  Three
 // FP64 cells take 142 or 164 VGPRs and leave three waves per SIMD, four or five
 // cells two; three FP32 cells are held to 96 VGPRs, five waves.
@@ -1465,10 +1471,12 @@ __device__ __forceinline__ void ring_min_store(double best, double *red, double 
 // PAIRS: ring i - 1, i or i + 1 stored as float pairs (its own instance, so that
 // the other rings run without the residuals' loads).
 // Bound: HBM on large grids (2048 x 4096: 478 MB by the counters, 470 of them
-// compulsory, in 112 us), latency on small
+// compulsory, in 117 us), latency on small
 // ones.  Was one lane's sum of the ring beside a pass that kept its terms in
-// registers (and two passes over rings beyond 3072 cells): 1024 x 3072 58 -> 51
-// us, 2048 x 4096 201 -> 112, 512 x 1536 24 -> 17; FP32 1024 x 3072 43 -> 34.
+// registers (and two passes over rings beyond 3072 cells): 1024 x 3072 61 -> 52
+// us, 2048 x 4096 198 -> 117, 512 x 1536 22 -> 17 (adiabatic 24 -> 23); FP32
+// 1024 x 3072 44 -> 36, 128 x 384 9.2 -> 8.1; FP64 at 128 x 384, where the pass was
+// one cell or two a thread, 7.2 -> 8.2.
 // Keeping that pass's terms unrolled over 12 or 16 cells was slower than the loop,
 // 512 threads a ring too (two rounds of workgroups).
 template <bool ADI, bool S32, bool PAIRS>
@@ -1755,7 +1763,7 @@ __device__ __forceinline__ float planet_potential_f(double x, double y, double x
 // star's gravity there, DREF the reference part of the shear.
 // Bound: VALU issue (~300 instructions a cell) and latency on small grids; as
 // 16 x 64 LDS tiles it evaluated 1.55 cells per cell and 590 instructions.
-// 1024 x 3072: 66 -> 42 us; 64 disks of 128 to 384 rings: 216 -> 106 us.
+// 1024 x 3072: 66 -> 42 us; 64 disks of 128 to 384 rings: 214 -> 108 us.
 #define SRC32_WAVES 4  // per SIMD
 enum { S3_MED, S3_CS, S3_VB, S3_IINF, S3_STAR, S3_VREF, S3_SBAR, S3_N };
 enum { S3F_IDMED, S3F_IDXT, S3F_SUPP, S3F_IMED, S3F_IDSUP, S3F_SUP, S3F_INF, S3F_NU, S3F_IINF, S3F_MED, S3F_DREF, S3F_N = 12 };
@@ -2374,8 +2382,9 @@ __global__ __launch_bounds__(RED_TPB) void k_forces_partial(forces_args a) {
 // are compared in); then the result block's sequence slots.  RINGS: the star's
 // force from k_fin's ring partials (FP32 mode).
 // Bound: latency, the chain of B = 1024 additions and the write to host memory:
-// 10.5 us however many planets there are, where two planets' own pairs of
-// launches took 36 (301 x 998 with two planets: 135 us per substep, now 104).
+// 11 us however many planets there are, where two planets' own pairs of
+// launches took 36 (301 x 998 with two planets: 135 us per substep before it, 104
+// with it).
 struct results_args {
   const double *partial;
   int B, star;
@@ -2674,19 +2683,23 @@ static int march_band(const int2 *disks, int n, int most, int resident = 3, doub
   }
   return band;
 }
-// Measured for k_src (us, FP64 isothermal): 128x384 1 ring 11.7, 8 rings 19;
-// 512x1536 7-8 rings 24, 4 rings 28, 20 rings 36; 1024x3072 18-20 rings 50,
-// 8 rings 57, 26 rings 57; 2048x4096 18-26 rings 107, 8 rings 121.
+// Measured for k_src (us by events, FP64 isothermal; *: what the estimate picks):
+// 128x384 1* ring 13.4, 2 rings 13.9, 8 rings 18.6; 512x1536 4 rings 27.8, 6 rings
+// 25.3, 7* rings 27.1, 9 rings 26.4, 20 rings 35; 2048x4096 8 rings 127, 18 rings 112,
+// 27* rings 113; 1024x3072 8 rings 57, 18-20 rings 50-52, 24 rings 55, 27* rings 62.
+// There the estimate is off: 27 rings make two full rounds of waves, which it
+// takes for quicker than three of 18 to 20 rings; the substep pays 4 % (261 us, 250
+// with 20 rings).  Elsewhere it is within 8 % of the best band tried.
 static int src_band(int nr, int nstrips) {
   const int2 disk = make_int2(nr + 1, nstrips);
   return march_band(&disk, 1, SRC_MAX_BAND);
 }
-// Measured for k_src32, four waves per SIMD at 1.4 us a step (us with 3 of
-// launch): 128x384 1 ring 12.7, 8 rings 19, 16 rings 29; 256x768 2 rings 14.8, 8
-// rings 20; 512x1536 6 rings 21.9, 13 rings 27.6; 1024x3072 20 rings 42, 10
-// rings 44, 27 rings 53.  fg_set_tiles fixes the band instead.
+// Measured for k_src32, four waves per SIMD at 1.4 us a step (us by events):
+// 128x384 1* ring 12.7, 8 rings 19, 16 rings 29; 256x768 2* rings 14.8, 8
+// rings 20; 512x1536 6 rings 21.9, 13 rings 27.6 (7* picked); 1024x3072 10 rings 42,
+// 18* rings 43, 20 rings 40, 27 rings 51.  fg_set_tiles fixes the band instead.
 static int src32_band(const int2 *disks, int n) { return march_band(disks, n, SRC_MAX_BAND, SRC32_WAVES, 0.44); }
-// Measured for k_trad (us): 128x384 2-3 rings 11.9, 16 rings 21.5; 301x998
+// Measured for k_trad (us by events): 128x384 2-3 rings 11.9, 16 rings 21.5; 301x998
 // (with energy) 3-6 rings 18, 16 rings 25; 512x1536 8 rings 23, 16 rings 26;
 // from 1024x3072 on, where HBM bounds it, 10 to 16 rings are within 3 % and
 // 20 to 32 cost 5 %; k_trad32 256x768 3-4 rings 14, 16 rings 23.5.  fg_set_tiles
@@ -2967,10 +2980,10 @@ extern "C" fg_status fg_step_fused(fg_ctx *c, double dt, double omega_frame, dou
 // ------------------------------------------- per-routine transport ----
 // Transport (TransportEuler.cu:30) with the fused path's sweeps: two
 // launches instead of one per quantity and step (86 with the copies), and the
-// fields that the routines leave (k_cells forms the velocities).  9 + 9 us at
-// 128 x 384, 18 + 18 us at 384 x 1152; bound as the fused path's sweeps are.  A 128 x 384 substep with
-// an open edge went from 393 to 121 us with it, one wait for all of a substep's
-// reductions, and results that the kernels write to host memory.
+// fields that the routines leave (k_cells forms the velocities).  9 + 7 us at
+// 128 x 384, 18 + 17 us at 384 x 1152; bound as the fused path's sweeps are.  A
+// 128 x 384 substep with an open edge went from 393 to 121 us with it, one wait for
+// all of a substep's reductions, and results that the kernels write to host memory.
 fg_status fg_transport_sweeps(fg_ctx *c, double dt, double omega_frame) {
   const int nr = c->nr, ns = c->ns;
   const bool adi = c->p.adiabatic;
@@ -3255,7 +3268,7 @@ static fg_status upload_items(const std::vector<T> &v, T **dev) {
 
 // rings per band of a batched disk's source march and radial sweep: those that
 // suit all the disks together (8 disks of 128 to 384 rings: 8 rings of the radial
-// sweep 187 us per substep, 16 rings 194; 64 disks 891 and 879)
+// sweep 130 us per substep, 16 rings 135; 64 disks 625 and 617)
 static int batch_src_band(const fg_batch_dev *b, const fg_ctx *c) {
   return c->tile_src_th ? std::min(c->tile_src_th, SRC_MAX_BAND) : b->src_band;
 }

@@ -315,9 +315,10 @@ __device__ __forceinline__ void mlp_store_rows(mlp_b *t, const bf16_t (&h)[V]) {
 // passage through the CU's L1 (1.3 MB both ways for the emulator network)
 // are what bounds the kernel, the products are not.  GELU' is formed on the
 // way up, where erff is at hand, and kept for the way back.
-// 512 rows of 5-256-256-256-256-512: 28.6 us; with k_mlp_weights 41 us a
+// 512 rows of 5-256-256-256-256-512: 28 us; with k_mlp_weights 41 us a
 // training step, where fourteen k_gemm_bf16, five k_colsum (114 us each), k_mse
-// and k_adam took 1160 us.  Forward alone, 128 rows: 13 us, was 5 x 24 us.
+// and k_adam took 1160 us.  Forward alone, 128 rows: 13 us, was 5 x 24 us; 18 us
+// with its rows and output in pinned host memory.
 // Workgroups are dispatched round-robin over the 8 XCDs; each XCD takes a
 // contiguous run of rows, so that the tiles they fill together are written
 // through one L2 (with neighbouring rows on different XCDs, k_mlp_weights

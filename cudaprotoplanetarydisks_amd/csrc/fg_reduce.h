@@ -318,8 +318,8 @@ __device__ __forceinline__ double dpp_move(double x) {
 // a binade (about log2 n of them in a sum of one sign), and sums with infinities
 // and NaN, are added up one by one.
 // Rings shorter than RING_SEQ_MIN are added up by one lane (k_fin with the one and
-// the other, us: 384 cells 10.8 and 12.0, 576 12.7 and 12.8, 768 14.7 and 13.8,
-// 1536 26.8 and 19.7).
+// the other, us by events around it: 384 cells 10.8 and 12.0, 576 12.7 and 12.8, 768
+// 14.7 and 13.8, 1536 26.8 and 19.7).
 #define RING_SEQ_MIN 640
 struct seq_map {
   double d0, d1;  // what the lanes up to this one, from the last single one on, add to an even, odd sum

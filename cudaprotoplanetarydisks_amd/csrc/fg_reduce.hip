@@ -225,8 +225,8 @@ extern "C" fg_status fg_circumplanetary_mass(fg_ctx *c, double xpl, double ypl, 
 // three rings runs them one after the other.  Bound: a dozen dependent
 // barriers and memory round trips.  As one launch per ring sum and copy, with
 // the host computing the shifts, a boundary pass was 22 launches and four
-// waits; this is 12 us at NSEC = 1152, and a 384 x 1152 substep with three of
-// them went from 605 to 126 us with it and fg_transport's sweeps.
+// waits; this is 13 us at NSEC = 1152, and a 384 x 1152 substep with three of
+// them takes 166 us with it, fg_transport's sweeps and k_cells, was 880.
 struct nr_args {
   double *dens, *energy, *vr, *press, *temp;  // press, temp: NULL or formed anew on the edge rings
   const double *cs, *fpress;

@@ -209,9 +209,9 @@ __device__ __forceinline__ double2 bfly2(double2 x0, double2 x1, double2 w0, dou
 // k_fft_lines), with half the LDS round trips and barriers.
 // Bound: the levels' chain of LDS round trips, 112 FP64 operations a group and
 // barriers, at eight waves per SIMD (62 VGPRs, which the attribute keeps).
-// 512 x 1536 (us): columns with the product 51 -> 46, inverse columns 39 -> 33, rows
-// 39 and 23 as before, since a pair's twiddles are loaded before the barriers in
-// front of it and a deepest factor of 2 is a radix-2 level like the others.
+// 512 x 1536 (us): columns with the product 53 -> 47, inverse columns 39 -> 34, rows
+// 40 and 24 (39 and 23 before), since a pair's twiddles are loaded before the barriers
+// in front of it and a deepest factor of 2 is a radix-2 level like the others.
 template <int CB, int MODE, int TPB>
 __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(8))) void k_fft_pow2(fft_args a) {
   extern __shared__ double2 buf[];
